@@ -513,6 +513,20 @@ int halma_pot_soft_self_batched(int64_t n_halo, const int64_t *offsets, const fl
                                 double eps, double *pot, double *acc, double *wsum,
                                 void *workspace, size_t workspace_bytes, void *stream);
 
+/* Potential-minimum centre of every halo (centring; the reference's discrete counterpart
+ * is most_bound_particle, halo_gas.py:498-634).  Particles m, x, y, z (device FP32) in halo
+ * order, HOST offsets (n_halo+1).  centres (device, 3 doubles per halo) holds the seeds and
+ * receives the result of c <- c + a(c) / w(c), a and w as halma_pot_soft_batched's gradient
+ * and wsum at c (no step where w is not positive), repeated per halo until a step is at
+ * most tol * eps, or max_iter times.  S (FP64 per halo): the softened sum at the centres;
+ * iters (int32): steps taken; steps (FP64): the last step's length (infinity with no
+ * step).  Waits for the iterations; S is stream-ordered. */
+size_t halma_refine_centres_workspace_size(int64_t n_halo, const int64_t *offsets, int max_iter);
+int halma_refine_centres(int64_t n_halo, const int64_t *offsets, const float *m, const float *x,
+                         const float *y, const float *z, double eps, double tol, int max_iter,
+                         double *centres, double *S, int32_t *iters, double *steps,
+                         void *workspace, size_t workspace_bytes, void *stream);
+
 /* Tuning knobs of the FP32 pair kernels (set by the autotuner; read back with get).
  *   HALMA_TUNE_TESTS_PER_LANE : test particles per lane (1, 2, 4)
  *   HALMA_TUNE_SUBTILE        : sources per plain FP32 sub-tile before the Kahan add

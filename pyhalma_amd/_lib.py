@@ -47,6 +47,9 @@ SIGNATURES = {
                                           _dbl, _p, _p, _p, _p, _size, _p]),
     "halma_pot_soft_batched_packed": (_c.c_int, [_i64, _i64p, _p, _i64p, _p, _p, _p, _dbl, _p,
                                                  _p, _p, _p, _size, _p]),
+    "halma_refine_centres_workspace_size": (_size, [_i64, _i64p, _c.c_int]),
+    "halma_refine_centres": (_c.c_int, [_i64, _i64p, _p, _p, _p, _p, _dbl, _dbl, _c.c_int, _p,
+                                        _p, _p, _p, _p, _size, _p]),
     "halma_soft_self_workspace_size": (_size, [_i64, _i64p]),
     "halma_pot_soft_self_batched": (_c.c_int, [_i64, _i64p, _p, _dbl, _p, _p, _p, _p, _size,
                                                _p]),

@@ -18,9 +18,8 @@ terms), through ``HaloPotentialEnergy``: the forward pass is the library's softe
 of every member against its halo (tests = the members' own FP32 positions, so the rule
 drops each self pair), the backward pass its hand-written acceleration kernel over the
 same pairs, recomputed.  ``refine_centres`` moves a seed centre per halo downhill on
-the potential Phi(c) = -G S(c): every step takes the autograd gradient of -S at the
-current centres and scales it per halo by 1 / w(c), w = sum_j m_j (r^2+eps^2)^(-3/2),
-which makes the step the fixed-point update c <- sum_j m_j w_j x_j / sum_j m_j w_j and
+the potential Phi(c) = -G S(c): every step is the gradient of S at the current centres
+scaled per halo by 1 / w(c), w = sum_j m_j (r^2+eps^2)^(-3/2), which makes the step the fixed-point update c <- sum_j m_j w_j x_j / sum_j m_j w_j and
 never increases Phi (the kernel (r^2 + eps^2)^(-1/2) is convex and decreasing in r^2).
 The reference's discrete counterpart is the most-bound particle of
 halo_gas.py:498-634.
@@ -217,33 +216,8 @@ def refine_centres(x, y, z, m, offsets, seeds, eps, max_iter=200, tol=1e-6):
     """Potential-minimum centre per halo.  Particles x, y, z, m in halo order (CSR
     host offsets, H+1 entries); seeds (H, 3) starting centres; eps the softening
     length (scalar or one per halo is not supported: one value).  Iterates until
-    every halo's step is below tol * eps, or max_iter.  Each step is autograd's
-    gradient of -sum S at the centres through SoftPotential, scaled by 1 / w."""
-    offsets = np.asarray(offsets, np.int64)
-    H = len(offsets) - 1
-    dev = engine.to_dev(np.zeros(1), np.float64).device
-    pos = torch.stack([engine.to_dev(a, np.float32) for a in (x, y, z)], dim=1)
-    mt = engine.to_dev(m, np.float32)
-    c = torch.as_tensor(np.asarray(seeds, np.float64), device=dev).clone()
-    tst_off = np.arange(H + 1, dtype=np.int64)
-    iters = torch.zeros(H, dtype=torch.int32, device=dev)
-    active = torch.ones(H, dtype=torch.bool, device=dev)
-    step_len = torch.full((H,), float("inf"), dtype=torch.float64, device=dev)
-    S = None
-    for _ in range(max_iter):
-        cc = c.detach().requires_grad_(True)
-        aux = {}
-        S = soft_potential(cc, pos, mt, offsets, tst_off, eps, aux)
-        (grad,) = torch.autograd.grad(-S.sum(), cc)   # = -acc(c)
-        w = aux["wsum"]
-        step = torch.where(w[:, None] > 0, -grad / w[:, None], torch.zeros_like(grad))
-        step = torch.where(active[:, None], step, torch.zeros_like(step))
-        c = c + step
-        step_len = torch.where(active, step.norm(dim=1), step_len)
-        iters += active.to(torch.int32)
-        active = active & (step_len > tol * eps)
-        if not bool(active.any()):
-            break
-    S = soft_potential(c, pos, mt, offsets, tst_off, eps).detach()
-    clear_cache()  # the columns of this call's source array
-    return CentringResult(c.detach(), S, iters, step_len)
+    every halo's step is at most tol * eps, or max_iter.  A step is the gradient of S at
+    the centre over w, the same as autograd's through SoftPotential; the iteration runs on
+    the device (halma_refine_centres)."""
+    c, S, iters, steps = engine.refine_centres(offsets, m, x, y, z, seeds, eps, tol, max_iter)
+    return CentringResult(c, S, iters, steps)

@@ -30,6 +30,7 @@
 #include <vector>
 
 #include "halma_common.h"
+#include "soft_pair.h"
 #include "staging.h"
 #include "tuning.h"
 
@@ -37,70 +38,15 @@ namespace halma {
 
 namespace {
 
-constexpr int kSub = 8;
 constexpr int kFewTests = 8;       // haloes with at most this many tests: lanes over sources
 constexpr int kFewChunk = 4096;    // sources of a few-test item (64 per lane)
 constexpr int kTileItems = 256;    // a tile halo's chunks aim at this many items ...
 constexpr int kTileMinChunk = 1024;  // ... with chunks of at least this many sources
 
-// pair quantities: bit 0 the potential S, bit 1 the gradient a and w
-constexpr int kModePot = 1;
-constexpr int kModeAcc = 2;
-constexpr int kModeBoth = 3;
-__host__ __device__ constexpr int n_planes(int mode) {
-    return ((mode & kModePot) ? 1 : 0) + ((mode & kModeAcc) ? 4 : 0);
-}
-
 struct __attribute__((aligned(8))) SoftDesc {
     int64_t src_off, tst_off, part_off;
     int32_t src_len, tst_len, chunk, few;
 };
-
-struct TestPt {
-    float hx, hy, hz, lx, ly, lz;
-};
-
-__device__ __forceinline__ TestPt split_test(double x, double y, double z) {
-    TestPt t;
-    t.hx = static_cast<float>(x);
-    t.hy = static_cast<float>(y);
-    t.hz = static_cast<float>(z);
-    t.lx = static_cast<float>(x - static_cast<double>(t.hx));
-    t.ly = static_cast<float>(y - static_cast<double>(t.hy));
-    t.lz = static_cast<float>(z - static_cast<double>(t.hz));
-    return t;
-}
-
-// Kahan-compensated addition: c holds the low part lost so far (s + c is the sum; the
-// sequence of s is that of the textbook form, whose compensation is -c)
-__device__ __forceinline__ void kahan(float& s, float& c, float v) {
-    const float y = v + c;
-    const float t = s + y;
-    c = y - (t - s);
-    s = t;
-}
-
-// One pair term added into the plain sub-tile sums ps (planes as n_planes(MODE): the
-// potential first when present, then ax, ay, az, w).  FP64 tests (SELF false) subtract
-// their lo part after the hi part.
-template <int MODE, bool SELF>
-__device__ __forceinline__ void pair_term(float* ps, float4 p, const TestPt& t, float e2) {
-    const float dx = SELF ? p.x - t.hx : (p.x - t.hx) - t.lx;
-    const float dy = SELF ? p.y - t.hy : (p.y - t.hy) - t.ly;
-    const float dz = SELF ? p.z - t.hz : (p.z - t.hz) - t.lz;
-    const float mn = fminf(fminf(fabsf(dx), fabsf(dy)), fabsf(dz));
-    const float d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, __builtin_fmaf(dx, dx, e2)));
-    const float inv = mn != 0.0f ? __builtin_amdgcn_rsqf(d2) : 0.0f;
-    constexpr int A = (MODE & kModePot) ? 1 : 0;
-    if (MODE & kModePot) ps[0] = __builtin_fmaf(p.w, inv, ps[0]);
-    if (MODE & kModeAcc) {
-        const float w = p.w * (inv * (inv * inv));
-        ps[A + 0] = __builtin_fmaf(w, dx, ps[A + 0]);
-        ps[A + 1] = __builtin_fmaf(w, dy, ps[A + 1]);
-        ps[A + 2] = __builtin_fmaf(w, dz, ps[A + 2]);
-        ps[A + 3] += w;
-    }
-}
 
 template <bool SELF>
 __device__ __forceinline__ TestPt load_test(const float4* src, const double* tx,

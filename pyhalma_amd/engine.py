@@ -199,6 +199,35 @@ def pot_soft_self(offsets, packed, eps, pot=True, acc=False, wsum=False):
     return out
 
 
+def refine_centres(offsets, m, x, y, z, seeds, eps, tol, max_iter):
+    """The centring iteration (halma_refine_centres) of every halo (CSR host offsets over
+    FP32 particles) from seeds (H, 3).  Returns device tensors (centres (H, 3) float64,
+    S float64, iters int32, last step lengths float64)."""
+    L = _lib_()
+    offsets = np.asarray(offsets, np.int64)
+    H = len(offsets) - 1
+    m, x, y, z = (to_dev(a.detach() if isinstance(a, torch.Tensor) else a, np.float32)
+                  for a in (m, x, y, z))
+    if not (x.numel() == y.numel() == z.numel() == m.numel()):
+        raise ValueError("particle arrays must have equal lengths")
+    if int(offsets[-1]) > x.numel() or int(offsets[0]) < 0:
+        raise ValueError("offsets beyond the particles")
+    c = to_dev(np.array(seeds, np.float64), np.float64)
+    if tuple(c.shape) != (H, 3):
+        raise ValueError("seeds must hold 3 values per halo")
+    S, steps = empty(H, np.float64), empty(H, np.float64)
+    iters = empty(H, np.int32)
+    if H == 0:
+        return c, S, iters, steps
+    off = _lib.i64_array(offsets)
+    ws = workspace(L.halma_refine_centres_workspace_size(H, off, int(max_iter)))
+    rc = L.halma_refine_centres(H, off, ptr(m), ptr(x), ptr(y), ptr(z), float(eps), float(tol),
+                                int(max_iter), ptr(c), ptr(S), ptr(iters), ptr(steps), ptr(ws),
+                                ws.numel(), stream_ptr())
+    _lib.check(rc, "halma_refine_centres")
+    return c, S, iters, steps
+
+
 def energy_test_batched(src_off, m, x, y, z, tst_off, tx, ty, tz, vx, vy, vz, halo_v,
                         factor, with_pot=False, stats=None):
     """One energy test per test particle, every halo at once (halma_energy_test_batched):
