@@ -23,7 +23,8 @@
 // adds a test's chunk partials in FP64 in chunk order whatever the launch shape (a
 // thread per test, or a wavefront per test for calls with few tests): a test's result
 // depends on its halo's inputs only.  Nothing of the N^2 pair terms is stored: the
-// gradient kernels recompute every term.
+// gradient kernels recompute every term.  Sums of the members over themselves without wsum
+// take the symmetric kernel of soft_sym.hip instead.
 #include <math.h>
 
 #include <algorithm>
@@ -31,6 +32,7 @@
 
 #include "halma_common.h"
 #include "soft_pair.h"
+#include "soft_sym.h"
 #include "staging.h"
 #include "tuning.h"
 
@@ -474,6 +476,14 @@ int soft_run(int64_t n_halo, const int64_t* src_off, const float* sm, const floa
         return set_error(HALMA_E_ARG, "packed sources must be 16-byte aligned");
     if (!pot && !acc && !wsum) return 0;
     hipStream_t st = static_cast<hipStream_t>(stream);
+    // the members as their own tests, without wsum: each pair once (soft_sym.hip; 18.1 ms
+    // for S and a of six haloes of 2e4-2e5 members, 26.6 ms one-sided); its slots grow with
+    // the halo, so a call with a halo of more than 2^23 members stays here
+    if (self && !wsum && soft_sym_takes(n_halo, src_off))
+        return soft_sym_run(n_halo, src_off,
+                            reinterpret_cast<const float4*>(src_xyzm) + src_off[0],
+                            static_cast<float>(eps * eps), pot ? pot + src_off[0] : nullptr,
+                            acc ? acc + 3 * src_off[0] : nullptr, ws, ws_bytes, st);
     SoftPlan plan;
     rc = plan_soft(n_halo, src_off, tst_off, plan);
     if (rc) return rc;
@@ -568,7 +578,9 @@ int halma_pot_soft_batched_packed(int64_t n_halo, const int64_t* src_off,
 }
 
 size_t halma_soft_self_workspace_size(int64_t n_halo, const int64_t* offsets) {
-    return soft_ws_bytes(n_halo, offsets, offsets, false);
+    const size_t one_sided = soft_ws_bytes(n_halo, offsets, offsets, false);
+    if (one_sided == 0 || !soft_sym_takes(n_halo, offsets)) return one_sided;
+    return std::max(one_sided, soft_sym_bytes(n_halo, offsets));
 }
 
 int halma_pot_soft_self_batched(int64_t n_halo, const int64_t* offsets, const float* src_xyzm,
