@@ -112,6 +112,44 @@ __device__ __forceinline__ void kahan_add(float& s, float& c, float v) {
     s = t;
 }
 
+__device__ __forceinline__ float min3(float a, float b, float c) { return fminf(fminf(a, b), c); }
+
+// 1 / r of N wave-uniform sources (an even number) from one test per lane, 0 where a
+// coordinate is equal (pair_acc's rule).  The rule costs 1.5 of 9.5 issue slots per pair
+// where pair_acc's costs 3 of 11: one running minimum of the |differences| of the N pairs,
+// a compare and a branch, and the rule pair by pair behind it only where some lane has an
+// equal coordinate.
+template <int N>
+__device__ __forceinline__ void inv_r_group(const float4 q[N], float x, float y, float z,
+                                            float v[N]) {
+    static_assert(N % 2 == 0, "the minimum takes two pairs at a time");
+    float mn = INFINITY;
+#pragma unroll
+    for (int s = 0; s < N; s += 2) {
+        const float dx0 = q[s].x - x, dy0 = q[s].y - y, dz0 = q[s].z - z;
+        const float dx1 = q[s + 1].x - x, dy1 = q[s + 1].y - y, dz1 = q[s + 1].z - z;
+        mn = min3(mn, fabsf(dx0), fabsf(dy0));
+        mn = min3(mn, fabsf(dz0), fabsf(dx1));
+        mn = min3(mn, fabsf(dy1), fabsf(dz1));
+        v[s] = __builtin_amdgcn_rsqf(
+            __builtin_fmaf(dz0, dz0, __builtin_fmaf(dy0, dy0, dx0 * dx0)));
+        v[s + 1] = __builtin_amdgcn_rsqf(
+            __builtin_fmaf(dz1, dz1, __builtin_fmaf(dy1, dy1, dx1 * dx1)));
+    }
+    if (__builtin_expect(__any(mn == 0.0f), 0)) {
+#pragma unroll
+        for (int s = 0; s < N; ++s) {
+            const float m1 = min3(fabsf(q[s].x - x), fabsf(q[s].y - y), fabsf(q[s].z - z));
+            v[s] = m1 != 0.0f ? v[s] : 0.0f;
+        }
+    }
+}
+
+// an FP64 sum as a pair of floats (hi, lo) whose sum keeps it to u^2
+__device__ __forceinline__ float2 split_sum(double S) {
+    const float hi = static_cast<float>(S);
+    return make_float2(hi, static_cast<float>(S - static_cast<double>(hi)));
+}
 
 // FP64 sum in the oracle's fixed order for one test position against ns sources:
 // kOrdWidth strided partials L[k] = sum over j = k, k + kOrdWidth, ... ascending (each

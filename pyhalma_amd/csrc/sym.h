@@ -6,7 +6,7 @@
 
 namespace halma {
 
-constexpr int kSymK = 4;  // tiles of 128 members per block
+constexpr int kSymK = 4;  // blocks of kSymK * 128 members
 
 // The partial slots of a halo take (nb + 1) * n * 8 bytes when its block pairs run in one
 // launch, quadratic in n: the unbinding keeps haloes above this size on the chunked

@@ -3,26 +3,37 @@
 // sources, as the unbinding's full passes need), each pair distance computed once and
 // its two terms, m_j / r to S_i and m_i / r to S_j, accumulated together.
 //
-// A halo of n members is cut into tiles of kTile = 128 members and the tiles into blocks
-// of kSymK = 4 tiles.  A work item is a pair of blocks (A, B), A <= B.  Tests are held in
-// registers (a tile of A: 2 per lane), the members of B's tiles streamed as wave-uniform
-// sources; accumulated are
-//   - test side: FP32 sums of 8 terms, Kahan-added, per test;
-//   - source side: per source, the wave-wide sum of its terms over a tile's tests (a
-//     fixed reduction tree across the lanes), Kahan-added in LDS over the tiles of A in
-//     order.
-// The test side keeps one Kahan sum per source tile; the tiles' sums are added in FP64
-// in tile order.  A launch with many items gives each item to one wavefront (all tiles of
-// B in turn); a launch with fewer (a lone large halo, the last passes of an unbinding)
-// gives each to a workgroup whose wavefront w takes tile w of B, so that an item lasts
-// four tile pairs instead of sixteen, and one with fewer than 1024 items to a 1024-thread
-// workgroup with one tile pair per wavefront (k_pot_sym_fine).  Both forms do the same arithmetic in
-// the same order: a halo's sums do not depend on the other haloes of the call.  Within a diagonal item
-// (A == B) only pairs of tiles a <= b are taken, and a tile against itself is summed on
-// the test side alone.  Every member then has kSymK-block partial sums in nb + 1 slots
-// (nb = blocks of its halo), each written by exactly one item: slot s < I (its block) from the source side of item (s, I), slot I from the test
-// side of item (I, I), slots s > I from the test side of item (I, s), and slot nb from
-// the source side of item (I, I).  The slots are merged in FP64 in slot order.
+// A halo of n members is cut into blocks of kBlock = 512 members.  A work item is a pair of
+// blocks (A, B), A <= B.  The members of A are the tests, kTests = 8 per lane in registers
+// (test strip t: members 64 t .. 64 t + 63 of A); the members of B stream through as
+// wave-uniform sources, eight at a time, in segments of kSeg = 32:
+//   - test side: per test an FP32 sum of the eight terms, added in FP64 over the segment,
+//     the segments' sums in FP64 in order;
+//   - source side: per source two FP32 chains over a lane's tests 0-3 and 4-7, their sum
+//     through a fixed tree over the lanes (reduce8, its last levels in FP64).  The lanes hold every test of the
+//     item, so the total goes straight to the member's slot.
+// In a diagonal item (A == B) a source of strip s meets the strips t < s on both sides and
+// strip s on the test side alone (all its ordered pairs); the strips above it are another
+// source's.  Every member then has partial sums in nb + 1 slots (nb = blocks of its halo),
+// each written by exactly one item: slot s < I (its block) from the source side of item
+// (s, I), slot I from the test side of item (I, I), slots s > I from the test side of item
+// (I, s), and slot nb from the source side of item (I, I).  The slots are merged in FP64 in
+// slot order.
+//
+// A launch of kWaveItems items or more gives each item to a wavefront, which takes its
+// segments in turn; one with fewer (a lone halo, the later passes of an unbinding) to a
+// workgroup of sixteen wavefronts, a segment each, whose test sums meet in LDS and are
+// added in segment order.  The same operations in the same order: a halo's sums do not
+// depend on the other haloes of the call.
+//
+// Bound by the FP32 vector ALUs.  Per pair distance 11.5 issue slots (3 differences, 3 for
+// r^2, 1.5 for the coordinate rule, 2 for the reciprocal root, 2 sums), 0.25 for the FP64
+// sums, 0.5 for the two chains and the tree.  The rule is a running minimum of the
+// |differences| of a strip's eight pairs per lane, one compare and a branch; the branch's
+// side evaluates the rule pair by pair (a tenth of the eights in the clumps' FP32
+// coordinates).  Pair by pair for all of them costs 3 slots.  The clump step's launches (8.0e9
+// distances in the first) 2.80 -> 2.46 ms, the gas step's 16.8 -> 14.6 ms against two tests
+// per lane with Kahan sums, the pair-by-pair rule and a tree per 128 tests.
 #include <math.h>
 
 #include <algorithm>
@@ -39,73 +50,132 @@ namespace halma {
 
 namespace {
 
-constexpr int kTile = 2 * kWave;  // 128 members: two tests per lane
+constexpr int kTests = 8;                 // tests per lane
+constexpr int kBlock = kTests * kWave;    // members of a block
+constexpr int kSeg = 32;                  // sources of a segment
+constexpr int kSegs = kBlock / kSeg;
+static_assert(kBlock == 128 * kSymK, "blocks of the plans");
 
-__device__ __forceinline__ float inv_r(float4 q, float x, float y, float z) {
-    const float dx = q.x - x;
-    const float dy = q.y - y;
-    const float dz = q.z - z;
-    const float d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
-    const float mn = fminf(fminf(fabsf(dx), fabsf(dy)), fabsf(dz));
-    return mn != 0.0f ? __builtin_amdgcn_rsqf(d2) : 0.0f;  // the rule of pair_acc
-}
+// Below this many items a launch gives each to a workgroup (k_pot_sym_fine): the clump step
+// (33k items in the first pass) is the same from 1024 to 8192, the bridged pairs' later passes
+// (1-8k items) take 8.2 ms at 1024, 8.0 at 2048, 7.6 at 4096, 7.9 at 8192
+constexpr int kWaveItems = 4096;
 
-// Kahan-compensated addition: c holds the low part lost so far (s + c is the sum; the
-// sequence of s is that of the textbook form, whose compensation is -c)
-__device__ __forceinline__ void kahan(float& s, float& c, float v) {
-    const float y = v + c;
-    const float t = s + y;
-    c = y - (t - s);
-    s = t;
-}
+struct SymTests {
+    float x[kTests], y[kTests], z[kTests], m[kTests];
+};
 
-// Sources q[g .. g+7] of a tile (cnt of them exist) against the lane's two tests: the
-// test-side partial sums ps[r] (8 terms, source order) and the per-source pair terms
-// pj[s] = m_i0 / r + m_i1 / r.  A full group (g + 8 <= cnt, wave-uniform) needs no
-// padding select; the tail group clamps its loads and gives padding sources no mass.
-template <bool kFull>
-__device__ __forceinline__ void pair_group(const float4* __restrict__ q0, int g, int cnt,
-                                           const float xi[2], const float yi[2],
-                                           const float zi[2], const float mi[2], float ps[2],
-                                           float pj[8]) {
+__device__ __forceinline__ void load_tests(const float4* __restrict__ sp, int i0, int n, int lane,
+                                           SymTests& T) {
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-        const int j = g + s;
-        const float4 q = uniform_load(q0 + (kFull ? j : min(j, cnt - 1)));
-        const float qw = (kFull || j < cnt) ? q.w : 0.0f;
-        const float v0 = inv_r(q, xi[0], yi[0], zi[0]);
-        const float v1 = inv_r(q, xi[1], yi[1], zi[1]);
-        ps[0] = __builtin_fmaf(qw, v0, ps[0]);
-        ps[1] = __builtin_fmaf(qw, v1, ps[1]);
-        pj[s] = __builtin_fmaf(mi[1], v1, mi[0] * v0);
+    for (int t = 0; t < kTests; ++t) {
+        const int i = i0 + t * kWave + lane;
+        const float4 p = sp[min(i, n - 1)];
+        T.x[t] = p.x;
+        T.y[t] = p.y;
+        T.z[t] = p.z;
+        T.m[t] = i < n ? p.w : 0.0f;  // padding lanes add nothing to sources
     }
 }
 
-// Below this many items in a launch an item is taken by a workgroup (four wavefronts,
-// one source tile each), else by one wavefront: a wavefront per item fills the device
-// once there are a few items per SIMD and keeps diagonal items balanced; with fewer
-// items the workgroup form cuts an item's latency fourfold.
-constexpr int kGroupItems = 2048;
+// Eight sources (cnt of them exist; kFull: all of them): strips t < lim on both sides, strip
+// lim on the test side.  R: the tests' FP64 sums of the segment.  Returns the source side's
+// total of source (lane >> 3) & 7, valid in the lanes with lane % 8 == 0.
+template <bool kFull>
+__device__ __forceinline__ double sym_group(const float4* __restrict__ q0, int cnt, int lim,
+                                           const SymTests& T, double R[kTests], int lane) {
+    float4 q[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        q[s] = uniform_load(q0 + (kFull ? s : min(s, cnt - 1)));
+        if (!kFull && s >= cnt) q[s].w = 0.0f;
+    }
+    float p[2][8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) p[0][s] = p[1][s] = 0.0f;
+#pragma unroll
+    for (int t = 0; t < kTests; ++t) {
+        if (t <= lim) {
+            float v[8];
+            inv_r_group<8>(q, T.x[t], T.y[t], T.z[t], v);
+            float ps = q[0].w * v[0];
+#pragma unroll
+            for (int s = 1; s < 8; ++s) ps = __builtin_fmaf(q[s].w, v[s], ps);
+            R[t] += static_cast<double>(ps);
+            if (t < lim) {
+#pragma unroll
+                for (int s = 0; s < 8; ++s)
+                    p[t / 4][s] = __builtin_fmaf(T.m[t], v[s], p[t / 4][s]);
+            }
+        }
+        // a strip's terms stay together (registers)
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (lim == 0) return 0.0;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) p[0][s] += p[1][s];
+    return reduce8(p[0], lane);
+}
 
-// Below this many items an item is taken by a 1024-thread workgroup whose sixteen
-// wavefronts take its sixteen tile pairs (k_pot_sym_fine): an item then lasts one tile
-// pair, for the last passes of an unbinding where a few small haloes take full passes.
-constexpr int kFineItems = 1024;
+// Sources j0 .. j0 + cnt - 1 (a segment) of item (A, B): the source side to its slot (out,
+// by member), the test side to R.
+__device__ __forceinline__ void sym_segment(const float4* __restrict__ sp, int j0, int cnt,
+                                            int lim, const SymTests& T, double R[kTests],
+                                            float2* __restrict__ out, int lane) {
+    const int s = (lane >> 3) & 7;
+    for (int g = 0; g < cnt; g += 8) {
+        const double tot = g + 8 <= cnt ? sym_group<true>(sp + j0 + g, 8, lim, T, R, lane)
+                                        : sym_group<false>(sp + j0 + g, cnt - g, lim, T, R, lane);
+        if ((lane & 7) == 0 && g + s < cnt) out[j0 + g + s] = split_sum(tot);
+    }
+}
 
-// One item per wavefront: tiles of A in turn against all tiles of B; test side a Kahan
-// sum per tile of B, the tiles' sums added in FP64 in tile order; source side in the
-// wavefront's LDS (ls, lc: kSymK tiles each).  Same arithmetic, in the same order, as
-// the workgroup form below, so both give the same bits.
-__device__ __forceinline__ void sym_items_wave(const float4* __restrict__ src,
-                                               const SymDesc* __restrict__ halos,
-                                               const int* __restrict__ live_n,
-                                               const int4* __restrict__ items, int n_items,
-                                               float2* __restrict__ part, int* __restrict__ head,
-                                               float* ls, float* lc) {
+struct SymItem {
+    const float4* sp;  // the halo's members
+    float2* pp;        // its slots
+    int64_t stride;    // slots are laid out for the planned size
+    int n, A, B, tslot, sslot;
+    bool ok;
+};
+
+__device__ __forceinline__ SymItem sym_item(const float4* __restrict__ src,
+                                            const SymDesc* __restrict__ halos,
+                                            const int* __restrict__ live_n,
+                                            const int4* __restrict__ items, int k,
+                                            float2* __restrict__ part) {
+    const int4 it = uniform_load(items + k);
+    const SymDesc d = uniform_load(halos + it.x);
+    SymItem r;
+    r.n = live_n ? __builtin_amdgcn_readfirstlane(uniform_load(live_n + it.x)) : d.n;
+    const int nb = (r.n + kBlock - 1) / kBlock;
+    r.A = it.y;
+    r.B = it.z;
+    r.ok = r.B < nb && r.A <= r.B;
+    r.sp = src + d.off;
+    r.pp = part + d.part_off;
+    r.stride = d.n;
+    // test side: slot B (mod the band width); source side: slot A, or the diagonal slot
+    r.tslot = r.B % d.wb;
+    r.sslot = r.A < r.B ? r.A % d.wb : min(d.wb, nb);
+    return r;
+}
+
+__global__ __launch_bounds__(256, 4) void k_pot_sym(const float4* __restrict__ src,
+                                                 const SymDesc* __restrict__ halos,
+                                                 const int* __restrict__ live_n,
+                                                 const int4* __restrict__ items, int n_items,
+                                                 const int64_t* __restrict__ n_items_dev,
+                                                 float2* __restrict__ part,
+                                                 int* __restrict__ head) {
     const int lane = __lane_id();
-    const int wv = threadIdx.x / kWave;
+    if (n_items_dev) {
+        const int64_t nd = uniform_load(n_items_dev);
+        n_items = static_cast<int>(nd < n_items ? nd : n_items);
+    }
+    if (n_items < kWaveItems) return;  // k_pot_sym_fine takes the launch
     const int n_waves = static_cast<int>(gridDim.x * (blockDim.x / kWave));
-    int k = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x * (blockDim.x / kWave) + wv));
+    int k = __builtin_amdgcn_readfirstlane(
+        static_cast<int>(blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave));
     for (bool first = true;; first = false) {
         if (!first) {
             int t = 0;
@@ -113,245 +183,35 @@ __device__ __forceinline__ void sym_items_wave(const float4* __restrict__ src,
             k = n_waves + __builtin_amdgcn_readfirstlane(t);
         }
         if (k >= n_items) break;
-        const int4 it = uniform_load(items + k);
-        const SymDesc d = uniform_load(halos + it.x);
-        const int n = live_n ? __builtin_amdgcn_readfirstlane(uniform_load(live_n + it.x)) : d.n;
-        const int nt = (n + kTile - 1) / kTile;
-        const int nb = (nt + kSymK - 1) / kSymK;
-        const int A = it.y, B = it.z;
-        if (B >= nb || A > B) continue;
-        const float4* sp = src + d.off;
-        float2* pp = part + d.part_off;
-        const int64_t stride = d.n;  // slots are laid out for the planned size
+        const SymItem it = sym_item(src, halos, live_n, items, k, part);
+        if (!it.ok) continue;
+        SymTests T;
+        load_tests(it.sp, it.A * kBlock, it.n, lane, T);
+        double S[kTests];
 #pragma unroll
-        for (int e = 0; e < kSymK * kTile / kWave; ++e) {
-            ls[e * kWave + lane] = 0.0f;
-            lc[e * kWave + lane] = 0.0f;
+        for (int t = 0; t < kTests; ++t) S[t] = 0.0;
+        float2* out = it.pp + static_cast<int64_t>(it.sslot) * it.stride;
+        const int j1 = min(it.n, (it.B + 1) * kBlock);
+        int sg = 0;
+        for (int j0 = it.B * kBlock; j0 < j1; j0 += kSeg, ++sg) {
+            double R[kTests];
+#pragma unroll
+            for (int t = 0; t < kTests; ++t) R[t] = 0.0;
+            sym_segment(it.sp, j0, min(kSeg, j1 - j0),
+                        it.A == it.B ? sg * kSeg / kWave : kTests, T, R, out, lane);
+#pragma unroll
+            for (int t = 0; t < kTests; ++t) S[t] += R[t];
         }
-        for (int ta = 0; ta < kSymK; ++ta) {
-            const int a = A * kSymK + ta;
-            if (a >= nt) break;
-            float xi[2], yi[2], zi[2], mi[2];
-            double S[2] = {0.0, 0.0};
-            int ii[2];
+        out = it.pp + static_cast<int64_t>(it.tslot) * it.stride;
 #pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                ii[r] = a * kTile + r * kWave + lane;
-                const float4 p = sp[min(ii[r], n - 1)];
-                xi[r] = p.x;
-                yi[r] = p.y;
-                zi[r] = p.z;
-                mi[r] = ii[r] < n ? p.w : 0.0f;  // padding lanes add nothing to sources
-            }
-            for (int tb = 0; tb < kSymK; ++tb) {
-                const int b = B * kSymK + tb;
-                if (b >= nt) break;
-                if (A == B && b < a) continue;
-                const int j0 = b * kTile;
-                const int cnt = min(kTile, n - j0);
-                const bool diag = b == a;
-                float as[2] = {0.0f, 0.0f}, ac[2] = {0.0f, 0.0f};
-                for (int g = 0; g < cnt; g += 8) {
-                    float ps[2] = {0.0f, 0.0f};
-                    float pj[8];
-                    if (g + 8 <= cnt)
-                        pair_group<true>(sp + j0, g, cnt, xi, yi, zi, mi, ps, pj);
-                    else
-                        pair_group<false>(sp + j0, g, cnt, xi, yi, zi, mi, ps, pj);
-                    kahan(as[0], ac[0], ps[0]);
-                    kahan(as[1], ac[1], ps[1]);
-                    if (!diag) {
-                        const float tot = reduce8(pj, lane);
-                        const int s = (lane >> 3) & 7;
-                        if ((lane & 7) == 0 && g + s < cnt) {
-                            const int e = tb * kTile + g + s;
-                            float sv = ls[e], cv = lc[e];
-                            kahan(sv, cv, tot);
-                            ls[e] = sv;
-                            lc[e] = cv;
-                        }
-                    }
-                }
-#pragma unroll
-                for (int r = 0; r < 2; ++r)
-                    S[r] += static_cast<double>(as[r]) + static_cast<double>(ac[r]);
-            }
-            // test side of tile a from this item: slot B (mod the band width), the source
-            // tiles' sums added in FP64 in tile order (the same bits as a workgroup's)
-            const int tslot = B % d.wb;
-#pragma unroll
-            for (int r = 0; r < 2; ++r)
-                if (ii[r] < n) {
-                    const float hi = static_cast<float>(S[r]);
-                    pp[static_cast<int64_t>(tslot) * stride + ii[r]] =
-                        make_float2(hi, static_cast<float>(S[r] - static_cast<double>(hi)));
-                }
-        }
-        // source side of B's tiles from this item: slot A (mod the band width), or the
-        // diagonal slot min(wb, nb)
-        const int slot = A < B ? A % d.wb : min(d.wb, nb);
-        for (int tb = 0; tb < kSymK; ++tb) {
-            const int b = B * kSymK + tb;
-            if (b >= nt) break;
-            const int j0 = b * kTile;
-            const int cnt = min(kTile, n - j0);
-#pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                const int e = r * kWave + lane;
-                if (e < cnt)
-                    pp[static_cast<int64_t>(slot) * stride + j0 + e] =
-                        make_float2(ls[tb * kTile + e], lc[tb * kTile + e]);
-            }
+        for (int t = 0; t < kTests; ++t) {
+            const int i = it.A * kBlock + t * kWave + lane;
+            if (i < it.n) out[i] = split_sum(S[t]);
         }
     }
 }
 
-// One item per workgroup: wavefront w streams tile w of B against each tile of A in turn;
-// its source side stays in its LDS (ls, lc: one tile), its test-side sums per tile of A go
-// to tpart[ta][w] and are added in FP64 in tile order once the four are done.
-__device__ __forceinline__ void sym_items_group(const float4* __restrict__ src,
-                                                const SymDesc* __restrict__ halos,
-                                                const int* __restrict__ live_n,
-                                                const int4* __restrict__ items, int n_items,
-                                                float2* __restrict__ part,
-                                                int* __restrict__ head, float* ls, float* lc,
-                                                float2* tpart, int* next_item) {
-    const int lane = __lane_id();
-    const int wv = threadIdx.x / kWave;
-    int k = static_cast<int>(blockIdx.x);
-    for (bool first = true;; first = false) {
-        if (!first) {
-            __syncthreads();  // the previous item's LDS has been read
-            if (threadIdx.x == 0) *next_item = atomicAdd(head, 1);
-            __syncthreads();
-            k = static_cast<int>(gridDim.x) + *next_item;
-        }
-        if (k >= n_items) break;
-        const int4 it = uniform_load(items + k);
-        const SymDesc d = uniform_load(halos + it.x);
-        const int n = live_n ? __builtin_amdgcn_readfirstlane(uniform_load(live_n + it.x)) : d.n;
-        const int nt = (n + kTile - 1) / kTile;
-        const int nb = (nt + kSymK - 1) / kSymK;
-        const int A = it.y, B = it.z;
-        if (B >= nb || A > B) continue;
-        const float4* sp = src + d.off;
-        float2* pp = part + d.part_off;
-        const int64_t stride = d.n;  // slots are laid out for the planned size
-        const int b = B * kSymK + wv;  // this wavefront's source tile
-        const int j0 = b * kTile;
-        const int cnt = b < nt ? min(kTile, n - j0) : 0;
-#pragma unroll
-        for (int e = 0; e < kTile / kWave; ++e) {
-            ls[e * kWave + lane] = 0.0f;
-            lc[e * kWave + lane] = 0.0f;
-        }
-        for (int ta = 0; ta < kSymK; ++ta) {
-            const int a = A * kSymK + ta;
-            if (a >= nt) break;
-            float as[2] = {0.0f, 0.0f}, ac[2] = {0.0f, 0.0f};
-            if (cnt > 0 && !(A == B && b < a)) {
-                float xi[2], yi[2], zi[2], mi[2];
-#pragma unroll
-                for (int r = 0; r < 2; ++r) {
-                    const int i = a * kTile + r * kWave + lane;
-                    const float4 p = sp[min(i, n - 1)];
-                    xi[r] = p.x;
-                    yi[r] = p.y;
-                    zi[r] = p.z;
-                    mi[r] = i < n ? p.w : 0.0f;  // padding lanes add nothing to sources
-                }
-                const bool diag = b == a;
-                for (int g = 0; g < cnt; g += 8) {
-                    float ps[2] = {0.0f, 0.0f};
-                    float pj[8];
-                    if (g + 8 <= cnt)
-                        pair_group<true>(sp + j0, g, cnt, xi, yi, zi, mi, ps, pj);
-                    else
-                        pair_group<false>(sp + j0, g, cnt, xi, yi, zi, mi, ps, pj);
-                    kahan(as[0], ac[0], ps[0]);
-                    kahan(as[1], ac[1], ps[1]);
-                    if (!diag) {
-                        const float tot = reduce8(pj, lane);
-                        const int s = (lane >> 3) & 7;
-                        if ((lane & 7) == 0 && g + s < cnt) {
-                            float sv = ls[g + s], cv = lc[g + s];
-                            kahan(sv, cv, tot);
-                            ls[g + s] = sv;
-                            lc[g + s] = cv;
-                        }
-                    }
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < 2; ++r)
-                tpart[(ta * kSymK + wv) * kTile + r * kWave + lane] = make_float2(as[r], ac[r]);
-        }
-        __syncthreads();
-        // test side of A's tiles from this item: slot B (mod the band width); the four
-        // source tiles' compensated sums added in FP64 in tile order, stored as a pair of
-        // floats (hi, lo) whose sum keeps the FP64 value to u^2
-        const int tslot = B % d.wb;
-        for (int t = threadIdx.x; t < kSymK * kTile; t += blockDim.x) {
-            const int ta = t / kTile, e = t % kTile;
-            const int i = (A * kSymK + ta) * kTile + e;
-            if (A * kSymK + ta >= nt || i >= n) continue;
-            double S = 0.0;
-#pragma unroll
-            for (int w = 0; w < kSymK; ++w) {
-                const float2 v = tpart[(ta * kSymK + w) * kTile + e];
-                S += static_cast<double>(v.x) + static_cast<double>(v.y);
-            }
-            const float hi = static_cast<float>(S);
-            pp[static_cast<int64_t>(tslot) * stride + i] =
-                make_float2(hi, static_cast<float>(S - static_cast<double>(hi)));
-        }
-        // source side of this wavefront's tile of B: slot A (mod the band width), or the
-        // diagonal slot min(wb, nb)
-        const int slot = A < B ? A % d.wb : min(d.wb, nb);
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            const int e = r * kWave + lane;
-            if (e < cnt)
-                pp[static_cast<int64_t>(slot) * stride + j0 + e] = make_float2(ls[e], lc[e]);
-        }
-    }
-}
-
-__global__ __launch_bounds__(256) void k_pot_sym(const float4* __restrict__ src,
-                                                 const SymDesc* __restrict__ halos,
-                                                 const int* __restrict__ live_n,
-                                                 const int4* __restrict__ items, int n_items,
-                                                 const int64_t* __restrict__ n_items_dev,
-                                                 float2* __restrict__ part,
-                                                 int* __restrict__ head) {
-    static_assert(kSymK * kWave == 256, "one wavefront per tile of a block");
-    // LDS of either form: a wavefront per item keeps (sum, comp) of kSymK source tiles
-    // per wavefront (16 KiB); a workgroup per item one source tile per wavefront (4 KiB)
-    // and the test-side sums of each (tile of A, wavefront) (16 KiB)
-    __shared__ float2 lds[2560];
-    __shared__ int next_item;
-    float* f = reinterpret_cast<float*>(lds);
-    const int wv = threadIdx.x / kWave;
-    if (n_items_dev) {
-        const int64_t nd = uniform_load(n_items_dev);
-        n_items = static_cast<int>(nd < n_items ? nd : n_items);
-    }
-    if (n_items < kFineItems) return;  // k_pot_sym_fine takes the launch
-    if (n_items >= kGroupItems)
-        sym_items_wave(src, halos, live_n, items, n_items, part, head,
-                       f + wv * kSymK * kTile, f + (kSymK + wv) * kSymK * kTile);
-    else
-        sym_items_group(src, halos, live_n, items, n_items, part, head, f + wv * kTile,
-                        f + (kSymK + wv) * kTile, lds + kSymK * kTile, &next_item);
-}
-
-// One item per 1024-thread workgroup (launches of fewer than kFineItems items): wavefront
-// 4 ta + w takes tile ta of A against tile w of B.  The pair's test-side compensated sum
-// goes to tpart[ta][w], its source-side terms (one per source of tile w, the wave-wide sum
-// over tile ta's tests) to spart[ta][w]; then the test side of each tile of A is added in
-// FP64 over the tiles of B in tile order and the source side of each tile of B is
-// Kahan-added over the tiles of A in order, skipping the pairs the other forms skip: the
-// same operations in the same order as the other forms, so the same bits.
+// One item per workgroup of sixteen wavefronts, a segment each.
 __global__ __launch_bounds__(1024) void k_pot_sym_fine(const float4* __restrict__ src,
                                                        const SymDesc* __restrict__ halos,
                                                        const int* __restrict__ live_n,
@@ -360,110 +220,47 @@ __global__ __launch_bounds__(1024) void k_pot_sym_fine(const float4* __restrict_
                                                        const int64_t* __restrict__ n_items_dev,
                                                        float2* __restrict__ part,
                                                        int* __restrict__ head) {
-    static_assert(kSymK * kSymK * kWave == 1024, "one wavefront per tile pair of an item");
-    __shared__ float2 tpart[kSymK * kSymK * kTile];  // 16 KiB
-    __shared__ float spart[kSymK * kSymK * kTile];   // 8 KiB
+    static_assert(kSegs * kWave == 1024, "one wavefront per segment of an item");
+    __shared__ double seg[kSegs][kBlock];  // 64 KiB
     __shared__ int next_item;
     if (n_items_dev) {
         const int64_t nd = uniform_load(n_items_dev);
         n_items = static_cast<int>(nd < n_items ? nd : n_items);
     }
-    if (n_items >= kFineItems) return;  // k_pot_sym takes the launch
+    if (n_items >= kWaveItems) return;  // k_pot_sym takes the launch
     const int lane = __lane_id();
-    const int wv = threadIdx.x / kWave;
-    const int ta = wv / kSymK, w = wv % kSymK;
-    float2* tp = tpart + wv * kTile;
-    float* spw = spart + wv * kTile;
+    const int sg = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
     int k = static_cast<int>(blockIdx.x);
     for (bool first = true;; first = false) {
         if (!first) {
             __syncthreads();  // the previous item's LDS has been read
             if (threadIdx.x == 0) next_item = atomicAdd(head, 1);
             __syncthreads();
-            k = static_cast<int>(gridDim.x) + next_item;
+            k = static_cast<int>(gridDim.x) + __builtin_amdgcn_readfirstlane(next_item);
         }
         if (k >= n_items) break;
-        const int4 it = uniform_load(items + k);
-        const SymDesc d = uniform_load(halos + it.x);
-        const int n = live_n ? __builtin_amdgcn_readfirstlane(uniform_load(live_n + it.x)) : d.n;
-        const int nt = (n + kTile - 1) / kTile;
-        const int nb = (nt + kSymK - 1) / kSymK;
-        const int A = it.y, B = it.z;
-        if (B >= nb || A > B) continue;  // the same for the whole workgroup
-        const float4* sp = src + d.off;
-        float2* pp = part + d.part_off;
-        const int64_t stride = d.n;  // slots are laid out for the planned size
-        const int a = A * kSymK + ta, b = B * kSymK + w;
-        const int j0 = b * kTile;
-        const int cnt = b < nt ? min(kTile, n - j0) : 0;
+        const SymItem it = sym_item(src, halos, live_n, items, k, part);
+        if (!it.ok) continue;  // the same for the whole workgroup
+        const int j0 = it.B * kBlock + sg * kSeg;
+        const int cnt = min(kSeg, it.n - j0);
+        if (cnt > 0) {
+            SymTests T;
+            load_tests(it.sp, it.A * kBlock, it.n, lane, T);
+            double R[kTests];
 #pragma unroll
-        for (int r = 0; r < 2; ++r) spw[r * kWave + lane] = 0.0f;
-        float as[2] = {0.0f, 0.0f}, ac[2] = {0.0f, 0.0f};
-        if (a < nt && cnt > 0 && !(A == B && b < a)) {
-            float xi[2], yi[2], zi[2], mi[2];
+            for (int t = 0; t < kTests; ++t) R[t] = 0.0;
+            sym_segment(it.sp, j0, cnt, it.A == it.B ? sg * kSeg / kWave : kTests, T, R,
+                        it.pp + static_cast<int64_t>(it.sslot) * it.stride, lane);
 #pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                const int i = a * kTile + r * kWave + lane;
-                const float4 p = sp[min(i, n - 1)];
-                xi[r] = p.x;
-                yi[r] = p.y;
-                zi[r] = p.z;
-                mi[r] = i < n ? p.w : 0.0f;  // padding lanes add nothing to sources
-            }
-            const bool diag = b == a;
-            for (int g = 0; g < cnt; g += 8) {
-                float ps[2] = {0.0f, 0.0f};
-                float pj[8];
-                if (g + 8 <= cnt)
-                    pair_group<true>(sp + j0, g, cnt, xi, yi, zi, mi, ps, pj);
-                else
-                    pair_group<false>(sp + j0, g, cnt, xi, yi, zi, mi, ps, pj);
-                kahan(as[0], ac[0], ps[0]);
-                kahan(as[1], ac[1], ps[1]);
-                if (!diag) {
-                    const float tot = reduce8(pj, lane);
-                    const int s = (lane >> 3) & 7;
-                    if ((lane & 7) == 0 && g + s < cnt) spw[g + s] = tot;
-                }
-            }
+            for (int t = 0; t < kTests; ++t) seg[sg][t * kWave + lane] = R[t];
         }
-#pragma unroll
-        for (int r = 0; r < 2; ++r) tp[r * kWave + lane] = make_float2(as[r], ac[r]);
         __syncthreads();
-        // test side of A's tiles: slot B (mod the band width), the four source tiles'
-        // compensated sums added in FP64 in tile order, kept as a float pair (hi, lo)
-        const int tslot = B % d.wb;
-        for (int t = threadIdx.x; t < kSymK * kTile; t += blockDim.x) {
-            const int t_a = t / kTile, e = t % kTile;
-            const int i = (A * kSymK + t_a) * kTile + e;
-            if (A * kSymK + t_a >= nt || i >= n) continue;
+        const int n_segs = min(kSegs, (it.n - it.B * kBlock + kSeg - 1) / kSeg);
+        const int e = threadIdx.x, i = it.A * kBlock + e;
+        if (e < kBlock && i < it.n) {
             double S = 0.0;
-#pragma unroll
-            for (int t_b = 0; t_b < kSymK; ++t_b) {
-                const float2 v = tpart[(t_a * kSymK + t_b) * kTile + e];
-                S += static_cast<double>(v.x) + static_cast<double>(v.y);
-            }
-            const float hi = static_cast<float>(S);
-            pp[static_cast<int64_t>(tslot) * stride + i] =
-                make_float2(hi, static_cast<float>(S - static_cast<double>(hi)));
-        }
-        // source side of B's tiles: slot A (mod the band width), or the diagonal slot
-        // min(wb, nb); the terms from the tiles of A Kahan-added in tile order
-        const int slot = A < B ? A % d.wb : min(d.wb, nb);
-        for (int t = threadIdx.x; t < kSymK * kTile; t += blockDim.x) {
-            const int t_b = t / kTile, e = t % kTile;
-            const int bb = B * kSymK + t_b;
-            if (bb >= nt) continue;
-            const int jb = bb * kTile;
-            if (e >= min(kTile, n - jb)) continue;
-            float sv = 0.0f, cv = 0.0f;
-            for (int t_a = 0; t_a < kSymK; ++t_a) {
-                const int aa = A * kSymK + t_a;
-                if (aa >= nt) break;
-                if ((A == B && bb < aa) || bb == aa) continue;
-                kahan(sv, cv, spart[(t_a * kSymK + t_b) * kTile + e]);
-            }
-            pp[static_cast<int64_t>(slot) * stride + jb + e] = make_float2(sv, cv);
+            for (int g = 0; g < n_segs; ++g) S += seg[g][e];
+            it.pp[static_cast<int64_t>(it.tslot) * it.stride + i] = split_sum(S);
         }
     }
 }
@@ -671,13 +468,13 @@ int launch_pot_sym(const SymPlan& plan, const float4* src4, const SymDesc* d_hal
     // both forms are queued when the item count is known only on the device and the plan
     // allows either (the one not chosen returns at once); the device count never exceeds
     // the planned n_items
-    if (n_items >= kFineItems) {
-        const int grid = std::max(1, std::min(cus * 8, n_items));  // a workgroup or more per item
+    if (n_items >= kWaveItems) {
+        const int grid = std::max(1, std::min(cus * 8, (n_items + 3) / 4));
         k_pot_sym<<<grid, 256, 0, st>>>(src4, d_halos, live_n, d_items, n_items, n_items_dev,
                                         part, head);
         HALMA_LAUNCH_CHECK();
     }
-    if (n_items < kFineItems || n_items_dev) {
+    if (n_items < kWaveItems || n_items_dev) {
         const int grid = std::max(1, std::min(cus, n_items));
         k_pot_sym_fine<<<grid, 1024, 0, st>>>(src4, d_halos, live_n, d_items, n_items,
                                               n_items_dev, part, head);
@@ -749,8 +546,8 @@ int halma_pot_sum_self_batched(int64_t n_halo, const int64_t* offsets, const flo
         if (ni > 0) {
             k_sym_clear<<<1, 64, 0, st>>>(w.head);
             HALMA_LAUNCH_CHECK();
-            if (ni >= kFineItems) {
-                const int grid = static_cast<int>(std::min<int64_t>(cus * 8, ni));
+            if (ni >= kWaveItems) {
+                const int grid = static_cast<int>(std::min<int64_t>(cus * 8, (ni + 3) / 4));
                 k_pot_sym<<<grid, 256, 0, st>>>(w.src4, w.halos, nullptr, w.items + i0,
                                                 static_cast<int>(ni), nullptr, w.part, w.head);
             } else {

@@ -24,7 +24,7 @@
 //                    kernels' item lists (haloes in the plan's largest-first order) and,
 //                    in its other blocks, the compacted lists;
 //   2. pair kernels  full passes on the symmetric kernel (k_pot_sym, or k_pot_sym_fine
-//                    for fewer than 1024 block pairs), incremental passes (and full
+//                    for fewer than 4096 block pairs), incremental passes (and full
 //                    passes of haloes planned without slots) on the chunked FP32 kernel
 //                    k_pot_f32;
 //   3. k_energy      merges the slots or chunk partials (FP64), updates S and its error

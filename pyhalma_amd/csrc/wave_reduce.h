@@ -11,14 +11,23 @@ __device__ __forceinline__ float dpp_move(float v) {
                                                       true));
 }
 
+// a double from another lane of the row, half by half
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
 // v[0..7] per lane -> the sum over all 64 lanes of v[k], for k = source index of the lane:
 // k = 4*bit5 + 2*bit4 + bit3 of the lane id, valid in the lanes with lane % 8 == 0.
 // A fixed binary tree of depth 6 per total: recursive halving over lane bits 5 and 4 with
 // the CDNA4 half-wave and row swaps (v_permlane32_swap / v_permlane16_swap: each lane
 // ends with its half's pair sum of v[k] or v[k + 4], then of w[k] or w[k + 2]), over
 // bit 3 with a row rotation by 8, then lane + (lane + 4), + (lane + 2), + (lane + 1)
-// within the row (DPP row shifts).
-__device__ __forceinline__ float reduce8(const float v[8], int lane) {
+// within the row (DPP row shifts).  The last three levels, whose roundings no other sum
+// averages out, are FP64: 8 issue slots more per eight sources, and half the error.
+__device__ __forceinline__ double reduce8(const float v[8], int lane) {
     float w[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -34,10 +43,11 @@ __device__ __forceinline__ float reduce8(const float v[8], int lane) {
         u[k] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
     }
     const bool h3 = (lane & 8) != 0;
-    float t = (h3 ? u[1] : u[0]) + dpp_move<0x128>(h3 ? u[0] : u[1]);  // row_ror:8
-    t += dpp_move<0x104>(t);                                           // row_shl:4
-    t += dpp_move<0x102>(t);                                           // row_shl:2
-    t += dpp_move<0x101>(t);                                           // row_shl:1
+    const float w8 = (h3 ? u[1] : u[0]) + dpp_move<0x128>(h3 ? u[0] : u[1]);  // row_ror:8
+    double t = static_cast<double>(w8);
+    t += dpp_move<0x104>(t);  // row_shl:4
+    t += dpp_move<0x102>(t);  // row_shl:2
+    t += dpp_move<0x101>(t);  // row_shl:1
     return t;
 }
 
