@@ -16,21 +16,20 @@ struct Tuning {
 
 extern Tuning g_tuning;
 
-// Rigorous relative error bound of the compensated FP32 sum for subtile SUB:
+// Rigorous relative error bound of the FP32 sums with sub-tiles of SUB terms, u = 2^-24:
 // per term 5.5u (FP32 differences and squares 2.5u after the square root, v_rsq_f32
-// <= 1 ulp = 2u, the mass product u), plain sub-tile sums (SUB-1)u, Kahan 2u, plus
-// FP64 merge and higher-order terms (covered by the extra 0.5u and 1e-11).
+// <= 1 ulp = 2u, the mass product u), the plain sub-tile sum (SUB-1)u, and 0.5u + 1e-11 for
+// the FP64 sums of the sub-tiles, the float pair they are kept in, the merge and the
+// higher-order terms.
 inline double pot_error_bound(int sub) {
     const double u = 5.9604644775390625e-08;  // 2^-24
-    return (sub + 7.0) * u + 1e-11;
+    return (sub + 5.0) * u + 1e-11;
 }
 
-// The symmetric self-potential kernel: test side as above with sub-tiles of 8 terms (a
-// Kahan sum per source tile, the tiles' sums added in FP64 and kept as a float pair:
-// relative error below 1e-15, inside the 0.5u);
-// source side per term 4.5u (differences, squares, v_rsq_f32), the lane's two-term
-// product sum 2u, the 6-level reduction tree across the wave 6u, Kahan 2u, + 0.5u:
-// 15u either way.
+// The symmetric self-potential kernel: test side as above with sub-tiles of 8 terms;
+// source side per term 4.5u (differences, squares, v_rsq_f32), a lane's chain over four
+// tests 4u (the products included), the two chains' sum u, the tree's three FP32 levels 3u,
+// its FP64 levels and the merge 0.5u: 13u either way.
 inline double pot_sym_error_bound() { return pot_error_bound(8); }
 
 }  // namespace halma
