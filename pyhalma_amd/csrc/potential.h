@@ -103,15 +103,6 @@ __device__ __forceinline__ float pair_acc(const float4 s, float xi, float yi, fl
     return __builtin_fmaf(s.w, inv, acc);
 }
 
-// Kahan-compensated addition: c holds the low part lost so far (s + c is the sum; the
-// sequence of s is that of the textbook form, whose compensation is -c)
-__device__ __forceinline__ void kahan_add(float& s, float& c, float v) {
-    const float y = v + c;
-    const float t = s + y;
-    c = y - (t - s);
-    s = t;
-}
-
 __device__ __forceinline__ float min3(float a, float b, float c) { return fminf(fminf(a, b), c); }
 
 // 1 / r of N wave-uniform sources (an even number) from one test per lane, 0 where a

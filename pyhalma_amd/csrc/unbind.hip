@@ -130,9 +130,8 @@ __device__ __forceinline__ bool pass_is_full(int pass_no, int run, int rrun, int
 // bound (the full pass's, plus that of every incremental subtraction since) goes above it
 // is stale.  Its decision is exact (it lies outside the decision band), so it only needs
 // a fresh S: when its halo has few stale members (at most 1/kStaleDiv of the live set)
-// the re-test kernel re-sums them in FP32 with every term Kahan-added (bound 8u =
-// 4.8e-7); otherwise the
-// halo's next pass is a full one (the symmetric kernel recomputes every S), and a halo
+// the re-test kernel re-sums them, FP32 terms added in FP64 (bound 6u = 3.6e-7);
+// otherwise the halo's next pass is a full one (the symmetric kernel recomputes every S), and a halo
 // that removed nobody takes that full pass only to refresh its S (not counted as an
 // iteration: its decisions are exact and do not change).  Both full-pass kernels stay
 // below the limit (halma_pot_error_bound at sub-tiles of 4 or 8, halma_pot_sym_error_bound).
@@ -661,23 +660,23 @@ __device__ void finish_haloes(const EnergyArgs& a, int h) {
 }
 
 // A stale member (kept, outside the decision band: its decision is exact) only needs a
-// fresh S within kPotRelMax: one FP32 sum over its halo's live set with the chunked
-// kernel's term and every term Kahan-added (relative bound pot_error_bound(1), 8u), the
+// fresh S within kPotRelMax: one sum over its halo's live set of the chunked kernel's FP32
+// terms, each added in FP64 (relative bound pot_error_bound(1), 6u), the
 // threads of a wavefront or block in stride over the sources (four loads in flight),
 // merged in FP64.  About five times cheaper per term than the FP64 ordered sum.
 __device__ __forceinline__ double resum_f32_part(const float4* __restrict__ src, int n,
                                                  float4 t, int i0, int step) {
-    float s = 0.0f, c = 0.0f;
+    double s = 0.0;
     int j = i0;
     for (; j + 3 * step < n; j += 4 * step) {
         float4 q[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) q[u] = src[j + u * step];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) kahan_add(s, c, pair_acc(q[u], t.x, t.y, t.z, 0.0f));
+        for (int u = 0; u < 4; ++u) s += static_cast<double>(pair_acc(q[u], t.x, t.y, t.z, 0.0f));
     }
-    for (; j < n; j += step) kahan_add(s, c, pair_acc(src[j], t.x, t.y, t.z, 0.0f));
-    return static_cast<double>(s) + static_cast<double>(c);
+    for (; j < n; j += step) s += static_cast<double>(pair_acc(src[j], t.x, t.y, t.z, 0.0f));
+    return s;
 }
 
 __device__ __forceinline__ double wave_resum_f32(const float4* __restrict__ src, int n, float4 t) {
