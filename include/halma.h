@@ -388,7 +388,8 @@ int halma_progenitors(int64_t n_new, int64_t n_new_members, const int64_t *new_o
  * keeps is within 1e-6 of the FP64 direct sum).  Full passes (first pass, or
  * more than a quarter of the live set removed) go to the symmetric kernel for haloes of
  * at most HALMA_TUNE_SYM_MAX members, to the chunked kernel otherwise; incremental passes
- * go to the chunked kernel.  Passes are queued one ahead of the host: the counters of
+ * go to the chunked kernel; small haloes take the passes after that in a workgroup each,
+ * several per queued pass.  Passes are queued one ahead of the host: the counters of
  * pass p are read back (pinned buffer, event) while pass p + 1 is already queued, so
  * the call ends with one extra pass that finds no active halo.  flags:
  * HALMA_UNBIND_GRAPHS captures each part of a pass (prepare, symmetric kernel, chunked

@@ -36,7 +36,10 @@
 //                    and the decision are the oracle's bit for bit (S and its bound are
 //                    reset to that value); stale members: a fresh FP32 S;
 //   5. k_finish      per-halo pass counts, convergence flags, the removed total (a thread
-//                    per halo).
+//                    per halo);
+//   6. k_halo_tail   the passes that follow, a workgroup per halo, where none of the active
+//                    haloes is large and until a halo's next pass is too much for a
+//                    workgroup.
 // The parts are plain launches (or, on request, hipGraphs captured once and replayed);
 // the host reads one counter per pass to stop.
 #include <math.h>
@@ -58,6 +61,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kIncChunk = 256;      // smallest source chunk of an incremental pass
+constexpr int kCounters = 16;       // words of the counters (EnergyArgs)
 constexpr int kRetestBlock = 2048;  // live sets from this size are re-summed by a block
 
 // member states
@@ -106,9 +110,12 @@ __global__ void k_member_halo(const int64_t* __restrict__ off, int H, int32_t* _
 __global__ void k_init_halo(const int64_t* __restrict__ off, int H, int32_t* __restrict__ active,
                             int32_t* __restrict__ iters, int32_t* __restrict__ removed,
                             int32_t* __restrict__ stale, int32_t* __restrict__ need_full,
-                            int32_t* __restrict__ refresh) {
+                            int32_t* __restrict__ refresh, int32_t* __restrict__ hpass,
+                            int32_t* __restrict__ last_gone) {
     const int h = blockIdx.x * blockDim.x + threadIdx.x;
     if (h >= H) return;
+    hpass[h] = 0;
+    last_gone[h] = 0;
     active[h] = off[h + 1] > off[h] ? 1 : 0;
     iters[h] = 0;
     removed[h] = 0;
@@ -146,6 +153,12 @@ constexpr int kStaleDiv = 32;
 __device__ __forceinline__ bool too_stale(int stale, int live) {
     return kStaleDiv * static_cast<int64_t>(stale) > live;
 }
+
+// k_halo_tail's workgroup, and the most it takes on (see there)
+constexpr int kTailThreads = 512;
+constexpr int kTailLive = 4096;         // live members
+constexpr int64_t kTailPairs = 1 << 20;  // pairs of an incremental pass
+constexpr int64_t kTailFull = 1 << 19;   // pairs of a full pass
 
 // band-list entries of stale members carry this bit (members of the decision band do not)
 constexpr uint32_t kStaleBit = 0x80000000u;
@@ -296,6 +309,8 @@ __global__ __launch_bounds__(kThreads) void k_halo_sets(
     if (pos == 0 && lane == 0) {
         counters[0] = 0;
         counters[5] = 0;
+        counters[9] = 0;
+        counters[11] = 0;
     }
     if (pos >= H) return;  // wave-uniform
     const int h = order[pos];
@@ -467,6 +482,7 @@ struct EnergyArgs {
     const float2* sym_part;
     const double* vel;
     const double* vcm;
+    double* vcm_out;   // the same array (k_halo_tail)
     double cg;         // factor * G
     double bound_rel;  // FP32 relative error bound B of one pair sum (incremental passes)
     double bound_sym;  // the same for the symmetric kernel (full passes)
@@ -484,7 +500,9 @@ struct EnergyArgs {
                                    // [3] pairs, [4] symmetric-kernel pairs, [5] haloes
                                    // still active after the pass, [6] members re-summed
                                    // for their error bound alone, [8] the band
-                                   // count of large live sets
+                                   // count of large live sets, [9] haloes still active
+                                   // after k_halo_tail, [10] most passes of a halo, [11] active
+                                   // haloes of more than kTailLive members
     double* s_out;     // optional: S per member position (FP64)
     int64_t nm;
     // the end of a pass (k_finish)
@@ -492,6 +510,9 @@ struct EnergyArgs {
     int32_t* active;
     int32_t* iters;
     int32_t* pass_no;
+    int32_t* hpass;      // per halo: passes taken
+    int32_t* last_gone;  // per halo: members removed by its last pass
+    int max_iter;
 };
 
 __device__ __forceinline__ double kinetic(const double* vel, int64_t k, const double* vc) {
@@ -627,6 +648,8 @@ __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v)
 // symmetric kernel's passes, [5] haloes still active.
 __device__ void finish_haloes(const EnergyArgs& a, int h) {
     unsigned long long rem = 0, pairs = 0, full_pairs = 0, live = 0;
+    int most = 0;
+    unsigned long long large = 0;
     if (h < a.H && a.active[h]) {
         const int nb = a.n_bound[h];
         const int r = a.removed[h];
@@ -642,20 +665,29 @@ __device__ void finish_haloes(const EnergyArgs& a, int h) {
         a.need_full[h] = redo ? 1 : 0;
         const bool refresh = !stay && redo && !refreshing;
         a.refresh[h] = refresh ? 1 : 0;
-        if (!stay && !refresh) a.active[h] = 0;
-        live = (stay || refresh) ? 1 : 0;
+        const int passes = a.hpass[h] + 1;
+        a.hpass[h] = passes;
+        a.last_gone[h] = r;
+        live = (stay || refresh) && passes < a.max_iter ? 1 : 0;
+        if (!live) a.active[h] = 0;
         rem = static_cast<unsigned long long>(r);
         a.removed[h] = 0;
+        most = passes;
+        large = live && nb > kTailLive ? 1 : 0;
     }
+    for (int o = kWave / 2; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o, kWave));
     rem = wave_sum_u64(rem);
     pairs = wave_sum_u64(pairs);
     full_pairs = wave_sum_u64(full_pairs);
     live = wave_sum_u64(live);
+    large = wave_sum_u64(large);
     if ((threadIdx.x & (kWave - 1)) == 0) {
         if (rem) atomicAdd(a.counters + 0, rem);
         if (pairs) atomicAdd(a.counters + 3, pairs);
         if (full_pairs) atomicAdd(a.counters + 4, full_pairs);
         if (live) atomicAdd(a.counters + 5, live);
+        if (most) atomicMax(a.counters + 10, static_cast<unsigned long long>(most));
+        if (large) atomicAdd(a.counters + 11, large);
     }
 }
 
@@ -783,6 +815,248 @@ __global__ __launch_bounds__(kThreads) void k_finish(EnergyArgs a) {
         a.counters[8] = 0;
         *a.pass_no += 1;
     }
+}
+
+// The passes that follow a launched one, halo by halo: a workgroup takes an active halo
+// through pass after pass (compaction, v_cm, the removed members' terms, decisions,
+// re-tests, the end of the pass -- the steps of the launched passes with the same terms,
+// rules and orders of the exact sums) until the halo is done or its next pass is too much
+// for one workgroup; that one is left, untouched, to the next launched pass.  A launched
+// pass is nine kernels, most of them waiting for the one before; here a pass of a few
+// thousand members is about 10 us of a compute unit's latency, and the haloes run
+// through theirs independently: 2000 bridged pairs of 2000 members (up to 46 passes) go
+// from 47 launched passes to 6, 7.6 -> 4.5 ms.  While a halo of more than kTailLive
+// members is active, launched passes go on anyway and the small haloes ride along: then
+// nothing is done here (the clump step, its largest haloes at 20000 members and 8 passes,
+// 4.55 ms; with this kernel after every launched pass 4.67).  512 threads: 1024 take
+// 5.8 ms on the pairs, 256 5.2.
+constexpr int kTailRem = 736;            // removed members: at most half the live ones in an
+                                         // incremental pass, so fewer than sqrt(kTailPairs / 2)
+static_assert(2 * int64_t(kTailRem) * kTailRem > kTailPairs, "removed members of a pass");
+
+struct TailShared {
+    float4 rem[kTailRem];
+    double dd[kTailThreads / kWave][8];
+    double vcm[3];
+    int scan[kTailThreads / kWave];
+    int n_gone, n_stale, n_list;
+};
+
+// sum of the sources' terms at one test per lane, in sub-tiles of four added in FP64 (the
+// chunked kernel's sum, bound pot_error_bound(4)); every lane of the wavefront takes part
+__device__ __forceinline__ double tail_sum(const float4* src, int n, float4 t) {
+    double S = 0.0;
+    int j = 0;
+    for (; j + 4 <= n; j += 4) {
+        float4 q[4];
+        float v[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) q[s] = src[j + s];
+        inv_r_group<4>(q, t.x, t.y, t.z, v);
+        float ps = q[0].w * v[0];
+#pragma unroll
+        for (int s = 1; s < 4; ++s) ps = __builtin_fmaf(q[s].w, v[s], ps);
+        S += static_cast<double>(ps);
+    }
+    for (; j < n; ++j) S += static_cast<double>(pair_acc(src[j], t.x, t.y, t.z, 0.0f));
+    return S;
+}
+
+__global__ __launch_bounds__(kTailThreads, 4) void k_halo_tail(
+    EnergyArgs a, const int32_t* __restrict__ order, const int64_t* __restrict__ off,
+    const double* __restrict__ m64, float4* src4, int32_t* cidx) {
+    __shared__ TailShared sh;
+    const int h = order[blockIdx.x];
+    if (!a.active[h]) return;
+    if (a.counters[11] != 0) {  // launched passes go on anyway
+        if (threadIdx.x == 0) atomicAdd(a.counters + 9, 1ull);
+        return;
+    }
+    const int lane = __lane_id();
+    const int tid = static_cast<int>(threadIdx.x);
+    const int wv = tid / kWave;
+    const int64_t o = off[h];
+    float4* live = src4 + o;   // the live set, in member order
+    int32_t* idx = cidx + o;   // its member positions
+    int32_t* list = a.band + o;
+    int n = a.n_bound[h];      // entries of the set: live ones and those just removed
+    int gone = a.last_gone[h];
+    int need_full = a.need_full[h], refresh = a.refresh[h];
+    int passes = a.hpass[h], iters = a.iters[h];
+    bool on = true;
+    unsigned long long pairs = 0, n_retest = 0, n_resum = 0;
+    while (on) {
+        const int run = n - gone;
+        const bool full = pass_is_full(1, run, gone, need_full);
+        if (n > kTailLive ||
+            static_cast<int64_t>(run) * (full ? run : gone) > (full ? kTailFull : kTailPairs))
+            break;
+        // compaction in place (a round's entries are read before any is written, and land
+        // at or before their own places), masses and momenta of the kept
+        double acc[4][2] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+        int kept = 0, rem = 0;
+        for (int base = 0; base < n; base += kTailThreads) {
+            const int i = base + tid;
+            const bool in = i < n;
+            const int k = in ? idx[i] : 0;
+            const float4 p = in ? live[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            const uint8_t st = in ? a.state[k] : kGone;
+            const double m = st == kBound ? m64[k] : 0.0;
+            double v[3];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) v[d] = st == kBound ? a.vel[3 * static_cast<int64_t>(k) + d] : 0.0;
+            const int f = st == kBound ? 1 : (st == kJustGone ? (1 << 16) : 0);
+            int x = f;
+            for (int s = 1; s < kWave; s <<= 1) {
+                const int y = __shfl_up(x, s, kWave);
+                if (lane >= s) x += y;
+            }
+            if (lane == kWave - 1) sh.scan[wv] = x;
+            __syncthreads();
+            int before = x - f, tot = 0;
+#pragma unroll
+            for (int q = 0; q < kTailThreads / kWave; ++q) {
+                if (q < wv) before += sh.scan[q];
+                tot += sh.scan[q];
+            }
+            if (st == kBound) {
+                const int at = kept + (before & 0xffff);
+                live[at] = p;
+                idx[at] = k;
+                dd_add(acc[0][0], acc[0][1], m);
+#pragma unroll
+                for (int d = 0; d < 3; ++d) dd_add(acc[1 + d][0], acc[1 + d][1], m * v[d]);
+            } else if (st == kJustGone) {
+                const int at = rem + (before >> 16);
+                if (at < kTailRem) sh.rem[at] = p;  // read in an incremental pass only
+                a.state[k] = kGone;
+            }
+            kept += tot & 0xffff;
+            rem += tot >> 16;
+            __syncthreads();  // the scan array is free again
+        }
+        for (int m = kWave / 2; m >= 1; m >>= 1)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const double h2 = __shfl_xor(acc[q][0], m, kWave);
+                const double l2 = __shfl_xor(acc[q][1], m, kWave);
+                dd_add_dd(acc[q][0], acc[q][1], h2, l2);
+            }
+        if (lane == 0)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                sh.dd[wv][2 * q] = acc[q][0];
+                sh.dd[wv][2 * q + 1] = acc[q][1];
+            }
+        __syncthreads();
+        if (tid == 0) {
+            double s[4][2] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+            for (int w = 0; w < kTailThreads / kWave; ++w)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    dd_add_dd(s[q][0], s[q][1], sh.dd[w][2 * q], sh.dd[w][2 * q + 1]);
+            const double M = s[0][0] + s[0][1];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) sh.vcm[d] = M > 0.0 ? (s[1 + d][0] + s[1 + d][1]) / M : 0.0;
+            sh.n_gone = sh.n_stale = sh.n_list = 0;
+        }
+        __syncthreads();
+        const double vc[3] = {sh.vcm[0], sh.vcm[1], sh.vcm[2]};
+        // S and the decisions outside the band, a member per lane
+        const int ns = full ? kept : rem;
+        for (int i0 = wv * kWave; i0 < kept; i0 += kTailThreads) {
+            const int i = min(i0 + lane, kept - 1);
+            const int64_t k = idx[i];
+            const double s_old = full ? 0.0 : a.sacc[k], e_old = full ? 0.0 : a.eacc[k];
+            const double kin = kinetic(a.vel, k, vc);
+            const float4 t = live[i];
+            const double sum = full ? tail_sum(live, ns, t) : tail_sum(sh.rem, ns, t);
+            const double S = full ? sum : s_old - sum;
+            const double err = e_old + a.bound_rel * sum;
+            const double pot = a.cg * S;
+            const double E = kin - pot;
+            const double band = a.cg * err * 1.01 + 8.0 * 0x1p-53 * (kin + fabs(pot)) +
+                                1e-10 * fabs(pot);
+            const bool in = i0 + lane < kept;
+            const bool in_band = in && fabs(E) <= band;
+            const bool out = in && !in_band && E > 0.0;
+            const bool stale = in && !out && !in_band && err > kPotRelMax * S;
+            if (in) {
+                a.sacc[k] = S;
+                a.eacc[k] = err;
+                if (a.s_out) a.s_out[k] = S;
+            }
+            if (out) a.state[k] = kJustGone;
+            const unsigned long long m_out = __ballot(out), m_st = __ballot(stale);
+            const unsigned long long m_list = __ballot(in_band || stale);
+            int at = 0;
+            if (lane == 0) {
+                if (m_out) atomicAdd(&sh.n_gone, __popcll(m_out));
+                if (m_st) atomicAdd(&sh.n_stale, __popcll(m_st));
+                if (m_list) at = atomicAdd(&sh.n_list, __popcll(m_list));
+            }
+            at = __shfl(at, 0, kWave);
+            const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+            if (in_band || stale)
+                list[at + __popcll(m_list & below)] =
+                    static_cast<int32_t>(static_cast<uint32_t>(i) | (stale ? kStaleBit : 0u));
+        }
+        __syncthreads();
+        // band members: the oracle's sum and decision; stale ones, when few, a fresh S
+        const int n_list = sh.n_list, n_stale = sh.n_stale;
+        const bool resum = !too_stale(n_stale, kept);
+        for (int e = wv; e < n_list; e += kTailThreads / kWave) {
+            const uint32_t entry = static_cast<uint32_t>(list[e]);
+            const int i = static_cast<int>(entry & ~kStaleBit);
+            const bool stale = (entry & kStaleBit) != 0;
+            if (stale && !resum) continue;
+            const float4 t = live[i];
+            const int64_t k = idx[i];
+            const double S = stale ? wave_resum_f32(live, kept, t)
+                                   : wave_pot_f64_ordered(SrcAoS{live}, kept, t.x, t.y, t.z);
+            if (lane == 0) {
+                a.sacc[k] = S;
+                a.eacc[k] = (stale ? a.bound_resum : 1e-12) * S;
+                if (a.s_out) a.s_out[k] = S;
+                if (!stale && kinetic(a.vel, k, vc) - a.cg * S > 0.0) {
+                    a.state[k] = kJustGone;
+                    atomicAdd(&sh.n_gone, 1);
+                }
+                ++n_retest;
+                if (stale) ++n_resum;
+            }
+        }
+        __syncthreads();
+        // the end of the pass, as finish_haloes
+        n = kept;
+        gone = sh.n_gone;
+        if (n > 0) {
+            if (!(refresh && gone == 0)) iters += 1;
+            pairs += static_cast<unsigned long long>(n) * static_cast<unsigned long long>(ns);
+        }
+        passes += 1;
+        const bool stay = gone > 0 && n > 0;
+        const bool redo = n > 0 && too_stale(n_stale, n);
+        need_full = redo ? 1 : 0;
+        refresh = !stay && redo && !refresh ? 1 : 0;
+        on = (stay || refresh) && passes < a.max_iter;
+        if (tid == 0)
+#pragma unroll
+            for (int d = 0; d < 3; ++d) a.vcm_out[3 * h + d] = vc[d];
+        __syncthreads();  // the counters have been read
+        if (!on && tid == 0) a.active[h] = 0;
+    }
+    if (tid == 0) {
+        a.need_full[h] = need_full;
+        a.refresh[h] = refresh;
+        a.hpass[h] = passes;
+        a.iters[h] = iters;
+        if (pairs) atomicAdd(a.counters + 3, pairs);
+        if (on) atomicAdd(a.counters + 9, 1ull);
+        atomicMax(a.counters + 10, static_cast<unsigned long long>(passes));
+    }
+    if (n_retest) atomicAdd(a.counters + 2, n_retest);
+    if (n_resum) atomicAdd(a.counters + 6, n_resum);
 }
 
 // The pass's item list: the items of the haloes with live work, in the plan's halo
@@ -967,6 +1241,8 @@ struct UnbWs {
     int32_t* stale;
     int32_t* need_full;
     int32_t* refresh;
+    int32_t* hpass;
+    int32_t* last_gone;
     int32_t* pass_no;
     double* vcm;
     int32_t* band;
@@ -1061,10 +1337,12 @@ UnbWs carve_unb(void* base, int64_t H, int64_t nm, const PotPlan& plan, const Sy
     w.stale = c.take<int32_t>(h1);
     w.need_full = c.take<int32_t>(h1);
     w.refresh = c.take<int32_t>(h1);
+    w.hpass = c.take<int32_t>(h1);
+    w.last_gone = c.take<int32_t>(h1);
     w.pass_no = c.take<int32_t>(64);
     w.vcm = c.take<double>(3 * h1);
     w.band = c.take<int32_t>(n1);
-    w.counters = c.take<unsigned long long>(16);
+    w.counters = c.take<unsigned long long>(kCounters);
     w.items = c.take<int4>(std::max<int64_t>(plan.n_items, 1));
     w.icnt = c.take<int64_t>(h1);
     w.ioff = c.take<int64_t>(h1);
@@ -1307,9 +1585,10 @@ int unbind_run(int64_t H, const int64_t* h_off, const int32_t* members, Inputs i
         HALMA_LAUNCH_CHECK();
     }
     k_init_halo<<<blocks_for(H), kThreads, 0, st>>>(w.off, static_cast<int>(H), w.active, w.iters,
-                                                    w.removed, w.stale, w.need_full, w.refresh);
+                                                    w.removed, w.stale, w.need_full, w.refresh, w.hpass,
+                                                    w.last_gone);
     HALMA_LAUNCH_CHECK();
-    k_zero_counters<<<1, 64, 0, st>>>(w.counters, 16);
+    k_zero_counters<<<1, 64, 0, st>>>(w.counters, kCounters);
     HALMA_LAUNCH_CHECK();
     k_zero_counters<<<1, 64, 0, st>>>(reinterpret_cast<unsigned long long*>(w.pass_no), 1);
     HALMA_LAUNCH_CHECK();
@@ -1347,6 +1626,7 @@ int unbind_run(int64_t H, const int64_t* h_off, const int32_t* members, Inputs i
     L.ea.sym_part = w.sym_part;
     L.ea.vel = w.vel;
     L.ea.vcm = w.vcm;
+    L.ea.vcm_out = w.vcm;
     L.ea.cg = factor * G;
     L.ea.bound_rel = pot_error_bound(plan.subtile);
     L.ea.bound_sym = pot_sym_error_bound();
@@ -1367,14 +1647,18 @@ int unbind_run(int64_t H, const int64_t* h_off, const int32_t* members, Inputs i
     L.ea.active = w.active;
     L.ea.iters = w.iters;
     L.ea.pass_no = w.pass_no;
+    L.ea.hpass = w.hpass;
+    L.ea.last_gone = w.last_gone;
+    L.ea.max_iter = max_iter;
 
     const bool use_graph = (flags & HALMA_UNBIND_GRAPHS) != 0;
     const bool timing = (flags & HALMA_UNBIND_TIME_POT) != 0;
-    // Passes are launched one ahead of the host: pass p + 1 is queued before pass p's
-    // counters are read, so the GPU never waits for the host between passes.  Pass p's
-    // counters go to slot p % 2 of a pinned buffer, with slot events; when pass p removes
-    // nobody, the queued pass p + 1 finds no active halo and does nothing.
-    hipEvent_t ev[2][3] = {{nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}};
+    // A round is a launched pass of every active halo, then k_halo_tail for the passes that
+    // a workgroup can take.  Rounds are launched one ahead of the host: round p + 1 is
+    // queued before round p's counters are read, so the GPU never waits for the host
+    // between them.  Round p's counters go to slot p % 2 of a pinned buffer, with slot
+    // events; when round p leaves no halo active, the queued round does nothing.
+    hipEvent_t ev[2][5] = {};
     hipEvent_t done[2] = {nullptr, nullptr};
     for (auto& d : done) HALMA_HIP(hipEventCreateWithFlags(&d, hipEventDisableTiming));
     if (timing)
@@ -1419,7 +1703,7 @@ int unbind_run(int64_t H, const int64_t* h_off, const int32_t* members, Inputs i
         }
         return parts[q](L, st);
     };
-    long long* host = pinned_words(16);
+    long long* host = pinned_words(2 * kCounters);
     if (!host) {
         cleanup();
         return set_error(HALMA_E_STATE, "pinned host buffer unavailable");
@@ -1429,7 +1713,7 @@ int unbind_run(int64_t H, const int64_t* h_off, const int32_t* members, Inputs i
                    ? 0
                    : set_error(HALMA_E_STATE, "event record failed");
     };
-    auto launch_pass = [&](int p) -> int {
+    auto launch_round = [&](int p) -> int {
         const int q = p & 1;
         int r = run_part(0);
         if (!r && timing) r = record(ev[q][0]);
@@ -1438,13 +1722,20 @@ int unbind_run(int64_t H, const int64_t* h_off, const int32_t* members, Inputs i
         if (!r) r = run_part(2);
         if (!r && timing) r = record(ev[q][2]);
         if (!r) r = run_part(3);
+        if (!r && timing) r = record(ev[q][3]);
         if (r) return r;
-        const hipError_t e = hipMemcpyAsync(host + 8 * q, w.counters, 7 * sizeof(long long),
+        k_halo_tail<<<static_cast<unsigned>(H), kTailThreads, 0, st>>>(L.ea, w.order, w.off,
+                                                                       w.m64, w.src4, w.cidx);
+        HALMA_LAUNCH_CHECK();
+        if (timing) r = record(ev[q][4]);
+        if (r) return r;
+        const hipError_t e = hipMemcpyAsync(host + kCounters * q, w.counters,
+                                            kCounters * sizeof(long long),
                                             hipMemcpyDeviceToHost, st);
         if (e != hipSuccess) return hip_fail(e, "counter read-back", __FILE__, __LINE__);
         return record(done[q]);
     };
-    // waits for pass p and adds its pair-kernel times
+    // waits for the round and adds its pair-kernel times (k_halo_tail counted whole)
     auto collect = [&](int p) -> int {
         const int q = p & 1;
         const hipError_t e = hipEventSynchronize(done[q]);
@@ -1452,37 +1743,38 @@ int unbind_run(int64_t H, const int64_t* h_off, const int32_t* members, Inputs i
         sym_launches += 1;
         f32_launches += 1;
         if (timing) {
-            float ms_all = 0.0f, ms_sym = 0.0f;
+            float ms_all = 0.0f, ms_sym = 0.0f, ms_tail = 0.0f;
             hipError_t e4 = hipEventElapsedTime(&ms_all, ev[q][0], ev[q][2]);
             if (e4 == hipSuccess) e4 = hipEventElapsedTime(&ms_sym, ev[q][0], ev[q][1]);
+            if (e4 == hipSuccess) e4 = hipEventElapsedTime(&ms_tail, ev[q][3], ev[q][4]);
             if (e4 != hipSuccess) return hip_fail(e4, "pair-kernel timing", __FILE__, __LINE__);
-            pot_ms += ms_all;
+            pot_ms += ms_all + ms_tail;
             sym_ms += ms_sym;
             ++pot_launches;
         }
         return 0;
     };
-    int passes = 0, launched = 0;
-    long long band_total = 0;
+    std::fill(host, host + 2 * kCounters, 0ll);
+    // every launched pass takes each active halo a pass further, so max_iter rounds do
     const long long* last = host;
-    int status = max_iter > 0 ? launch_pass(0) : 0;
+    int rounds = 0, launched = 0;
+    int status = max_iter > 0 ? launch_round(0) : 0;
     if (max_iter > 0) launched = 1;
-    while (!status && passes < launched) {
-        const int p = passes;
+    while (!status && rounds < launched) {
+        const int p = rounds;
         if (launched < max_iter) {
-            status = launch_pass(launched);
+            status = launch_round(launched);
             if (status) break;
             ++launched;
         }
         status = collect(p);
         if (status) break;
-        last = host + 8 * (p & 1);
-        band_total = last[2];
-        passes = p + 1;
-        if (last[5] == 0) break;  // converged: a queued pass, if any, does nothing
+        last = host + kCounters * (p & 1);
+        rounds = p + 1;
+        if (last[9] == 0) break;  // no halo left: a queued round, if any, does nothing
     }
-    // the queued pass after convergence: its (empty) kernels are counted like the others
-    if (!status && launched > passes) status = collect(passes);
+    // the queued round after convergence: its (empty) kernels are counted like the others
+    if (!status && launched > rounds) status = collect(rounds);
     cleanup();
     if (status) return status;
     if (nm > 0) {
@@ -1494,8 +1786,8 @@ int unbind_run(int64_t H, const int64_t* h_off, const int32_t* members, Inputs i
     if (vcm_out) HALMA_HIP(hipMemcpyAsync(vcm_out, w.vcm, 3 * H * sizeof(double),
                                           hipMemcpyDeviceToDevice, st));
     if (stats) {
-        stats[0] = passes;
-        stats[1] = band_total;
+        stats[0] = last[10];
+        stats[1] = last[2];
         stats[2] = splan.n_items;
         stats[3] = plan.tests_per_lane;
         stats[4] = plan.subtile;
