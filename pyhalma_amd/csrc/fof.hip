@@ -13,18 +13,18 @@
 //    consecutive and ordered by z, columns are in (x, y) order, particles ascending within
 //    a cell; coordinates are gathered into that order as one vector per particle, each
 //    cell is one 8-byte record
-//    (first position, z), and each column enters a hash table whose 16-byte entry holds
-//    its key, cell count, first cell and (between the rounds) shared root, so that a
-//    neighbour column costs one line; the table is sized from the column count;
-// 4. links, in two rounds (Chebyshev distance 1, then 2), one lane per (segment of up to
-//    4 cells of a column, neighbour column): the half-stencil's 12 columns (dx > 0, or
-//    dx = 0 and dy > 0) and the column itself (cells above); one table probe finds the
-//    neighbour column, then the two z-ordered cell lists are merged for the cell pairs
-//    within the round's dz.  Pairs
-//    of cells with at most 8 particle pairs are tested at once (roots are looked up only
-//    for a link); larger ones already joined are skipped, the rest tested by the lane or,
+//    (first position, z), and each column one 16-byte record (key, cell count, first cell,
+//    and between the rounds its shared root).  The columns are sorted by (x, y), so the
+//    neighbour columns of a row x + 1 or x + 2 are adjacent records: one search per column
+//    and row finds the first, and a bit per neighbour tells which of them exist;
+// 4. links between cells of one stretch of consecutive cells, a workgroup per stretch with
+//    its forest in LDS (k_fof_local); then those between stretches in two rounds (Chebyshev
+//    distance 1, then 2), one lane per (segment of up to 4 cells of a column, neighbour
+//    column of the half stencil's 12, or the column itself): the two z-ordered cell lists
+//    are merged, as records that hold each cell's root before the round, so that a joined
+//    pair costs one sequential load.  Pairs of cells not joined are tested by the lane or,
 //    beyond 64 particle pairs, listed for one wavefront each (64 lanes over the larger
-//    cell, early exit); linked cells are joined in a lock-free union-find over cells (the
+//    cell, early exit).  Linked cells are joined in a lock-free union-find over cells (the
 //    larger root index is hooked under the smaller, so parents only decrease and no cycle
 //    can form; finds halve paths);
 // 5. roots are read back with atomic reads (see k_roots), each component's minimum
@@ -43,7 +43,6 @@ namespace halma {
 
 namespace {
 
-constexpr uint64_t kEmpty = ~0ull;
 constexpr double kCellLimit = 2097152.0;  // 2^21 cells per axis
 constexpr int kBoxBlocks = 1024;
 
@@ -52,35 +51,34 @@ constexpr int kBoxBlocks = 1024;
 constexpr int kKeyBits = 42;
 constexpr uint64_t kKeyMask = (uint64_t{1} << kKeyBits) - 1;
 
-// 16-byte column table entry, everything a lane needs of a neighbour column in one line:
-// the word (kEmpty when free), the first cell, and between the rounds the root shared by
-// all its cells (-1 when they differ)
+// A column's record, everything a lane needs of a neighbour column in one vector: the word,
+// the first cell, and between the rounds the root shared by all its cells (-1 when they
+// differ).  Records are in (x, y) order.
 struct __attribute__((aligned(16))) ColEntry {
     uint64_t word;
     int32_t c0;
     int32_t root;
 };
 
+// Where a column's neighbours are: the first record of row x + 1 and of row x + 2 from
+// y - 2 on, and which neighbours exist (bits 0-1: (0, 1), (0, 2); bits 2-6: row x + 1,
+// dy = -2 .. 2; bits 7-11: row x + 2); last: the last cell of the column and its neighbours.
+struct __attribute__((aligned(16))) ColNeigh {
+    int32_t row1, row2;
+    uint32_t mask;
+    int32_t last;
+};
+
 // A column segment in link-lane order: its word (the column's key in the low bits, the
 // segment's cell count above them, then how many cells of the column follow the segment,
-// at most 2: all that an own-column pair can reach), its first cell and the column's
-// table slot
+// at most 2: all that an own-column pair can reach), its first cell and the column
 struct __attribute__((aligned(16))) ColRec {
     uint64_t word;
     int32_t c0;
-    int32_t slot;
+    int32_t col;
 };
 constexpr int kSegLenShift = kKeyBits;       // 10 bits
 constexpr int kSegMoreShift = kKeyBits + 10;  // 2 bits
-
-__device__ __forceinline__ uint64_t mix64(uint64_t k) {
-    k ^= k >> 30;
-    k *= 0xbf58476d1ce4e5b9ull;
-    k ^= k >> 27;
-    k *= 0x94d049bb133111ebull;
-    k ^= k >> 31;
-    return k;
-}
 
 template <typename T>
 __device__ __forceinline__ int ld_relaxed(const T* p) {
@@ -291,34 +289,14 @@ __global__ void k_fof_heads(const uint64_t* __restrict__ skey, int64_t n, uint64
     heads[j] = cell | (col << 32);
 }
 
-// the column table's size from the column count (power of two >= 2 columns, >= 1024,
-// <= cap), kept as its mask in totals[1]; then cleared
-__global__ void k_col_table_size(int64_t* __restrict__ totals, int64_t cap) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    const int64_t ncol = totals[0] >> 32;
-    int64_t c = 1024;
-    while (c < 2 * ncol && c < cap) c <<= 1;
-    totals[1] = c - 1;
-}
-
-__global__ void k_clear_cols(const int64_t* __restrict__ totals, ColEntry* __restrict__ tab) {
-    const int64_t m = totals[1] + 1;
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < m;
-         i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-        tab[i].word = kEmpty;
-        tab[i].c0 = -1;
-        tab[i].root = -1;
-    }
-}
-
 // Cells and columns from the sorted keys.  Cell c: its record (first sorted position,
 // z = key mod nz), its smallest particle index (the sort is stable, so the first one),
-// the union-find root; column q: its first cell and its packed key (x << by | y, from
-// key / nz = x * ny + y).
+// its column; column q: its first cell and its packed key (x << by | y, from
+// key / nz = x * ny + y).  The forest starts in k_fof_local.
 __global__ __launch_bounds__(256) void k_fof_cells(
     const uint64_t* __restrict__ skey, const int32_t* __restrict__ perm,
     const int64_t* __restrict__ heads, const int64_t* __restrict__ before, int64_t n, Grid g,
-    int2* __restrict__ crec, int* __restrict__ cell_min, int* __restrict__ parent,
+    int2* __restrict__ crec, int* __restrict__ cell_min, int* __restrict__ cell_col,
     int* __restrict__ comp_min, int* __restrict__ col_cell, uint64_t* __restrict__ col_key) {
     const int64_t j = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (j >= n) return;
@@ -330,7 +308,7 @@ __global__ __launch_bounds__(256) void k_fof_cells(
     if (h & 0xffffffff) {
         crec[c] = make_int2(static_cast<int>(j), static_cast<int>(k - ck * g.n[2]));
         cell_min[c] = perm[j];
-        parent[c] = c;
+        cell_col[c] = q;
         comp_min[c] = INT32_MAX;
     }
     if (h >> 32) {
@@ -342,23 +320,6 @@ __global__ __launch_bounds__(256) void k_fof_cells(
         crec[c + 1] = make_int2(static_cast<int>(n), INT32_MAX);
         col_cell[q + 1] = c + 1;
     }
-}
-
-// The table entry of a column key, or an entry whose word is kEmpty when the column has
-// no cells.  Every word is final before the link kernels run.
-__device__ __forceinline__ ColEntry col_find(const ColEntry* __restrict__ tab, uint64_t mask,
-                                             uint64_t key) {
-    uint64_t s = mix64(key) & mask;
-    for (uint64_t probe = 0; probe <= mask; ++probe) {
-        const ColEntry e = tab[s];
-        if (e.word == kEmpty || (e.word & kKeyMask) == key) return e;
-        s = (s + 1) & mask;
-    }
-    ColEntry e;
-    e.word = kEmpty;
-    e.c0 = -1;
-    e.root = -1;
-    return e;
 }
 
 // Read-only find with plain loads, for the "already joined?" test before a pair search.
@@ -379,22 +340,37 @@ __device__ __forceinline__ bool within(const V& a, const V& b, double ll2) {
     return (dx * dx + dy * dy) + dz * dz <= ll2;
 }
 
-// Every cell pointed straight at its root (between the candidate passes, when no union
-// runs): the read-only root checks of the next pass then take one or two steps instead
-// of walking the chains that hooking by index builds in dense regions.  Concurrent
+// Every cell pointed straight at its root (between the rounds, when no union runs), and
+// the cells' records for the next round: {first position, z, end position, root}.  Concurrent
 // writers store each cell's own root, so a reader sees either its old parent or the root.
-__global__ void k_flatten(const int64_t* __restrict__ totals, int* __restrict__ parent) {
+__global__ void k_flatten(const int64_t* __restrict__ totals, int* __restrict__ parent,
+                          const int2* __restrict__ crec, int4* __restrict__ frec) {
     const int64_t ncell = totals[0] & 0xffffffff;
     for (int64_t c = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; c < ncell;
          c += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+        const int2 r0 = crec[c];
+        const int end = crec[c + 1].x;
         int r = static_cast<int>(c);
         for (int p = parent[r]; p != r; p = parent[r]) r = p;
         parent[c] = r;
+        frec[c] = make_int4(r0.x, r0.y, end, r);
     }
 }
 
+// Stretches: runs of consecutive cells, one workgroup of k_fof_local each.  Cells are in
+// (x, y, z) order, so a stretch of kStretchMax holds a few dozen rows of columns of a
+// clustered catalogue and most links of its cells; smaller catalogues are cut finer, down
+// to kStretchMin, so that every compute unit has a stretch.
+constexpr int kStretchMax = 2048;
+constexpr int kStretchMin = 256;
 
-// Link lanes: a column of more than kSegMin cells is cut into segments of kSegCells
+__device__ __forceinline__ int stretch_cells(int64_t ncell) {
+    const int64_t s = (ncell / 1024 + 63) & ~int64_t{63};
+    return static_cast<int>(s < kStretchMin ? kStretchMin : (s > kStretchMax ? kStretchMax : s));
+}
+
+// The link lanes of the rounds between stretches: the segments with a neighbour in another
+// stretch.  A column of more than kSegMin cells is cut into segments of kSegCells
 // cells, and each segment takes its own lanes (a long column's cells are then linked by
 // several lanes at once instead of one long chain of finds and unions).  Lane order:
 // segments grouped by the log2 of their particle count, largest first, so that the lanes
@@ -405,6 +381,7 @@ __global__ void k_flatten(const int64_t* __restrict__ totals, int* __restrict__ 
 // not fixed; the links do not depend on it).
 constexpr int kColClasses = 8;
 constexpr int kClassBlocks = 256;
+constexpr int kBigLists = 3;  // fillings of the list of large pairs: local, cross 1, cross 2
 constexpr int kSegMin = 4;
 constexpr int kSegCells = 4;
 static_assert(kSegCells < 1024 && kSegMin < 1024, "a segment's cell count has 10 bits");
@@ -419,46 +396,89 @@ __device__ __forceinline__ int seg_class(const int2* __restrict__ crec, int c0, 
     return lg < kColClasses - 1 ? lg : kColClasses - 1;
 }
 
-// counts[0..7]: segments per class; counts[8..15]: the class cursors (zero here).  Also
-// enters each column in the table (word, first cell) and keeps its slot.
+// first column from `from` on whose key is at least `key`
+__device__ __forceinline__ int64_t col_lower(const uint64_t* __restrict__ col_key, int64_t from,
+                                             int64_t ncol, uint64_t key) {
+    int64_t lo = from, hi = ncol;
+    while (lo < hi) {
+        const int64_t mid = (lo + hi) >> 1;
+        if (col_key[mid] < key) lo = mid + 1;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// Each column's record and where its neighbours are.  The lanes of a wavefront hold
+// consecutive columns and search nearly the same places, so the searches run in the
+// caches: 2.6M columns (8M bridged stars) take 120 us; entered into a hash table (one
+// compare-and-swap per column, then a probe of a line of its own per neighbour) 0.32 ms
+// and most of the link rounds' misses.
+__global__ __launch_bounds__(256) void k_col_neigh(const int64_t* __restrict__ totals,
+                                                   const int* __restrict__ col_cell,
+                                                   const uint64_t* __restrict__ col_key, int by,
+                                                   ColEntry* __restrict__ cols,
+                                                   ColNeigh* __restrict__ neigh) {
+    const int64_t ncol = totals[0] >> 32;
+    const uint64_t ymask = (uint64_t{1} << by) - 1;
+    for (int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; q < ncol;
+         q += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+        const uint64_t key = col_key[q];
+        const int a0 = col_cell[q], a1 = col_cell[q + 1];
+        ColEntry e;
+        e.word = key | (static_cast<uint64_t>(a1 - a0) << kKeyBits);
+        e.c0 = a0;
+        e.root = -1;
+        cols[q] = e;
+        const uint64_t x = key >> by, y = key & ymask;
+        const uint64_t ylo = y < 2 ? 0 : y - 2, yhi = y + 2;
+        uint32_t mask = 0;
+        int64_t last = q;  // the last neighbour
+        for (int i = 1; i <= 2 && q + i < ncol; ++i) {
+            const uint64_t k = col_key[q + i];
+            if ((k >> by) != x || (k & ymask) > yhi) break;
+            mask |= 1u << ((k & ymask) - y - 1);
+            last = q + i;
+        }
+        int64_t row[2];
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+            const uint64_t xr = x + 1 + d;
+            row[d] = col_lower(col_key, d == 0 ? q + 1 : row[0], ncol, (xr << by) | ylo);
+            for (int i = 0; i < 5 && row[d] + i < ncol; ++i) {
+                const uint64_t k = col_key[row[d] + i];
+                if ((k >> by) != xr || (k & ymask) > yhi) break;
+                mask |= 1u << (2 + 5 * d + static_cast<int>((k & ymask) + 2 - y));
+                last = row[d] + i;
+            }
+        }
+        ColNeigh nb;
+        nb.row1 = static_cast<int32_t>(row[0]);
+        nb.row2 = static_cast<int32_t>(row[1]);
+        nb.mask = mask;
+        nb.last = col_cell[last + 1] - 1;
+        neigh[q] = nb;
+    }
+}
+
+// counts[0..7]: segments per class; counts[8..15]: the class cursors (zero here)
 __global__ __launch_bounds__(256) void k_col_class_count(const int64_t* __restrict__ totals,
                                                          const int* __restrict__ col_cell,
-                                                         const uint64_t* __restrict__ col_key,
-                                                         int* __restrict__ col_slot,
+                                                         const ColNeigh* __restrict__ neigh,
                                                          const int2* __restrict__ crec,
-                                                         ColEntry* __restrict__ tab,
-                                                         int* __restrict__ counts,
-                                                         int* __restrict__ err) {
+                                                         int* __restrict__ counts) {
     __shared__ int h[kColClasses];
     if (threadIdx.x < kColClasses) h[threadIdx.x] = 0;
     __syncthreads();
     const int64_t ncol = totals[0] >> 32;
+    const int str = stretch_cells(totals[0] & 0xffffffff);
     const int64_t per = (ncol + gridDim.x - 1) / gridDim.x;
     const int64_t q0 = blockIdx.x * per, q1 = q0 + per < ncol ? q0 + per : ncol;
-    const uint64_t mask = static_cast<uint64_t>(totals[1]);
     for (int64_t q = q0 + threadIdx.x; q < q1; q += blockDim.x) {
         const int a0 = col_cell[q], a1 = col_cell[q + 1];
         const int step = seg_step(a1 - a0);
-        for (int c = a0; c < a1; c += step) atomicAdd(&h[seg_class(crec, c, min(c + step, a1))], 1);
-        const uint64_t key = col_key[q];
-        const uint64_t word = key | (static_cast<uint64_t>(a1 - a0) << kKeyBits);
-        uint64_t s = mix64(key) & mask;
-        for (uint64_t probe = 0;; ++probe) {
-            uint64_t expected = kEmpty;
-            if (__hip_atomic_compare_exchange_strong(&tab[s].word, &expected, word,
-                                                     __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                     __HIP_MEMORY_SCOPE_AGENT)) {
-                tab[s].c0 = a0;
-                col_slot[q] = static_cast<int>(s);
-                break;
-            }
-            if (probe > mask) {  // table full (cannot happen: capacity >= 2 columns)
-                atomicOr(err, 2);
-                col_slot[q] = 0;
-                break;
-            }
-            s = (s + 1) & mask;
-        }
+        const int last = neigh[q].last / str;
+        for (int c = a0; c < a1; c += step)
+            if (c / str != last) atomicAdd(&h[seg_class(crec, c, min(c + step, a1))], 1);
     }
     __syncthreads();
     if (threadIdx.x < kColClasses && h[threadIdx.x] > 0) atomicAdd(counts + threadIdx.x, h[threadIdx.x]);
@@ -467,7 +487,7 @@ __global__ __launch_bounds__(256) void k_col_class_count(const int64_t* __restri
 __global__ __launch_bounds__(256) void k_col_class_scatter(const int64_t* __restrict__ totals,
                                                            const int* __restrict__ col_cell,
                                                            const uint64_t* __restrict__ col_key,
-                                                           const int* __restrict__ col_slot,
+                                                           const ColNeigh* __restrict__ neigh,
                                                            const int2* __restrict__ crec,
                                                            int* __restrict__ counts,
                                                            ColRec* __restrict__ lanes) {
@@ -476,12 +496,15 @@ __global__ __launch_bounds__(256) void k_col_class_scatter(const int64_t* __rest
     if (threadIdx.x < kColClasses) h[threadIdx.x] = 0;
     __syncthreads();
     const int64_t ncol = totals[0] >> 32;
+    const int str = stretch_cells(totals[0] & 0xffffffff);
     const int64_t per = (ncol + gridDim.x - 1) / gridDim.x;
     const int64_t q0 = blockIdx.x * per, q1 = q0 + per < ncol ? q0 + per : ncol;
     for (int64_t q = q0 + threadIdx.x; q < q1; q += blockDim.x) {
         const int a0 = col_cell[q], a1 = col_cell[q + 1];
         const int step = seg_step(a1 - a0);
-        for (int c = a0; c < a1; c += step) atomicAdd(&h[seg_class(crec, c, min(c + step, a1))], 1);
+        const int last = neigh[q].last / str;
+        for (int c = a0; c < a1; c += step)
+            if (c / str != last) atomicAdd(&h[seg_class(crec, c, min(c + step, a1))], 1);
     }
     __syncthreads();
     if (threadIdx.x < kColClasses) {
@@ -495,31 +518,31 @@ __global__ __launch_bounds__(256) void k_col_class_scatter(const int64_t* __rest
     for (int64_t q = q0 + threadIdx.x; q < q1; q += blockDim.x) {
         const int a0 = col_cell[q], a1 = col_cell[q + 1];
         const int step = seg_step(a1 - a0);
+        const int last = neigh[q].last / str;
         for (int c = a0; c < a1; c += step) {
+            if (c / str == last) continue;
             const int c1 = min(c + step, a1);
             const int k = seg_class(crec, c, c1);
             ColRec r;
             r.word = col_key[q] | (static_cast<uint64_t>(c1 - c) << kSegLenShift) |
                      (static_cast<uint64_t>(min(a1 - c1, 2)) << kSegMoreShift);
             r.c0 = c;
-            r.slot = col_slot[q];
+            r.col = static_cast<int32_t>(q);
             lanes[base[k] + atomicAdd(&h[k], 1)] = r;
         }
     }
 }
 
 // Between the rounds, after k_flatten (parent[c] is then c's root): the root shared by
-// all cells of a column, or -1 when they differ, into the column's table entry (the
-// table is walked in slot order).  Two columns with the same shared root are joined
-// throughout, so round 2 skips the pair without looking at its cells.
+// all cells of a column, or -1 when they differ, into the column's record.  Two columns
+// with the same shared root are joined throughout: the next round skips the pair without
+// looking at its cells.
 __global__ void k_col_roots(const int64_t* __restrict__ totals, const int* __restrict__ parent,
-                            ColEntry* __restrict__ tab) {
-    const int64_t m = totals[1] + 1;
-    for (int64_t s = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; s < m;
+                            ColEntry* __restrict__ cols) {
+    const int64_t ncol = totals[0] >> 32;
+    for (int64_t s = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; s < ncol;
          s += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-        const uint64_t word = tab[s].word;
-        if (word == kEmpty) continue;
-        const int a0 = tab[s].c0, a1 = a0 + static_cast<int>(word >> kKeyBits);
+        const int a0 = cols[s].c0, a1 = a0 + static_cast<int>(cols[s].word >> kKeyBits);
         const int r = parent[a0];
         int u = r;
         for (int c = a0 + 1; c < a1; ++c)
@@ -527,7 +550,7 @@ __global__ void k_col_roots(const int64_t* __restrict__ totals, const int* __res
                 u = -1;
                 break;
             }
-        tab[s].root = u;
+        cols[s].root = u;
     }
 }
 
@@ -536,149 +559,277 @@ __global__ void k_col_roots(const int64_t* __restrict__ totals, const int* __res
 __constant__ signed char kCol[12][2] = {{0, 1}, {1, -1}, {1, 0}, {1, 1},  // near
                                         {0, 2}, {1, -2}, {1, 2}, {2, -2},
                                         {2, -1}, {2, 0}, {2, 1}, {2, 2}};
+// the neighbour's record, or -1 when the column does not exist
+__device__ __forceinline__ int col_neighbour(const ColNeigh& nb, int q, int k) {
+    const int dx = kCol[k][0], dy = kCol[k][1];
+    if (dx == 0)
+        return (nb.mask >> (dy - 1)) & 1 ? q + 1 + (dy == 2 ? static_cast<int>(nb.mask & 1) : 0) : -1;
+    const uint32_t row = (nb.mask >> (dx == 1 ? 2 : 7)) & 31;
+    if (!((row >> (dy + 2)) & 1)) return -1;
+    return (dx == 1 ? nb.row1 : nb.row2) + __popc(row & ((1u << (dy + 2)) - 1));
+}
 constexpr int kLaneTest = 64;  // pair tests a lane does alone
-// Round 1: pairs of cells this small are tested before any root lookup.  Round 2 looks
-// the roots up first (after round 1 most of its pairs are already joined).
+
+// One candidate pair of cells c (particles [sc, sc + nc)) and d (particles [sd, sd + nd))
+// whose records hold different roots.  Pairs of at most kTestFirst particle pairs are
+// tested at once (a test costs less than looking up whether they were joined meanwhile);
+// larger ones are skipped when already joined, else tested here when below kLaneTest pairs,
+// else listed for k_fof_big (tested here too when the list is full).  rc caches c's root
+// (-1: not looked up yet; from a read-only find, possibly out of date: equal roots still
+// prove the cells joined); it is refreshed after a link.
 constexpr int kTestFirst = 8;
 
-// One candidate pair of cells c (particles [sc, sc + nc)) and d (particles [sd, sd + nd)).
-// Pairs of at most TF particle pairs are tested first, and the roots looked at only when
-// a pair is within ll (a test costs less than the root lookups).  Larger pairs are skipped
-// when already joined, else tested here when below kLaneTest pairs, else listed for
-// k_fof_big (tested here too when the list is full).  rc caches c's root (-1: not looked
-// up yet; from a read-only find, possibly out of date: equal roots still prove the cells
-// joined); it is refreshed after a link.
-template <int TF, typename V>
+template <typename V>
 __device__ __forceinline__ void candidate(int c, int& rc, int sc, int nc, int d, int sd,
                                           int nd, const V* __restrict__ spk, double ll2,
                                           int* __restrict__ parent, int2* __restrict__ big,
                                           int64_t big_cap,
                                           unsigned long long* __restrict__ n_big) {
-    const int64_t pairs = static_cast<int64_t>(nc) * nd;
-    if (pairs > TF) {
+    const bool small = static_cast<int64_t>(nc) * nd <= kTestFirst;
+    if (!small) {
         if (rc < 0) rc = find_ro(parent, c);
         if (rc == find_ro(parent, d)) return;
-        if (pairs > kLaneTest) {
-            // neighbouring dense cells nearly always hold a close pair among their first
-            // members: a 2 x 2 sample first, the whole pair to a wavefront only without one
-            const int sa = nc < 2 ? nc : 2, sb = nd < 2 ? nd : 2;
-            for (int b = 0; b < sb; ++b) {
-                const V pb = spk[sd + b];
-                for (int a = 0; a < sa; ++a)
-                    if (within(spk[sc + a], pb, ll2)) {
-                        uf_union(parent, c, d);
-                        rc = find_ro(parent, c);
-                        return;
-                    }
-            }
-            const unsigned long long at = atomicAdd(n_big, 1ull);
-            if (static_cast<int64_t>(at) < big_cap) {
-                big[at] = make_int2(c, d);
-                return;
-            }
+    }
+    const bool sample = static_cast<int64_t>(nc) * nd > kLaneTest;
+    // neighbouring dense cells nearly always hold a close pair among their first members: a
+    // 2 x 2 sample first, the whole pair to a wavefront only without one
+    const int sa = sample && nc > 2 ? 2 : nc, sb = sample && nd > 2 ? 2 : nd;
+    bool linked = false;
+    for (int b = 0; b < sb && !linked; ++b) {
+        const V pb = spk[sd + b];
+        for (int a = 0; a < sa && !linked; ++a) linked = within(spk[sc + a], pb, ll2);
+    }
+    if (!linked && sample) {
+        const unsigned long long at = atomicAdd(n_big, 1ull);
+        if (static_cast<int64_t>(at) < big_cap) {
+            big[at] = make_int2(c, d);
+            return;
+        }
+        for (int b = 0; b < nd && !linked; ++b) {
+            const V pb = spk[sd + b];
+            for (int a = 0; a < nc && !linked; ++a) linked = within(spk[sc + a], pb, ll2);
         }
     }
-    for (int b = 0; b < nd; ++b) {
-        const V pb = spk[sd + b];
-        for (int a = 0; a < nc; ++a)
-            if (within(spk[sc + a], pb, ll2)) {
-                if (rc < 0) rc = find_ro(parent, c);
-                if (rc != find_ro(parent, d)) {
-                    uf_union(parent, c, d);
-                    rc = find_ro(parent, c);
-                }
-                return;
-            }
+    if (!linked) return;
+    if (small) {
+        if (rc < 0) rc = find_ro(parent, c);
+        if (rc == find_ro(parent, d)) return;
+    }
+    uf_union(parent, c, d);
+    rc = find_ro(parent, c);
+}
+
+// The links between cells of one stretch, a workgroup per stretch with its forest and its
+// cells' records in LDS: first the pairs at Chebyshev distance 1, then those at distance 2
+// (in a dense region the first have joined what the second would search).  A lane takes a
+// cell and a column offset: the column's cells within reach (a binary search in a long
+// column), skipped where the forest has joined them, else tested; pairs of more than
+// kLaneTest particle pairs without a link in their first 2 x 2 are listed for k_fof_big.
+// At the end every cell of the stretch is pointed at its root: this starts the global
+// forest.
+//
+// What bounds the links of sparse cells are finds and hooks in memory shared by all XCDs
+// (8M bridged stars, 6.5M cells: 1.1 of the 1.9 ms of a distance-1 round over all cells;
+// merging the columns 0.5, testing 0.3) and dependent loads of roots and records; here
+// both
+// are LDS accesses.  @N1@
+__device__ __forceinline__ int lds_parent(int* P, int x) {
+    return __hip_atomic_load(P + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+__device__ __forceinline__ int lds_find(int* P, int x) {
+    int p = lds_parent(P, x);
+    while (p != x) {
+        const int g = lds_parent(P, p);
+        if (g != p)  // halve the path; concurrent writers store ancestors too
+            __hip_atomic_store(P + x, g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        x = p;
+        p = g;
+    }
+    return x;
+}
+
+__device__ __forceinline__ void lds_join(int* P, int a, int b) {
+    for (;;) {
+        a = lds_find(P, a);
+        b = lds_find(P, b);
+        if (a == b) return;
+        if (a < b) {
+            const int t = a;
+            a = b;
+            b = t;
+        }
+        if (atomicCAS(P + a, a, b) == a) return;  // root a (> b) hooked under b
     }
 }
 
-// Link candidates, one lane per (column segment, column offset) of one round: the
-// segment's cells against the cells ROUND apart above them in their own column, or
-// against a neighbour column.  ROUND 1: the own cells one z apart, and the four near
-// columns with |dz| <= 1 (the 13 cell offsets at Chebyshev distance 1).  ROUND 2,
-// launched after every distance-1 link is in the forest (so that dense regions are
-// recognised as joined and need no search): the own cells two apart, the near columns
-// with |dz| = 2, the far columns with |dz| <= 2 (the other 49 offsets).  The lanes of
-// one segment are consecutive and read its record together; a neighbour column costs
-// one table line (first cell, cell count, shared root), its cell records and its
-// particles.
-template <typename T, int ROUND>
-__global__ __launch_bounds__(256) void k_fof_cols(
-    const ColEntry* __restrict__ tab, const ColRec* __restrict__ lanes,
-    const int2* __restrict__ crec, const typename Packed<T>::type* __restrict__ spk,
-    const int64_t* __restrict__ totals, int bx, int by, double ll2, int* __restrict__ parent,
-    int2* __restrict__ big, int64_t big_cap, unsigned long long* __restrict__ n_big,
-    const int* __restrict__ seg_counts) {
-    constexpr int K = ROUND == 1 ? 5 : 13;  // own column + neighbour columns
+// Distance DIST (1 or 2) of one stretch: cells base .. base + m - 1, records R (m + 1)
+template <int DIST, typename V>
+__device__ __forceinline__ void local_links(int* P, const int2* R, int base, int m,
+                                            const ColEntry* __restrict__ cols,
+                                            const ColNeigh* __restrict__ neigh,
+                                            const int* __restrict__ cell_col,
+                                            const V* __restrict__ spk, double ll2,
+                                            int2* __restrict__ big, int64_t big_cap,
+                                            unsigned long long* __restrict__ n_big) {
+    constexpr int K = DIST == 1 ? 5 : 13;  // the own column, the four near ones, the far ones
+    for (int i = threadIdx.x; i < m * K; i += blockDim.x) {
+        const int c = i / K, o = i % K;
+        const int q = cell_col[base + c];
+        const int2 cc = R[c];
+        const int nc = R[c + 1].x - cc.x;
+        int d, d1, lo = 0;  // lo: smallest |dz|
+        if (o == 0) {
+            d = c + 1;
+            d1 = cols[q].c0 + static_cast<int>(cols[q].word >> kKeyBits) - base;
+            lo = DIST;
+        } else {
+            const int at = col_neighbour(neigh[q], q, o - 1);
+            if (at < 0) continue;
+            const ColEntry e = cols[at];
+            d = e.c0 - base;
+            d1 = d + static_cast<int>(e.word >> kKeyBits);
+            if (DIST == 2 && o <= 4) lo = 2;
+        }
+        d1 = min(d1, m);
+        if (o != 0) {  // first cell with z >= zc - DIST
+            int hi = d1;
+            while (d < hi) {
+                const int mid = (d + hi) >> 1;
+                if (R[mid].y < cc.y - DIST) d = mid + 1;
+                else hi = mid;
+            }
+        }
+        for (; d < d1; ++d) {
+            const int2 dd = R[d];
+            const int dz = dd.y - cc.y;
+            if (dz > DIST) break;
+            if (dz < lo && -dz < lo) continue;
+            if (lds_find(P, c) == lds_find(P, d)) continue;
+            const int nd = R[d + 1].x - dd.x;
+            const bool sample = static_cast<int64_t>(nc) * nd > kLaneTest;
+            const int sa = sample && nc > 2 ? 2 : nc, sb = sample && nd > 2 ? 2 : nd;
+            bool linked = false;
+            for (int b = 0; b < sb && !linked; ++b) {
+                const V pb = spk[dd.x + b];
+                for (int a = 0; a < sa && !linked; ++a) linked = within(spk[cc.x + a], pb, ll2);
+            }
+            if (!linked && sample) {
+                const unsigned long long at = atomicAdd(n_big, 1ull);
+                if (static_cast<int64_t>(at) < big_cap) {
+                    big[at] = make_int2(base + c, base + d);
+                    continue;
+                }
+                for (int b = 0; b < nd && !linked; ++b) {  // the list is full
+                    const V pb = spk[dd.x + b];
+                    for (int a = 0; a < nc && !linked; ++a)
+                        linked = within(spk[cc.x + a], pb, ll2);
+                }
+            }
+            if (linked) lds_join(P, c, d);
+        }
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(512) void k_fof_local(
+    const ColEntry* __restrict__ cols, const ColNeigh* __restrict__ neigh,
+    const int* __restrict__ cell_col, const int2* __restrict__ crec,
+    const typename Packed<T>::type* __restrict__ spk, const int64_t* __restrict__ totals,
+    double ll2, int* __restrict__ parent, int2* __restrict__ big, int64_t big_cap,
+    unsigned long long* __restrict__ n_big) {
+    __shared__ int P[kStretchMax];
+    __shared__ int2 R[kStretchMax + 1];
+    const int64_t ncell = totals[0] & 0xffffffff;
+    const int str = stretch_cells(ncell);
+    for (int64_t b0 = static_cast<int64_t>(blockIdx.x) * str; b0 < ncell;
+         b0 += static_cast<int64_t>(gridDim.x) * str) {
+        const int base = static_cast<int>(b0);
+        const int m = static_cast<int>(ncell - b0 < str ? ncell - b0 : str);
+        for (int i = threadIdx.x; i <= m; i += blockDim.x) {
+            if (i < m) P[i] = i;
+            R[i] = crec[base + i];
+        }
+        __syncthreads();
+        local_links<1>(P, R, base, m, cols, neigh, cell_col, spk, ll2, big, big_cap, n_big);
+        __syncthreads();
+        local_links<2>(P, R, base, m, cols, neigh, cell_col, spk, ll2, big, big_cap, n_big);
+        __syncthreads();
+        for (int i = threadIdx.x; i < m; i += blockDim.x) {
+            int x = i;
+            for (int p = P[x]; p != x; p = P[x]) x = p;
+            parent[base + i] = base + x;
+        }
+        __syncthreads();
+    }
+}
+
+// The links between stretches, in two rounds (Chebyshev distance 1, then 2 after
+// flattening the forest), one lane per (column segment, column offset): the segment's
+// cells against those above them in their own column, or against a neighbour column.  The
+// lanes of one segment are consecutive and read its record and its neighbours' places
+// together.  Cells whose records hold the same root are joined; the others look at the
+// forest as it is now.
+template <typename T, int DIST>
+__global__ __launch_bounds__(256) void k_fof_cross(
+    const ColEntry* __restrict__ cols, const ColNeigh* __restrict__ neigh,
+    const ColRec* __restrict__ lanes, const int4* __restrict__ frec,
+    const typename Packed<T>::type* __restrict__ spk, const int64_t* __restrict__ totals,
+    double ll2, int* __restrict__ parent, int2* __restrict__ big, int64_t big_cap,
+    unsigned long long* __restrict__ n_big, const int* __restrict__ seg_counts) {
+    constexpr int K = DIST == 1 ? 5 : 13;  // own column + neighbour columns
     int64_t nseg = 0;
 #pragma unroll
     for (int k = 0; k < kColClasses; ++k) nseg += seg_counts[k];
-    const uint64_t mask = static_cast<uint64_t>(totals[1]);
     const int64_t total = nseg * K;
-    const int64_t ymask = (int64_t{1} << by) - 1;
-    const int64_t nxc = int64_t{1} << bx, nyc = int64_t{1} << by;
+    const int str = stretch_cells(totals[0] & 0xffffffff);
     for (int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
          idx < total; idx += static_cast<int64_t>(gridDim.x) * blockDim.x) {
         const ColRec col = lanes[idx / K];
         const int o = static_cast<int>(idx % K);
         const int a0 = col.c0;  // the segment's cells [a0, a1)
         const int a1 = a0 + static_cast<int>((col.word >> kSegLenShift) & 1023);
-        const int ra = ROUND == 2 ? tab[col.slot].root : -1;  // the column's shared root
-        if (o == 0) {  // the segment's cells against those ROUND above them in the column
+        const int ra = cols[col.col].root;  // the column's shared root
+        if (o == 0) {  // the segment's cells against those above them in the column
             if (ra >= 0) continue;  // one component already
             const int e1 = a1 + static_cast<int>((col.word >> kSegMoreShift) & 3);
-            int2 cc = crec[a0];
-            for (int c = a0; c < a1 && c + 1 < e1; ++c) {
-                const int2 cn = crec[c + 1];
+            if (a0 / str == (e1 - 1) / str) continue;
+            for (int c = a0; c < a1; ++c) {
+                const int4 cc = frec[c];
                 int rc = -1;
-                const int sc = cc.x, nc = cn.x - cc.x;
-                int2 dd = cn;
-                for (int d = c + 1; d < e1 && dd.y - cc.y <= ROUND; ++d) {
-                    const int2 dn = crec[d + 1];
-                    if (dd.y - cc.y == ROUND)
-                        candidate<ROUND == 1 ? kTestFirst : 0>(c, rc, sc, nc, d, dd.x,
-                                                               dn.x - dd.x, spk, ll2, parent,
-                                                               big, big_cap, n_big);
-                    dd = dn;
+                for (int d = c + 1; d < e1; ++d) {
+                    const int4 dd = frec[d];
+                    if (dd.y - cc.y > DIST) break;
+                    if (dd.y - cc.y == DIST && dd.w != cc.w)
+                        candidate(c, rc, cc.x, cc.z - cc.x, d, dd.x, dd.z - dd.x, spk, ll2,
+                                  parent, big, big_cap, n_big);
                 }
-                cc = cn;
             }
             continue;
         }
-        const int k = o - 1;  // round 1: the near columns; round 2: all twelve
-        const uint64_t key = col.word & kKeyMask;
-        const int64_t nx = static_cast<int64_t>(key >> by) + kCol[k][0];
-        const int64_t ny = static_cast<int64_t>(key & ymask) + kCol[k][1];
-        if (nx < 0 || ny < 0 || nx >= nxc || ny >= nyc) continue;
-        const ColEntry e = col_find(tab, mask, (static_cast<uint64_t>(nx) << by) |
-                                                   static_cast<uint64_t>(ny));
-        if (e.word == kEmpty) continue;
+        const int at = col_neighbour(neigh[col.col], col.col, o - 1);
+        if (at < 0) continue;
+        const ColEntry e = cols[at];
         if (ra >= 0 && ra == e.root) continue;  // joined throughout
         const int b0 = e.c0, b1 = b0 + static_cast<int>(e.word >> kKeyBits);
-        // |dz| range of this (round, column): near columns take |dz| <= 1 in round 1 and
-        // |dz| = 2 in round 2, far columns |dz| <= 2
-        const bool near = k < 4;
-        const int lo = (ROUND == 2 && near) ? 2 : 0;
-        const int hi = ROUND == 1 ? 1 : 2;
+        if (a0 / str == (b1 - 1) / str) continue;  // one stretch: k_fof_local's
+        const int lo = DIST == 2 && o <= 4 ? 2 : 0;  // smallest |dz|
         int p = b0;
-        int2 pp = crec[b0];
-        int2 cc = crec[a0];
         for (int c = a0; c < a1; ++c) {
-            const int2 cn = crec[c + 1];
-            const int zc = cc.y;
+            const int4 cc = frec[c];
             int rc = -1;
-            while (p < b1 && pp.y < zc - hi) pp = crec[++p];
-            int2 dd = pp;
-            for (int d = p; d < b1 && dd.y <= zc + hi; ++d) {
-                const int2 dn = crec[d + 1];
-                const int dz = dd.y > zc ? dd.y - zc : zc - dd.y;
-                if (dz >= lo)
-                    candidate<ROUND == 1 ? kTestFirst : 0>(c, rc, cc.x, cn.x - cc.x, d, dd.x,
-                                                           dn.x - dd.x, spk, ll2, parent, big,
-                                                           big_cap, n_big);
-                dd = dn;
+            for (int d = p; d < b1; ++d) {
+                const int4 dd = frec[d];
+                const int dz = dd.y - cc.y;
+                if (dz < -DIST) {
+                    p = d + 1;
+                    continue;
+                }
+                if (dz > DIST) break;
+                if (dd.w != cc.w && (dz >= lo || -dz >= lo))
+                    candidate(c, rc, cc.x, cc.z - cc.x, d, dd.x, dd.z - dd.x, spk, ll2, parent,
+                              big, big_cap, n_big);
             }
-            cc = cn;
         }
     }
 }
@@ -810,8 +961,10 @@ __global__ void k_labels(int64_t n, const int32_t* __restrict__ perm,
 struct FofWs {
     double* box_part;
     double* box;
-    ColEntry* tab;
-    int64_t* totals;  // [0] cells | columns << 32, [1] column table mask
+    ColEntry* cols;   // the columns' records
+    ColNeigh* neigh;
+    int4* frec;       // per cell: its record with its root
+    int64_t* totals;  // cells | columns << 32
     void* scan_ws;
     void* sort_ws;
     uint32_t* klo;    // low / high 32 bits of each particle's cell key
@@ -827,37 +980,31 @@ struct FofWs {
     int2* crec;       // per cell: first sorted position, z (n_cells + 1 entries)
     int* col_cell;    // first cell of each column (n_cols + 1 entries)
     uint64_t* col_key;
-    int* col_slot;    // table slot of each column
     ColRec* lanes;    // the column segments in link-lane order (by class)
     int* class_counts;
     int* parent;
     int* root;
     int* comp_min;
     int* cell_min;
+    int* cell_col;    // column of each cell
     void* spk;        // (x, y, z, 0) per sorted position
     void* pk;         // (x, y, z, 0) per particle in input order
     int2* big;        // large pairs of cells left for k_fof_big
-    unsigned long long* n_big;
+    unsigned long long* n_big;  // kBigLists counts (the list is refilled for each)
     int64_t big_cap;
     int* err;
     size_t bytes;
-    int64_t cap;      // column table capacity for n particles (the largest it gets)
 };
-
-int64_t table_capacity(int64_t n) {
-    int64_t cap = 1024;
-    while (cap < 2 * n) cap <<= 1;
-    return cap;
-}
 
 FofWs carve_fof(void* base, int64_t n, size_t elt) {
     Carver c(base);
     FofWs w;
     const int64_t nn = n > 0 ? n : 1;
-    w.cap = table_capacity(n);
     w.box_part = c.take<double>(kBoxBlocks * 6);
     w.box = c.take<double>(8);
-    w.tab = c.take<ColEntry>(w.cap);
+    w.cols = c.take<ColEntry>(nn);
+    w.neigh = c.take<ColNeigh>(nn);
+    w.frec = c.take<int4>(nn);
     w.totals = c.take<int64_t>(4);
     w.scan_ws = c.take<char>(scan_workspace_bytes(nn));
     w.sort_ws = c.take<char>(radix_workspace_bytes(nn));
@@ -874,18 +1021,18 @@ FofWs carve_fof(void* base, int64_t n, size_t elt) {
     w.crec = c.take<int2>(nn + 1);
     w.col_cell = c.take<int>(nn + 1);
     w.col_key = c.take<uint64_t>(nn);
-    w.col_slot = c.take<int>(nn);
     w.lanes = c.take<ColRec>(nn + nn / kSegCells + 1);  // segments <= columns + cells / 4
     w.class_counts = c.take<int>(2 * kColClasses);
     w.parent = c.take<int>(nn);
     w.root = c.take<int>(nn);
     w.comp_min = c.take<int>(nn);
     w.cell_min = c.take<int>(nn);
+    w.cell_col = c.take<int>(nn);
     w.spk = c.take<char>(nn * 4 * elt);
     w.pk = c.take<char>(nn * 4 * elt);
     w.big_cap = 2 * nn;
     w.big = c.take<int2>(w.big_cap);
-    w.n_big = c.take<unsigned long long>(4);
+    w.n_big = c.take<unsigned long long>(kBigLists);
     w.err = c.take<int>(64);
     w.bytes = c.used;
     return w;
@@ -966,46 +1113,43 @@ int fof_run(const T* x, const T* y, const T* z, int64_t n, double ll, int* label
     HALMA_LAUNCH_CHECK();
     rc = exclusive_scan_i64(w.heads, w.before, n, w.totals, w.scan_ws, st);
     if (rc) return rc;
-    k_col_table_size<<<1, 64, 0, st>>>(w.totals, w.cap);
-    HALMA_LAUNCH_CHECK();
-    k_clear_cols<<<grid_cells, 256, 0, st>>>(w.totals, w.tab);
-    HALMA_LAUNCH_CHECK();
     k_fof_cells<<<blocks_for(n), 256, 0, st>>>(w.skey, perm, w.heads, w.before, n, g,
-                                               w.crec, w.cell_min, w.parent, w.comp_min,
+                                               w.crec, w.cell_min, w.cell_col, w.comp_min,
                                                w.col_cell, w.col_key);
     HALMA_LAUNCH_CHECK();
-    k_clear_words<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(w.n_big), 4);
+    k_clear_words<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(w.n_big), 2 * kBigLists);
     HALMA_LAUNCH_CHECK();
     k_clear_words<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(w.class_counts), 2 * kColClasses);
     HALMA_LAUNCH_CHECK();
-    k_col_class_count<<<kClassBlocks, 256, 0, st>>>(w.totals, w.col_cell, w.col_key,
-                                                     w.col_slot, w.crec, w.tab,
-                                                     w.class_counts, w.err);
+    k_col_neigh<<<grid_cells, 256, 0, st>>>(w.totals, w.col_cell, w.col_key, g.by, w.cols,
+                                            w.neigh);
     HALMA_LAUNCH_CHECK();
-    k_col_class_scatter<<<kClassBlocks, 256, 0, st>>>(w.totals, w.col_cell, w.col_key,
-                                                       w.col_slot, w.crec, w.class_counts,
-                                                       w.lanes);
+    k_col_class_count<<<kClassBlocks, 256, 0, st>>>(w.totals, w.col_cell, w.neigh, w.crec,
+                                                     w.class_counts);
+    HALMA_LAUNCH_CHECK();
+    k_col_class_scatter<<<kClassBlocks, 256, 0, st>>>(w.totals, w.col_cell, w.col_key, w.neigh,
+                                                       w.crec, w.class_counts, w.lanes);
     HALMA_LAUNCH_CHECK();
     const unsigned cand_grid = static_cast<unsigned>(cus * 32);
     const double ll2 = ll * ll;
-    k_fof_cols<T, 1><<<cand_grid, 256, 0, st>>>(w.tab, w.lanes, w.crec, spk, w.totals, g.bx,
-                                                g.by, ll2, w.parent, w.big, w.big_cap,
-                                                w.n_big, w.class_counts);
+    k_fof_local<T><<<cus * 16, 512, 0, st>>>(w.cols, w.neigh, w.cell_col, w.crec, spk, w.totals,
+                                             ll2, w.parent, w.big, w.big_cap, w.n_big);
     HALMA_LAUNCH_CHECK();
-    k_fof_big<T><<<grid_cells, 256, 0, st>>>(w.big, w.n_big, w.big_cap, w.crec, spk, ll2,
-                                             w.parent);
-    HALMA_LAUNCH_CHECK();
-    k_flatten<<<grid_cells, 256, 0, st>>>(w.totals, w.parent);
-    HALMA_LAUNCH_CHECK();
-    k_col_roots<<<grid_cells, 256, 0, st>>>(w.totals, w.parent, w.tab);
-    HALMA_LAUNCH_CHECK();
-    k_fof_cols<T, 2><<<cand_grid, 256, 0, st>>>(w.tab, w.lanes, w.crec, spk, w.totals, g.bx,
-                                                g.by, ll2, w.parent, w.big, w.big_cap,
-                                                w.n_big + 1, w.class_counts);
-    HALMA_LAUNCH_CHECK();
-    k_fof_big<T><<<grid_cells, 256, 0, st>>>(w.big, w.n_big + 1, w.big_cap, w.crec, spk, ll2,
-                                             w.parent);
-    HALMA_LAUNCH_CHECK();
+    for (int round = 0; round < kBigLists; ++round) {
+        k_fof_big<T><<<grid_cells, 256, 0, st>>>(w.big, w.n_big + round, w.big_cap, w.crec, spk,
+                                                 ll2, w.parent);
+        HALMA_LAUNCH_CHECK();
+        if (round == kBigLists - 1) break;
+        k_flatten<<<grid_cells, 256, 0, st>>>(w.totals, w.parent, w.crec, w.frec);
+        HALMA_LAUNCH_CHECK();
+        k_col_roots<<<grid_cells, 256, 0, st>>>(w.totals, w.parent, w.cols);
+        HALMA_LAUNCH_CHECK();
+        auto cross = round == 0 ? k_fof_cross<T, 1> : k_fof_cross<T, 2>;
+        cross<<<cand_grid, 256, 0, st>>>(w.cols, w.neigh, w.lanes, w.frec, spk, w.totals, ll2,
+                                         w.parent, w.big, w.big_cap, w.n_big + round + 1,
+                                         w.class_counts);
+        HALMA_LAUNCH_CHECK();
+    }
     k_roots<<<grid_cells, 256, 0, st>>>(w.totals, w.parent, w.root);
     HALMA_LAUNCH_CHECK();
     k_check_roots<<<grid_cells, 256, 0, st>>>(w.totals, w.parent, w.root, w.cell_min,
@@ -1053,7 +1197,6 @@ int fof_check_error(const int* d_err, hipStream_t st) {
         return set_error(HALMA_E_LIMIT,
                          "friends-of-friends: coordinates span more than 2^21 sub-cells of "
                          "side ll/sqrt(3) on an axis, or are not finite");
-    if (e & 2) return set_error(HALMA_E_STATE, "friends-of-friends: cell table overflow");
     if (e & 4) return set_error(HALMA_E_STATE, "friends-of-friends: inconsistent union-find roots");
     return 0;
 }
