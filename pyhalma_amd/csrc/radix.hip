@@ -1,33 +1,51 @@
 // Stable LSD radix sort (8-bit digits).  Per pass: a per-block digit histogram, an
 // exclusive scan of each digit's row of the digit-major [digit][block] table (a block per
 // digit, which also writes the digit's total), then a stable scatter (each block adds the
-// exclusive scan of the 256 digit totals, taken in LDS, to its row offsets) in
-// which each block ranks its tile's keys by digit (256 keys per round; ranks among equal
-// digits inside a wavefront from eight ballots, wavefronts of a round offset by their
-// predecessors' counts through LDS), sorts the tile by digit in LDS and writes each
-// digit's run to its place, consecutive threads to consecutive addresses.
+// exclusive scan of the 256 digit totals, taken in LDS, to its row offsets) in which each
+// wavefront ranks a contiguous part of the tile by digit on its own (ranks among equal
+// digits of 64 keys from eight ballots, the wavefront's running counts in LDS), the
+// wavefronts' counts are put together once, and the tile is sorted by digit in LDS and
+// written digit run by digit run, consecutive threads to consecutive addresses.
+//
+// Bound by memory latency and the barriers of a tile.  A scatter pass of 8M pairs takes
+// 45 us (2.8 TB/s), of 1.9M 16, of 24k 5.2; with 256 keys ranked per round by the whole
+// workgroup, four barriers each, it took 56, 19 and 11.5.  Large inputs take tiles of 4096 keys (longer runs per digit), small ones of 1024 (more
+// blocks).
 #include "radix.h"
+
+#include <algorithm>
 
 namespace halma {
 
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kRounds = 8;
-constexpr int kTile = kThreads * kRounds;
 constexpr int kWaves = kThreads / kWave;
+constexpr int kSmall = 4, kLarge = 16;         // keys per thread of a tile
+constexpr int64_t kLargeKeys = int64_t{1} << 20;  // inputs from this size take large tiles
 
+inline int64_t tiles_of(int64_t n) {
+    const int64_t tile = kThreads * (n >= kLargeKeys ? kLarge : kSmall);
+    return n > 0 ? (n + tile - 1) / tile : 1;
+}
+
+template <int kRounds>
 __global__ __launch_bounds__(kThreads) void k_radix_hist(const uint32_t* __restrict__ keys,
                                                          int64_t n, int shift, int64_t nb,
                                                          int32_t* __restrict__ hist) {
     __shared__ int h[256];
     h[threadIdx.x] = 0;
     __syncthreads();
-    const int64_t base = static_cast<int64_t>(blockIdx.x) * kTile;
+    const int64_t base = static_cast<int64_t>(blockIdx.x) * (kThreads * kRounds);
+    uint32_t k[kRounds];
+#pragma unroll
     for (int r = 0; r < kRounds; ++r) {
         const int64_t i = base + r * kThreads + threadIdx.x;
-        if (i < n) atomicAdd(&h[(keys[i] >> shift) & 0xff], 1);
+        k[r] = i < n ? keys[i] : 0;
     }
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r)
+        if (base + r * kThreads + threadIdx.x < n) atomicAdd(&h[(k[r] >> shift) & 0xff], 1);
     __syncthreads();
     hist[static_cast<int64_t>(threadIdx.x) * nb + blockIdx.x] = h[threadIdx.x];
 }
@@ -79,16 +97,16 @@ __global__ __launch_bounds__(kThreads) void k_radix_rows(const int32_t* __restri
     if (threadIdx.x == 0) tot[blockIdx.x] = run;
 }
 
-// Stable scatter of one tile: every key's rank among the tile's keys of its digit (rounds
-// in order, wavefronts in order, lanes by ballot), then the tile sorted by digit in LDS,
-// then written out digit run by digit run, consecutive threads to consecutive addresses.
+// Stable scatter of one tile: wavefront w ranks keys [w part, (w + 1) part) of the tile in
+// order, 64 at a time.
+template <int kRounds>
 __global__ __launch_bounds__(kThreads) void k_radix_scatter(
     const uint32_t* __restrict__ keys, const int32_t* __restrict__ vals, int64_t n, int shift,
     int64_t nb, const int32_t* __restrict__ offs, const int32_t* __restrict__ tot,
     uint32_t* __restrict__ keys_out, int32_t* __restrict__ vals_out) {
-    __shared__ int wcnt[kWaves][256];
-    __shared__ int tcnt[256];
-    __shared__ int loff[256];
+    constexpr int kTile = kThreads * kRounds;
+    __shared__ int wcnt[kWaves][256];  // counts of a wavefront, then its digits' first places
+    __shared__ int loff[256];          // a digit's first place in the sorted tile
     __shared__ int scan_sh[kWaves];
     __shared__ int64_t run[256];
     __shared__ uint32_t sk[kTile];
@@ -96,31 +114,28 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(
     const int tid = threadIdx.x;
     const int lane = __lane_id();
     const int w = tid / kWave;
-    {  // start of the digit's run: the totals of the smaller digits plus this block's row offset
-        const int before = block_excl_scan(tot[tid], scan_sh);
-        run[tid] = static_cast<int64_t>(before) + offs[static_cast<int64_t>(tid) * nb + blockIdx.x];
-    }
-    tcnt[tid] = 0;
-    const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
     const int64_t base = static_cast<int64_t>(blockIdx.x) * kTile;
+    const int64_t first = base + w * (kWave * kRounds) + lane;
     uint32_t kk[kRounds];
     int32_t vv[kRounds];
     int rk[kRounds];
 #pragma unroll
     for (int r = 0; r < kRounds; ++r) {
+        const int64_t i = first + r * kWave;
+        kk[r] = i < n ? keys[i] : 0;
+        vv[r] = i < n ? (vals ? vals[i] : static_cast<int32_t>(i)) : 0;
+    }
+    {  // start of the digit's run: the totals of the smaller digits plus this block's row offset
+        const int row = offs[static_cast<int64_t>(tid) * nb + blockIdx.x];
+        run[tid] = static_cast<int64_t>(block_excl_scan(tot[tid], scan_sh)) + row;
+    }
 #pragma unroll
-        for (int k = 0; k < kWaves; ++k) wcnt[k][tid] = 0;
-        __syncthreads();
-        const int64_t i = base + r * kThreads + tid;
-        const bool valid = i < n;
-        uint32_t key = 0;
-        int32_t val = 0;
-        int digit = 0;
-        if (valid) {
-            key = keys[i];
-            val = vals ? vals[i] : static_cast<int32_t>(i);
-            digit = (key >> shift) & 0xff;
-        }
+    for (int k = 0; k < 256; k += kWave) wcnt[w][k + lane] = 0;
+    const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+        const bool valid = first + r * kWave < n;
+        const int digit = (kk[r] >> shift) & 0xff;
         uint64_t peers = __ballot(valid);
 #pragma unroll
         for (int b = 0; b < 8; ++b) {
@@ -128,30 +143,33 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(
             const uint64_t m = __ballot(bit);
             peers &= bit ? m : ~m;
         }
+        // the wavefront's counts: read by every lane of the digit, then raised by its last
+        // (LDS accesses of one wavefront stay in order)
+        const int before = valid ? wcnt[w][digit] : 0;
         const int rank = __popcll(peers & lt);
-        if (valid && (peers >> lane) == 1ull) wcnt[w][digit] = rank + 1;
-        __syncthreads();
-        int lr = -1;
-        if (valid) {
-            lr = tcnt[digit] + rank;
-            for (int k = 0; k < w; ++k) lr += wcnt[k][digit];
-        }
-        kk[r] = key;
-        vv[r] = val;
-        rk[r] = lr;
-        __syncthreads();
-        int add = 0;
-#pragma unroll
-        for (int k = 0; k < kWaves; ++k) add += wcnt[k][tid];
-        tcnt[tid] += add;
+        __builtin_amdgcn_wave_barrier();
+        if (valid && (peers >> lane) == 1ull) wcnt[w][digit] = before + rank + 1;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        rk[r] = valid ? before + rank : -1;
     }
     __syncthreads();
-    loff[tid] = block_excl_scan(tcnt[tid], scan_sh);
+    int sum = 0;
+    int part[kWaves];
+#pragma unroll
+    for (int k = 0; k < kWaves; ++k) {
+        part[k] = sum;
+        sum += wcnt[k][tid];
+    }
+    const int at = block_excl_scan(sum, scan_sh);
+    loff[tid] = at;
+#pragma unroll
+    for (int k = 0; k < kWaves; ++k) wcnt[k][tid] = at + part[k];
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < kRounds; ++r)
         if (rk[r] >= 0) {
-            const int pos = loff[(kk[r] >> shift) & 0xff] + rk[r];
+            const int pos = wcnt[w][(kk[r] >> shift) & 0xff] + rk[r];
             sk[pos] = kk[r];
             sv[pos] = vv[r];
         }
@@ -173,8 +191,10 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(
 
 }  // namespace
 
+// Enough for every sort of at most n pairs: a caller may size it for its largest, and the
+// small tiles of just under kLargeKeys pairs need the longest tables up to 4M pairs.
 size_t radix_workspace_bytes(int64_t n) {
-    const int64_t nb = n > 0 ? (n + kTile - 1) / kTile : 1;
+    const int64_t nb = std::max(tiles_of(n), tiles_of(std::min(n, kLargeKeys - 1)));
     Carver c(nullptr);
     c.take<int32_t>(256 * nb);
     c.take<int32_t>(256 * nb);
@@ -188,7 +208,8 @@ int radix_sort_pairs(const uint32_t* keys_in, const int32_t* vals_in, uint32_t* 
                      int32_t* vals_out, int64_t n, int bits, void* ws, hipStream_t st) {
     if (n <= 0) return 0;
     if (n > INT32_MAX) return set_error(HALMA_E_LIMIT, "radix sort: too many keys");
-    const int64_t nb = (n + kTile - 1) / kTile;
+    const int64_t nb = tiles_of(n);
+    const bool large = n >= kLargeKeys;
     Carver c(ws);
     int32_t* hist = c.take<int32_t>(256 * nb);
     int32_t* offs = c.take<int32_t>(256 * nb);
@@ -203,12 +224,14 @@ int radix_sort_pairs(const uint32_t* keys_in, const int32_t* vals_in, uint32_t* 
         const bool to_out = ((passes - 1 - p) % 2) == 0;
         uint32_t* kout = to_out ? keys_out : tk;
         int32_t* vout = to_out ? vals_out : tv;
-        k_radix_hist<<<static_cast<unsigned>(nb), kThreads, 0, st>>>(kin, n, 8 * p, nb, hist);
+        auto hist_kernel = large ? k_radix_hist<kLarge> : k_radix_hist<kSmall>;
+        hist_kernel<<<static_cast<unsigned>(nb), kThreads, 0, st>>>(kin, n, 8 * p, nb, hist);
         HALMA_LAUNCH_CHECK();
         k_radix_rows<<<256, kThreads, 0, st>>>(hist, nb, offs, tot);
         HALMA_LAUNCH_CHECK();
-        k_radix_scatter<<<static_cast<unsigned>(nb), kThreads, 0, st>>>(kin, vin, n, 8 * p, nb,
-                                                                         offs, tot, kout, vout);
+        auto scatter = large ? k_radix_scatter<kLarge> : k_radix_scatter<kSmall>;
+        scatter<<<static_cast<unsigned>(nb), kThreads, 0, st>>>(kin, vin, n, 8 * p, nb, offs, tot,
+                                                                kout, vout);
         HALMA_LAUNCH_CHECK();
         kin = kout;
         vin = vout;
