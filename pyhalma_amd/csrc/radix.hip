@@ -9,8 +9,8 @@
 //
 // Bound by memory latency and the barriers of a tile.  A scatter pass of 8M pairs takes
 // 45 us (2.8 TB/s), of 1.9M 16, of 24k 5.2; with 256 keys ranked per round by the whole
-// workgroup, four barriers each, it took 56, 19 and 11.5.  Large inputs take tiles of 4096 keys (longer runs per digit), small ones of 1024 (more
-// blocks).
+// workgroup, four barriers each, it took 56, 19 and 11.5.  Large inputs take tiles of 4096
+// keys (longer runs per digit), small ones of 1024 (more blocks).
 #include "radix.h"
 
 #include <algorithm>
