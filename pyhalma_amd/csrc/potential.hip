@@ -236,7 +236,7 @@ int plan_pot(int64_t H, const int64_t* src_off, const int64_t* tst_off, PotPlan&
     const int64_t waves = static_cast<int64_t>(cus) * t.waves_per_cu;
     plan.grid = static_cast<int>(waves / 4);
     const int64_t target = waves * t.items_per_wave;
-    int64_t base_items = 0;
+    int64_t base_items = 0, min_items = 0;
     double work = 0.0;
     for (int64_t h = 0; h < H; ++h) {
         const int64_t ns = src_off[h + 1] - src_off[h];
@@ -244,8 +244,17 @@ int plan_pot(int64_t H, const int64_t* src_off, const int64_t* tst_off, PotPlan&
         if (ns < 0 || nt < 0 || ns > INT32_MAX || nt > INT32_MAX)
             return set_error(HALMA_E_ARG, "halo %lld: bad offsets", (long long)h);
         base_items += (nt + tile - 1) / tile;
+        min_items += (nt + tile - 1) / tile * ((ns + t.min_chunk - 1) / t.min_chunk);
         work += static_cast<double>(ns) * static_cast<double>(nt);
     }
+    // A launch that leaves SIMDs without two wavefronts at the tuned smallest chunk is a
+    // chain of one wavefront's latencies (3001 sources on 797 tests: 42 items, 74 us):
+    // smaller chunks until it has them, 64 sources at the least (329 items, 12 us).
+    int64_t min_chunk = t.min_chunk;
+    const int64_t two_waves = static_cast<int64_t>(cus) * 8;
+    if (min_items < two_waves)
+        min_chunk = std::min<int64_t>(
+            min_chunk, std::max<int64_t>(64, min_chunk * min_items / two_waves / 8 * 8));
     int64_t part = 0;
     std::vector<int64_t> key(H);
     for (int64_t h = 0; h < H; ++h) {
@@ -257,7 +266,7 @@ int plan_pot(int64_t H, const int64_t* src_off, const int64_t* tst_off, PotPlan&
             const double want = static_cast<double>(target) *
                                 (static_cast<double>(ns) * static_cast<double>(nt) / work) /
                                 static_cast<double>(tiles);
-            const int64_t max_ch = std::max<int64_t>(1, ns / t.min_chunk);
+            const int64_t max_ch = std::max<int64_t>(1, ns / min_chunk);
             nch = std::min<int64_t>(max_ch, std::max<int64_t>(1, static_cast<int64_t>(want)));
         }
         int64_t chunk = ns > 0 ? (ns + nch - 1) / nch : 1;
