@@ -268,7 +268,9 @@ __global__ __launch_bounds__(1024) void k_pot_sym_fine(const float4* __restrict_
 // The slots of one tile launch added into each affected member's FP64 sum (out, cleared
 // before the first launch): segment s = {halo, first member, count, role << 24 | local
 // slots}; the member adds its local slots 0 .. nloc - 1 in order, then, on a diagonal
-// tile, the diagonal slot.  With one band a member's slots 0..nb are added in order.
+// tile, the diagonal slot.  With one band a member's slots 0..nb are added in order.  Bound
+// by reading the slots: 128 workgroups to a segment, since a launch of few large haloes has
+// few segments (24 gas haloes of 1e3-2e5 cells: 62 -> 22.6 us a launch against 32).
 __global__ __launch_bounds__(256) void k_sym_merge_tile(const SymDesc* __restrict__ halos,
                                                         const int4* __restrict__ segs, int nseg,
                                                         const int64_t* __restrict__ member_base,
@@ -559,7 +561,7 @@ int halma_pot_sum_self_batched(int64_t n_halo, const int64_t* offsets, const flo
             HALMA_LAUNCH_CHECK();
         }
         if (ns > 0) {
-            const dim3 mg(32, static_cast<unsigned>(std::min<int64_t>(ns, 4096)));
+            const dim3 mg(128, static_cast<unsigned>(std::min<int64_t>(ns, 4096)));
             k_sym_merge_tile<<<mg, 256, 0, st>>>(w.halos, w.segs + s0, static_cast<int>(ns),
                                                  w.base, w.part, o);
             HALMA_LAUNCH_CHECK();
