@@ -528,6 +528,19 @@ int halma_refine_centres(int64_t n_halo, const int64_t *offsets, const float *m,
                          double *centres, double *S, int32_t *iters, double *steps,
                          void *workspace, size_t workspace_bytes, void *stream);
 
+/* Per-halo sums over CSR ranges (HOST offsets, n_halo+1, indexing the arrays), double-double,
+ * rounded once to FP64.  halma_gas_masses: four values per halo from cell masses,
+ * temperatures and bound flags: total mass, cold bound fraction (0 without mass), cold
+ * unbound mass, hot unbound mass (cold: T < 5e4; halo_gas.py:466-489).
+ * halma_weighted_sums: sum of m[i] * s[i] (FP64 products).  Stream-ordered. */
+size_t halma_halo_sums_workspace_size(int64_t n_halo, const int64_t *offsets);
+int halma_gas_masses(int64_t n_halo, const int64_t *offsets, const void *m, int m_dtype,
+                     const void *temp, int temp_dtype, const uint8_t *bound, double *out,
+                     void *workspace, size_t workspace_bytes, void *stream);
+int halma_weighted_sums(int64_t n_halo, const int64_t *offsets, const void *m, int m_dtype,
+                        const double *s, double *out, void *workspace, size_t workspace_bytes,
+                        void *stream);
+
 /* Tuning knobs of the FP32 pair kernels (set by the autotuner; read back with get).
  *   HALMA_TUNE_TESTS_PER_LANE : test particles per lane (1, 2, 4)
  *   HALMA_TUNE_SUBTILE        : sources per plain FP32 sub-tile before the Kahan add

@@ -47,6 +47,10 @@ SIGNATURES = {
                                           _dbl, _p, _p, _p, _p, _size, _p]),
     "halma_pot_soft_batched_packed": (_c.c_int, [_i64, _i64p, _p, _i64p, _p, _p, _p, _dbl, _p,
                                                  _p, _p, _p, _size, _p]),
+    "halma_halo_sums_workspace_size": (_size, [_i64, _i64p]),
+    "halma_gas_masses": (_c.c_int, [_i64, _i64p, _p, _c.c_int, _p, _c.c_int, _p, _p, _p, _size,
+                                    _p]),
+    "halma_weighted_sums": (_c.c_int, [_i64, _i64p, _p, _c.c_int, _p, _p, _p, _size, _p]),
     "halma_refine_centres_workspace_size": (_size, [_i64, _i64p, _c.c_int]),
     "halma_refine_centres": (_c.c_int, [_i64, _i64p, _p, _p, _p, _p, _dbl, _dbl, _c.c_int, _p,
                                         _p, _p, _p, _p, _size, _p]),

@@ -135,17 +135,6 @@ def soft_potential(tests, src_pos, src_m, src_off, tst_off, eps, aux=None):
                                np.asarray(tst_off, np.int64), float(eps), aux)
 
 
-def _halo_sums(v, offsets_dev, offsets):
-    """Per-halo FP64 sums of v over the CSR ranges (the library's double-double group
-    reduction: a fixed order, no atomics)."""
-    n = int(v.numel())
-    grp = engine.Groups(torch.arange(max(n, 1), dtype=torch.int32, device=v.device),
-                        offsets_dev, offsets)
-    z = torch.zeros(max(n, 1), dtype=torch.float32, device=v.device)
-    vv = v if n else torch.zeros(1, dtype=torch.float64, device=v.device)
-    return engine.group_reduce(grp, z, z, z, vv)[:, 0]
-
-
 class HaloPotentialEnergy(torch.autograd.Function):
     """W_h = -G/2 sum_{i in h} m_i S_i (one per halo, float64) for members pos (N, 3) and
     masses m (N,) in halo order (CSR host offsets), S_i the softened sum over the other
@@ -163,10 +152,9 @@ class HaloPotentialEnergy(torch.autograd.Function):
         fused = bool(fuse) and ctx.needs_input_grad[0]
         r = engine.pot_soft_self(offsets, packed, eps, pot=True, acc=fused)
         S = r["pot"]
-        off_dev = engine.to_dev(offsets, np.int64)
-        W = -0.5 * G * _halo_sums(m.detach().double() * S, off_dev, offsets)
+        W = -0.5 * G * engine.weighted_sums(offsets, m.detach(), S)
         ctx.save_for_backward(m, S)
-        ctx.packed, ctx.offsets, ctx.off_dev, ctx.eps, ctx.G = packed, offsets, off_dev, eps, G
+        ctx.packed, ctx.offsets, ctx.eps, ctx.G = packed, offsets, eps, G
         ctx.acc = r["acc"] if fused else None
         ctx.pos_dtype = pos.dtype
         return W

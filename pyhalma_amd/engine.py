@@ -228,6 +228,48 @@ def refine_centres(offsets, m, x, y, z, seeds, eps, tol, max_iter):
     return c, S, iters, steps
 
 
+def gas_masses(offsets, m, temp, bound):
+    """Per halo (CSR host offsets over the cells): total mass, cold bound fraction, cold
+    unbound mass, hot unbound mass (halma_gas_masses); (H, 4) float64 device tensor."""
+    from .device import dtype_flag
+    L = _lib_()
+    offsets = np.asarray(offsets, np.int64)
+    H = len(offsets) - 1
+    m, temp = _vec(m), _vec(temp)
+    n = int(m.numel())
+    if temp.numel() != n or bound.numel() != n or (H > 0 and int(offsets[-1]) > n):
+        raise ValueError("cell arrays must have equal lengths, not shorter than the offsets")
+    out = torch.empty((max(H, 0), 4), dtype=torch.float64, device=m.device)
+    if H <= 0:
+        return out
+    off = _lib.i64_array(offsets)
+    ws = workspace(L.halma_halo_sums_workspace_size(H, off))
+    rc = L.halma_gas_masses(H, off, ptr(m), dtype_flag(m), ptr(temp), dtype_flag(temp), ptr(bound),
+                            ptr(out), ptr(ws), ws.numel(), stream_ptr())
+    _lib.check(rc, "halma_gas_masses")
+    return out
+
+
+def weighted_sums(offsets, m, s):
+    """Per halo (CSR host offsets) the sum of m * s, s float64 (halma_weighted_sums)."""
+    from .device import dtype_flag
+    L = _lib_()
+    offsets = np.asarray(offsets, np.int64)
+    H = len(offsets) - 1
+    m, s = _vec(m), to_dev(s, np.float64)
+    if m.numel() != s.numel() or (H > 0 and int(offsets[-1]) > m.numel()):
+        raise ValueError("m and s must have equal lengths, not shorter than the offsets")
+    out = torch.empty(max(H, 0), dtype=torch.float64, device=m.device)
+    if H <= 0:
+        return out
+    off = _lib.i64_array(offsets)
+    ws = workspace(L.halma_halo_sums_workspace_size(H, off))
+    rc = L.halma_weighted_sums(H, off, ptr(m), dtype_flag(m), ptr(s), ptr(out), ptr(ws),
+                               ws.numel(), stream_ptr())
+    _lib.check(rc, "halma_weighted_sums")
+    return out
+
+
 def energy_test_batched(src_off, m, x, y, z, tst_off, tx, ty, tz, vx, vy, vz, halo_v,
                         factor, with_pot=False, stats=None):
     """One energy test per test particle, every halo at once (halma_energy_test_batched):

@@ -242,10 +242,7 @@ def RPS_batched(gas, gas_offsets, halo_v, dm=None, stars=None, stats=None):
     The gas self-term runs on the symmetric kernel (each cell pair once), the dark matter
     and stars against the cells on the chunked kernel (halma_energy_test_self_batched).
     ``stats`` (a dict) receives the energy test's counters (engine.energy_test_batched)."""
-    import torch
-
     from . import engine
-    from .device import to_dev
     gas_offsets = np.asarray(gas_offsets, np.int64)
     H = len(gas_offsets) - 1
     gx, gy, gz, gvx, gvy, gvz, gm, gt = gas
@@ -258,26 +255,4 @@ def RPS_batched(gas, gas_offsets, halo_v, dm=None, stars=None, stats=None):
         ext = dict(ext_off=ext_off, em=em, ex=ex, ey=ey, ez=ez)
     bound, _, _ = engine.energy_test_self_batched(gas_offsets, gm, gx, gy, gz, gvx, gvy, gvz,
                                                   halo_v, 2.0, stats=stats, **ext)
-    mass = to_dev(gm, np.float64)
-    temp = to_dev(gt, np.float64)
-    dev = mass.device
-    b = bound.to(torch.bool)
-    cold = temp < 5 * 1e4
-    zero = torch.zeros_like(mass)
-    # the four per-halo sums with the library's group reduction over the CSR ranges
-    # (double-double, fixed order, no atomics on the few hundred per-halo totals)
-    n = int(mass.numel())
-    grp = engine.Groups(torch.arange(max(n, 1), dtype=torch.int32, device=dev),
-                        to_dev(gas_offsets, np.int64), gas_offsets)
-    cx, cy, cz = engine._coords(gx, gy, gz)
-
-    def seg(v):
-        return engine.group_reduce(grp, cx, cy, cz, v)[:, 0]
-
-    total = seg(mass)
-    cold_bound = seg(torch.where(cold & b, mass, zero))
-    unb_cold = seg(torch.where(cold & ~b, mass, zero))
-    unb_hot = seg(torch.where(~cold & ~b, mass, zero))
-    frac = torch.where(total != 0, cold_bound / torch.where(total != 0, total, 1.0),
-                       torch.zeros_like(total))
-    return torch.stack([total, frac, unb_cold, unb_hot], 1).cpu().numpy(), bound
+    return engine.gas_masses(gas_offsets, gm, gt, bound).cpu().numpy(), bound
