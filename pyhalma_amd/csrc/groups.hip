@@ -228,43 +228,65 @@ struct Src {
 };
 
 // All of a group's block reductions in one LDS round: every wave reduces its eight
-// double-double sums (shuffle tree), three minima, three maxima and the grain exponent,
-// writes them to LDS, and thread q then folds quantity q over the waves in wave order (the
-// order of block_dd_sum / block_max), so the results are those of the separate
-// reductions with two barriers instead of forty-five.
-constexpr int kGrpQ = 8 * 2 + 6 + 1;
+// double-double sums and eight minima (three coordinates, the three negated, the grain
+// exponent), writes them to LDS, and thread q then folds quantity q over the waves in wave
+// order: two barriers.  Within a wave the trees are halved as they go: at each of the first
+// three levels a lane keeps half of its quantities and hands the other half to its partner,
+// so eight sums take 4 + 2 + 1 + 3 additions of a lane instead of 6 x 8 (the trees of 16
+// wavefronts were a quarter of the kernel's time).  Lane 8 q ends with quantity q.
+constexpr int kGrpQ = 8 * 2 + 8;
+
+template <int H>
+__device__ __forceinline__ void halve_dd(double (&v)[8][2]) {
+    const bool up = (__lane_id() & (8 * H)) != 0;
+#pragma unroll
+    for (int k = 0; k < H; ++k) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const double keep = up ? v[k + H][c] : v[k][c];
+            const double give = up ? v[k][c] : v[k + H][c];
+            v[k][c] = keep;
+            v[k + H][c] = __shfl_xor(give, 8 * H, kWave);
+        }
+        dd_add_dd(v[k][0], v[k][1], v[k + H][0], v[k + H][1]);
+    }
+}
+
+template <int H>
+__device__ __forceinline__ void halve_min(double (&v)[8]) {
+    const bool up = (__lane_id() & (8 * H)) != 0;
+#pragma unroll
+    for (int k = 0; k < H; ++k) {
+        const double keep = up ? v[k + H] : v[k], give = up ? v[k] : v[k + H];
+        v[k] = fmin(keep, __shfl_xor(give, 8 * H, kWave));
+    }
+}
 
 // Only the first nw wavefronts hold members (the others skip the trees and are left out
-// of the fold), so a small group pays for the trees of the wavefronts it uses.
-__device__ void block_group_reduce(double (&acc)[8][2], double (&lo)[3], double (&hi)[3],
-                                   int& gexp, double* sh /* kGrpQ * kMaxWaves */, int nw) {
+// of the fold), so a small group pays for the trees of the wavefronts it uses.  The result
+// is left in LDS: sums at 2 q, minima at 16 + q of the returned row.
+__device__ const double* block_group_reduce(double (&acc)[8][2], double (&mn)[8],
+                                            double* sh /* kGrpQ * (waves + 1) */, int nw) {
     const int w = threadIdx.x / kWave;
     if (w < nw) {
-        for (int k = 0; k < 8; ++k)
-            for (int s = 32; s >= 1; s >>= 1) {
-                const double h2 = __shfl_down(acc[k][0], s, kWave);
-                const double l2 = __shfl_down(acc[k][1], s, kWave);
-                dd_add_dd(acc[k][0], acc[k][1], h2, l2);
-            }
-        for (int d = 0; d < 3; ++d)
-            for (int s = 32; s >= 1; s >>= 1) {
-                lo[d] = fmin(lo[d], __shfl_down(lo[d], s, kWave));
-                hi[d] = fmax(hi[d], __shfl_down(hi[d], s, kWave));
-            }
-        for (int s = 32; s >= 1; s >>= 1) gexp = min(gexp, __shfl_down(gexp, s, kWave));
-    }
-    __syncthreads();
-    if (w < nw && __lane_id() == 0) {
-        double* o = sh + w * kGrpQ;
-        for (int k = 0; k < 8; ++k) {
-            o[2 * k] = acc[k][0];
-            o[2 * k + 1] = acc[k][1];
+        halve_dd<4>(acc);
+        halve_dd<2>(acc);
+        halve_dd<1>(acc);
+        halve_min<4>(mn);
+        halve_min<2>(mn);
+        halve_min<1>(mn);
+        for (int s = 4; s >= 1; s >>= 1) {
+            const double h2 = __shfl_down(acc[0][0], s, kWave);
+            const double l2 = __shfl_down(acc[0][1], s, kWave);
+            dd_add_dd(acc[0][0], acc[0][1], h2, l2);
+            mn[0] = fmin(mn[0], __shfl_down(mn[0], s, kWave));
         }
-        for (int d = 0; d < 3; ++d) {
-            o[16 + d] = lo[d];
-            o[19 + d] = hi[d];
+        const int q = __lane_id() / 8;
+        if ((__lane_id() & 7) == 0) {
+            sh[w * kGrpQ + 2 * q] = acc[0][0];
+            sh[w * kGrpQ + 2 * q + 1] = acc[0][1];
+            sh[w * kGrpQ + 16 + q] = mn[0];
         }
-        o[22] = static_cast<double>(gexp);
     }
     __syncthreads();
     const int q = threadIdx.x;
@@ -273,43 +295,33 @@ __device__ void block_group_reduce(double (&acc)[8][2], double (&lo)[3], double 
         for (int k = 1; k < nw; ++k) dd_add_dd(h, l, sh[k * kGrpQ + 2 * q], sh[k * kGrpQ + 2 * q + 1]);
         sh[nw * kGrpQ + 2 * q] = h;
         sh[nw * kGrpQ + 2 * q + 1] = l;
-    } else if (q < 11) {
-        double v = sh[16 + (q - 8)];
-        for (int k = 1; k < nw; ++k) v = fmin(v, sh[k * kGrpQ + 16 + (q - 8)]);
-        sh[nw * kGrpQ + 16 + (q - 8)] = v;
-    } else if (q < 14) {
-        double v = sh[19 + (q - 11)];
-        for (int k = 1; k < nw; ++k) v = fmax(v, sh[k * kGrpQ + 19 + (q - 11)]);
-        sh[nw * kGrpQ + 19 + (q - 11)] = v;
-    } else if (q == 14) {
-        double v = sh[22];
-        for (int k = 1; k < nw; ++k) v = fmin(v, sh[k * kGrpQ + 22]);
-        sh[nw * kGrpQ + 22] = v;
+    } else if (q < 16) {
+        double v = sh[q + 8];
+        for (int k = 1; k < nw; ++k) v = fmin(v, sh[k * kGrpQ + q + 8]);
+        sh[nw * kGrpQ + q + 8] = v;
     }
     __syncthreads();
-    const double* r = sh + nw * kGrpQ;
-    for (int k = 0; k < 8; ++k) {
-        acc[k][0] = r[2 * k];
-        acc[k][1] = r[2 * k + 1];
-    }
-    for (int d = 0; d < 3; ++d) {
-        lo[d] = r[16 + d];
-        hi[d] = r[19 + d];
-    }
-    gexp = static_cast<int>(r[22]);
-    __syncthreads();
+    return sh + nw * kGrpQ;
 }
 
-template <int DT>
-__global__ __launch_bounds__(kBig) void k_group_reduce(Src s, const int64_t* __restrict__ off,
-                                                           const int32_t* __restrict__ mem,
-                                                           int64_t G,
-                                                           const double* __restrict__ centres,
-                                                           double* __restrict__ out) {
-    __shared__ double sh[kGrpQ * (kMaxWaves + 1)];
+// One workgroup per group of first < members <= last: 1024 threads for the large groups,
+// 256 for those of at most kSmallGroup, of which a CU then holds several at once and whose
+// barriers, trees and folds span four wavefronts (2.1M members in 1000 groups of up to
+// 20000: 79 us with 1024 threads for every group, 68 us in the two launches; one group of 24k
+// 40 -> 32 us with the shorter trees).  Bound by one CU's gathers for its largest group.
+constexpr int64_t kSmallGroup = 4096;
+
+template <int DT, int T>
+__global__ __launch_bounds__(T, 4) void k_group_reduce(Src s, const int64_t* __restrict__ off,
+                                                    const int32_t* __restrict__ mem, int64_t G,
+                                                    int64_t first, int64_t last,
+                                                    const double* __restrict__ centres,
+                                                    double* __restrict__ out) {
+    __shared__ double sh[kGrpQ * (T / kWave + 1)];
     __shared__ double cen[3];
     for (int64_t g = blockIdx.x; g < G; g += gridDim.x) {
         const int64_t b = off[g], e = off[g + 1];
+        if (e - b <= first || e - b > last) continue;  // block-uniform
         double acc[8][2];  // M, Mx, My, Mz, Mvx, Mvy, Mvz, sum |m|
         for (int k = 0; k < 8; ++k) acc[k][0] = acc[k][1] = 0.0;
         double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
@@ -317,7 +329,7 @@ __global__ __launch_bounds__(kBig) void k_group_reduce(Src s, const int64_t* __r
         // wavefronts that take members: enough for four or more members per lane
         const int64_t ng = e - b;
         const int nw = static_cast<int>(std::min<int64_t>(
-            std::max<int64_t>((ng + 4 * kWave - 1) / (4 * kWave), 1), blockDim.x / kWave));
+            std::max<int64_t>((ng + 4 * kWave - 1) / (4 * kWave), 1), T / kWave));
         const int nthr = nw * kWave;
         // four members per thread in flight: their indices, then mass and position, then
         // velocity; every accumulator takes the members in the same order as one member
@@ -367,22 +379,23 @@ __global__ __launch_bounds__(kBig) void k_group_reduce(Src s, const int64_t* __r
                 for (int d = 0; d < 3; ++d) dd_add(acc[4 + d][0], acc[4 + d][1], mu[u] * f[u][d]);
             }
         }
-        block_group_reduce(acc, lo, hi, gexp, sh, nw);
-        const double* bl = lo;
-        const double* bh = hi;
+        double mn[8] = {lo[0], lo[1], lo[2], -hi[0], -hi[1], -hi[2],
+                        static_cast<double>(gexp), 0.0};
+        const double* r = block_group_reduce(acc, mn, sh, nw);
         if (threadIdx.x == 0) {
             double* o = out + g * kRedFields;
-            const double M = acc[0][0] + acc[0][1];
+            const double M = r[0] + r[1];
             o[0] = M;
             for (int d = 0; d < 3; ++d) {
-                const double num = acc[1 + d][0] + acc[1 + d][1];
+                const double num = r[2 + 2 * d] + r[3 + 2 * d];
                 o[1 + d] = M > 0.0 ? num / M : 0.0;
-                const double vn = acc[4 + d][0] + acc[4 + d][1];
+                const double vn = r[8 + 2 * d] + r[9 + 2 * d];
                 o[4 + d] = M > 0.0 ? vn / M : 0.0;
-                o[8 + d] = bl[d];
-                o[11 + d] = bh[d];
+                o[8 + d] = r[16 + d];
+                o[11 + d] = -r[19 + d];
             }
-            const double total_abs = (acc[7][0] + acc[7][1]) * (1.0 + 1e-12);
+            const double total_abs = (r[14] + r[15]) * (1.0 + 1e-12);
+            gexp = static_cast<int>(r[22]);
             o[14] = total_abs;
             // every partial sum of any subset is an integer multiple of 2^gexp below 2^53
             // of those units -> exact in FP64 whatever the order
@@ -417,13 +430,22 @@ __global__ __launch_bounds__(kBig) void k_group_reduce(Src s, const int64_t* __r
 // ------------------------------------------------------------- density peak ----
 struct Grid1 {
     double start, step, stop;
+    double inv, tie;  // 1 / step; how near a midpoint (in steps) the rounded nodes may differ
     __device__ __forceinline__ double node(int k) const {
         return k == kNodes - 1 ? stop : static_cast<double>(k) * step + start;
     }
 };
 
-// first k minimising |node(k) - v| (np.argmin over the 50 nodes)
+// first k minimising |node(k) - v| (np.argmin over the 50 nodes).  A value further than
+// `tie` from the middle of its two nodes is nearest to the one on its side whatever the
+// rounding (~10 instructions an axis instead of ~150 of the compared distances, which the
+// whole kernel was bound by); a value within it, outside the grid or not finite compares.
 __device__ int nearest_node(const Grid1& g, double v) {
+    {
+        const double t = (v - g.start) * g.inv, k = floor(t);
+        if (t >= 0.0 && t < static_cast<double>(kNodes - 1) && fabs((t - k) - 0.5) > g.tie)
+            return static_cast<int>(k) + (t - k > 0.5 ? 1 : 0);
+    }
     int best = 0;
     if (g.step > 0.0 && isfinite(v)) {
         const double t = (v - g.start) / g.step;
@@ -477,6 +499,12 @@ __device__ __forceinline__ void grids_of(const PeakArgs& a, int64_t g, Grid1* gr
         gr[d].start = start;
         gr[d].stop = stop;
         gr[d].step = (stop - start) / static_cast<double>(kNodes - 1);
+        // t is off by at most 49 * 5 * 2^-53 < 1e-13 steps (difference, reciprocal,
+        // product); a node by the rounding of k * step and of the sum, a distance by its own:
+        // 4 units of the larger end, twice for the two nodes.  Not a number or infinite
+        // (a grid of no width): every value compares.
+        gr[d].inv = 1.0 / gr[d].step;
+        gr[d].tie = 1e-13 + 16.0 * 0x1p-53 * fmax(fabs(start), fabs(stop)) * gr[d].inv;
     }
 }
 
@@ -511,6 +539,10 @@ __device__ void write_peak(const PeakArgs& a, const Grid1* gr, int64_t g, int no
     a.out[3 * g + 2] = gr[2].node(iz);
 }
 
+// slots of a thread read together: the dense grid's 125000 nodes are a chain of 122 loads a
+// thread otherwise (58 -> 36 us a group)
+constexpr int kPickBatch = 8;
+
 // Given (node, approximate mass) pairs held by the block (a thread-strided view through
 // get()), picks the winner: exact sums -> first node with the maximum; otherwise nodes
 // within the band of the maximum are re-summed in member order by one thread.
@@ -518,10 +550,18 @@ template <class Get>
 __device__ int pick_peak(const PeakArgs& a, const Grid1* gr, int64_t g, int64_t b, int64_t e,
                          int nslots, Get get, double* shd, int* shi, int* cand) {
     double vmax = -INFINITY;
-    for (int k = threadIdx.x; k < nslots; k += blockDim.x) {
-        int node;
-        double v;
-        if (get(k, node, v)) vmax = fmax(vmax, v);
+    for (int k0 = threadIdx.x; k0 < nslots; k0 += kPickBatch * blockDim.x) {
+        int node[kPickBatch];
+        double v[kPickBatch];
+        bool ok[kPickBatch];
+#pragma unroll
+        for (int u = 0; u < kPickBatch; ++u) {
+            const int k = min(k0 + u * static_cast<int>(blockDim.x), nslots - 1);
+            ok[u] = get(k, node[u], v[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < kPickBatch; ++u)
+            if (ok[u]) vmax = fmax(vmax, v[u]);
     }
     vmax = block_max(vmax, shd);
     if (!(vmax > 0.0)) return -1;
@@ -530,14 +570,22 @@ __device__ int pick_peak(const PeakArgs& a, const Grid1* gr, int64_t g, int64_t 
     const double band = exact ? 0.0 : 2.0 * static_cast<double>(e - b) * 0x1p-53 * r[14];
     int first = INT32_MAX;
     int ncand = 0;
-    for (int k = threadIdx.x; k < nslots; k += blockDim.x) {
-        int node;
-        double v;
-        if (get(k, node, v) && v >= vmax - 2.0 * band) {
-            first = min(first, node);
+    for (int k0 = threadIdx.x; k0 < nslots; k0 += kPickBatch * blockDim.x) {
+        int node[kPickBatch];
+        double v[kPickBatch];
+        bool ok[kPickBatch];
+#pragma unroll
+        for (int u = 0; u < kPickBatch; ++u) {
+            const int k = k0 + u * static_cast<int>(blockDim.x);
+            ok[u] = get(min(k, nslots - 1), node[u], v[u]) && k < nslots;
+        }
+#pragma unroll
+        for (int u = 0; u < kPickBatch; ++u) {
+            if (!ok[u] || !(v[u] >= vmax - 2.0 * band)) continue;
+            first = min(first, node[u]);
             if (!exact) {
                 const int at = atomicAdd(&shi[kMaxWaves], 1);
-                if (at < kMaxCandidates) cand[at] = node;
+                if (at < kMaxCandidates) cand[at] = node[u];
             }
         }
     }
@@ -565,6 +613,8 @@ __device__ int pick_peak(const PeakArgs& a, const Grid1* gr, int64_t g, int64_t 
     return winner;
 }
 
+// Bound by one CU's work for the largest group (2.1M members in 1000 groups of up to 20000:
+// 71 us when every value compared its distances to five nodes an axis, 53 us now).
 template <int DT>
 __global__ __launch_bounds__(kBig) void k_density_peak(PeakArgs a) {
     __shared__ int skey[kTable];
@@ -836,6 +886,19 @@ Src make_src(const void* x, const void* y, const void* z, int pos_t, const void*
 }
 
 bool bad_dtype(int t) { return t != HALMA_F32 && t != HALMA_F64; }
+
+template <int DT>
+int run_group_reduce(const Src& s, const int64_t* off, const int32_t* mem, int64_t G,
+                     const double* centres, double* out, hipStream_t st) {
+    const unsigned grid = static_cast<unsigned>(G < 65536 ? G : 65536);
+    k_group_reduce<DT, kBig><<<grid, kBig, 0, st>>>(s, off, mem, G, kSmallGroup, INT64_MAX,
+                                                    centres, out);
+    HALMA_LAUNCH_CHECK();
+    k_group_reduce<DT, kThreads><<<grid, kThreads, 0, st>>>(s, off, mem, G, -1, kSmallGroup,
+                                                            centres, out);
+    HALMA_LAUNCH_CHECK();
+    return 0;
+}
 }  // namespace
 
 extern "C" {
@@ -873,17 +936,11 @@ int halma_group_reduce(int64_t n_groups, const int64_t* offsets, const int32_t* 
         return set_error(HALMA_E_ARG, "bad dtype");
     if (vx && (!vy || !vz)) return set_error(HALMA_E_ARG, "velocities need vx, vy and vz");
     Src s = make_src(x, y, z, pos_dtype, vx, vy, vz, vel_dtype, m, mass_dtype);
-    const unsigned grid = static_cast<unsigned>(n_groups < 65536 ? n_groups : 65536);
     const int dt = common_dtype(pos_dtype, mass_dtype, vx ? vel_dtype : mass_dtype);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (dt == 1)
-        k_group_reduce<1><<<grid, kBig, 0, st>>>(s, offsets, members, n_groups, centres, out);
-    else if (dt == 2)
-        k_group_reduce<2><<<grid, kBig, 0, st>>>(s, offsets, members, n_groups, centres, out);
-    else
-        k_group_reduce<0><<<grid, kBig, 0, st>>>(s, offsets, members, n_groups, centres, out);
-    HALMA_LAUNCH_CHECK();
-    return 0;
+    return dt == 1   ? run_group_reduce<1>(s, offsets, members, n_groups, centres, out, st)
+           : dt == 2 ? run_group_reduce<2>(s, offsets, members, n_groups, centres, out, st)
+                     : run_group_reduce<0>(s, offsets, members, n_groups, centres, out, st);
 }
 
 size_t halma_density_peak_workspace_size(int64_t n_groups) {
