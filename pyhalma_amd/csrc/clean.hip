@@ -68,12 +68,18 @@ __device__ __forceinline__ double node(const GridArgs& g, int h, int64_t k) {
     return k == 0 ? g.start[h] : (k == 1 ? g.g1[h] : g.start[h] + static_cast<double>(k) * g.d[h]);
 }
 
-// first k minimising |node(k) - xh| (np.argmin: the first of equal distances).  The
-// estimate's window is refined by descending the distances, which are unimodal in k
+// first k minimising |node(k) - xh| (np.argmin: the first of equal distances).  Of nodes
+// start + k d (k >= 2) a value further than `tie` steps from the middle of two is nearest to
+// the one on its side whatever the rounding; the others compare.  The estimate's window is refined by descending the distances, which are unimodal in k
 // (the nodes increase); a non-finite xh has every distance non-finite: node 0.
-__device__ int nearest(const GridArgs& g, int h, double xh) {
+__device__ int nearest(const GridArgs& g, int h, double xh, double inv, double tie) {
     const int64_t n = g.n[h];
     if (!isfinite(xh)) return 0;
+    {
+        const double t = (xh - g.start[h]) * inv, k = floor(t);
+        if (t >= 2.0 && t < static_cast<double>(n - 1) && fabs((t - k) - 0.5) > tie)
+            return static_cast<int>(k) + (t - k > 0.5 ? 1 : 0);
+    }
     const double est = floor((xh - g.start[h]) / g.d[h] + 0.5);
     const int64_t kc = est >= 0.0 ? (est <= static_cast<double>(n - 1) ? static_cast<int64_t>(est)
                                                                         : n - 1)
@@ -104,7 +110,9 @@ __device__ int nearest(const GridArgs& g, int h, double xh) {
 }
 
 // per member of S: its three node indices and its cell key within the group,
-// (ix n + iy) n + iz as two 32-bit words
+// (ix n + iy) n + iz as two 32-bit words.  Bound by the FP64 arithmetic of the nodes: 2M
+// members 35.4 us comparing five distances an axis, 25.8 us where only values near a midpoint
+// compare.
 __global__ void k_clean_cells(int64_t ns, const int32_t* __restrict__ s_mem,
                               const int32_t* __restrict__ s_grp, Particles p, GridArgs g,
                               int kbits, int composite, int32_t* __restrict__ ijk,
@@ -114,9 +122,13 @@ __global__ void k_clean_cells(int64_t ns, const int32_t* __restrict__ s_mem,
     const int64_t i = s_mem[k];
     const int h = s_grp[k];
     const double* c = g.centre + 3 * static_cast<int64_t>(h);
-    const int ix = nearest(g, h, ldf(p.x, p.pos_t, i) - c[0]);
-    const int iy = nearest(g, h, ldf(p.y, p.pos_t, i) - c[1]);
-    const int iz = nearest(g, h, ldf(p.z, p.pos_t, i) - c[2]);
+    // t <= n is off by at most 3 units (difference, reciprocal, product), a node by the
+    // rounding of k d and of the sum, in steps: 32 units of the larger of n and |start| / d
+    const double inv = 1.0 / g.d[h];
+    const double tie = 0x1p-48 * (static_cast<double>(g.n[h]) + fabs(g.start[h]) * inv);
+    const int ix = nearest(g, h, ldf(p.x, p.pos_t, i) - c[0], inv, tie);
+    const int iy = nearest(g, h, ldf(p.y, p.pos_t, i) - c[1], inv, tie);
+    const int iz = nearest(g, h, ldf(p.z, p.pos_t, i) - c[2], inv, tie);
     ijk[3 * k + 0] = ix;
     ijk[3 * k + 1] = iy;
     ijk[3 * k + 2] = iz;
@@ -141,10 +153,12 @@ __global__ void k_gather_u32(const uint32_t* __restrict__ src, const int32_t* __
 // head flags of the (group, cell) runs in sorted order
 __global__ void k_cell_heads(int64_t ns, const int32_t* __restrict__ order,
                              const uint32_t* __restrict__ klo, const uint32_t* __restrict__ khi,
-                             const int32_t* __restrict__ s_grp, int32_t* __restrict__ head) {
+                             const int32_t* __restrict__ s_grp, int32_t* __restrict__ head,
+                             int64_t* __restrict__ n_items) {
     const int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (k >= ns) return;
     int h = 1;
+    if (k == 0) *n_items = 0;
     if (k > 0) {
         const int32_t a = order[k], b = order[k - 1];
         h = (klo[a] != klo[b] || khi[a] != khi[b] || s_grp[a] != s_grp[b]) ? 1 : 0;
@@ -177,9 +191,10 @@ __device__ __forceinline__ void wave_dd(double& hi, double& lo) {
     }
 }
 
-// Cell statistics over work items: item = (cell, chunk of kChunk consecutive members of
-// the cell in sorted order), one wavefront per item, double-double partial sums folded
-// per cell in item order (fixed order: deterministic).
+// Cell statistics.  A cell of at most kChunk members takes one wavefront that reads its
+// members once (k_cell_small); a larger one is cut into items of kChunk consecutive members
+// in sorted order, a wavefront each, with the double-double partial sums folded per cell in
+// item order.  Both orders are fixed: deterministic.
 constexpr int kChunk = 256;
 
 __device__ __forceinline__ int64_t cell_end(const int64_t* begin, int64_t c, int64_t nseg,
@@ -187,18 +202,22 @@ __device__ __forceinline__ int64_t cell_end(const int64_t* begin, int64_t c, int
     return c + 1 < nseg ? begin[c + 1] : ns;
 }
 
-__global__ void k_cell_chunks(int64_t nseg, int64_t ns, const int64_t* __restrict__ begin,
-                              int32_t* __restrict__ nch) {
+// counts: [0] cells, [1] items (zeroed by k_cell_heads).  The items of a cell are
+// consecutive; which cell comes first does not matter to any sum.
+__global__ void k_cell_items(int64_t ns, int64_t* __restrict__ counts,
+                             const int64_t* __restrict__ begin, int64_t* __restrict__ ioff,
+                             int32_t* __restrict__ nch, int32_t* __restrict__ item_cell) {
     const int64_t c = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t nseg = counts[0];
     if (c >= nseg) return;
-    nch[c] = static_cast<int32_t>((cell_end(begin, c, nseg, ns) - begin[c] + kChunk - 1) / kChunk);
-}
-
-__global__ void k_cell_items(int64_t nseg, const int64_t* __restrict__ ioff,
-                             const int32_t* __restrict__ nch, int32_t* __restrict__ item_cell) {
-    const int64_t c = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (c >= nseg) return;
-    for (int t = 0; t < nch[c]; ++t) item_cell[ioff[c] + t] = static_cast<int32_t>(c);
+    const int64_t n = cell_end(begin, c, nseg, ns) - begin[c];
+    const int items = n > kChunk ? static_cast<int>((n + kChunk - 1) / kChunk) : 0;
+    nch[c] = items;
+    if (items == 0) return;
+    const int64_t at = static_cast<int64_t>(atomicAdd(
+        reinterpret_cast<unsigned long long*>(counts + 1), static_cast<unsigned long long>(items)));
+    ioff[c] = at;
+    for (int t = 0; t < items; ++t) item_cell[at + t] = static_cast<int32_t>(c);
 }
 
 struct CellArgs {
@@ -221,6 +240,76 @@ __device__ __forceinline__ void item_range(const CellArgs& a, int64_t it, int64_
     b = a.begin[c] + (it - a.ioff[c]) * kChunk;
     const int64_t ce = cell_end(a.begin, c, a.nseg, a.ns);
     e = b + kChunk < ce ? b + kChunk : ce;
+}
+
+// The statistics of a cell of at most kChunk members in one pass over them: up to four
+// members a lane stay in registers between the sums of v m and m and the dispersion, and the
+// tree of the four sums is halved at its first two levels (lanes 16 q .. 16 q + 15 hold
+// sum q).  Bound by the gathers (order, member, four fields).  2M members of 1000 haloes: 12.7
+// us a round, the larger cells' items 49 us; as items with two passes and folds, all cells
+// took 99 us.
+__global__ __launch_bounds__(kThreads) void k_cell_small(CellArgs a, Particles p) {
+    const int64_t c = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
+    if (c >= a.nseg || a.nch[c] != 0) return;  // wave-uniform
+    const int lane = __lane_id();
+    const int64_t b = a.begin[c];
+    const int n = static_cast<int>(cell_end(a.begin, c, a.nseg, a.ns) - b);  // 1..kChunk
+    double v[kChunk / kWave][3];
+    double acc[4][2] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+#pragma unroll
+    for (int u = 0; u < kChunk / kWave; ++u) {
+        const int k = u * kWave + lane;
+        if (k >= n) break;
+        const int64_t i = a.s_mem[a.order[b + k]];
+        v[u][0] = ldf(p.vx, p.vel_t, i);
+        v[u][1] = ldf(p.vy, p.vel_t, i);
+        v[u][2] = ldf(p.vz, p.vel_t, i);
+        dd_add(acc[0][0], acc[0][1], vm_product(p.vx, p.vel_t, p.m, p.mass_t, i));
+        dd_add(acc[1][0], acc[1][1], vm_product(p.vy, p.vel_t, p.m, p.mass_t, i));
+        dd_add(acc[2][0], acc[2][1], vm_product(p.vz, p.vel_t, p.m, p.mass_t, i));
+        dd_add(acc[3][0], acc[3][1], ldf(p.m, p.mass_t, i));
+    }
+    const bool up2 = (lane & 32) != 0, up1 = (lane & 16) != 0;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const double kh = up2 ? acc[q + 2][0] : acc[q][0], kl = up2 ? acc[q + 2][1] : acc[q][1];
+        const double gh = up2 ? acc[q][0] : acc[q + 2][0], gl = up2 ? acc[q][1] : acc[q + 2][1];
+        acc[q][0] = kh;
+        acc[q][1] = kl;
+        dd_add_dd(acc[q][0], acc[q][1], __shfl_xor(gh, 32, kWave), __shfl_xor(gl, 32, kWave));
+    }
+    double hi = up1 ? acc[1][0] : acc[0][0], lo = up1 ? acc[1][1] : acc[0][1];
+    {
+        const double gh = up1 ? acc[0][0] : acc[1][0], gl = up1 ? acc[0][1] : acc[1][1];
+        dd_add_dd(hi, lo, __shfl_xor(gh, 16, kWave), __shfl_xor(gl, 16, kWave));
+    }
+    for (int s = 8; s >= 1; s >>= 1) {
+        const double h2 = __shfl_down(hi, s, kWave), l2 = __shfl_down(lo, s, kWave);
+        dd_add_dd(hi, lo, h2, l2);
+    }
+    const double sum = hi + lo;
+    const double mass = __shfl(sum, 48, kWave);
+    double vc[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) vc[d] = __shfl(sum, 16 * d, kWave) / mass;
+    double sh = 0.0, sl = 0.0;
+#pragma unroll
+    for (int u = 0; u < kChunk / kWave; ++u) {
+        if (u * kWave + lane >= n) break;
+        const double dx = vc[0] - v[u][0], dy = vc[1] - v[u][1], dz = vc[2] - v[u][2];
+        dd_add(sh, sl, (dx * dx + dy * dy) + dz * dz);
+    }
+    for (int s = kWave / 2; s >= 1; s >>= 1) {
+        const double h2 = __shfl_down(sh, s, kWave), l2 = __shfl_down(sl, s, kWave);
+        dd_add_dd(sh, sl, h2, l2);
+    }
+    if (lane == 0) {
+        double* o = a.stats + 6 * c;
+        for (int d = 0; d < 3; ++d) o[d] = vc[d];
+        o[3] = mass;
+        o[4] = static_cast<double>(n);
+        o[5] = sqrt((sh + sl) / 3.0 / o[4]);
+    }
 }
 
 // pass 1: sums of v m (3) and m per item
@@ -247,18 +336,22 @@ __global__ __launch_bounds__(kThreads) void k_cell_part1(CellArgs a, Particles p
     }
 }
 
-// per cell: fold the items' sums, then the mass-weighted velocity, mass and count
-__global__ void k_cell_fold1(CellArgs a) {
-    const int64_t c = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (c >= a.nseg) return;
-    const double* q0 = a.part + 8 * a.ioff[c];
-    double s[4][2];
-    for (int q = 0; q < 4; ++q) {
-        s[q][0] = q0[2 * q];
-        s[q][1] = q0[2 * q + 1];
-    }
-    for (int t = 1; t < a.nch[c]; ++t)
-        for (int q = 0; q < 4; ++q) dd_add_dd(s[q][0], s[q][1], q0[8 * t + 2 * q], q0[8 * t + 2 * q + 1]);
+// the items' sums of a cell by the wavefront of its first item (a chain of one thread took
+// 33 us for the core of a halo of 20000, 3 us this way): lanes over the items, then a
+// fixed tree; mass-weighted velocity, mass and count
+__global__ __launch_bounds__(kThreads) void k_cell_fold1(CellArgs a) {
+    const int64_t it = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
+    if (it >= a.nitems) return;  // wave-uniform
+    const int64_t c = a.item_cell[it];
+    if (it != a.ioff[c]) return;
+    double s[4][2] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+    for (int t = __lane_id(); t < a.nch[c]; t += kWave)
+        for (int q = 0; q < 4; ++q) {
+            const double* p = a.part + 8 * (it + t) + 2 * q;
+            dd_add_dd(s[q][0], s[q][1], p[0], p[1]);
+        }
+    for (int q = 0; q < 4; ++q) wave_dd(s[q][0], s[q][1]);
+    if (__lane_id() != 0) return;
     const double mass = s[3][0] + s[3][1];
     double* o = a.stats + 6 * c;
     for (int d = 0; d < 3; ++d) o[d] = (s[d][0] + s[d][1]) / mass;
@@ -288,19 +381,25 @@ __global__ __launch_bounds__(kThreads) void k_cell_part2(CellArgs a, Particles p
     }
 }
 
-__global__ void k_cell_fold2(CellArgs a) {
-    const int64_t c = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (c >= a.nseg) return;
-    const double* q0 = a.part + 2 * a.ioff[c];
-    double h = q0[0], l = q0[1];
-    for (int t = 1; t < a.nch[c]; ++t) dd_add_dd(h, l, q0[2 * t], q0[2 * t + 1]);
+__global__ __launch_bounds__(kThreads) void k_cell_fold2(CellArgs a) {
+    const int64_t it = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
+    if (it >= a.nitems) return;  // wave-uniform
+    const int64_t c = a.item_cell[it];
+    if (it != a.ioff[c]) return;
+    double h = 0.0, l = 0.0;
+    for (int t = __lane_id(); t < a.nch[c]; t += kWave)
+        dd_add_dd(h, l, a.part[2 * (it + t)], a.part[2 * (it + t) + 1]);
+    wave_dd(h, l);
+    if (__lane_id() != 0) return;
     double* o = a.stats + 6 * c;
     o[5] = sqrt((h + l) / 3.0 / o[4]);
 }
 
 // the test of every member of S (in sorted order); phase per group: 0 = first round
 // ("> 2" rule), 1 = later round (">= 2"), other = no test.  A removed member clears
-// control[target] and counts in cleaned[group].
+// control[target] and counts in cleaned[group].  Bound by the gathers; with an addition per
+// removed member the counters' own lines were the bound (2M members of 1000 haloes 72 us a
+// round, 37.6 us with one per group and wavefront).
 __global__ void k_clean_decide(int64_t ns, const int32_t* __restrict__ order,
                                const int32_t* __restrict__ seg_of,
                                const int32_t* __restrict__ s_mem,
@@ -311,29 +410,36 @@ __global__ void k_clean_decide(int64_t ns, const int32_t* __restrict__ order,
                                const double* __restrict__ fac, double q_fil, double sig_fil,
                                uint8_t* __restrict__ control, int32_t* __restrict__ cleaned) {
     const int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (k >= ns) return;
-    const int32_t s = order[k];
-    const int h = s_grp[s];
-    const int ph = phase[h];
-    if (ph != 0 && ph != 1) return;
-    const double* c = stats + 6 * static_cast<int64_t>(seg_of[k]);
-    const double q = c[4];
-    bool removed;
-    if (q > q_fil) {
-        const int64_t i = s_mem[s];
-        const double dx = c[0] - ldf(p.vx, p.vel_t, i);
-        const double dy = c[1] - ldf(p.vy, p.vel_t, i);
-        const double dz = c[2] - ldf(p.vz, p.vel_t, i);
-        double bas = sqrt((dx * dx + dy * dy) + dz * dz);
-        const bool scaled = ph == 0 ? q > 2.0 : q >= 2.0;
-        bas = scaled ? bas / c[5] : 0.0;
-        removed = bas >= fac[h] * sig_fil;
-    } else {
-        removed = true;
+    int h = -1;
+    bool removed = false;
+    if (k < ns) {
+        const int32_t s = order[k];
+        h = s_grp[s];
+        const int ph = phase[h];
+        if (ph == 0 || ph == 1) {
+            const double* c = stats + 6 * static_cast<int64_t>(seg_of[k]);
+            const double q = c[4];
+            removed = true;
+            if (q > q_fil) {
+                const int64_t i = s_mem[s];
+                const double dx = c[0] - ldf(p.vx, p.vel_t, i);
+                const double dy = c[1] - ldf(p.vy, p.vel_t, i);
+                const double dz = c[2] - ldf(p.vz, p.vel_t, i);
+                double bas = sqrt((dx * dx + dy * dy) + dz * dz);
+                const bool scaled = ph == 0 ? q > 2.0 : q >= 2.0;
+                bas = scaled ? bas / c[5] : 0.0;
+                removed = bas >= fac[h] * sig_fil;
+            }
+        }
+        if (removed) control[target[s]] = 0;
     }
-    if (removed) {
-        control[target[s]] = 0;
-        atomicAdd(cleaned + h, 1);
+    // one addition per group and wavefront: the members are in group order
+    for (unsigned long long left = __ballot(removed); left != 0;) {
+        const int first = __ffsll(left) - 1;
+        const int g = __shfl(h, first, kWave);
+        const unsigned long long same = __ballot(removed && h == g);
+        if (static_cast<int>(__lane_id()) == first) atomicAdd(cleaned + g, __popcll(same));
+        left &= ~same;
     }
 }
 
@@ -442,7 +548,7 @@ CleanWs carve_clean(void* base, int64_t n) {
     w.segid = c.take<int64_t>(n1);
     w.begin = c.take<int64_t>(n1);
     w.seg_of = c.take<int32_t>(n1);
-    const int64_t max_items = n1 + n1 / kChunk + 1;
+    const int64_t max_items = 2 * (n1 / kChunk) + 2;  // cells of more than kChunk members
     w.nch = c.take<int32_t>(n1);
     w.ioff = c.take<int64_t>(n1);
     w.item_cell = c.take<int32_t>(max_items);
@@ -530,35 +636,37 @@ int halma_clean_cells(int64_t n_set, int64_t n_groups, const int32_t* set_member
         if (rc) return rc;
     }
     k_cell_heads<<<blocks_for(n_set), kThreads, 0, st>>>(n_set, w.p1, w.klo, w.khi, set_groups,
-                                                         w.head);
+                                                         w.head, w.nseg + 1);
     HALMA_LAUNCH_CHECK();
     rc = exclusive_scan_i32_to_i64(w.head, w.segid, n_set, w.nseg, w.sws, st);
     if (rc) return rc;
     k_cell_begin<<<blocks_for(n_set), kThreads, 0, st>>>(n_set, w.head, w.segid, w.begin,
                                                          w.seg_of);
     HALMA_LAUNCH_CHECK();
-    HALMA_HIP(hipMemcpyAsync(n_cells, w.nseg, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    HALMA_HIP(hipStreamSynchronize(st));
-    const int64_t nseg = *n_cells;
-    k_cell_chunks<<<blocks_for(nseg), kThreads, 0, st>>>(nseg, n_set, w.begin, w.nch);
+    k_cell_items<<<blocks_for(n_set), kThreads, 0, st>>>(n_set, w.nseg, w.begin, w.ioff, w.nch,
+                                                         w.item_cell);
     HALMA_LAUNCH_CHECK();
-    rc = exclusive_scan_i32_to_i64(w.nch, w.ioff, nseg, w.nseg + 1, w.sws, st);
-    if (rc) return rc;
-    int64_t nitems = 0;
-    HALMA_HIP(hipMemcpyAsync(&nitems, w.nseg + 1, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+    int64_t counts[2] = {0, 0};
+    HALMA_HIP(hipMemcpyAsync(counts, w.nseg, sizeof(counts), hipMemcpyDeviceToHost, st));
     HALMA_HIP(hipStreamSynchronize(st));
-    k_cell_items<<<blocks_for(nseg), kThreads, 0, st>>>(nseg, w.ioff, w.nch, w.item_cell);
-    HALMA_LAUNCH_CHECK();
+    const int64_t nseg = counts[0], nitems = counts[1];
+    *n_cells = nseg;
     CellArgs a{nseg, n_set, nitems, w.begin, w.ioff, w.nch, w.item_cell, w.p1, set_members,
                w.part, cell_stats};
-    const unsigned item_blocks = static_cast<unsigned>((nitems * kWave + kThreads - 1) / kThreads);
+    const auto wave_blocks = [](int64_t n) {
+        return static_cast<unsigned>((n * kWave + kThreads - 1) / kThreads);
+    };
+    k_cell_small<<<wave_blocks(nseg), kThreads, 0, st>>>(a, p);
+    HALMA_LAUNCH_CHECK();
+    if (nitems == 0) return 0;
+    const unsigned item_blocks = wave_blocks(nitems);
     k_cell_part1<<<item_blocks, kThreads, 0, st>>>(a, p);
     HALMA_LAUNCH_CHECK();
-    k_cell_fold1<<<blocks_for(nseg), kThreads, 0, st>>>(a);
+    k_cell_fold1<<<item_blocks, kThreads, 0, st>>>(a);
     HALMA_LAUNCH_CHECK();
     k_cell_part2<<<item_blocks, kThreads, 0, st>>>(a, p);
     HALMA_LAUNCH_CHECK();
-    k_cell_fold2<<<blocks_for(nseg), kThreads, 0, st>>>(a);
+    k_cell_fold2<<<item_blocks, kThreads, 0, st>>>(a);
     HALMA_LAUNCH_CHECK();
     return 0;
 }
