@@ -3,14 +3,13 @@
 // the dark-matter mass inside a sphere the same way).
 //
 // The points are binned once into a uniform grid (cell keys (iz ny + iy) nx + ix, stable
-// radix sort, packed FP64 copies in cell order, dense cell start offsets), so the points
+// radix sort, packed copies in cell order, dense cell start offsets), so the points
 // of one (iy, iz) row of cells between two ix are contiguous.  One block per centre walks
 // the rows of the cells that can hold a point within R (the box of the sphere widened by
-// one cell against rounding), each wavefront a contiguous range of rows: a first kernel
-// counts the hits per wavefront (and sums their masses in double-double), a scan gives
-// each centre its output range, a second kernel writes every wavefront's hits after the
-// counts of the wavefronts before it (hits in row order), and an optional pair of stable
-// radix passes puts every centre's indices in ascending order.
+// one cell against rounding): a first kernel counts the hits (and sums their masses in
+// double-double), a scan gives each centre its output range, a second kernel writes the
+// hits in row order, and every centre's indices are put in ascending order if asked for,
+// in LDS up to kSortMost of them.
 //
 // Predicates: (dx^2 + dy^2) + dz^2 <= R^2 (the KD-tree's query_ball_point) or
 // sqrt((dx^2 + dy^2) + dz^2) < R (parallel_inside, halo_gas.py:218-220), in FP64.
@@ -21,6 +20,7 @@
 #include "halma_common.h"
 #include "radix.h"
 #include "scan.h"
+#include "staging.h"
 
 namespace halma {
 
@@ -29,6 +29,12 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kRB = 2048;                  // reduction blocks of the bounding box
 constexpr int kWavesPerBlock = kThreads / kWave;
+// A centre's rows or patches are walked by one workgroup: of 16 wavefronts while there are
+// few centres, since four leave the chip mostly idle (300 centres: counts 31 -> 20 us, hits
+// 45 -> 23 us, gas cells 41 -> 30 and 110 -> 77 us), of four beyond kFewPerCu centres a CU,
+// where small ones fill it by themselves.
+constexpr int kWideThreads = 1024;
+constexpr int kFewPerCu = 4;
 
 inline unsigned blocks_for(int64_t n) {
     return static_cast<unsigned>((n + kThreads - 1) / kThreads);
@@ -41,7 +47,26 @@ struct Pts {
     int t;
 };
 
-// bounding box: (min x, min y, min z, max x, max y, max z) partial per block ...
+// the block's (min x, min y, min z, max x, max y, max z) from its threads' (in v of thread 0)
+__device__ void block_bbox(double (&v)[6], double* sh /* 6 * kWavesPerBlock */) {
+    for (int s = kWave / 2; s >= 1; s >>= 1)
+        for (int d = 0; d < 3; ++d) {
+            v[d] = fmin(v[d], __shfl_down(v[d], s, kWave));
+            v[3 + d] = fmax(v[3 + d], __shfl_down(v[3 + d], s, kWave));
+        }
+    const int w = threadIdx.x / kWave;
+    if (__lane_id() == 0)
+        for (int d = 0; d < 6; ++d) sh[6 * w + d] = v[d];
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (int q = 1; q < kWavesPerBlock; ++q)
+            for (int d = 0; d < 3; ++d) {
+                v[d] = fmin(v[d], sh[6 * q + d]);
+                v[3 + d] = fmax(v[3 + d], sh[6 * q + 3 + d]);
+            }
+}
+
+// bounding box: a partial per block ...
 __global__ __launch_bounds__(kThreads) void k_bbox(Pts p, int64_t n, double* __restrict__ part) {
     __shared__ double sh[6 * kWavesPerBlock];
     double v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
@@ -53,40 +78,28 @@ __global__ __launch_bounds__(kThreads) void k_bbox(Pts p, int64_t n, double* __r
             v[3 + d] = fmax(v[3 + d], c[d]);
         }
     }
-    for (int s = kWave / 2; s >= 1; s >>= 1)
-        for (int d = 0; d < 3; ++d) {
-            v[d] = fmin(v[d], __shfl_down(v[d], s, kWave));
-            v[3 + d] = fmax(v[3 + d], __shfl_down(v[3 + d], s, kWave));
-        }
-    const int w = threadIdx.x / kWave;
-    if (__lane_id() == 0)
-        for (int d = 0; d < 6; ++d) sh[6 * w + d] = v[d];
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int q = 1; q < kWavesPerBlock; ++q)
-            for (int d = 0; d < 3; ++d) {
-                v[d] = fmin(v[d], sh[6 * q + d]);
-                v[3 + d] = fmax(v[3 + d], sh[6 * q + 3 + d]);
-            }
+    block_bbox(v, sh);
+    if (threadIdx.x == 0)
         for (int d = 0; d < 6; ++d) part[6 * blockIdx.x + d] = v[d];
-    }
 }
 
-// ... then over the partials (one wavefront)
-__global__ void k_bbox_final(const double* __restrict__ part, int np, double* __restrict__ out) {
+// ... then over the partials (one workgroup: a wavefront's chain of 2048 partials took 12 us,
+// four take 5); also clears the largest count
+__global__ __launch_bounds__(kThreads) void k_bbox_final(const double* __restrict__ part, int np,
+                                                         double* __restrict__ out,
+                                                         int64_t* __restrict__ most) {
+    __shared__ double sh[6 * kWavesPerBlock];
     double v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    for (int q = __lane_id(); q < np; q += kWave)
+    for (int q = threadIdx.x; q < np; q += kThreads)
         for (int d = 0; d < 3; ++d) {
             v[d] = fmin(v[d], part[6 * q + d]);
             v[3 + d] = fmax(v[3 + d], part[6 * q + 3 + d]);
         }
-    for (int s = kWave / 2; s >= 1; s >>= 1)
-        for (int d = 0; d < 3; ++d) {
-            v[d] = fmin(v[d], __shfl_down(v[d], s, kWave));
-            v[3 + d] = fmax(v[3 + d], __shfl_down(v[3 + d], s, kWave));
-        }
-    if (__lane_id() == 0)
+    block_bbox(v, sh);
+    if (threadIdx.x == 0) {
         for (int d = 0; d < 6; ++d) out[d] = v[d];
+        *most = 0;
+    }
 }
 
 struct Grid {
@@ -139,16 +152,34 @@ __global__ void k_zero_out(int64_t H, int64_t* __restrict__ off, double* __restr
     if (mass && h < H) mass[h] = 0.0;
 }
 
-// packed FP64 copies in input order (coalesced) ...
-__global__ void k_pack(Pts p, int64_t n, double4* __restrict__ tmp) {
+// A point as the queries read it: its coordinates in their own precision and its index
+// (FP32 points in half the bytes: packing and sorting 1.2M of them 57 -> 44 us).
+struct Rec32 {
+    float x, y, z;
+    int32_t i;
+};
+struct __attribute__((aligned(32))) Rec64 {
+    double x, y, z;
+    int64_t i;
+};
+
+// packed copies in input order (coalesced) ...
+template <typename R>
+__global__ void k_pack(Pts p, int64_t n, R* __restrict__ tmp) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    tmp[i] = make_double4(ldf(p.x, p.t, i), ldf(p.y, p.t, i), ldf(p.z, p.t, i), 0.0);
+    R r;
+    r.x = static_cast<decltype(r.x)>(ldf(p.x, p.t, i));
+    r.y = static_cast<decltype(r.x)>(ldf(p.y, p.t, i));
+    r.z = static_cast<decltype(r.x)>(ldf(p.z, p.t, i));
+    r.i = static_cast<decltype(r.i)>(i);
+    tmp[i] = r;
 }
 
-// ... then into cell order, one 32-byte record per point
-__global__ void k_pack_sorted(const double4* __restrict__ tmp, const int32_t* __restrict__ perm,
-                              int64_t n, double4* __restrict__ pk) {
+// ... then into cell order, one record per point
+template <typename R>
+__global__ void k_pack_sorted(const R* __restrict__ tmp, const int32_t* __restrict__ perm,
+                              int64_t n, R* __restrict__ pk) {
     const int64_t j = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (j < n) pk[j] = tmp[perm[j]];
 }
@@ -191,10 +222,11 @@ __device__ CellRows rows_of(const Grid& g, const double* c, double R) {
     return r;
 }
 
-__device__ __forceinline__ bool is_hit(const double4& q, const double* c, double R, int strict) {
-    const double dx = q.x - c[0];
-    const double dy = q.y - c[1];
-    const double dz = q.z - c[2];
+template <typename P>
+__device__ __forceinline__ bool is_hit(const P& q, const double* c, double R, int strict) {
+    const double dx = static_cast<double>(q.x) - c[0];
+    const double dy = static_cast<double>(q.y) - c[1];
+    const double dz = static_cast<double>(q.z) - c[2];
     const double d2 = (dx * dx + dy * dy) + dz * dz;
     return strict ? sqrt(d2) < R : d2 <= R * R;
 }
@@ -208,43 +240,86 @@ __device__ __forceinline__ void row_range(const Grid& g, const CellRows& cr, con
     b = start[cell_key(g, cr.ix1, iy, iz) + 1];
 }
 
-// the rows of a centre's cell box are split into kWavesPerBlock contiguous ranges, one
-// per wavefront (the same split in both kernels)
-__device__ __forceinline__ void wave_rows(int64_t nrows, int w, int64_t& r0, int64_t& r1) {
-    const int64_t per = (nrows + kWavesPerBlock - 1) / kWavesPerBlock;
-    r0 = w * per < nrows ? w * per : nrows;
-    r1 = r0 + per < nrows ? r0 + per : nrows;
+// The points of a centre's cell box in row order, spread over the W wavefronts of a workgroup
+// whatever rows they lie in (a halo's core is one row or two of the grid; a range of rows for
+// each wavefront left one of them with nearly all the points): a block's width of rows at a
+// time, f(total, at) with at(p) the sorted position of the p-th point of these rows.
+template <int W>
+struct RowSpan {
+    int32_t beg[W * kWave];
+    int32_t pre[W * kWave];
+    int32_t wsum[W];
+};
+
+template <int W, typename F>
+__device__ void for_row_points(const Grid& g, const CellRows& cr, const int32_t* start,
+                               RowSpan<W>& sh, F&& f) {
+    const int lane = __lane_id(), w = threadIdx.x / kWave;
+    const int64_t nrows = cr.rows();
+    for (int64_t r0 = 0; r0 < nrows; r0 += W * kWave) {
+        const int64_t r = r0 + threadIdx.x;
+        int64_t a = 0, b = 0;
+        if (r < nrows) row_range(g, cr, start, r, a, b);
+        const int len = static_cast<int>(b - a);
+        int inc = len;
+        for (int d = 1; d < kWave; d <<= 1) {
+            const int v = __shfl_up(inc, d, kWave);
+            if (lane >= d) inc += v;
+        }
+        if (lane == kWave - 1) sh.wsum[w] = inc;
+        __syncthreads();
+        int base = 0, total = 0;
+#pragma unroll 1
+        for (int v = 0; v < W; ++v) {
+            if (v < w) base += sh.wsum[v];
+            total += sh.wsum[v];
+        }
+        sh.beg[threadIdx.x] = static_cast<int32_t>(a);
+        sh.pre[threadIdx.x] = base + inc - len;
+        __syncthreads();
+        const int nr = static_cast<int>(nrows - r0 < W * kWave ? nrows - r0 : W * kWave);
+        f(total, [&](int p) {
+            int lo = 0, hi = nr - 1;  // the last row that begins at or before p holds it
+            while (lo < hi) {
+                const int mid = (lo + hi + 1) >> 1;
+                if (sh.pre[mid] <= p)
+                    lo = mid;
+                else
+                    hi = mid - 1;
+            }
+            return sh.beg[lo] + (p - sh.pre[lo]);
+        });
+        __syncthreads();
+    }
 }
 
-// one block per centre: hits per wavefront's rows (wcount, kWavesPerBlock per centre), their
-// total, and their mass (double-double, fixed order)
-__global__ __launch_bounds__(kThreads) void k_ball_count(int64_t H, Grid g, Query q,
-                                                         const int32_t* __restrict__ start,
-                                                         const int32_t* __restrict__ perm,
-                                                         const double4* __restrict__ pk,
-                                                         int64_t* __restrict__ count,
-                                                         int64_t* __restrict__ wcount,
-                                                         double* __restrict__ mass) {
-    __shared__ int64_t shc[kWavesPerBlock];
-    __shared__ double shm[2 * kWavesPerBlock];
+// one block of W wavefronts per centre: its hits (and the largest centre's), and their mass
+// (double-double, fixed order)
+template <int W, typename P>
+__global__ __launch_bounds__(W * kWave) void k_ball_count(int64_t H, Grid g, Query q,
+                                                          const int32_t* __restrict__ start,
+                                                          const P* __restrict__ pk,
+                                                          int64_t* __restrict__ count,
+                                                          int64_t* __restrict__ most,
+                                                          double* __restrict__ mass) {
+    __shared__ RowSpan<W> span;
+    __shared__ int64_t shc[W];
+    __shared__ double shm[2 * W];
     const int w = threadIdx.x / kWave;
     for (int64_t h = blockIdx.x; h < H; h += gridDim.x) {
         const double* c = q.centre + 3 * h;
         const double R = q.radius[h];
-        const CellRows cr = rows_of(g, c, R);
-        int64_t r0, r1;
-        wave_rows(cr.rows(), w, r0, r1);
         int64_t cnt = 0;
         double mh = 0.0, ml = 0.0;
-        for (int64_t r = r0; r < r1; ++r) {
-            int64_t a, b;
-            row_range(g, cr, start, r, a, b);
-            for (int64_t j = a + __lane_id(); j < b; j += kWave)
-                if (is_hit(pk[j], c, R, q.strict)) {
+        for_row_points<W>(g, rows_of(g, c, R), start, span, [&](int total, auto&& at) {
+            for (int p = threadIdx.x; p < total; p += W * kWave) {
+                const P rec = pk[at(p)];
+                if (is_hit(rec, c, R, q.strict)) {
                     ++cnt;
-                    if (q.m) dd_add(mh, ml, ldf(q.m, q.mt, perm[j]));
+                    if (q.m) dd_add(mh, ml, ldf(q.m, q.mt, rec.i));
                 }
-        }
+            }
+        });
         for (int s = kWave / 2; s >= 1; s >>= 1) cnt += __shfl_down(cnt, s, kWave);
         if (q.m) {
             for (int s = kWave / 2; s >= 1; s >>= 1) {
@@ -254,7 +329,6 @@ __global__ __launch_bounds__(kThreads) void k_ball_count(int64_t H, Grid g, Quer
         }
         if (__lane_id() == 0) {
             shc[w] = cnt;
-            wcount[kWavesPerBlock * h + w] = cnt;
             shm[2 * w] = mh;
             shm[2 * w + 1] = ml;
         }
@@ -262,48 +336,102 @@ __global__ __launch_bounds__(kThreads) void k_ball_count(int64_t H, Grid g, Quer
         if (threadIdx.x == 0) {
             int64_t t = shc[0];
             double th = shm[0], tl = shm[1];
-            for (int v = 1; v < kWavesPerBlock; ++v) {
+#pragma unroll 1  // unrolled it takes registers from every wavefront
+            for (int v = 1; v < W; ++v) {
                 t += shc[v];
                 dd_add_dd(th, tl, shm[2 * v], shm[2 * v + 1]);
             }
             count[h] = t;
+            atomicMax(reinterpret_cast<unsigned long long*>(most),
+                      static_cast<unsigned long long>(t));
             if (mass) mass[h] = th + tl;
         }
         __syncthreads();
     }
 }
 
-// one block per centre: every wavefront writes the hits of its rows, in row order, after
-// the counts of the wavefronts before it (rows in order -> hits in row order)
-__global__ __launch_bounds__(kThreads) void k_ball_emit(int64_t H, Grid g, Query q,
-                                                        const int32_t* __restrict__ start,
-                                                        const int32_t* __restrict__ perm,
-                                                        const double4* __restrict__ pk,
-                                                        const int64_t* __restrict__ off,
-                                                        const int64_t* __restrict__ wcount,
-                                                        int32_t* __restrict__ out) {
+// one block per centre: the points a block's width at a time in row order, each step's hits
+// written after the earlier ones (ballot and wavefront counts)
+template <int W, typename P>
+__global__ __launch_bounds__(W * kWave) void k_ball_emit(int64_t H, Grid g, Query q,
+                                                         const int32_t* __restrict__ start,
+                                                         const P* __restrict__ pk,
+                                                         const int64_t* __restrict__ off,
+                                                         int32_t* __restrict__ out) {
+    __shared__ RowSpan<W> span;
+    __shared__ int shc[2][W];  // steps in turn: one barrier each
     const int w = threadIdx.x / kWave;
     const int lane = __lane_id();
     const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (kWave - lane));
+    int turn = 0;
     for (int64_t h = blockIdx.x; h < H; h += gridDim.x) {
         const double* c = q.centre + 3 * h;
         const double R = q.radius[h];
-        const CellRows cr = rows_of(g, c, R);
-        int64_t r0, r1;
-        wave_rows(cr.rows(), w, r0, r1);
-        int64_t base = off[h];
-        for (int v = 0; v < w; ++v) base += wcount[kWavesPerBlock * h + v];
-        for (int64_t r = r0; r < r1; ++r) {
-            int64_t a, b;
-            row_range(g, cr, start, r, a, b);
-            for (int64_t j0 = a; j0 < b; j0 += kWave) {
-                const int64_t j = j0 + lane;
-                const bool hit = j < b && is_hit(pk[j], c, R, q.strict);
+        int64_t running = off[h];
+        for_row_points<W>(g, rows_of(g, c, R), start, span, [&](int total, auto&& at) {
+            for (int p0 = 0; p0 < total; p0 += W * kWave) {
+                const int p = p0 + static_cast<int>(threadIdx.x);
+                const P rec = pk[at(p < total ? p : total - 1)];
+                const bool hit = p < total && is_hit(rec, c, R, q.strict);
                 const unsigned long long mask = __ballot(hit);
-                if (hit) out[base + __popcll(mask & below)] = perm[j];
-                base += __popcll(mask);
+                if (lane == 0) shc[turn][w] = __popcll(mask);
+                __syncthreads();
+                int base = 0, all = 0;
+#pragma unroll
+                for (int v = 0; v < W; ++v) {
+                    const int n = shc[turn][v];
+                    base += v < w ? n : 0;
+                    all += n;
+                }
+                if (hit)
+                    out[running + base + __popcll(mask & below)] = static_cast<int32_t>(rec.i);
+                running += all;
+                turn ^= 1;
             }
-        }
+        });
+    }
+}
+
+// Every centre's hits (distinct indices, at most N) in ascending order: a bitonic sort of the
+// next power of two in LDS, one workgroup per centre.  One read and one write of the hits
+// instead of five radix passes and two gathers (1.2M hits of 300 centres 135 -> 41 us);
+// bound by the LDS steps, which grow with log^2 of the largest centre: with more than
+// kSortMost hits in one, all go by the radix passes (index, then stably centre).
+constexpr int kSortSmall = 2048, kSortMost = 16384;
+
+template <int T, int N>
+__global__ __launch_bounds__(T) void k_sort_hits(int64_t H, const int64_t* __restrict__ off,
+                                                 const int32_t* __restrict__ raw,
+                                                 int32_t* __restrict__ out) {
+    __shared__ uint32_t s[N];
+    for (int64_t h = blockIdx.x; h < H; h += gridDim.x) {
+        const int64_t b = off[h];
+        const int n = static_cast<int>(off[h + 1] - b);  // at most N: the caller looks
+        int m = 2;
+        while (m < n) m <<= 1;  // at most N
+        for (int k = threadIdx.x; k < m; k += T)
+            s[k] = k < n ? static_cast<uint32_t>(raw[b + k]) : 0xffffffffu;
+        __syncthreads();
+        for (int k = 2; k <= m; k <<= 1)
+            for (int j = k >> 1; j > 0; j >>= 1) {
+                // a wavefront's pairs at distances up to 64 stay within its own runs of 128
+                if (j >= kWave) {
+                    __syncthreads();
+                } else {
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                }
+                for (int t = threadIdx.x; t < m / 2; t += T) {
+                    const int lo = 2 * t - (t & (j - 1)), hi = lo + j;
+                    const uint32_t a = s[lo], c = s[hi];
+                    const bool keep = ((lo & k) == 0) == (a < c);
+                    s[lo] = keep ? a : c;
+                    s[hi] = keep ? c : a;
+                }
+            }
+        __syncthreads();
+        for (int k = threadIdx.x; k < n; k += T) out[b + k] = static_cast<int32_t>(s[k]);
+        __syncthreads();
     }
 }
 
@@ -338,10 +466,9 @@ struct BallWs {
     uint32_t* key;
     uint32_t* skey;
     int32_t* perm;
-    double4* pk;
-    double4* tmp;
+    Rec64* pk;   // Rec32 for FP32 points
+    Rec64* tmp;
     int32_t* start;
-    int64_t* wcount;
     int64_t* count;
     int64_t* total;
     int32_t* raw;
@@ -367,12 +494,11 @@ BallWs carve_ball(void* base, int64_t n, int64_t H, int64_t max_found) {
     w.key = c.take<uint32_t>(n1);
     w.skey = c.take<uint32_t>(n1);
     w.perm = c.take<int32_t>(n1);
-    w.pk = c.take<double4>(n1);
-    w.tmp = c.take<double4>(n1);
-    w.wcount = c.take<int64_t>(kWavesPerBlock * h1);
+    w.pk = c.take<Rec64>(n1);
+    w.tmp = c.take<Rec64>(n1);
     w.start = c.take<int32_t>(w.max_cells + 1);
     w.count = c.take<int64_t>(h1 + 1);
-    w.total = c.take<int64_t>(2);
+    w.total = c.take<int64_t>(4);  // [0] hits, [2] the largest centre's
     w.raw = c.take<int32_t>(f1);
     w.cid = c.take<uint32_t>(f1);
     w.k2 = c.take<uint32_t>(f1);
@@ -391,7 +517,7 @@ BallWs carve_ball(void* base, int64_t n, int64_t H, int64_t max_found) {
 // x0 + ix res (x0 = rx - res/2) lies strictly inside the query's box per axis, that are
 // neither refined nor overlapped (cr0amr and solapst) and, with a sphere, lie within
 // sqrt(d2) < R.  One block per halo culls the patches
-// 256 at a time (a box-overlap test, widened by a cell against rounding), then walks the
+// a block-width at a time (a box-overlap test, widened by a cell against rounding), then walks the
 // candidate patches in order, the cells of each patch's clip box a block-width at a time
 // in (ix, iy, iz) order -- the reference's loop order, kept by the chunk scan of the
 // emitting kernel.
@@ -489,8 +615,8 @@ __device__ __forceinline__ bool amr_hit(const PatchClip& c, const AmrCells& g, c
     return sqrt((dx * dx + dy * dy) + dz * dz) < R;
 }
 
-// the patches of a halo's box, in order, kThreads at a time into an LDS list
-template <typename F>
+// the patches of a halo's box, in order, W wavefronts of them at a time into an LDS list
+template <int W, typename F>
 __device__ void for_candidate_patches(const AmrPatches& pa, const double* box, int32_t* list,
                                       int* nlist, F&& f) {
     for (int64_t p0 = 0; p0 < pa.P; p0 += blockDim.x) {
@@ -498,7 +624,7 @@ __device__ void for_candidate_patches(const AmrPatches& pa, const double* box, i
         const bool cand = p < pa.P && clip_patch(pa, p, box).rows() > 0;
         const unsigned long long mask = __ballot(cand);
         const int w = threadIdx.x / kWave, lane = __lane_id();
-        __shared__ int wcnt[kWavesPerBlock];
+        __shared__ int wcnt[W];
         if (lane == 0) wcnt[w] = __popcll(mask);
         __syncthreads();
         int base = 0;
@@ -509,7 +635,7 @@ __device__ void for_candidate_patches(const AmrPatches& pa, const double* box, i
         }
         if (threadIdx.x == 0) {
             int t = 0;
-            for (int v = 0; v < kWavesPerBlock; ++v) t += wcnt[v];
+            for (int v = 0; v < W; ++v) t += wcnt[v];
             *nlist = t;
         }
         __syncthreads();
@@ -525,10 +651,19 @@ struct AmrHalo {
     const double* radius;
 };
 
-// cell q (0 .. cells()) of a patch's clip box in (ix, iy, iz) order
-__device__ __forceinline__ void clip_cell(const PatchClip& c, int64_t q, int64_t& ix, int64_t& iy,
-                                          int64_t& iz) {
+// cell q (0 .. nc - 1) of a patch's clip box in (ix, iy, iz) order, divided in 32 bits where
+// the box's nc cells fit them
+__device__ __forceinline__ void clip_cell(const PatchClip& c, int64_t nc, int64_t q, int64_t& ix,
+                                          int64_t& iy, int64_t& iz) {
     const int64_t niz = c.iz1 - c.iz0 + 1, niy = c.iy1 - c.iy0 + 1;
+    if (nc <= INT32_MAX) {
+        const uint32_t r = static_cast<uint32_t>(q) / static_cast<uint32_t>(niz);
+        const uint32_t x = r / static_cast<uint32_t>(niy);
+        iz = c.iz0 + (static_cast<uint32_t>(q) - r * static_cast<uint32_t>(niz));
+        iy = c.iy0 + (r - x * static_cast<uint32_t>(niy));
+        ix = c.ix0 + x;
+        return;
+    }
     iz = c.iz0 + q % niz;
     iy = c.iy0 + (q / niz) % niy;
     ix = c.ix0 + q / (niz * niy);
@@ -538,11 +673,13 @@ __device__ __forceinline__ int64_t clip_cells(const PatchClip& c) {
     return c.rows() * (c.iz1 - c.iz0 + 1);
 }
 
-__global__ __launch_bounds__(kThreads) void k_amr_count(int64_t H, AmrPatches pa, AmrCells g,
-                                                        AmrHalo hq, int64_t* __restrict__ count) {
-    __shared__ int32_t list[kThreads];
+template <int W>
+__global__ __launch_bounds__(W * kWave) void k_amr_count(int64_t H, AmrPatches pa, AmrCells g,
+                                                         AmrHalo hq,
+                                                         int64_t* __restrict__ count) {
+    __shared__ int32_t list[W * kWave];
     __shared__ int nlist;
-    __shared__ int64_t shc[kWavesPerBlock];
+    __shared__ int64_t shc[W];
     const int w = threadIdx.x / kWave;
     for (int64_t h = blockIdx.x; h < H; h += gridDim.x) {
         const double* cen = hq.centre ? hq.centre + 3 * h : nullptr;
@@ -550,13 +687,13 @@ __global__ __launch_bounds__(kThreads) void k_amr_count(int64_t H, AmrPatches pa
         const double* box = hq.box + 6 * h;
         int64_t cnt = 0;
         if (!cen || R >= 0.0)
-            for_candidate_patches(pa, box, list, &nlist, [&](int64_t p) {
+            for_candidate_patches<W>(pa, box, list, &nlist, [&](int64_t p) {
                 const PatchClip c = clip_patch(pa, p, box);
                 const int64_t nc = clip_cells(c);
                 for (int64_t q = threadIdx.x; q < nc; q += blockDim.x) {
                     int64_t ix, iy, iz, cell;
                     double x, y, z;
-                    clip_cell(c, q, ix, iy, iz);
+                    clip_cell(c, nc, q, ix, iy, iz);
                     if (amr_hit(c, g, box, cen, R, ix, iy, iz, cell, x, y, z)) ++cnt;
                 }
             });
@@ -565,7 +702,7 @@ __global__ __launch_bounds__(kThreads) void k_amr_count(int64_t H, AmrPatches pa
         __syncthreads();
         if (threadIdx.x == 0) {
             int64_t t = 0;
-            for (int v = 0; v < kWavesPerBlock; ++v) t += shc[v];
+            for (int v = 0; v < W; ++v) t += shc[v];
             count[h] = t;
         }
         __syncthreads();
@@ -574,22 +711,26 @@ __global__ __launch_bounds__(kThreads) void k_amr_count(int64_t H, AmrPatches pa
 
 // the same traversal, the clip box's cells a block-width at a time in (ix, iy, iz) order:
 // each chunk's hits are written after the chunk's earlier hits (ballot + wave counts)
-__global__ __launch_bounds__(kThreads) void k_amr_emit(int64_t H, AmrPatches pa, AmrCells g,
-                                                       AmrHalo hq, const int64_t* __restrict__ off,
-                                                       int64_t stride, double* __restrict__ out) {
-    __shared__ int32_t list[kThreads];
+template <int W>
+__global__ __launch_bounds__(W * kWave) void k_amr_emit(int64_t H, AmrPatches pa, AmrCells g,
+                                                        AmrHalo hq,
+                                                        const int64_t* __restrict__ off,
+                                                        int64_t stride,
+                                                        double* __restrict__ out) {
+    __shared__ int32_t list[W * kWave];
     __shared__ int nlist;
-    __shared__ int64_t shc[kWavesPerBlock];
+    __shared__ int shc[2][W];  // chunks in turn: one barrier each
     const int w = threadIdx.x / kWave;
     const int lane = __lane_id();
     const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (kWave - lane));
+    int turn = 0;
     for (int64_t h = blockIdx.x; h < H; h += gridDim.x) {
         const double* cen = hq.centre ? hq.centre + 3 * h : nullptr;
         const double R = hq.centre ? hq.radius[h] : 0.0;
         const double* box = hq.box + 6 * h;
         int64_t running = off[h];
         if (cen && !(R >= 0.0)) continue;  // block-uniform
-        for_candidate_patches(pa, box, list, &nlist, [&](int64_t p) {
+        for_candidate_patches<W>(pa, box, list, &nlist, [&](int64_t p) {
             const PatchClip c = clip_patch(pa, p, box);
             const int64_t nc = clip_cells(c);
             for (int64_t q0 = 0; q0 < nc; q0 += blockDim.x) {
@@ -598,16 +739,16 @@ __global__ __launch_bounds__(kThreads) void k_amr_emit(int64_t H, AmrPatches pa,
                 double x = 0, y = 0, z = 0;
                 bool hit = false;
                 if (q < nc) {
-                    clip_cell(c, q, ix, iy, iz);
+                    clip_cell(c, nc, q, ix, iy, iz);
                     hit = amr_hit(c, g, box, cen, R, ix, iy, iz, cell, x, y, z);
                 }
                 const unsigned long long mask = __ballot(hit);
-                if (lane == 0) shc[w] = __popcll(mask);
+                if (lane == 0) shc[turn][w] = __popcll(mask);
                 __syncthreads();
                 int64_t base = running;
-                for (int v = 0; v < w; ++v) base += shc[v];
+                for (int v = 0; v < w; ++v) base += shc[turn][v];
                 int64_t total = 0;
-                for (int v = 0; v < kWavesPerBlock; ++v) total += shc[v];
+                for (int v = 0; v < W; ++v) total += shc[turn][v];
                 if (hit) {
                     const int64_t o = base + __popcll(mask & below);
                     out[o] = x;
@@ -621,10 +762,46 @@ __global__ __launch_bounds__(kThreads) void k_amr_emit(int64_t H, AmrPatches pa,
                     out[7 * stride + o] = ldf(g.temp, g.t, cell);
                 }
                 running += total;
-                __syncthreads();
+                turn ^= 1;
             }
         });
     }
+}
+
+// the points in cell order, then every centre's count (and mass)
+template <typename R>
+int ball_count(const Pts& p, int64_t n, int64_t H, const Grid& g, const Query& q, const BallWs& w,
+               bool wide, double* mass, hipStream_t st) {
+    R* tmp = reinterpret_cast<R*>(w.tmp);
+    R* pk = reinterpret_cast<R*>(w.pk);
+    k_pack<R><<<blocks_for(n), kThreads, 0, st>>>(p, n, tmp);
+    HALMA_LAUNCH_CHECK();
+    k_pack_sorted<R><<<blocks_for(n), kThreads, 0, st>>>(tmp, w.perm, n, pk);
+    HALMA_LAUNCH_CHECK();
+    const unsigned hb = static_cast<unsigned>(std::min<int64_t>(H, 65536));
+    if (wide)
+        k_ball_count<kWideThreads / kWave, R><<<hb, kWideThreads, 0, st>>>(
+            H, g, q, w.start, pk, w.count, w.total + 2, mass);
+    else
+        k_ball_count<kWavesPerBlock, R><<<hb, kThreads, 0, st>>>(H, g, q, w.start, pk, w.count,
+                                                                 w.total + 2, mass);
+    HALMA_LAUNCH_CHECK();
+    return 0;
+}
+
+template <typename R>
+int ball_emit(int64_t H, const Grid& g, const Query& q, const BallWs& w, const int64_t* off,
+              bool wide, int32_t* out, hipStream_t st) {
+    const R* pk = reinterpret_cast<const R*>(w.pk);
+    const unsigned hb = static_cast<unsigned>(std::min<int64_t>(H, 65536));
+    if (wide)
+        k_ball_emit<kWideThreads / kWave, R><<<hb, kWideThreads, 0, st>>>(H, g, q, w.start, pk,
+                                                                          off, out);
+    else
+        k_ball_emit<kWavesPerBlock, R><<<hb, kThreads, 0, st>>>(H, g, q, w.start, pk, off,
+                                                                out);
+    HALMA_LAUNCH_CHECK();
+    return 0;
 }
 
 }  // namespace
@@ -667,7 +844,7 @@ int halma_ball_query(int64_t n_points, const void* x, const void* y, const void*
     if (n_points > 0) {
         k_bbox<<<kRB, kThreads, 0, st>>>(p, n_points, w.part);
         HALMA_LAUNCH_CHECK();
-        k_bbox_final<<<1, kWave, 0, st>>>(w.part, kRB, w.bbox);
+        k_bbox_final<<<1, kThreads, 0, st>>>(w.part, kRB, w.bbox, w.total + 2);
         HALMA_LAUNCH_CHECK();
         double bb[6];
         HALMA_HIP(hipMemcpyAsync(bb, w.bbox, sizeof(bb), hipMemcpyDeviceToHost, st));
@@ -703,25 +880,29 @@ int halma_ball_query(int64_t n_points, const void* x, const void* y, const void*
         if (rc) return rc;
         k_starts<<<blocks_for(ncell + 1), kThreads, 0, st>>>(w.skey, n_points, ncell, w.start);
         HALMA_LAUNCH_CHECK();
-        k_pack<<<blocks_for(n_points), kThreads, 0, st>>>(p, n_points, w.tmp);
-        HALMA_LAUNCH_CHECK();
-        k_pack_sorted<<<blocks_for(n_points), kThreads, 0, st>>>(w.tmp, w.perm, n_points, w.pk);
-        HALMA_LAUNCH_CHECK();
     } else {
         g.cs = 1.0;
         g.n[0] = g.n[1] = g.n[2] = 1;
     }
     Query q{centres, radii, strict, mass_sums ? m : nullptr, mass_dtype};
     const unsigned hb = static_cast<unsigned>(std::min<int64_t>(n_centres, 65536));
+    const bool wide = n_centres <= static_cast<int64_t>(kFewPerCu) * device_cu_count();
+    const bool f32 = pos_dtype == HALMA_F32;
+    int64_t most = 0;
     if (n_points > 0) {
-        k_ball_count<<<hb, kThreads, 0, st>>>(n_centres, g, q, w.start, w.perm, w.pk, w.count,
-                                              w.wcount, mass_sums);
-        HALMA_LAUNCH_CHECK();
-        int rc = exclusive_scan_i64(w.count, offsets, n_centres + 1, w.total, w.sws, st);
+        int rc = f32 ? ball_count<Rec32>(p, n_points, n_centres, g, q, w, wide, mass_sums, st)
+                     : ball_count<Rec64>(p, n_points, n_centres, g, q, w, wide, mass_sums, st);
         if (rc) return rc;
-        HALMA_HIP(hipMemcpyAsync(n_found, offsets + n_centres, sizeof(int64_t),
-                                 hipMemcpyDeviceToHost, st));
+        rc = exclusive_scan_i64(w.count, offsets, n_centres + 1, w.total, w.sws, st);
+        if (rc) return rc;
+        long long* h = pinned_words(2);
+        if (!h) return set_error(HALMA_E_STATE, "pinned host buffer unavailable");
+        HALMA_HIP(hipMemcpyAsync(h, offsets + n_centres, sizeof(int64_t), hipMemcpyDeviceToHost,
+                                 st));
+        HALMA_HIP(hipMemcpyAsync(h + 1, w.total + 2, sizeof(int64_t), hipMemcpyDeviceToHost, st));
         HALMA_HIP(hipStreamSynchronize(st));
+        *n_found = h[0];
+        most = h[1];
     } else {  // no points: empty ranges, zero masses
         k_zero_out<<<blocks_for(n_centres + 1), kThreads, 0, st>>>(n_centres, offsets, mass_sums);
         HALMA_LAUNCH_CHECK();
@@ -733,13 +914,22 @@ int halma_ball_query(int64_t n_points, const void* x, const void* y, const void*
                          static_cast<long long>(F), static_cast<long long>(max_found));
     if (F > INT32_MAX) return set_error(HALMA_E_LIMIT, "at most 2^31-1 points found");
     if (F == 0) return 0;
-    k_ball_emit<<<hb, kThreads, 0, st>>>(n_centres, g, q, w.start, w.perm, w.pk, offsets,
-                                         w.wcount, sorted ? w.raw : indices);
-    HALMA_LAUNCH_CHECK();
-    if (sorted) {  // ascending indices per centre: by index, then stably by centre
+    int32_t* hits = sorted ? w.raw : indices;
+    int rc = f32 ? ball_emit<Rec32>(n_centres, g, q, w, offsets, wide, hits, st)
+                 : ball_emit<Rec64>(n_centres, g, q, w, offsets, wide, hits, st);
+    if (rc) return rc;
+    if (sorted && most <= kSortMost) {
+        if (most > kSortSmall)
+            k_sort_hits<kWideThreads, kSortMost><<<hb, kWideThreads, 0, st>>>(n_centres, offsets,
+                                                                              w.raw, indices);
+        else
+            k_sort_hits<2 * kThreads, kSortSmall><<<hb, 2 * kThreads, 0, st>>>(
+                n_centres, offsets, w.raw, indices);
+        HALMA_LAUNCH_CHECK();
+    } else if (sorted) {  // ascending indices per centre: by index, then stably by centre
         k_entry_centre<<<hb, kThreads, 0, st>>>(offsets, n_centres, w.cid);
         HALMA_LAUNCH_CHECK();
-        int rc = radix_sort_pairs(reinterpret_cast<const uint32_t*>(w.raw), nullptr, w.k2, w.p0,
+        rc = radix_sort_pairs(reinterpret_cast<const uint32_t*>(w.raw), nullptr, w.k2, w.p0,
                                   F, bits_for(static_cast<uint64_t>(n_points - 1)), w.rws, st);
         if (rc) return rc;
         k_gather_u32<<<blocks_for(F), kThreads, 0, st>>>(w.cid, w.p0, F, w.k3);
@@ -809,7 +999,11 @@ int halma_amr_particles(int64_t n_patches, const int32_t* level, const int32_t* 
     AmrCells g{delta, vx, vy, vz, temp, gas_dtype, cr0amr, solapst, rho_B, mass_scale, vel_scale};
     AmrHalo hq{boxes, centres, radii};
     const unsigned hb = static_cast<unsigned>(std::min<int64_t>(n_haloes, 65536));
-    k_amr_count<<<hb, kThreads, 0, st>>>(n_haloes, pa, g, hq, count);
+    const bool wide = n_haloes <= static_cast<int64_t>(kFewPerCu) * device_cu_count();
+    if (wide)
+        k_amr_count<kWideThreads / kWave><<<hb, kWideThreads, 0, st>>>(n_haloes, pa, g, hq, count);
+    else
+        k_amr_count<kWavesPerBlock><<<hb, kThreads, 0, st>>>(n_haloes, pa, g, hq, count);
     HALMA_LAUNCH_CHECK();
     int rc = exclusive_scan_i64(count, offsets, n_haloes + 1, total, sws, st);
     if (rc) return rc;
@@ -822,7 +1016,12 @@ int halma_amr_particles(int64_t n_patches, const int32_t* level, const int32_t* 
         return set_error(HALMA_E_LIMIT, "%lld gas cells found exceed max_found = %lld",
                          static_cast<long long>(F), static_cast<long long>(max_found));
     if (F == 0) return 0;
-    k_amr_emit<<<hb, kThreads, 0, st>>>(n_haloes, pa, g, hq, offsets, max_found, out);
+    if (wide)
+        k_amr_emit<kWideThreads / kWave><<<hb, kWideThreads, 0, st>>>(n_haloes, pa, g, hq, offsets,
+                                                                      max_found, out);
+    else
+        k_amr_emit<kWavesPerBlock><<<hb, kThreads, 0, st>>>(n_haloes, pa, g, hq, offsets,
+                                                            max_found, out);
     HALMA_LAUNCH_CHECK();
     return 0;
 }
