@@ -30,11 +30,13 @@ constexpr int kThreads = 256;
 constexpr int kRB = 2048;                  // reduction blocks of the bounding box
 constexpr int kWavesPerBlock = kThreads / kWave;
 // A centre's rows or patches are walked by one workgroup: of 16 wavefronts while there are
-// few centres, since four leave the chip mostly idle (300 centres: counts 31 -> 20 us, hits
-// 45 -> 23 us, gas cells 41 -> 30 and 110 -> 77 us), of four beyond kFewPerCu centres a CU,
-// where small ones fill it by themselves.
+// few centres, since four leave the chip mostly idle, of four beyond kFewPerCu centres a CU.
+// Whole calls, four against 16: 300 spheres of 4000 hits 384 / 370 us, 1000 of 1200 359 / 364,
+// 3000 of 400 389 / 475; gas cells of 300 haloes 327 / 280 us, 1000 363 / 437, 3000 574 / 893.
+// The kernels for 300 haloes: counts 31 -> 20 us, hits 45 -> 23 us, gas cells 41 -> 30 (count)
+// and 110 -> 77 us.
 constexpr int kWideThreads = 1024;
-constexpr int kFewPerCu = 4;
+constexpr int kFewPerCu = 2;
 
 inline unsigned blocks_for(int64_t n) {
     return static_cast<unsigned>((n + kThreads - 1) / kThreads);

@@ -28,8 +28,8 @@ def _balls(counts, dtype, seed):
     [2047, 2048, 2049, 0, 1, 4096, 4097],             # both
     [16383, 16384, 5, 2048],                          # up to the largest sorted in LDS
     [16385, 70, 0, 2000],                             # one more: the radix passes
-    [3] * 1024,                                       # 16 wavefronts a centre on 256 CUs
-    [2, 0, 4] * 500,                                  # four
+    [3] * 512,                                        # 16 wavefronts a centre on 256 CUs
+    [2, 0, 4] * 171,                                  # four
 ])
 def test_sphere_forms(gpu, counts, dtype):
     from pyhalma_amd import engine
@@ -69,8 +69,8 @@ def test_gas_cells_of_many_haloes(gpu, sphere):
 
     off, gas = run(0, Q)
     assert off[-1] > 0
-    for a in range(0, Q, 600):
-        po, pg = run(a, a + 600)
-        assert np.array_equal(po, off[a:a + 601] - off[a])
+    for a in range(0, Q, 500):
+        po, pg = run(a, a + 500)
+        assert np.array_equal(po, off[a:a + 501] - off[a])
         for k in gas:
-            assert torch.equal(pg[k], gas[k][off[a]:off[a + 600]])
+            assert torch.equal(pg[k], gas[k][off[a]:off[a + 500]])
