@@ -20,6 +20,7 @@
 #include "halma_common.h"
 #include "radix.h"
 #include "scan.h"
+#include "staging.h"
 
 namespace halma {
 
@@ -646,8 +647,9 @@ int halma_clean_cells(int64_t n_set, int64_t n_groups, const int32_t* set_member
     k_cell_items<<<blocks_for(n_set), kThreads, 0, st>>>(n_set, w.nseg, w.begin, w.ioff, w.nch,
                                                          w.item_cell);
     HALMA_LAUNCH_CHECK();
-    int64_t counts[2] = {0, 0};
-    HALMA_HIP(hipMemcpyAsync(counts, w.nseg, sizeof(counts), hipMemcpyDeviceToHost, st));
+    long long* counts = pinned_words(2);
+    if (!counts) return set_error(HALMA_E_STATE, "pinned host buffer unavailable");
+    HALMA_HIP(hipMemcpyAsync(counts, w.nseg, 2 * sizeof(int64_t), hipMemcpyDeviceToHost, st));
     HALMA_HIP(hipStreamSynchronize(st));
     const int64_t nseg = counts[0], nitems = counts[1];
     *n_cells = nseg;
@@ -731,8 +733,11 @@ int halma_clean_select(int64_t n_groups, int64_t n_members, const int64_t* offse
         n_members, offsets, members, w.flag, w.grp, w.pos, set_offsets, set_members, set_groups,
         set_target);
     HALMA_LAUNCH_CHECK();
-    HALMA_HIP(hipMemcpyAsync(n_set, w.total, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+    long long* total = pinned_words(1);
+    if (!total) return set_error(HALMA_E_STATE, "pinned host buffer unavailable");
+    HALMA_HIP(hipMemcpyAsync(total, w.total, sizeof(int64_t), hipMemcpyDeviceToHost, st));
     HALMA_HIP(hipStreamSynchronize(st));
+    *n_set = *total;
     return 0;
 }
 

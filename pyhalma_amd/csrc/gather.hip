@@ -848,8 +848,9 @@ int halma_ball_query(int64_t n_points, const void* x, const void* y, const void*
         HALMA_LAUNCH_CHECK();
         k_bbox_final<<<1, kThreads, 0, st>>>(w.part, kRB, w.bbox, w.total + 2);
         HALMA_LAUNCH_CHECK();
-        double bb[6];
-        HALMA_HIP(hipMemcpyAsync(bb, w.bbox, sizeof(bb), hipMemcpyDeviceToHost, st));
+        double* bb = reinterpret_cast<double*>(pinned_words(6));
+        if (!bb) return set_error(HALMA_E_STATE, "pinned host buffer unavailable");
+        HALMA_HIP(hipMemcpyAsync(bb, w.bbox, 6 * sizeof(double), hipMemcpyDeviceToHost, st));
         HALMA_HIP(hipStreamSynchronize(st));
         for (int d = 0; d < 3; ++d)
             if (!std::isfinite(bb[d]) || !std::isfinite(bb[3 + d]))
@@ -1009,9 +1010,12 @@ int halma_amr_particles(int64_t n_patches, const int32_t* level, const int32_t* 
     HALMA_LAUNCH_CHECK();
     int rc = exclusive_scan_i64(count, offsets, n_haloes + 1, total, sws, st);
     if (rc) return rc;
-    HALMA_HIP(hipMemcpyAsync(n_found, offsets + n_haloes, sizeof(int64_t), hipMemcpyDeviceToHost,
+    long long* found = pinned_words(1);
+    if (!found) return set_error(HALMA_E_STATE, "pinned host buffer unavailable");
+    HALMA_HIP(hipMemcpyAsync(found, offsets + n_haloes, sizeof(int64_t), hipMemcpyDeviceToHost,
                              st));
     HALMA_HIP(hipStreamSynchronize(st));
+    *n_found = *found;
     const int64_t F = *n_found;
     if (!out) return 0;  // counting only
     if (F > max_found)

@@ -20,6 +20,7 @@
 #include <algorithm>
 
 #include "halma_common.h"
+#include "staging.h"
 
 namespace halma {
 
@@ -442,8 +443,9 @@ int halma_progenitors(int64_t n_new, int64_t n_new_members, const int64_t* new_o
         HALMA_LAUNCH_CHECK();
         k_range_final<<<1, kWave, 0, st>>>(w.part, 2 * kRangeBlocks, w.range);
         HALMA_LAUNCH_CHECK();
-        unsigned long long r[2];
-        HALMA_HIP(hipMemcpyAsync(r, w.range, sizeof(r), hipMemcpyDeviceToHost, st));
+        unsigned long long* r = reinterpret_cast<unsigned long long*>(pinned_words(2));
+        if (!r) return set_error(HALMA_E_STATE, "pinned host buffer unavailable");
+        HALMA_HIP(hipMemcpyAsync(r, w.range, 2 * sizeof(*r), hipMemcpyDeviceToHost, st));
         HALMA_HIP(hipStreamSynchronize(st));
         if (r[1] - r[0] == kEmpty)
             return set_error(HALMA_E_LIMIT, "IDs span the whole int64 range");

@@ -8,7 +8,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .device import ptr, stream_ptr, to_dev, workspace, empty
+from .device import ptr, stream_ptr, to_dev, to_dev_all, workspace, empty
 
 
 def _lib_():
@@ -26,8 +26,7 @@ def pot_sum(m, x, y, z, tx, ty, tz, out_dtype=np.float32, with_f64=False):
     Returns a device tensor (float32 by default; float64 if out_dtype is float64).
     With with_f64=True returns (out, out_f64)."""
     L = _lib_()
-    m, x, y, z = (to_dev(a, np.float32) for a in (m, x, y, z))
-    tx, ty, tz = (to_dev(a, np.float32) for a in (tx, ty, tz))
+    m, x, y, z, tx, ty, tz = to_dev_all((m, x, y, z, tx, ty, tz), np.float32)
     ns, nt = int(m.numel()), int(tx.numel())
     if not (x.numel() == y.numel() == z.numel() == ns):
         raise ValueError("source arrays must have equal lengths")
@@ -724,21 +723,20 @@ def _centres(red, counts):
 
 
 def _clean_cells(L, ns, H, s_mem, s_grp, x, y, z, vx, vy, vz, m, c, grid, used, ijk, stats,
-                 ws):
+                 ws, more=()):
     """halma_clean_cells over the set (s_mem, s_grp) with per-group centres c (H, 3) and
     grids (start, second node, delta, length); ``used`` marks the groups with members in
     the set.  Returns the number of cells and the device copies of the per-group
-    arguments (to be held until the stream has used them)."""
+    arguments (to be held until the stream has used them) followed by those of ``more``,
+    which go up with them."""
     from .device import dtype_flag
-    dev = x.device
     start, g1, d, n = grid
     max_n = int(n[used].max())
-    dv = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)  # noqa: E731
-    held = (dv(c), dv(start), dv(g1), dv(d), dv(np.clip(n, 1, 2 ** 30).astype(np.int32)))
+    held = to_dev_all((c, start, g1, d, np.clip(n, 1, 2 ** 30).astype(np.int32)) + tuple(more))
     ncells = ctypes_i64()
     rc = L.halma_clean_cells(ns, H, ptr(s_mem), ptr(s_grp), ptr(x), ptr(y), ptr(z),
                              dtype_flag(x), ptr(vx), ptr(vy), ptr(vz), dtype_flag(vx), ptr(m),
-                             dtype_flag(m), *(ptr(t) for t in held), max_n, ptr(ijk), ptr(stats),
+                             dtype_flag(m), *(ptr(t) for t in held[:5]), max_n, ptr(ijk), ptr(stats),
                              ncells, ptr(ws), ws.numel(), stream_ptr())
     _lib.check(rc, "halma_clean_cells")
     return int(ncells.value), held
@@ -779,6 +777,14 @@ def _select(L, H, goff, nm, members, control, live, force, out, ws):
                               stream_ptr())
     _lib.check(rc, "halma_clean_select")
     return int(n.value)
+
+
+def _reduce_set(s_mem, s_off, off, A):
+    """group_reduce of the cleaning's set and the set's offsets, on the host in one transfer
+    (``off``: any host offsets of as many groups)."""
+    red = group_reduce(Groups(s_mem, s_off, off), A[0], A[1], A[2], A[6])
+    both = torch.cat([red.reshape(-1), s_off.view(torch.float64)]).cpu().numpy()
+    return both[:red.numel()].reshape(red.shape), both[red.numel():].view(np.int64)
 
 
 def phase_space_clean(groups, x, y, z, vx, vy, vz, m, ll, q_fil, sig_fil, psc=True,
@@ -864,9 +870,8 @@ def phase_space_clean(groups, x, y, z, vx, vy, vz, m, ll, q_fil, sig_fil, psc=Tr
     while (phase < 3).any():
         live = dv((phase < 3).astype(np.uint8))
         ns = _select(L, H, goff, nm, by, control, live, None, sel, sel_ws)
-        s_off_h = s_off.cpu().numpy()
+        red, s_off_h = _reduce_set(s_mem, s_off, off, A)
         counts_h = np.diff(s_off_h)
-        red = group_reduce(Groups(s_mem, s_off, s_off_h), A[0], A[1], A[2], A[6]).cpu().numpy()
         c, M, R = _centres(red, counts_h)
         if given is not None:
             c, R = given  # the caller's first grid (every group is in its first round)
@@ -876,10 +881,10 @@ def phase_space_clean(groups, x, y, z, vx, vy, vz, m, ll, q_fil, sig_fil, psc=Tr
         n_cell[first] = grid[3][first]
         if ns:
             _, held = _clean_cells(L, ns, H, s_mem, s_grp, *A, c, grid, counts_h > 0, ijk,
-                                   stats, ws)
+                                   stats, ws, (phase, fac))
             which.index_copy_(0, target[:ns], ijk[:ns])
             cleaned.zero_()
-            phase_d, fac_d = dv(phase), dv(fac)  # held until the kernel has read them
+            phase_d, fac_d = held[5:]  # held until the kernel has read them
             rc = L.halma_clean_decide(ns, ptr(s_mem), ptr(s_grp), ptr(target), ptr(A[3]),
                                       ptr(A[4]), ptr(A[5]), vf, ptr(stats), ptr(phase_d),
                                       ptr(fac_d), float(q_fil), float(sig_fil), ptr(control),
@@ -924,15 +929,16 @@ def phase_space_clean(groups, x, y, z, vx, vy, vz, m, ll, q_fil, sig_fil, psc=Tr
     if redo.any():
         ns = _select(L, H, goff, nm, by, control, dv(redo.astype(np.uint8)), force, sel,
                      sel_ws)
-        cnt = np.diff(s_off.cpu().numpy())
-        kred = group_reduce(Groups(s_mem, s_off, np.concatenate([[0], np.cumsum(cnt)])),
-                            A[0], A[1], A[2], A[6]).cpu().numpy()
+        kred, s_off_h = _reduce_set(s_mem, s_off, off, A)
+        cnt = np.diff(s_off_h)
         rcen, rM, rR = _centres(kred, cnt)
         kc[redo], kM[redo], kR[redo], kcount[redo] = rcen[redo], rM[redo], rR[redo], cnt[redo]
     ok = kcount >= minp
-    grp_of = torch.repeat_interleave(torch.arange(H, device=dev),
-                                     torch.from_numpy(sizes).to(dev))
-    final = control_clean | force.bool()[grp_of]
+    if keep_all.any():
+        grp_of = torch.repeat_interleave(torch.arange(H, device=dev), dv(sizes), output_size=nm)
+        final = control_clean | force.bool()[grp_of]
+    else:
+        final = control_clean.clone()
     ns = _select(L, H, goff, nm, mem, control, dv(ok.astype(np.uint8)), force, sel, sel_ws)
     out_off = np.concatenate([[0], np.cumsum(kcount[ok])]).astype(np.int64)
     kept = Groups(s_mem[:max(ns, 1)].clone(), torch.from_numpy(out_off).to(dev), out_off)
@@ -957,10 +963,12 @@ def progenitors(new_groups, oripa, masses, old_npart, old_oripas, omm):
     nm = new_groups.n_members
     ids = to_dev(oripa, np.int64)
     new_ids = ids[new_groups.members[:nm].long()] if nm else ids[:0]
-    new_mass = to_dev(np.asarray(masses, np.float64).reshape(H), np.float64)
     old_npart = np.asarray(old_npart, np.int64).ravel()
     G = old_npart.size
-    old_off = to_dev(np.concatenate([[0], np.cumsum(old_npart)]).astype(np.int64), np.int64)
+    new_mass, old_off, old_mass = to_dev_all(
+        (np.asarray(masses, np.float64).reshape(H),
+         np.concatenate([[0], np.cumsum(old_npart)]).astype(np.int64),
+         np.asarray(omm, np.float64).ravel()[:G] if G else np.zeros(1)))
     no = int(old_npart.sum())
     if no == 0:
         old_ids = new_ids[:0]
@@ -968,15 +976,13 @@ def progenitors(new_groups, oripa, masses, old_npart, old_oripas, omm):
         old_ids = to_dev(old_oripas.reshape(-1)[:no], np.int64)
     else:
         old_ids = to_dev(np.asarray(old_oripas).ravel()[:no], np.int64)
-    old_mass = to_dev(np.asarray(omm, np.float64).ravel()[:G], np.float64) if G else new_mass
-    dev = new_mass.device
-    res = [torch.empty(H, dtype=torch.int32, device=dev) for _ in range(4)]
+    res = torch.empty((4, H), dtype=torch.int32, device=new_mass.device)
     ws = workspace(L.halma_progenitors_workspace_size(H, nm, G, no))
     rc = L.halma_progenitors(H, nm, ptr(new_groups.offsets), ptr(new_ids), ptr(new_mass), G, no,
                              ptr(old_off), ptr(old_ids), ptr(old_mass), *(ptr(r) for r in res),
                              ptr(ws), ws.numel(), stream_ptr())
     _lib.check(rc, "halma_progenitors")
-    return tuple(r.cpu().numpy() for r in res)
+    return tuple(res.cpu().numpy())
 
 
 def ball_query(x, y, z, centres, radii, strict=False, m=None, cell=0.0, sorted=True,
@@ -991,9 +997,9 @@ def ball_query(x, y, z, centres, radii, strict=False, m=None, cell=0.0, sorted=T
     L = _lib_()
     x, y, z = _coords(x, y, z)
     dev = x.device
-    c = to_dev(np.asarray(centres, np.float64).reshape(-1, 3), np.float64)
-    H = int(c.shape[0])
-    r = to_dev(np.asarray(radii, np.float64).reshape(H), np.float64)
+    c = np.asarray(centres, np.float64).reshape(-1, 3)
+    H = len(c)
+    c, r = to_dev_all((c, np.asarray(radii, np.float64).reshape(H)))
     n = int(x.numel())
     mm = _vec(m) if m is not None else None
     sums = torch.zeros(max(H, 1), dtype=torch.float64, device=dev) if m is not None else None

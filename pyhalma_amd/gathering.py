@@ -16,7 +16,7 @@ import numpy as np
 import torch
 
 from . import _lib, engine
-from .device import ptr, stream_ptr, to_dev, workspace
+from .device import ptr, stream_ptr, to_dev, to_dev_all, workspace
 
 MASS_TO_SUN = 9.1717e18
 
@@ -96,12 +96,14 @@ def amr_particles(grid, rho_B, boxes, centres=None, radii=None, mass_scale=1.0,
     (offsets (numpy int64, Q+1), dict x, y, z, vx, vy, vz, mass, temp of FP64 device
     tensors)."""
     L = _lib.load()
-    boxes_d = to_dev(np.asarray(boxes, np.float64).reshape(-1, 6), np.float64)
-    Q = int(boxes_d.shape[0])
+    boxes_d = np.asarray(boxes, np.float64).reshape(-1, 6)
+    Q = len(boxes_d)
     cen = rad = None
     if centres is not None:
-        cen = to_dev(np.asarray(centres, np.float64).reshape(Q, 3), np.float64)
-        rad = to_dev(np.asarray(radii, np.float64).reshape(Q), np.float64)
+        boxes_d, cen, rad = to_dev_all((boxes_d, np.asarray(centres, np.float64).reshape(Q, 3),
+                                        np.asarray(radii, np.float64).reshape(Q)))
+    else:
+        boxes_d = to_dev(boxes_d, np.float64)
     dev = boxes_d.device
     off = torch.zeros(Q + 1, dtype=torch.int64, device=dev)
     found = engine.ctypes_i64()
