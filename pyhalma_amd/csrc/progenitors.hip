@@ -27,7 +27,7 @@ namespace halma {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kRangeBlocks = 256;
+constexpr int kRangeBlocks = 256;  // per catalogue
 constexpr unsigned long long kEmpty = ~0ull;
 
 inline unsigned blocks_for(int64_t n) {
@@ -42,16 +42,30 @@ __device__ __forceinline__ unsigned long long fib_hash(unsigned long long k, int
     return (k * 0x9E3779B97F4A7C15ull) >> shift;
 }
 
-// smallest and largest key of ids[0..n): one (lo, hi) partial per block ...
-__global__ __launch_bounds__(kThreads) void k_range(const int64_t* __restrict__ ids, int64_t n,
+// smallest and largest key of both catalogues' IDs, the old ones by the first half of the
+// blocks: one (lo, hi) partial per block, four IDs of a thread in flight (2M IDs each: two
+// launches of one ID at a time 24.5 us, 10 us this way) ...
+__global__ __launch_bounds__(kThreads) void k_range(const int64_t* __restrict__ old_ids,
+                                                    int64_t n_old,
+                                                    const int64_t* __restrict__ new_ids,
+                                                    int64_t n_new,
                                                     unsigned long long* __restrict__ part) {
     __shared__ unsigned long long sh[2 * (kThreads / kWave)];
+    const bool old = blockIdx.x < kRangeBlocks;
+    const int64_t* ids = old ? old_ids : new_ids;
+    const int64_t n = old ? n_old : n_new;
+    constexpr int64_t kAll = int64_t{kRangeBlocks} * kThreads;
     unsigned long long lo = ~0ull, hi = 0ull;
-    for (int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; k < n;
-         k += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-        const unsigned long long v = id_key(ids[k]);
-        lo = v < lo ? v : lo;
-        hi = v > hi ? v : hi;
+    for (int64_t k0 = static_cast<int64_t>(blockIdx.x % kRangeBlocks) * kThreads + threadIdx.x;
+         k0 < n; k0 += 4 * kAll) {
+        unsigned long long v[4];  // past the end the last one again
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = id_key(ids[k0 + u * kAll < n ? k0 + u * kAll : n - 1]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            lo = v[u] < lo ? v[u] : lo;
+            hi = v[u] > hi ? v[u] : hi;
+        }
     }
     for (int s = kWave / 2; s >= 1; s >>= 1) {
         const unsigned long long a = __shfl_down(lo, s, kWave);
@@ -206,6 +220,7 @@ __device__ __forceinline__ void top2_add(Top2& t, int32_t oh, double m) {
 }
 
 constexpr int kRankThreads = 512;
+constexpr int kRankBatch = 8;  // members of a thread in flight
 constexpr int kLdsSet = 4096;  // LDS set slots; a halo filling more than half -> fallback
 
 // insert oh into a set of cap slots (-1 free): 1 inserted, 0 already there, -1 no free slot
@@ -280,7 +295,8 @@ __device__ void rank_set(const int32_t* set, int64_t cap, int64_t ih,
 
 // one block per new halo: its members' chains into an LDS set of old haloes, then
 // rank_set; a halo with more than kLdsSet / 2 distinct old haloes is flagged for
-// k_rank_fallback
+// k_rank_fallback.  Bound by the latency of the members' reads in the largest halo (20000
+// members, 40 a thread: 35 us one at a time, 26 us eight at a time).
 __global__ __launch_bounds__(kRankThreads) void k_halo_rank(
     int64_t H, const int64_t* __restrict__ noff, const int32_t* __restrict__ mhalo,
     const int32_t* __restrict__ mrest, Table t, const double* __restrict__ new_mass,
@@ -298,14 +314,24 @@ __global__ __launch_bounds__(kRankThreads) void k_halo_rank(
             full = 0;
         }
         __syncthreads();
-        for (int64_t k = b + threadIdx.x; k < e; k += blockDim.x) {
-            int32_t oh = mhalo[k];
-            int32_t j = mrest[k];
-            while (oh >= 0 && !full) {
-                const int rc = set_insert(lset, kLdsSet, oh);
-                if (rc < 0 || (rc > 0 && atomicAdd(&count, 1) + 1 > kLdsSet / 2)) full = 1;
-                oh = j >= 0 ? t.halo[j] : -1;
-                j = j >= 0 ? t.next[j] : -1;
+        for (int64_t k0 = b + threadIdx.x; k0 < e; k0 += kRankBatch * kRankThreads) {
+            int32_t head[kRankBatch], rest[kRankBatch];
+#pragma unroll
+            for (int u = 0; u < kRankBatch; ++u) {
+                const int64_t k = k0 + u * kRankThreads;
+                head[u] = k < e ? mhalo[k] : -1;
+                rest[u] = k < e ? mrest[k] : -1;
+            }
+#pragma unroll
+            for (int u = 0; u < kRankBatch; ++u) {
+                int32_t oh = head[u];
+                int32_t j = rest[u];
+                while (oh >= 0 && !full) {
+                    const int rc = set_insert(lset, kLdsSet, oh);
+                    if (rc < 0 || (rc > 0 && atomicAdd(&count, 1) + 1 > kLdsSet / 2)) full = 1;
+                    oh = j >= 0 ? t.halo[j] : -1;
+                    j = j >= 0 ? t.next[j] : -1;
+                }
             }
             if (full) break;
         }
@@ -436,10 +462,8 @@ int halma_progenitors(int64_t n_new, int64_t n_new_members, const int64_t* new_o
     const bool none = n_new_members == 0 || n_old_members == 0 || n_old == 0;
     if (!none) {
         // 1. key range, ID table of the old members
-        k_range<<<kRangeBlocks, kThreads, 0, st>>>(old_ids, n_old_members, w.part);
-        HALMA_LAUNCH_CHECK();
-        k_range<<<kRangeBlocks, kThreads, 0, st>>>(new_ids, n_new_members,
-                                                   w.part + 2 * kRangeBlocks);
+        k_range<<<2 * kRangeBlocks, kThreads, 0, st>>>(old_ids, n_old_members, new_ids,
+                                                       n_new_members, w.part);
         HALMA_LAUNCH_CHECK();
         k_range_final<<<1, kWave, 0, st>>>(w.part, 2 * kRangeBlocks, w.range);
         HALMA_LAUNCH_CHECK();
