@@ -372,7 +372,10 @@ __device__ __forceinline__ int stretch_cells(int64_t ncell) {
 // The link lanes of the rounds between stretches: the segments with a neighbour in another
 // stretch.  A column of more than kSegMin cells is cut into segments of kSegCells
 // cells, and each segment takes its own lanes (a long column's cells are then linked by
-// several lanes at once instead of one long chain of finds and unions).  Lane order:
+// several lanes at once instead of one long chain of finds and unions).  Up to kFewCells
+// cells, which leave most of the chip idle, every cell is a segment: FoF of a 24k Plummer
+// sphere 397 -> 339 us (its first round 113 -> 60), 98k clump stars 279 -> 255, 654k 430 -> 405,
+// 240k bridged 427 -> 405, 800k (650k cells) 670 and 667; 2.4M 1325 -> 1339.  Lane order:
 // segments grouped by the log2 of their particle count, largest first, so that the lanes
 // of a wavefront walk segments of similar length (a wavefront lasts as long as its
 // longest lane) and the longest start first.  A counting sort over kColClasses classes;
@@ -384,10 +387,14 @@ constexpr int kClassBlocks = 256;
 constexpr int kBigLists = 3;  // fillings of the list of large pairs: local, cross 1, cross 2
 constexpr int kSegMin = 4;
 constexpr int kSegCells = 4;
+constexpr int64_t kFewCells = 1 << 19;
 static_assert(kSegCells < 1024 && kSegMin < 1024, "a segment's cell count has 10 bits");
 
-// cells per segment of a column of n cells
-__device__ __forceinline__ int seg_step(int n) { return n > kSegMin ? kSegCells : (n > 0 ? n : 1); }
+// cells per segment of a column of n cells, of ncell in all
+__device__ __forceinline__ int seg_step(int n, int64_t ncell) {
+    if (ncell <= kFewCells) return 1;
+    return n > kSegMin ? kSegCells : (n > 0 ? n : 1);
+}
 
 // a segment's class: log2 of its particle count
 __device__ __forceinline__ int seg_class(const int2* __restrict__ crec, int c0, int c1) {
@@ -470,12 +477,13 @@ __global__ __launch_bounds__(256) void k_col_class_count(const int64_t* __restri
     if (threadIdx.x < kColClasses) h[threadIdx.x] = 0;
     __syncthreads();
     const int64_t ncol = totals[0] >> 32;
-    const int str = stretch_cells(totals[0] & 0xffffffff);
+    const int64_t ncell = totals[0] & 0xffffffff;
+    const int str = stretch_cells(ncell);
     const int64_t per = (ncol + gridDim.x - 1) / gridDim.x;
     const int64_t q0 = blockIdx.x * per, q1 = q0 + per < ncol ? q0 + per : ncol;
     for (int64_t q = q0 + threadIdx.x; q < q1; q += blockDim.x) {
         const int a0 = col_cell[q], a1 = col_cell[q + 1];
-        const int step = seg_step(a1 - a0);
+        const int step = seg_step(a1 - a0, ncell);
         const int last = neigh[q].last / str;
         for (int c = a0; c < a1; c += step)
             if (c / str != last) atomicAdd(&h[seg_class(crec, c, min(c + step, a1))], 1);
@@ -496,12 +504,13 @@ __global__ __launch_bounds__(256) void k_col_class_scatter(const int64_t* __rest
     if (threadIdx.x < kColClasses) h[threadIdx.x] = 0;
     __syncthreads();
     const int64_t ncol = totals[0] >> 32;
-    const int str = stretch_cells(totals[0] & 0xffffffff);
+    const int64_t ncell = totals[0] & 0xffffffff;
+    const int str = stretch_cells(ncell);
     const int64_t per = (ncol + gridDim.x - 1) / gridDim.x;
     const int64_t q0 = blockIdx.x * per, q1 = q0 + per < ncol ? q0 + per : ncol;
     for (int64_t q = q0 + threadIdx.x; q < q1; q += blockDim.x) {
         const int a0 = col_cell[q], a1 = col_cell[q + 1];
-        const int step = seg_step(a1 - a0);
+        const int step = seg_step(a1 - a0, ncell);
         const int last = neigh[q].last / str;
         for (int c = a0; c < a1; c += step)
             if (c / str != last) atomicAdd(&h[seg_class(crec, c, min(c + step, a1))], 1);
@@ -517,7 +526,7 @@ __global__ __launch_bounds__(256) void k_col_class_scatter(const int64_t* __rest
     __syncthreads();
     for (int64_t q = q0 + threadIdx.x; q < q1; q += blockDim.x) {
         const int a0 = col_cell[q], a1 = col_cell[q + 1];
-        const int step = seg_step(a1 - a0);
+        const int step = seg_step(a1 - a0, ncell);
         const int last = neigh[q].last / str;
         for (int c = a0; c < a1; c += step) {
             if (c / str == last) continue;
@@ -1168,7 +1177,7 @@ int fof_run(const T* x, const T* y, const T* z, int64_t n, double ll, int* label
 }  // namespace
 
 // Runs FoF into `labels` (the cell structures stay in the workspace).  Asynchronous
-// after one read-back of the bounding box; *err (device) is non-zero on a range or table
+// after one read-back of the bounding box; *err (device) is non-zero on a range
 // failure.
 int fof_labels_async(const void* x, const void* y, const void* z, int dtype, int64_t n,
                      double ll, int* labels, void* ws, size_t ws_bytes, int** err_out,
