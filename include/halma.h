@@ -51,8 +51,8 @@ int halma_device_cu_count(void);
  *
  * out[i] = sum_j m[j] / |x_j - x_i| over the sources j whose three coordinates all
  * differ from test i's (particle_subroutines.f90:499-501), inputs FP32 (the caller
- * casts, as halo_gas.py:172-178 does).  Summed in FP32 on the vector ALUs with
- * Kahan-compensated tiles; the FP64 value of the compensated sum is written to
+ * casts, as halo_gas.py:172-178 does).  Summed on the vector ALUs in FP32 sub-tiles
+ * that are added in FP64; the FP64 value of the sum is written to
  * out_f64 when that pointer is non-NULL, and out (float32, the reference's output
  * type) may be NULL when only out_f64 is wanted.  The relative error against the
  * FP64 direct sum is below halma_pot_error_bound() (a rigorous bound).  The rule is
@@ -371,7 +371,7 @@ int halma_progenitors(int64_t n_new, int64_t n_new_members, const int64_t *new_o
  * most max_iter passes); max_iter = 1 is the reference's single test with v_cm over all
  * members.  Haloes are the CSR ranges offsets[h]..offsets[h+1] of `members` (particle
  * indices into the global arrays); offsets is a HOST array of n_halo+1 entries.
- * Decisions are exact with respect to the FP64 oracle: members whose FP32-compensated E
+ * Decisions are exact with respect to the FP64 oracle: members whose E from FP32 terms
  * lies inside the rigorous error band are re-tested with an FP64 sum in the oracle's
  * fixed order.  Outputs (device): bound[k] per member position (1 bound, 0 not); iters
  * (n_halo int32, may be NULL) passes per halo; vcm (3 per halo, may be NULL); pot (per
@@ -476,7 +476,7 @@ int halma_energy_test_self_batched(int64_t n_halo, const int64_t *tst_off, const
  * over the sources j of h (FP32 sm, sx, sy, sz) whose three coordinates all differ
  * from the test's (particle_subroutines.f90:499-501; drops the self pair).  Any of
  * pot, acc, wsum may be NULL; when pot and acc or wsum are asked for together, one pass
- * over the pairs computes them all.  FP32 compensated sums merged in FP64: pot within
+ * over the pairs computes them all.  FP32 sub-tiles merged in FP64: pot within
  * halma_pot_error_bound() relative; acc and wsum within the same bound relative to
  * sum_j |term_j|.  A halo with at most 8 tests spreads each test's sources over the lanes
  * of a wavefront (chunks of 4096 sources); larger haloes hold 64 tests per wavefront.
@@ -543,7 +543,7 @@ int halma_weighted_sums(int64_t n_halo, const int64_t *offsets, const void *m, i
 
 /* Tuning knobs of the FP32 pair kernels (set by the autotuner; read back with get).
  *   HALMA_TUNE_TESTS_PER_LANE : test particles per lane (1, 2, 4)
- *   HALMA_TUNE_SUBTILE        : sources per plain FP32 sub-tile before the Kahan add
+ *   HALMA_TUNE_SUBTILE        : sources per plain FP32 sub-tile before the FP64 add
  *                               (4 or 8)
  *   HALMA_TUNE_MIN_CHUNK      : smallest source chunk when a halo's source range is
  *                               split across waves (multiple of 64, >= 64)

@@ -6,7 +6,7 @@
 // with S_i the pair sum of particle_subroutines.f90:466-514 of test i against its halo's
 // sources (any CSR source set: gas cells, dark matter, stars) and v_h the halo's bulk
 // velocity given by the caller (halo_gas.py:468 uses the halo's vx, vy, vz).  S comes
-// from the persistent FP32 compensated kernel (one launch for every halo); members
+// from the persistent FP32 pair kernel (one launch for every halo); members
 // whose |E| lies inside the FP32 error band are re-tested with the FP64 sum in the
 // oracle's fixed order (one block each), so the mask equals the FP64 oracle's.
 #include <math.h>
@@ -40,7 +40,7 @@ struct TestArgs {
     const double* halo_v;
     double cg;        // factor * G
     double bound_rel; // B of the FP32 sums
-    const double* S;  // FP32-compensated sums (FP64 values)
+    const double* S;  // sums of FP32 sub-tiles (FP64 values)
     uint8_t* bound;
     int32_t* band;
     unsigned long long* counters;  // [0] band members

@@ -53,7 +53,7 @@ struct DynSets {
     const int* chunk = nullptr;  // per-halo source chunk of this launch (else the plan's)
 };
 
-// Batched FP32 compensated pair sums over H haloes (HOST CSR offsets), FP64 (and/or
+// Batched FP32 pair sums over H haloes (HOST CSR offsets), FP64 (and/or
 // FP32) result per test; scratch from pot_batched_workspace_bytes.  Stream-ordered.
 size_t pot_batched_workspace_bytes(int64_t H, const int64_t* src_off, const int64_t* tst_off);
 // ev_begin / ev_end (may be null): events recorded on the stream right before and after

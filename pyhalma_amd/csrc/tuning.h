@@ -7,7 +7,7 @@ namespace halma {
 // pass 4.34 ms against 4.99 ms for R=2, SUB=8, 16 waves/CU, 4 items/wave).
 struct Tuning {
     int tests_per_lane = 2;   // R: test particles held in registers per lane
-    int subtile = 4;          // sources summed in plain FP32 before each Kahan add
+    int subtile = 4;          // sources summed in plain FP32 before each FP64 add
     int min_chunk = 512;      // smallest source chunk when a source range is split
     int items_per_wave = 8;   // queue items targeted per resident wave
     int waves_per_cu = 32;    // persistent waves per compute unit

@@ -16,13 +16,13 @@ def _lib_():
 
 
 def pot_error_bound():
-    """Rigorous relative error bound of the FP32 compensated pair sums."""
+    """Rigorous relative error bound of the FP32 pair sums."""
     return float(_lib_().halma_pot_error_bound())
 
 
 def pot_sum(m, x, y, z, tx, ty, tz, out_dtype=np.float32, with_f64=False):
     """S_i = sum_j m_j / r_ij over sources with all three coordinates different from
-    test i's (particle_subroutines.f90:466-514), FP32 compensated on the GPU.
+    test i's (particle_subroutines.f90:466-514), FP32 sub-tiles added in FP64 on the GPU.
     Returns a device tensor (float32 by default; float64 if out_dtype is float64).
     With with_f64=True returns (out, out_f64)."""
     L = _lib_()

@@ -14,8 +14,8 @@ libhalma GPU kernels:
       (particle_subroutines.f90:517-556)
 
 Like f2py, array arguments are converted to float32 and a length that does not match
-the declared dimension raises ValueError.  The sum is FP32 with compensated
-accumulation; its relative error is below ``pyhalma_amd.engine.pot_error_bound()``
+the declared dimension raises ValueError.  The sum is FP32 in sub-tiles
+added in FP64; its relative error is below ``pyhalma_amd.engine.pot_error_bound()``
 (the reference's plain FP32 loop has no such bound).
 
 The same Fortran module also holds ``halo_shape`` and ``sigma_projections``
