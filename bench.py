@@ -47,7 +47,7 @@ FOF_BYTES_PER_PARTICLE = 16  # 12 B FP32 xyz read + 4 B label written
 # step (the first pass carries almost all of it): FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0 from
 # two rocprofv3 --pmc passes, each scaled by what the counter reads for a 256 MiB device
 # copy (profiles/clumps_2M_hbm_traffic.md)
-SYM_TRAFFIC_BYTES = 80.0e6
+SYM_TRAFFIC_BYTES = 90.0e6
 MINP = 50
 VALU_ROOF = ("FP32 vector ALU (157.3 TFLOP/s, MI355X's dense FP32 figure, which counts "
              "packed FMA); the kernel issues FP32 vector instructions, no matrix "
@@ -1097,8 +1097,9 @@ def bench_centring(args):
     roofline = {"bound": "valu", "achieved": round(fwd_tf, 3), "peak": PEAK_FP32_TFLOPS,
                 "unit": "TFLOP/s", "frac": round(fwd_tf / PEAK_FP32_TFLOPS, 4),
                 "traffic": None, "roof": VALU_ROOF,
-                "kernel": "k_soft_tile<S and acceleration, tests = the halo's members> (the "
-                          "potential-energy forward with the gradient fused)",
+                "kernel": "k_soft_sym<S and acceleration, tests = the halo's members, each pair "
+                          "once> (every launch of the potential-energy forward with the "
+                          "gradient fused)",
                 "flop_per_pair": fused_flop, "pairs_per_launch": pairs,
                 "launch_ms": round(fwd_s * 1e3, 3), "launches_per_step": 1,
                 "unfused": {"S": {"ms": pot_ms, "flop_per_pair": FLOP_PER_SOFT_PAIR,
