@@ -57,7 +57,7 @@ def to_dev_all(arrays, dtype=None):
             if dtype is not None:
                 arr = arr.astype(dtype, copy=False)
             a = torch.from_numpy(np.ascontiguousarray(arr))
-            if total + a.numel() * a.element_size() <= PACK_BYTES:
+            if 0 < a.numel() and total + a.numel() * a.element_size() <= PACK_BYTES:
                 host.append((k, a, total))
                 total += -(-a.numel() * a.element_size() // 256) * 256
                 continue

@@ -24,3 +24,5 @@ def test_packed_like_single(gpu, dtype, big):
         assert t.dtype == want.dtype and t.shape == want.shape and t.is_contiguous()
         assert t.device == want.device and torch.equal(t, want)
     assert device.to_dev_all([]) == []
+    for t in device.to_dev_all([np.zeros((0, 3)), np.zeros(0, np.int64)], dtype):
+        assert t.numel() == 0 and t.is_cuda
