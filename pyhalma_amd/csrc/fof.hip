@@ -927,9 +927,20 @@ __global__ void k_roots(const int64_t* __restrict__ totals, int* __restrict__ pa
     }
 }
 
-// Also folds every cell's minimum particle index into its component's minimum.  The
-// lanes of a wavefront whose root is the first lane's (consecutive cells mostly share
-// one) are merged into one check and one atomic; the others act alone.
+// Also folds every cell's minimum particle index into its component's minimum.  Up to
+// kRootGroups sets of lanes of a wavefront that share a root (consecutive cells mostly have
+// few) are merged into one check and one atomic each; the others act alone.  A component's
+// minimum only falls, so a value that is not below what is read of it needs no atomic,
+// however old the read.  Bound by the atomics on the few large components' words: 6.5M cells
+// of 4000 bridged pairs 183 us with one set and every atomic, 101 us this way.
+constexpr int kRootGroups = 4;
+
+__device__ __forceinline__ void root_min(int* parent, int* comp_min, int r, int v, int* err) {
+    if (coherent_read(parent + r) != r) atomicOr(err, 4);
+    if (v < __hip_atomic_load(comp_min + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))
+        atomicMin(comp_min + r, v);
+}
+
 __global__ __launch_bounds__(256) void k_check_roots(const int64_t* __restrict__ totals,
                                                      int* __restrict__ parent,
                                                      const int* __restrict__ root,
@@ -944,18 +955,16 @@ __global__ __launch_bounds__(256) void k_check_roots(const int64_t* __restrict__
         const bool valid = c < n_cells;  // lane 0 always is
         const int r = valid ? root[c] : -1;
         const int m = valid ? cell_min[c] : INT32_MAX;
-        const int r0 = __shfl(r, 0, kWave);
-        const bool same = r == r0;
-        int v = same ? m : INT32_MAX;
-        for (int s = 32; s >= 1; s >>= 1) v = min(v, __shfl_xor(v, s, kWave));
-        if (lane == 0) {
-            if (coherent_read(parent + r0) != r0) atomicOr(err, 4);
-            atomicMin(comp_min + r0, v);
+        unsigned long long left = __ballot(valid);
+        for (int k = 0; k < kRootGroups && left != 0; ++k) {
+            const int first = __ffsll(left) - 1;
+            const int g = __shfl(r, first, kWave);
+            int v = r == g ? m : INT32_MAX;
+            for (int s = 32; s >= 1; s >>= 1) v = min(v, __shfl_xor(v, s, kWave));
+            if (lane == first) root_min(parent, comp_min, g, v, err);
+            left &= ~__ballot(r == g);
         }
-        if (valid && !same) {
-            if (coherent_read(parent + r) != r) atomicOr(err, 4);
-            atomicMin(comp_min + r, m);
-        }
+        if ((left >> lane) & 1) root_min(parent, comp_min, r, m, err);
     }
 }
 
