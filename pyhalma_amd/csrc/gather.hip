@@ -314,8 +314,8 @@ __global__ __launch_bounds__(W * kWave) void k_ball_count(int64_t H, Grid g, Que
         int64_t cnt = 0;
         double mh = 0.0, ml = 0.0;
         for_row_points<W>(g, rows_of(g, c, R), start, span, [&](int total, auto&& at) {
-            for (int p = threadIdx.x; p < total; p += W * kWave) {
-                const P rec = pk[at(p)];
+            for (int64_t p = threadIdx.x; p < total; p += W * kWave) {
+                const P rec = pk[at(static_cast<int>(p))];
                 if (is_hit(rec, c, R, q.strict)) {
                     ++cnt;
                     if (q.m) dd_add(mh, ml, ldf(q.m, q.mt, rec.i));
@@ -371,9 +371,9 @@ __global__ __launch_bounds__(W * kWave) void k_ball_emit(int64_t H, Grid g, Quer
         const double R = q.radius[h];
         int64_t running = off[h];
         for_row_points<W>(g, rows_of(g, c, R), start, span, [&](int total, auto&& at) {
-            for (int p0 = 0; p0 < total; p0 += W * kWave) {
-                const int p = p0 + static_cast<int>(threadIdx.x);
-                const P rec = pk[at(p < total ? p : total - 1)];
+            for (int64_t p0 = 0; p0 < total; p0 += W * kWave) {
+                const int64_t p = p0 + threadIdx.x;
+                const P rec = pk[at(p < total ? static_cast<int>(p) : total - 1)];
                 const bool hit = p < total && is_hit(rec, c, R, q.strict);
                 const unsigned long long mask = __ballot(hit);
                 if (lane == 0) shc[turn][w] = __popcll(mask);
