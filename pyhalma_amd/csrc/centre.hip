@@ -42,18 +42,15 @@ __global__ void k_centre_pack(const float* __restrict__ m, const float* __restri
     if (i < n) out[i] = make_float4(x[i], y[i], z[i], m[i]);
 }
 
-__global__ void k_centre_init(int n_halo, int max_iter, int* __restrict__ moving,
-                              int* __restrict__ iters, double* __restrict__ steps,
-                              int* __restrict__ left) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < max(n_halo, max_iter + 1);
-         i += gridDim.x * blockDim.x) {
-        if (i < n_halo) {
-            moving[i] = 1;
-            iters[i] = 0;
-            steps[i] = INFINITY;
-        }
-        if (i <= max_iter) left[i] = 0;
+__global__ void k_centre_init(int n_halo, int* __restrict__ moving, int* __restrict__ iters,
+                              double* __restrict__ steps, int* __restrict__ left) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < n_halo) {
+        moving[i] = 1;
+        iters[i] = 0;
+        steps[i] = INFINITY;
     }
+    if (i < 2) left[i] = 0;
 }
 
 // The sums of one chunk at its halo's centre: a and w (kModeAcc, part[4 k ..]) or S
@@ -127,17 +124,19 @@ __device__ __forceinline__ void halo_sums(const CentreDesc& d, const double* __r
         for (int q = 0; q < NQ; ++q) v[q] = v[q] + __shfl_xor(v[q], m, kWave);
 }
 
-// One wavefront per halo: the step of a moving halo, and whether it moves on; *left counts
-// the haloes that do.
+// One wavefront per halo: the step of a moving halo, and whether it moves on; left[turn]
+// counts the haloes that do, and the other word, whose count was copied to the host before
+// this launch, is cleared for the next iteration.
 __global__ __launch_bounds__(256) void k_centre_step(const CentreDesc* __restrict__ halos,
                                                      int n_halo, const double* __restrict__ part,
                                                      double limit, double* __restrict__ c,
                                                      int* __restrict__ moving,
                                                      int* __restrict__ iters,
                                                      double* __restrict__ steps,
-                                                     int* __restrict__ left) {
+                                                     int* __restrict__ left, int turn) {
     const int lane = __lane_id();
     const int h = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
+    if (blockIdx.x == 0 && threadIdx.x == 0) left[turn ^ 1] = 0;
     if (h >= n_halo || !moving[h]) return;
     double v[4];
     halo_sums<4>(halos[h], part, lane, v);
@@ -154,7 +153,7 @@ __global__ __launch_bounds__(256) void k_centre_step(const CentreDesc* __restric
     iters[h] += 1;
     const bool on = len > limit;
     moving[h] = on;
-    if (on) atomicAdd(left, 1);
+    if (on) atomicAdd(left + turn, 1);
 }
 
 __global__ __launch_bounds__(256) void k_centre_pot(const CentreDesc* __restrict__ halos,
@@ -174,7 +173,7 @@ struct CentreWs {
     int* chunk_halo;
     double* part;
     int* moving;
-    int* left;  // haloes still moving after iteration i
+    int* left;  // haloes still moving after iteration i, at i % 2
     size_t bytes;
 };
 
@@ -184,7 +183,7 @@ int64_t centre_chunks(int64_t H, const int64_t* off) {
     return n;
 }
 
-CentreWs carve_centre(void* base, int64_t H, int64_t n, int64_t n_chunks, int max_iter) {
+CentreWs carve_centre(void* base, int64_t H, int64_t n, int64_t n_chunks) {
     Carver c(base);
     CentreWs w;
     w.src4 = c.take<float4>(std::max<int64_t>(n, 1));
@@ -192,13 +191,13 @@ CentreWs carve_centre(void* base, int64_t H, int64_t n, int64_t n_chunks, int ma
     w.chunk_halo = c.take<int>(std::max<int64_t>(n_chunks, 1));
     w.part = c.take<double>(4 * std::max<int64_t>(n_chunks, 1));
     w.moving = c.take<int>(std::max<int64_t>(H, 1));
-    w.left = c.take<int>(static_cast<size_t>(max_iter) + 1);
+    w.left = c.take<int>(2);
     w.bytes = c.used;
     return w;
 }
 
 int check_centre(int64_t H, const int64_t* off, int max_iter) {
-    if (H < 0 || !off || H > INT32_MAX || max_iter < 0 || max_iter == INT32_MAX)
+    if (H < 0 || !off || H > INT32_MAX || max_iter < 0)
         return set_error(HALMA_E_ARG, "halma_refine_centres: bad halo count, offsets or max_iter");
     for (int64_t h = 0; h < H; ++h) {
         if (off[h + 1] < off[h]) return set_error(HALMA_E_ARG, "offsets must not decrease");
@@ -221,9 +220,9 @@ extern "C" {
 
 size_t halma_refine_centres_workspace_size(int64_t n_halo, const int64_t* offsets, int max_iter) {
     if (check_centre(n_halo, offsets, max_iter)) return 0;
-    if (n_halo == 0) return carve_centre(nullptr, 0, 0, 0, max_iter).bytes;
+    if (n_halo == 0) return carve_centre(nullptr, 0, 0, 0).bytes;
     return carve_centre(nullptr, n_halo, offsets[n_halo] - offsets[0],
-                        centre_chunks(n_halo, offsets), max_iter)
+                        centre_chunks(n_halo, offsets))
         .bytes;
 }
 
@@ -240,7 +239,7 @@ int halma_refine_centres(int64_t n_halo, const int64_t* offsets, const float* m,
         return set_error(HALMA_E_ARG, "halma_refine_centres: null pointer");
     const int64_t n_chunks = centre_chunks(n_halo, offsets);
     const int H = static_cast<int>(n_halo), nc = static_cast<int>(n_chunks);
-    CentreWs w = carve_centre(ws, n_halo, n, n_chunks, max_iter);
+    CentreWs w = carve_centre(ws, n_halo, n, n_chunks);
     if (!ws || ws_bytes < w.bytes)
         return set_error(HALMA_E_WORKSPACE, "workspace %zu < required %zu", ws_bytes, w.bytes);
     hipStream_t st = static_cast<hipStream_t>(stream);
@@ -262,8 +261,8 @@ int halma_refine_centres(int64_t n_halo, const int64_t* offsets, const float* m,
             m + s0, x + s0, y + s0, z + s0, n, w.src4);
         HALMA_LAUNCH_CHECK();
     }
-    k_centre_init<<<std::max(1, std::min(256, H / 256 + 1)), 256, 0, st>>>(H, max_iter, w.moving,
-                                                                          iters, steps, w.left);
+    k_centre_init<<<static_cast<unsigned>((n_halo + 256) / 256), 256, 0, st>>>(H, w.moving, iters,
+                                                                               steps, w.left);
     HALMA_LAUNCH_CHECK();
     const float e2 = static_cast<float>(eps * eps);
     const unsigned gc = static_cast<unsigned>((n_chunks + 3) / 4);
@@ -283,12 +282,12 @@ int halma_refine_centres(int64_t n_halo, const int64_t* offsets, const float* m,
                 k_centre_part<kModeAcc><<<gc, 256, 0, st>>>(w.src4, w.halos, w.chunk_halo, nc,
                                                             centres, w.moving, e2, w.part);
             k_centre_step<<<gh, 256, 0, st>>>(w.halos, H, w.part, tol * eps, centres, w.moving,
-                                              iters, steps, w.left + launched);
+                                              iters, steps, w.left, launched & 1);
             e = hipGetLastError();
         }
         if (e == hipSuccess)
-            e = hipMemcpyAsync(const_cast<int*>(host) + q, w.left + launched - 1, sizeof(int),
-                               hipMemcpyDeviceToHost, st);
+            e = hipMemcpyAsync(const_cast<int*>(host) + q, w.left + ((launched - 1) & 1),
+                               sizeof(int), hipMemcpyDeviceToHost, st);
         if (e == hipSuccess) e = hipEventRecord(done[q], st);
         if (e != hipSuccess) break;
         pending[q] = true;

@@ -219,9 +219,11 @@ def refine_centres(offsets, m, x, y, z, seeds, eps, tol, max_iter):
     if H == 0:
         return c, S, iters, steps
     off = _lib.i64_array(offsets)
-    ws = workspace(L.halma_refine_centres_workspace_size(H, off, int(max_iter)))
+    # a C int, as the step counts are: any larger limit is as good as none, one below 0 is 0
+    max_iter = min(max(int(max_iter), 0), 2 ** 31 - 1)
+    ws = workspace(L.halma_refine_centres_workspace_size(H, off, max_iter))
     rc = L.halma_refine_centres(H, off, ptr(m), ptr(x), ptr(y), ptr(z), float(eps), float(tol),
-                                int(max_iter), ptr(c), ptr(S), ptr(iters), ptr(steps), ptr(ws),
+                                max_iter, ptr(c), ptr(S), ptr(iters), ptr(steps), ptr(ws),
                                 ws.numel(), stream_ptr())
     _lib.check(rc, "halma_refine_centres")
     return c, S, iters, steps

@@ -1,6 +1,7 @@
 """The centring iteration on the device (halma_refine_centres) against the same iteration
 in FP64 torch: haloes of sizes around its 2048-particle chunks and its 512-particle inner
-step, empty and one-particle haloes, iteration limits around its batches of four."""
+step, empty and one-particle haloes, iteration limits around its batches of four,
+limits below 0 and beyond any count."""
 import numpy as np
 import pytest
 
@@ -63,3 +64,28 @@ def test_refine_centres_chunk_edges(gpu, max_iter):
             assert abs(steps[h] - length) <= 2e-5 * EPS, h
         elif it == 0:
             assert np.isinf(steps[h])
+
+
+def test_refine_centres_any_limit(gpu):
+    """Limits beyond any count (2^31 - 1 and 10^10 among them) are no limit, those below 0
+    are 0, as a loop over range(max_iter) has it."""
+    from pyhalma_amd import centring
+
+    rng = np.random.default_rng(8)
+    off = np.array([0, 700, 3000])
+    x = rng.normal(scale=0.004, size=(3000, 3)).astype(np.float32)
+    m = rng.uniform(1e4, 1e6, 3000).astype(np.float32)
+    seeds = rng.normal(scale=1e-3, size=(2, 3))
+    print("limits", flush=True)
+
+    def run(max_iter):
+        r = centring.refine_centres(*x.T, m, off, seeds, EPS, max_iter=max_iter, tol=1e-3)
+        return [a.cpu().numpy() for a in (r.centres, r.S, r.iters, r.steps)]
+
+    want, none = run(2000), run(0)
+    assert 0 < want[2].max() < 2000 and none[2].max() == 0
+    for max_iter in (2 ** 31 - 2, 2 ** 31 - 1, 2 ** 31, 10 ** 10):
+        for a, b in zip(run(max_iter), want):
+            assert np.array_equal(a, b), max_iter
+    for a, b in zip(run(-1), none):
+        assert np.array_equal(a, b)
