@@ -476,7 +476,7 @@ int soft_run(int64_t n_halo, const int64_t* src_off, const float* sm, const floa
         return set_error(HALMA_E_ARG, "packed sources must be 16-byte aligned");
     if (!pot && !acc && !wsum) return 0;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    // the members as their own tests, without wsum: each pair once (soft_sym.hip; 18.1 ms
+    // the members as their own tests, without wsum: each pair once (soft_sym.hip; 18.9 ms
     // for S and a of six haloes of 2e4-2e5 members, 26.6 ms one-sided); its slots grow with
     // the halo, so a call with a halo of more than 2^23 members stays here
     if (self && !wsum && soft_sym_takes(n_halo, src_off))

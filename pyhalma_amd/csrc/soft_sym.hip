@@ -8,8 +8,9 @@
 //   - test side: FP32 sums of the eight terms, added in FP64 per test and quantity (two
 //     instructions, where a Kahan sum takes four);
 //   - source side: per source the T terms of a lane in FP32, then the fixed tree over the
-//     lanes (reduce8, its last levels in FP64).  A holds every test of the item, so the total is the item's and goes
-//     straight to its slot.
+//     lanes (reduce8), FP64 from the first level at T = 8, from the third at T = 2: eight
+//     terms meet in FP32, as on the test side.  A holds every test of the item, so the total
+//     is the item's and goes straight to its slot.
 // A diagonal item (A == B) takes all its ordered pairs on the test side.  A member's sums
 // of one item go to the slot of the other block (mod the band width), in FP64: slot B for
 // the members of A, slot A for the members of B; k_soft_sym_merge adds a member's slots in
@@ -23,8 +24,10 @@
 //
 // Bound by the FP32 vector ALUs: 23 issue slots per pair distance (3 differences, 3 for
 // r^2, 3 for the rule, 2 for the reciprocal root, 2 for its cube, 2 + 8 for the sums of the
-// two sides), 1 for the FP64 sums and 1.6 for the tree at T = 8, i.e. 12.8 per ordered pair;
-// the one-sided kernel of soft.hip takes 21.5.
+// two sides), 1 for the FP64 sums and 2.4 for the tree at T = 8 (1.6 with its first three
+// levels in FP32, i.e. 64 terms instead of 8: six haloes of 2e4-2e5 members 18.2 instead of
+// 19.0 ms a call, the spread of S 1.27 times the one-sided kernel's instead of 0.9), i.e. 13.2
+// per ordered pair; the one-sided kernel of soft.hip takes 21.5.
 #include <math.h>
 
 #include <algorithm>
@@ -191,7 +194,7 @@ __global__ __launch_bounds__(256, 2) void k_soft_sym(const float4* __restrict__ 
                     ss_group<MODE, T, true, false>(sp + j0 + g, cnt - g, e2, x, y, z, m, R, pj);
 #pragma unroll
                 for (int q = 0; q < NP; ++q) {
-                    const double tot = reduce8(pj[q], lane);
+                    const double tot = reduce8<T == 8 ? 0 : 2>(pj[q], lane);
                     if ((lane & 7) == 0 && g + s < cnt)
                         out[q * n_part + g + s] = q < A0 ? tot : -tot;
                 }

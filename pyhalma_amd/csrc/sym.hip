@@ -114,7 +114,7 @@ __device__ __forceinline__ double sym_group(const float4* __restrict__ q0, int c
     if (lim == 0) return 0.0;
 #pragma unroll
     for (int s = 0; s < 8; ++s) p[0][s] += p[1][s];
-    return reduce8(p[0], lane);
+    return reduce8<3>(p[0], lane);
 }
 
 // Sources j0 .. j0 + cnt - 1 (a segment) of item (A, B): the source side to its slot (out,

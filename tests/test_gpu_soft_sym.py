@@ -55,10 +55,11 @@ def test_self_sums_block_and_band_edges(gpu, sizes):
         for k in range(0, i.numel(), step):
             q = i[k:k + step]
             ws, wa, mag = _fp64(p, q)
-            # per term: differences and r^2 2.5u, the root 2u, products u, chain and tree 12u
-            # (S); three times the root's error, two products more and the sums for a
+            # per term: differences and r^2 2.5u, the root 2u, the product and eight terms in
+            # FP32 8u, 0.5u for the FP64 sums (S); three times the root's error, two products,
+            # the difference and the sums for a
             es = (S[off[h] + q] - ws).abs() / ws.clamp(min=1e-300)
-            assert float(es.max()) <= 18 * U or n == 1, (h, float(es.max()))
+            assert float(es.max()) <= 13 * U or n == 1, (h, float(es.max()))
             ea = (a[off[h] + q] - wa).abs() / mag.clamp(min=1e-300)
             assert float(ea.max()) <= 26 * U or n == 1, (h, float(ea.max()))
     one = engine.pot_soft_self(off, rows, EPS, pot=True, acc=False)["pot"]
@@ -69,6 +70,32 @@ def test_self_sums_block_and_band_edges(gpu, sizes):
     assert torch.equal(alone["pot"], S[off[h]:]) and torch.equal(alone["acc"], a[off[h]:])
     based = engine.pot_soft_self(off[h:], rows, EPS, pot=True, acc=True)  # offsets not from 0
     assert torch.equal(based["pot"][off[h]:], S[off[h]:])
-    # the sums with wsum run one-sided: the same values to both bounds
+    # the sums with wsum run one-sided: the same values to both bounds (13u and 15u)
     old = engine.pot_soft_self(off, rows, EPS, pot=True, acc=True, wsum=True)
-    assert float(((old["pot"] - S).abs() / S.clamp(min=1e-300)).max()) <= 36 * U
+    assert float(((old["pot"] - S).abs() / S.clamp(min=1e-300)).max()) <= 28 * U
+
+
+@pytest.mark.parametrize("n", [1000, 16383, 17000])
+def test_self_sums_are_as_exact_as_the_one_sided_ones(gpu, n):
+    """Both forms add eight terms in FP32 before FP64 (or a Kahan pair), on either side of a
+    pair: the spread of S about its FP64 value is no larger (the mean, the root's bias, is
+    common to both).  With 64 terms in FP32 on the source side it is 1.27 of it at 17000."""
+    import torch
+
+    from pyhalma_amd import engine
+
+    rng = np.random.default_rng(n)
+    u = np.sqrt(rng.uniform(1e-6, 0.98, n))
+    v = rng.normal(size=(n, 3))
+    x = (0.02 * u / (1 - u))[:, None] * v / np.linalg.norm(v, axis=1, keepdims=True)
+    m = np.exp(rng.uniform(np.log(1e4), np.log(1e6), n))
+    rows = torch.from_numpy(np.concatenate([x + 7, m[:, None]], 1).astype(np.float32)).cuda()
+    print(f"n={n}", flush=True)
+    off, p = np.array([0, n]), rows.double()
+    S = engine.pot_soft_self(off, rows, EPS, pot=True)["pot"]
+    T = engine.pot_soft_self(off, rows, EPS, pot=True, wsum=True)["pot"]
+    want = torch.cat([_fp64(p, torch.arange(k, min(k + 500, n), device="cuda"))[0]
+                      for k in range(0, n, 500)])
+    sym, one = ((S - want) / want).std(), ((T - want) / want).std()
+    print(f"symmetric {float(sym):.3e} one-sided {float(one):.3e}", flush=True)
+    assert float(sym) <= 1.05 * float(one)
