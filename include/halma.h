@@ -476,9 +476,10 @@ int halma_energy_test_self_batched(int64_t n_halo, const int64_t *tst_off, const
  * over the sources j of h (FP32 sm, sx, sy, sz) whose three coordinates all differ
  * from the test's (particle_subroutines.f90:499-501; drops the self pair).  Any of
  * pot, acc, wsum may be NULL; when pot and acc or wsum are asked for together, one pass
- * over the pairs computes them all.  FP32 sub-tiles merged in FP64: pot within
- * halma_pot_error_bound() relative; acc and wsum within the same bound relative to
- * sum_j |term_j|.  A halo with at most 8 tests spreads each test's sources over the lanes
+ * over the pairs computes them all.  FP32 terms in plain sub-tiles of eight, the sub-tiles
+ * in Kahan pairs (self sums without wsum: in FP64), the chunks in FP64.  Against FP64: pot
+ * within 2^-20 relative, acc and wsum within 2^-19 relative to sum_j |term_j|, whatever the
+ * tuning (halma_pot_error_bound() is the plain sums').  A halo with at most 8 tests spreads each test's sources over the lanes
  * of a wavefront (chunks of 4096 sources); larger haloes hold 64 tests per wavefront.
  * Chunk sizes follow from each halo's own source and test counts and the chunk
  * partials are added in chunk order, so a test's bits depend on its halo's inputs only
@@ -495,8 +496,8 @@ int halma_pot_soft_batched(int64_t n_halo, const int64_t *src_off, const float *
                            void *stream);
 /* The same with the sources packed by the caller: src_xyzm holds (x, y, z, m) per source
  * as 4 consecutive floats (16-byte aligned), indexed like sm, sx, sy, sz above.  For
- * callers that evaluate the same sources many times (the centring iterations): the
- * sources are not repacked on every call.  Same workspace size, results bit-identical
+ * callers that evaluate the same sources many times: the sources are not repacked on every
+ * call.  Same workspace size, results bit-identical
  * to halma_pot_soft_batched on the same values. */
 int halma_pot_soft_batched_packed(int64_t n_halo, const int64_t *src_off,
                                   const float *src_xyzm, const int64_t *tst_off,

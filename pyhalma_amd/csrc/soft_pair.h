@@ -39,6 +39,15 @@ __device__ __forceinline__ void kahan(float& s, float& c, float v) {
     s = t;
 }
 
+// Error bounds of the softened sums, u = 2^-24 (tests FP64 points; the members as tests lack
+// the lo part's share).  A difference is off by 2u (the lo part's rounding or the first
+// subtraction's, and the second's), r^2 + eps^2 by 7u, its root by 3.5u, v_rsq_f32 by 1 ulp =
+// 2u: 5.5u for 1 / r.  S: 5.5u, at most 8 roundings of a term in its sub-tile (the product's
+// included), the Kahan sum 2u, 0.5u for the FP64 sums and the higher orders: 16u = 2^-20.
+// a: three times 5.5u, the products of the cube and the mass 3u, the difference 2u, the
+// sub-tile 8u, Kahan 2u and 0.5u: 32u = 2^-19 of the sum of |terms|; w less.  The symmetric
+// form (soft_sym.hip) has neither the lo part nor Kahan sums: 13u and 26u.
+
 // One pair term added into the plain sub-tile sums ps (planes as n_planes(MODE): the
 // potential first when present, then ax, ay, az, w).  FP64 tests (SELF false) subtract
 // their lo part after the hi part.

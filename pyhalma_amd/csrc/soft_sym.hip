@@ -26,7 +26,7 @@
 // r^2, 3 for the rule, 2 for the reciprocal root, 2 for its cube, 2 + 8 for the sums of the
 // two sides), 1 for the FP64 sums and 2.4 for the tree at T = 8 (1.6 with its first three
 // levels in FP32, i.e. 64 terms instead of 8: six haloes of 2e4-2e5 members 18.2 instead of
-// 19.0 ms a call, the spread of S 1.27 times the one-sided kernel's instead of 0.9), i.e. 13.2
+// 19.0 ms a call, the spread of S 1.36 times the one-sided kernel's instead of 0.94), i.e. 13.2
 // per ordered pair; the one-sided kernel of soft.hip takes 21.5.
 #include <math.h>
 

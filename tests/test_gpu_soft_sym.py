@@ -79,7 +79,7 @@ def test_self_sums_block_and_band_edges(gpu, sizes):
 def test_self_sums_are_as_exact_as_the_one_sided_ones(gpu, n):
     """Both forms add eight terms in FP32 before FP64 (or a Kahan pair), on either side of a
     pair: the spread of S about its FP64 value is no larger (the mean, the root's bias, is
-    common to both).  With 64 terms in FP32 on the source side it is 1.27 of it at 17000."""
+    common to both).  With 64 terms in FP32 on the source side it is 1.36 of it at 17000."""
     import torch
 
     from pyhalma_amd import engine
