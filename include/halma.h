@@ -507,7 +507,10 @@ int halma_pot_soft_batched_packed(int64_t n_halo, const int64_t *src_off,
 /* The halo potential-energy form: the tests are the sources themselves (halo h's
  * members src_xyzm rows [offsets[h], offsets[h+1]), packed as above), so pot[k], acc and
  * wsum are the sums of member k over the other members of its halo (the coordinate rule
- * drops k itself).  Outputs indexed like the rows.  This is the forward (pot) and
+ * drops k itself).  Outputs indexed like the rows.  Without wsum a halo of at most 2^21
+ * members takes each pair once, in partial sums of up to 2 kB a member: the workspace grows
+ * to 4 GiB of them and no further.  Larger haloes, and calls with wsum, are one-sided; a
+ * halo's form follows from its own size.  This is the forward (pot) and
  * backward (acc: dW/dx_k = -G m_k acc_k for W_h = -G/2 sum m_k pot_k) of the halo
  * potential energy. */
 size_t halma_soft_self_workspace_size(int64_t n_halo, const int64_t *offsets);

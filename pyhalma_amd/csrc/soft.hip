@@ -24,7 +24,7 @@
 // thread per test, or a wavefront per test for calls with few tests): a test's result
 // depends on its halo's inputs only.  Nothing of the N^2 pair terms is stored: the
 // gradient kernels recompute every term.  Sums of the members over themselves without wsum
-// take the symmetric kernel of soft_sym.hip instead.
+// take the symmetric kernel of soft_sym.hip instead, in haloes that it takes.
 #include <math.h>
 
 #include <algorithm>
@@ -452,7 +452,20 @@ int launch_mode(const SoftPlan& plan, const SoftWs& w, const float4* src4, const
     return 0;
 }
 
-// The body of every entry: sources as separate arrays (packed here into the workspace)
+// the symmetric form's arguments, as soft_run checks them
+int check_self(int64_t H, const int64_t* off, const float* rows, double eps) {
+    if (!(eps >= 0.0) || !isfinite(eps)) return set_error(HALMA_E_ARG, "eps must be >= 0");
+    int rc = check_offsets(H, off);
+    if (rc || off[H] == off[0]) return rc;
+    if (reinterpret_cast<uintptr_t>(rows) % alignof(float4) != 0)
+        return set_error(HALMA_E_ARG, "packed sources must be 16-byte aligned");
+    for (int64_t h = 0; h < H; ++h)
+        if (off[h + 1] - off[h] > INT32_MAX)
+            return set_error(HALMA_E_ARG, "halo %lld: bad offsets", (long long)h);
+    return 0;
+}
+
+// The one-sided body of every entry: sources as separate arrays (packed here into the workspace)
 // or already packed by the caller as (x, y, z, m) float4; tests FP64 points, or the
 // sources themselves (self).
 int soft_run(int64_t n_halo, const int64_t* src_off, const float* sm, const float* sx,
@@ -476,14 +489,6 @@ int soft_run(int64_t n_halo, const int64_t* src_off, const float* sm, const floa
         return set_error(HALMA_E_ARG, "packed sources must be 16-byte aligned");
     if (!pot && !acc && !wsum) return 0;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    // the members as their own tests, without wsum: each pair once (soft_sym.hip; 18.9 ms
-    // for S and a of six haloes of 2e4-2e5 members, 26.6 ms one-sided); its slots grow with
-    // the halo, so a call with a halo of more than 2^23 members stays here
-    if (self && !wsum && soft_sym_takes(n_halo, src_off))
-        return soft_sym_run(n_halo, src_off,
-                            reinterpret_cast<const float4*>(src_xyzm) + src_off[0],
-                            static_cast<float>(eps * eps), pot ? pot + src_off[0] : nullptr,
-                            acc ? acc + 3 * src_off[0] : nullptr, ws, ws_bytes, st);
     SoftPlan plan;
     rc = plan_soft(n_halo, src_off, tst_off, plan);
     if (rc) return rc;
@@ -579,7 +584,7 @@ int halma_pot_soft_batched_packed(int64_t n_halo, const int64_t* src_off,
 
 size_t halma_soft_self_workspace_size(int64_t n_halo, const int64_t* offsets) {
     const size_t one_sided = soft_ws_bytes(n_halo, offsets, offsets, false);
-    if (one_sided == 0 || !soft_sym_takes(n_halo, offsets)) return one_sided;
+    if (one_sided == 0) return 0;
     return std::max(one_sided, soft_sym_bytes(n_halo, offsets));
 }
 
@@ -588,8 +593,28 @@ int halma_pot_soft_self_batched(int64_t n_halo, const int64_t* offsets, const fl
                                 size_t ws_bytes, void* stream) {
     if (!src_xyzm && n_halo > 0 && offsets && offsets[n_halo] > offsets[0])
         return set_error(HALMA_E_ARG, "halma_pot_soft_self_batched: null sources");
-    return soft_run(n_halo, offsets, nullptr, nullptr, nullptr, nullptr, src_xyzm, offsets,
-                    nullptr, nullptr, nullptr, true, eps, pot, acc, wsum, ws, ws_bytes, stream);
+    const auto one_sided = [&](int64_t H, const int64_t* off) {
+        return soft_run(H, off, nullptr, nullptr, nullptr, nullptr, src_xyzm, off, nullptr, nullptr,
+                        nullptr, true, eps, pot, acc, wsum, ws, ws_bytes, stream);
+    };
+    if (wsum || n_halo <= 0 || !offsets || (!pot && !acc)) return one_sided(n_halo, offsets);
+    int rc = check_self(n_halo, offsets, src_xyzm, eps);
+    if (rc || offsets[n_halo] == offsets[0]) return rc;
+    const auto left_out = [&](int64_t h) { return !soft_sym_takes(offsets[h + 1] - offsets[h]); };
+    for (int64_t h = 0; h < n_halo; ++h) {
+        const size_t need = left_out(h) ? soft_ws_bytes(1, offsets + h, offsets + h, false) : 0;
+        if (ws_bytes < need)
+            return set_error(HALMA_E_WORKSPACE, "workspace %zu < required %zu", ws_bytes, need);
+    }
+    // without wsum each pair once, halo by halo where the path takes it (soft_sym.hip; 18.9 ms
+    // for S and a of six haloes of 2e4-2e5 members, 26.6 ms one-sided)
+    rc = soft_sym_run(n_halo, offsets, reinterpret_cast<const float4*>(src_xyzm) + offsets[0],
+                      static_cast<float>(eps * eps), pot ? pot + offsets[0] : nullptr,
+                      acc ? acc + 3 * offsets[0] : nullptr, ws, ws_bytes,
+                      static_cast<hipStream_t>(stream));
+    for (int64_t h = 0; !rc && h < n_halo; ++h)
+        if (left_out(h)) rc = one_sided(1, offsets + h);
+    return rc;
 }
 
 }  // extern "C"

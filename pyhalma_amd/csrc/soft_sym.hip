@@ -45,8 +45,13 @@ namespace {
 
 constexpr int kSsBand = 64;          // blocks per band
 constexpr int kSsBig = 16384;        // members from which a halo is cut into blocks of 512
-constexpr int kSsMax = 1 << 23;      // members of the largest halo this path takes
-constexpr size_t kSsSlots = size_t(4) << 30;  // slot bytes of haloes that share a launch
+// Slot bytes of the haloes that share a launch, at 32 bytes a slot (room for S and a, whatever
+// the call asks for): the workspace grows by 2 kB a member up to here and no further, and a
+// halo that would need more is left to soft.hip (a quarter of the room makes 20 haloes of 1e5
+// members 60 -> 68 ms in more launches, and one of 1e6 413 -> 516 in narrower bands).
+constexpr size_t kSsSlots = size_t(4) << 30;
+constexpr size_t kSsSlotBytes = 32;
+constexpr int64_t kSsMax = static_cast<int64_t>(kSsSlots / (kSsSlotBytes * kSsBand));
 
 // members rows[off, off + n); slot s, plane q of member i at
 // part[q * n_part + part_off + s * n + i]
@@ -274,12 +279,13 @@ int plan_ss(int64_t H, const int64_t* off, SsPlan& p) {
         SsDesc& d = p.halos[h];
         const int64_t n = off[h + 1] - off[h];
         d.off = off[h] - off[0];
-        d.n = static_cast<int32_t>(n);
+        d.n = static_cast<int32_t>(std::min<int64_t>(n, INT32_MAX));  // larger: not taken
         d.bs = n >= kSsBig ? 512 : 128;
         d.nb = static_cast<int32_t>((n + d.bs - 1) / d.bs);
         d.wb = std::max(1, std::min(d.nb, kSsBand));
         d.part_off = 0;
-        if (n > 0) order.push_back(static_cast<int32_t>(h));
+        if (n == 0 || !soft_sym_takes(n)) continue;
+        order.push_back(static_cast<int32_t>(h));
     }
     std::stable_sort(order.begin(), order.end(),
                      [&](int32_t a, int32_t b) { return p.halos[a].n > p.halos[b].n; });
@@ -293,7 +299,7 @@ int plan_ss(int64_t H, const int64_t* off, SsPlan& p) {
             SsDesc& d = p.halos[order[end]];
             const int64_t s = static_cast<int64_t>(d.wb) * d.n;
             if ((d.bs == 512) != big) break;
-            if (end > at && static_cast<size_t>(slots + s) * 32 > kSsSlots) break;
+            if (end > at && static_cast<size_t>(slots + s) * kSsSlotBytes > kSsSlots) break;
             d.part_off = slots;
             slots += s;
             ++end;
@@ -394,15 +400,11 @@ int launch_ss(const SsPlan& p, const SsWs& w, const float4* rows, float e2, doub
 
 }  // namespace
 
-bool soft_sym_takes(int64_t H, const int64_t* off) {
-    for (int64_t h = 0; h < H; ++h)
-        if (off[h + 1] - off[h] > kSsMax) return false;
-    return true;
-}
+bool soft_sym_takes(int64_t n) { return n <= kSsMax; }
 
 size_t soft_sym_bytes(int64_t H, const int64_t* off) {
     SsPlan p;
-    if (!soft_sym_takes(H, off) || plan_ss(H, off, p)) return 0;
+    if (plan_ss(H, off, p)) return 0;
     return carve_ss(nullptr, p).bytes;
 }
 
@@ -418,6 +420,7 @@ int soft_sym_run(int64_t H, const int64_t* off, const float4* rows, float e2, do
     if (!rc) rc = upload_async(w.tiles, p.tiles.data(), p.tiles.size() * sizeof(int4), st);
     if (!rc) rc = upload_async(w.segs, p.segs.data(), p.segs.size() * sizeof(int4), st);
     if (rc) return rc;
+    if (p.launches.empty()) return 0;
     if (pot && acc) return launch_ss<kModeBoth>(p, w, rows, e2, pot, acc, st);
     if (pot) return launch_ss<kModePot>(p, w, rows, e2, pot, nullptr, st);
     return launch_ss<kModeAcc>(p, w, rows, e2, nullptr, acc, st);

@@ -99,3 +99,29 @@ def test_self_sums_are_as_exact_as_the_one_sided_ones(gpu, n):
     sym, one = ((S - want) / want).std(), ((T - want) / want).std()
     print(f"symmetric {float(sym):.3e} one-sided {float(one):.3e}", flush=True)
     assert float(sym) <= 1.05 * float(one)
+
+
+@pytest.mark.parametrize("n", [1 << 21, (1 << 21) + 1])
+def test_self_sums_large_haloes_by_their_own_size(gpu, n):
+    """Above 2^21 members a halo is one-sided; a small halo of the same call keeps its bits
+    either way, and the large one is within the bound."""
+    import torch
+
+    from pyhalma_amd import engine
+
+    rng = np.random.default_rng(n)
+    rows = torch.from_numpy(np.concatenate([_halo(rng, n, True), _halo(rng, 700, True)])).cuda()
+    off = np.array([0, n, n + 700])
+    print(f"n={n}", flush=True)
+    r = engine.pot_soft_self(off, rows, EPS, pot=True, acc=True)
+    p = rows[:n].double()
+    i = torch.from_numpy(np.concatenate([np.arange(9), rng.integers(0, n, 40),
+                                         np.arange(n - 9, n)])).cuda()
+    for q in i.split(16):
+        ws, wa, mag = _fp64(p, q)
+        assert float(((r["pot"][q] - ws).abs() / ws).max()) <= 15 * U
+        assert float(((r["acc"][q] - wa).abs() / mag).max()) <= 28 * U
+    alone = engine.pot_soft_self(off[1:] - n, rows[n:], EPS, pot=True, acc=True)
+    assert torch.equal(alone["pot"], r["pot"][n:]) and torch.equal(alone["acc"], r["acc"][n:])
+    one = engine.pot_soft_self(off[:2], rows, EPS, pot=True, acc=True, wsum=True)
+    assert torch.equal(one["pot"], r["pot"][:n]) == (n > 1 << 21)
