@@ -373,9 +373,12 @@ __device__ __forceinline__ int stretch_cells(int64_t ncell) {
 // stretch.  A column of more than kSegMin cells is cut into segments of kSegCells
 // cells, and each segment takes its own lanes (a long column's cells are then linked by
 // several lanes at once instead of one long chain of finds and unions).  Up to kFewCells
-// cells, which leave most of the chip idle, every cell is a segment: FoF of a 24k Plummer
-// sphere 397 -> 339 us (its first round 113 -> 60), 98k clump stars 279 -> 255, 654k 430 -> 405,
-// 240k bridged 427 -> 405, 800k (650k cells) 670 and 667; 2.4M 1325 -> 1339.  Lane order:
+// cells, kFewCross of them with a neighbour in another stretch, which leave most of the chip
+// idle, every cell is a segment: FoF of a 24k Plummer sphere 397 -> 339 us (its first round 113 ->
+// 60), 98k clump stars 279 -> 255, 654k 430 -> 405, 240k bridged 427 -> 405, 800k (650k cells) 670
+// and 667; 2.4M 1325 -> 1339.  With more between stretches the lanes fill the chip as
+// segments of kSegCells: 200k uniform points 0.8-1.2 linking lengths apart 485 -> 427 and 434 -> 401 us
+// (100k, all of them between stretches: 360 and 323 either way).  Lane order:
 // segments grouped by the log2 of their particle count, largest first, so that the lanes
 // of a wavefront walk segments of similar length (a wavefront lasts as long as its
 // longest lane) and the longest start first.  A counting sort over kColClasses classes;
@@ -388,11 +391,17 @@ constexpr int kBigLists = 3;  // fillings of the list of large pairs: local, cro
 constexpr int kSegMin = 4;
 constexpr int kSegCells = 4;
 constexpr int64_t kFewCells = 1 << 19;
+constexpr int kFewCross = 1 << 17;
 static_assert(kSegCells < 1024 && kSegMin < 1024, "a segment's cell count has 10 bits");
 
-// cells per segment of a column of n cells, of ncell in all
-__device__ __forceinline__ int seg_step(int n, int64_t ncell) {
-    if (ncell <= kFewCells) return 1;
+// whether every cell is a segment (counts: k_col_class_count's)
+__device__ __forceinline__ bool few_cells(int64_t ncell, const int* __restrict__ counts) {
+    return ncell <= kFewCells && counts[2 * kColClasses] <= kFewCross;
+}
+
+// cells per segment of a column of n cells
+__device__ __forceinline__ int seg_step(int n, bool few) {
+    if (few) return 1;
     return n > kSegMin ? kSegCells : (n > 0 ? n : 1);
 }
 
@@ -424,9 +433,13 @@ __global__ __launch_bounds__(256) void k_col_neigh(const int64_t* __restrict__ t
                                                    const int* __restrict__ col_cell,
                                                    const uint64_t* __restrict__ col_key, int by,
                                                    ColEntry* __restrict__ cols,
-                                                   ColNeigh* __restrict__ neigh) {
+                                                   ColNeigh* __restrict__ neigh,
+                                                   int* __restrict__ n_cross) {
     const int64_t ncol = totals[0] >> 32;
+    const int64_t ncell = totals[0] & 0xffffffff;
+    const int str = stretch_cells(ncell);
     const uint64_t ymask = (uint64_t{1} << by) - 1;
+    int cross = 0;  // cells with a neighbour in another stretch
     for (int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; q < ncol;
          q += static_cast<int64_t>(gridDim.x) * blockDim.x) {
         const uint64_t key = col_key[q];
@@ -464,10 +477,15 @@ __global__ __launch_bounds__(256) void k_col_neigh(const int64_t* __restrict__ t
         nb.mask = mask;
         nb.last = col_cell[last + 1] - 1;
         neigh[q] = nb;
+        cross += max(0, min(a1, nb.last / str * str) - a0);
     }
+    if (ncell > kFewCells) return;  // not asked for
+    for (int s = kWave / 2; s >= 1; s >>= 1) cross += __shfl_xor(cross, s, kWave);
+    if (__lane_id() == 0 && cross > 0) atomicAdd(n_cross, cross);
 }
 
-// counts[0..7]: segments per class; counts[8..15]: the class cursors (zero here)
+// counts[0..7]: segments per class; counts[8..15]: the class cursors (zero here);
+// counts[16]: k_col_neigh's count of cells with a neighbour in another stretch
 __global__ __launch_bounds__(256) void k_col_class_count(const int64_t* __restrict__ totals,
                                                          const int* __restrict__ col_cell,
                                                          const ColNeigh* __restrict__ neigh,
@@ -479,11 +497,12 @@ __global__ __launch_bounds__(256) void k_col_class_count(const int64_t* __restri
     const int64_t ncol = totals[0] >> 32;
     const int64_t ncell = totals[0] & 0xffffffff;
     const int str = stretch_cells(ncell);
+    const bool few = few_cells(ncell, counts);
     const int64_t per = (ncol + gridDim.x - 1) / gridDim.x;
     const int64_t q0 = blockIdx.x * per, q1 = q0 + per < ncol ? q0 + per : ncol;
     for (int64_t q = q0 + threadIdx.x; q < q1; q += blockDim.x) {
         const int a0 = col_cell[q], a1 = col_cell[q + 1];
-        const int step = seg_step(a1 - a0, ncell);
+        const int step = seg_step(a1 - a0, few);
         const int last = neigh[q].last / str;
         for (int c = a0; c < a1; c += step)
             if (c / str != last) atomicAdd(&h[seg_class(crec, c, min(c + step, a1))], 1);
@@ -506,11 +525,12 @@ __global__ __launch_bounds__(256) void k_col_class_scatter(const int64_t* __rest
     const int64_t ncol = totals[0] >> 32;
     const int64_t ncell = totals[0] & 0xffffffff;
     const int str = stretch_cells(ncell);
+    const bool few = few_cells(ncell, counts);
     const int64_t per = (ncol + gridDim.x - 1) / gridDim.x;
     const int64_t q0 = blockIdx.x * per, q1 = q0 + per < ncol ? q0 + per : ncol;
     for (int64_t q = q0 + threadIdx.x; q < q1; q += blockDim.x) {
         const int a0 = col_cell[q], a1 = col_cell[q + 1];
-        const int step = seg_step(a1 - a0, ncell);
+        const int step = seg_step(a1 - a0, few);
         const int last = neigh[q].last / str;
         for (int c = a0; c < a1; c += step)
             if (c / str != last) atomicAdd(&h[seg_class(crec, c, min(c + step, a1))], 1);
@@ -526,7 +546,7 @@ __global__ __launch_bounds__(256) void k_col_class_scatter(const int64_t* __rest
     __syncthreads();
     for (int64_t q = q0 + threadIdx.x; q < q1; q += blockDim.x) {
         const int a0 = col_cell[q], a1 = col_cell[q + 1];
-        const int step = seg_step(a1 - a0, ncell);
+        const int step = seg_step(a1 - a0, few);
         const int last = neigh[q].last / str;
         for (int c = a0; c < a1; c += step) {
             if (c / str == last) continue;
@@ -642,10 +662,11 @@ __device__ __forceinline__ void candidate(int c, int& rc, int sc, int nc, int d,
 // merging the columns 0.5, testing 0.3) and dependent loads of roots and records; here both
 // are LDS accesses: 1.47 ms for all pairs within stretches, and 0.35 for those between
 // them, where the two rounds over all cells took 4.0 (the call 6.43 -> 4.3 ms).  512
-// threads per stretch: 256 take 1.63 ms, 1024 1.72.  Where rows are longer than a stretch (a
-// uniform box of 2M cells: 126 x 126 columns a side) most links are left to the rounds
-// between stretches: 2.2-2.4 ms a call at 0.8-1.2 linking lengths of mean spacing, against
-// 2.0-2.3 with the two rounds alone, and 1.6 against 2.8 at 0.5.
+// threads per stretch: 256 take 1.63 ms, 1024 1.72.  Where a slab of one x is longer than a
+// stretch (a uniform box) a stretch holds no neighbours in x: then its columns' own and y
+// neighbours are all it looks at, both distances at once (2M points 2.0, 1.2 and 0.8 linking
+// lengths apart: 306 -> 80, 357 -> 110 us and, in the call, 2140 -> 1850; the two rounds alone
+// took 1150, 1965 and 2300 us a call, with the stretches 1165, 1910 and 1850).
 __device__ __forceinline__ int lds_parent(int* P, int x) {
     return __hip_atomic_load(P + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
@@ -676,18 +697,23 @@ __device__ __forceinline__ void lds_join(int* P, int a, int b) {
     }
 }
 
-// Distance DIST (1 or 2) of one stretch: cells base .. base + m - 1, records R (m + 1)
-template <int DIST, typename V>
-__device__ __forceinline__ void local_links(int* P, const int2* R, int base, int m,
+// The pairs of one stretch at distance LO .. DIST: cells base .. base + m - 1, records R
+// (m + 1), the last of its columns qlast.  ROWS: a column of it may have a neighbour in row
+// x + 1 or x + 2 within it; else only its own column and those at (0, 1) and (0, 2) can.
+template <int LO, int DIST, bool ROWS, typename V>
+__device__ __forceinline__ void local_links(int* P, const int2* R, int base, int m, int qlast,
                                             const ColEntry* __restrict__ cols,
                                             const ColNeigh* __restrict__ neigh,
                                             const int* __restrict__ cell_col,
                                             const V* __restrict__ spk, double ll2,
                                             int2* __restrict__ big, int64_t big_cap,
                                             unsigned long long* __restrict__ n_big) {
-    constexpr int K = DIST == 1 ? 5 : 13;  // the own column, the four near ones, the far ones
+    // the own column, the four near ones, the far ones; without rows the own column, (0, 1)
+    // and (0, 2), the first of the far ones
+    constexpr int K = ROWS ? (DIST == 1 ? 5 : 13) : 3;
     for (int i = threadIdx.x; i < m * K; i += blockDim.x) {
-        const int c = i / K, o = i % K;
+        const int c = i / K;
+        const int o = !ROWS && i % K == 2 ? 5 : i % K;
         const int q = cell_col[base + c];
         const int2 cc = R[c];
         const int nc = R[c + 1].x - cc.x;
@@ -695,14 +721,14 @@ __device__ __forceinline__ void local_links(int* P, const int2* R, int base, int
         if (o == 0) {
             d = c + 1;
             d1 = cols[q].c0 + static_cast<int>(cols[q].word >> kKeyBits) - base;
-            lo = DIST;
+            lo = LO;
         } else {
             const int at = col_neighbour(neigh[q], q, o - 1);
-            if (at < 0) continue;
+            if (at < 0 || at > qlast) continue;
             const ColEntry e = cols[at];
             d = e.c0 - base;
             d1 = d + static_cast<int>(e.word >> kKeyBits);
-            if (DIST == 2 && o <= 4) lo = 2;
+            if (LO == 2 && o <= 4) lo = 2;
         }
         d1 = min(d1, m);
         if (o != 0) {  // first cell with z >= zc - DIST
@@ -764,9 +790,18 @@ __global__ __launch_bounds__(512) void k_fof_local(
             R[i] = crec[base + i];
         }
         __syncthreads();
-        local_links<1>(P, R, base, m, cols, neigh, cell_col, spk, ll2, big, big_cap, n_big);
-        __syncthreads();
-        local_links<2>(P, R, base, m, cols, neigh, cell_col, spk, ll2, big, big_cap, n_big);
+        // the first row x + 1 record of the stretch's first column bounds those of the others
+        const int qlast = cell_col[base + m - 1];
+        if (neigh[cell_col[base]].row1 <= qlast) {
+            local_links<1, 1, true>(P, R, base, m, qlast, cols, neigh, cell_col, spk, ll2, big,
+                                    big_cap, n_big);
+            __syncthreads();
+            local_links<2, 2, true>(P, R, base, m, qlast, cols, neigh, cell_col, spk, ll2, big,
+                                    big_cap, n_big);
+        } else {
+            local_links<1, 2, false>(P, R, base, m, qlast, cols, neigh, cell_col, spk, ll2, big,
+                                     big_cap, n_big);
+        }
         __syncthreads();
         for (int i = threadIdx.x; i < m; i += blockDim.x) {
             int x = i;
@@ -929,11 +964,14 @@ __global__ void k_roots(const int64_t* __restrict__ totals, int* __restrict__ pa
 
 // Also folds every cell's minimum particle index into its component's minimum.  Up to
 // kRootGroups sets of lanes of a wavefront that share a root (consecutive cells mostly have
-// few) are merged into one check and one atomic each; the others act alone.  A component's
-// minimum only falls, so a value that is not below what is read of it needs no atomic,
-// however old the read.  Bound by the atomics on the few large components' words: 6.5M cells
-// of 4000 bridged pairs 183 us with one set and every atomic, 101 us this way.
+// few), of kRootMerge lanes or more, are merged into one check and one atomic each; the
+// others act alone.  A component's minimum only falls, so a value that is not below what is
+// read of it needs no atomic, however old the read.  Bound by the atomics on the few large
+// components' words: 6.5M cells of 4000 bridged pairs 183 us with one set and every atomic,
+// 101 us this way; 2M points two linking lengths apart, mostly alone, 37 us with a tree for
+// every set, 24 us with the small ones left out.
 constexpr int kRootGroups = 4;
+constexpr int kRootMerge = 4;
 
 __device__ __forceinline__ void root_min(int* parent, int* comp_min, int r, int v, int* err) {
     if (coherent_read(parent + r) != r) atomicOr(err, 4);
@@ -955,16 +993,21 @@ __global__ __launch_bounds__(256) void k_check_roots(const int64_t* __restrict__
         const bool valid = c < n_cells;  // lane 0 always is
         const int r = valid ? root[c] : -1;
         const int m = valid ? cell_min[c] : INT32_MAX;
-        unsigned long long left = __ballot(valid);
+        unsigned long long left = __ballot(valid), alone = 0;
         for (int k = 0; k < kRootGroups && left != 0; ++k) {
             const int first = __ffsll(left) - 1;
             const int g = __shfl(r, first, kWave);
+            const unsigned long long same = __ballot(r == g);
+            left &= ~same;
+            if (__popcll(same) < kRootMerge) {  // too few for the tree
+                alone |= same;
+                continue;
+            }
             int v = r == g ? m : INT32_MAX;
             for (int s = 32; s >= 1; s >>= 1) v = min(v, __shfl_xor(v, s, kWave));
             if (lane == first) root_min(parent, comp_min, g, v, err);
-            left &= ~__ballot(r == g);
         }
-        if ((left >> lane) & 1) root_min(parent, comp_min, r, m, err);
+        if (((left | alone) >> lane) & 1) root_min(parent, comp_min, r, m, err);
     }
 }
 
@@ -1044,7 +1087,7 @@ FofWs carve_fof(void* base, int64_t n, size_t elt) {
     w.col_cell = c.take<int>(nn + 1);
     w.col_key = c.take<uint64_t>(nn);
     w.lanes = c.take<ColRec>(nn + nn / kSegCells + 1);  // segments <= columns + cells / 4
-    w.class_counts = c.take<int>(2 * kColClasses);
+    w.class_counts = c.take<int>(2 * kColClasses + 1);
     w.parent = c.take<int>(nn);
     w.root = c.take<int>(nn);
     w.comp_min = c.take<int>(nn);
@@ -1141,10 +1184,11 @@ int fof_run(const T* x, const T* y, const T* z, int64_t n, double ll, int* label
     HALMA_LAUNCH_CHECK();
     k_clear_words<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(w.n_big), 2 * kBigLists);
     HALMA_LAUNCH_CHECK();
-    k_clear_words<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(w.class_counts), 2 * kColClasses);
+    k_clear_words<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(w.class_counts),
+                                     2 * kColClasses + 1);
     HALMA_LAUNCH_CHECK();
     k_col_neigh<<<grid_cells, 256, 0, st>>>(w.totals, w.col_cell, w.col_key, g.by, w.cols,
-                                            w.neigh);
+                                            w.neigh, w.class_counts + 2 * kColClasses);
     HALMA_LAUNCH_CHECK();
     k_col_class_count<<<kClassBlocks, 256, 0, st>>>(w.totals, w.col_cell, w.neigh, w.crec,
                                                      w.class_counts);

@@ -42,3 +42,19 @@ def test_fof_uniform_boxes(gpu, n, mean):
     # ll = 1, mean spacing `mean`: 0.86 percolates
     rng = np.random.default_rng(n)
     _check(rng.uniform(0, mean * n ** (1 / 3), (n, 3)).astype(np.float32), 1.0)
+
+
+@pytest.mark.parametrize("side", [8, 15, 16, 17, 23])
+@pytest.mark.parametrize("spacing", [0.6, 0.99, 1.02])
+def test_fof_slabs_about_a_stretch(gpu, side, spacing):
+    """Slabs of one x of side^2 cells, shorter and longer than a stretch (256 cells), so that
+    some stretches hold neighbours in x and others only own columns and neighbours in y; full
+    slabs beside sparse and empty ones."""
+    rng = np.random.default_rng(side)
+    g = np.stack(np.meshgrid(*[np.arange(side)] * 2, indexing="ij"), -1).reshape(-1, 2)
+    parts = []
+    for k in range(40):
+        yz = g if k % 7 < 4 else g[rng.permutation(len(g))[: (0, 9, len(g) // 2)[k % 3]]]
+        parts.append(np.concatenate([np.full((len(yz), 1), k), yz], 1))
+    x = np.concatenate(parts) * spacing
+    _check(x[rng.permutation(len(x))], 1.0)
