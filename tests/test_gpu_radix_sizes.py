@@ -1,6 +1,7 @@
 """Group lists from labels through the radix sort at the edges of its tiles: sizes around
 1024, 4096 and 2^20 keys (where the tile size changes), labels few and many, sorted and
-shuffled: members ascending within a group, groups by smallest member."""
+shuffled: members ascending within a group, groups by smallest member; a
+sort of fewer keys than its workspace was sized for."""
 import numpy as np
 import pytest
 
@@ -30,16 +31,18 @@ def test_groups_of_sorted_labels(gpu, n, groups):
     assert np.array_equal(r.offsets_host, np.concatenate([[0], np.cumsum(cnt)]))
 
 
-def test_sort_workspace_holds_every_smaller_sort():
-    # on the host: the tables of a sort of up to n pairs fit the workspace of n pairs
-    def need(n, small=1024, large=4096):
-        nb = -(-n // (large if n >= 1 << 20 else small))
-        return 2 * 256 * 4 * nb + 8 * n
+def test_sort_of_fewer_keys_than_its_workspace(gpu):
+    """A sphere query's workspace holds the sort of all its points in large tiles; one sphere
+    with 2^20 - 1 of them sorts its hits in small tiles, whose tables are four times longer."""
+    from pyhalma_amd import engine
 
-    def given(n):
-        nb = max(-(-n // (4096 if n >= 1 << 20 else 1024)), -(-min(n, (1 << 20) - 1) // 1024))
-        return 2 * 256 * 4 * nb + 8 * n
-
-    for n in (1 << 20, (1 << 20) + 1, 1200000, 5000000):
-        for m in (n, (1 << 20) - 1, 1 << 20, 1000):
-            assert need(m) <= given(n)
+    n, hits = (1 << 20) + 5000, (1 << 20) - 1
+    rng = np.random.default_rng(1)
+    x = rng.uniform(-0.5, 0.5, (n, 3))
+    inside = np.zeros(n, bool)
+    inside[rng.permutation(n)[:hits]] = True
+    x[~inside] += 5.0
+    print(f"points={n} hits={hits}", flush=True)
+    off, idx, _ = engine.ball_query(*x.T, [[0.0, 0.0, 0.0]], [1.0])
+    assert list(off) == [0, hits]
+    assert np.array_equal(idx.cpu().numpy(), np.nonzero(inside)[0])

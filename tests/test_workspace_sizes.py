@@ -28,3 +28,21 @@ def test_soft_self_workspace_is_bounded():
                   [1 << 21, 1 << 23, 1 << 21, 100], [200000] * 20):
         H, off, _keep = _off(*sizes)
         assert 0 < size(H, off) <= (4 << 30) + 200 * sum(sizes), sizes
+
+
+def test_sort_workspaces_never_shrink():
+    """Callers size for their largest input and sort fewer: the tables of the small tiles just
+    under 2^20 keys are longer than those of the large tiles from there on."""
+    from pyhalma_amd import _lib
+
+    L = _lib.load()
+    sizes = [1, 1000, 1 << 19, (1 << 20) - 1, 1 << 20, (1 << 20) + 1, 1200000, 1 << 21, 5000000]
+    for query in (lambda n: L.halma_fof_workspace_size(n, 0),
+                  lambda n: L.halma_clean_workspace_size(n),
+                  lambda n: L.halma_ball_query_workspace_size(1000, 1, n)):
+        got = [query(n) for n in sizes]
+        assert got[0] > 0 and got == sorted(got)
+    # the tables of the small tiles (1024 keys, 256 counts and offsets a tile) within a size
+    # that is otherwise proportional
+    per = lambda n: L.halma_ball_query_workspace_size(1000, 1, n) / n  # noqa: E731
+    assert per(1 << 20) >= 0.999 * per((1 << 20) - 1)
