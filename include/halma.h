@@ -384,14 +384,17 @@ int halma_progenitors(int64_t n_new, int64_t n_new_members, const int64_t *new_o
  * [10] pairs of the symmetric kernel's passes (part of [7]; it evaluates each unordered
  * pair once for two of them), [11] chunked-kernel launches, [12] members of [1] re-summed
  * because their S had an error bound above 1e-6 of S (a kept member whose incremental
- * updates took its rigorous bound past 1e-6 gets a fresh FP64 sum, so every S the call
- * keeps is within 1e-6 of the FP64 direct sum).  Full passes (first pass, or
- * more than a quarter of the live set removed) go to the symmetric kernel for haloes of
- * at most HALMA_TUNE_SYM_MAX members, to the chunked kernel otherwise; incremental passes
- * go to the chunked kernel; small haloes take the passes after that in a workgroup each,
- * several per queued pass.  Passes are queued one ahead of the host: the counters of
- * pass p are read back (pinned buffer, event) while pass p + 1 is already queued, so
- * the call ends with one extra pass that finds no active halo.  flags:
+ * updates took its rigorous bound past 1e-6 gets a fresh sum of FP32 terms, so every S the
+ * call keeps is within 1e-6 of the FP64 direct sum).  Full passes (first pass, more than
+ * half as many members removed as kept by the last one, or too many stale S) go to the
+ * symmetric kernel for haloes of at most HALMA_TUNE_SYM_MAX members, to the chunked kernel
+ * otherwise; incremental passes go to the chunked kernel; while every active halo has at
+ * most 4096 live members they take the passes after that in a workgroup each, several per
+ * queued pass.  bound and iters do not depend on the other haloes of the call; S (within its
+ * bound) and the last bit of v_cm can, through the chunks of a launch and through who takes
+ * a pass.  Passes are queued one ahead of the host: the counters of pass p are read back
+ * (pinned buffer, event) while pass p + 1 is already queued, so the call ends with one extra
+ * pass that finds no active halo.  flags:
  * HALMA_UNBIND_GRAPHS captures each part of a pass (prepare, symmetric kernel, chunked
  * kernel, decisions) into a hipGraph replayed every pass; by default the parts are plain
  * launches (a few passes do not repay the capture).

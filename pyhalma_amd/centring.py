@@ -19,10 +19,10 @@ of every member against its halo (tests = the members' own FP32 positions, so th
 drops each self pair), the backward pass its hand-written acceleration kernel over the
 same pairs, recomputed.  ``refine_centres`` moves a seed centre per halo downhill on
 the potential Phi(c) = -G S(c): every step is the gradient of S at the current centres
-scaled per halo by 1 / w(c), w = sum_j m_j (r^2+eps^2)^(-3/2), which makes the step the fixed-point update c <- sum_j m_j w_j x_j / sum_j m_j w_j and
-never increases Phi (the kernel (r^2 + eps^2)^(-1/2) is convex and decreasing in r^2).
-The reference's discrete counterpart is the most-bound particle of
-halo_gas.py:498-634.
+scaled per halo by 1 / w(c), w = sum_j m_j (r^2+eps^2)^(-3/2), which makes the step the
+fixed-point update c <- sum_j m_j w_j x_j / sum_j m_j w_j and never increases Phi (the
+kernel (r^2 + eps^2)^(-1/2) is convex and decreasing in r^2).  The reference's discrete
+counterpart is the most-bound particle of halo_gas.py:498-634.
 """
 import numpy as np
 import torch
@@ -41,7 +41,8 @@ _src_cache = {}
 
 def _src_cols(src_pos):
     """FP32 columns of the source positions, kept for the next call on the same unchanged
-    tensor (the centring iterations pass one source array to every forward and backward).
+    tensor (an iteration over soft_potential passes one source array to every forward and
+    backward).
     The key holds the storage address, shape, strides, dtype and the version counter
     (bumped by every in-place change); the entry holds the tensor itself, so its storage
     cannot be freed and reused under the same address while it is cached."""
@@ -87,7 +88,7 @@ class SoftPotential(torch.autograd.Function):
     @staticmethod
     def forward(ctx, tests, src_pos, src_m, src_off, tst_off, eps, aux=None):
         tx, ty, tz = _cols(tests.detach().double())
-        # with aux (the centring, which always takes the test gradient next) the gradient
+        # with aux (an iteration on the tests, which takes their gradient next) the gradient
         # and w come from the same launch as S: one pass over the sources per step
         fused = aux is not None and ctx.needs_input_grad[0]
         r = engine.pot_soft_batched(src_off, None, None, None, None, tst_off, tx, ty, tz,

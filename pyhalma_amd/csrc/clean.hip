@@ -71,8 +71,9 @@ __device__ __forceinline__ double node(const GridArgs& g, int h, int64_t k) {
 
 // first k minimising |node(k) - xh| (np.argmin: the first of equal distances).  Of nodes
 // start + k d (k >= 2) a value further than `tie` steps from the middle of two is nearest to
-// the one on its side whatever the rounding; the others compare.  The estimate's window is refined by descending the distances, which are unimodal in k
-// (the nodes increase); a non-finite xh has every distance non-finite: node 0.
+// the one on its side whatever the rounding; the others compare.  The estimate's window is
+// refined by descending the distances, which are unimodal in k (the nodes increase); a
+// non-finite xh has every distance non-finite: node 0.
 __device__ int nearest(const GridArgs& g, int h, double xh, double inv, double tie) {
     const int64_t n = g.n[h];
     if (!isfinite(xh)) return 0;

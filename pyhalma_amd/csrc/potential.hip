@@ -8,9 +8,10 @@
 // is pure VALU: 3 sub, mul + 2 fma, v_rsq_f32, the skip test (inv_r_group), fma.  SUB terms
 // are summed plainly in FP32, the sub-tiles in FP64 (two instructions, where a Kahan pair
 // takes four); partials of split source ranges, stored as (hi, lo) floats, are merged in
-// FP64 in chunk order (deterministic).  Bound by the issue of the vector ALUs: 11 slots per
-// pair at SUB = 4 (13 with Kahan sums and the rule pair by pair).  24 gas
-// haloes against their dark matter and stars (2.4e10 pairs): 12.6 -> 11.3 ms.
+// FP64 in chunk order (deterministic).  Bound by the issue of the vector ALUs: 10.25
+// instructions per pair at SUB = 4 (12.25 with Kahan sums and the rule pair by pair).  24 gas
+// haloes against their dark matter and stars (4.5e10 pairs): 12.6 -> 11.3 ms, 9.9 issue slots
+// of a SIMD a pair.
 #include <algorithm>
 #include <mutex>
 #include <numeric>
