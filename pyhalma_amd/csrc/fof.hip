@@ -373,12 +373,12 @@ __device__ __forceinline__ int stretch_cells(int64_t ncell) {
 // stretch.  A column of more than kSegMin cells is cut into segments of kSegCells
 // cells, and each segment takes its own lanes (a long column's cells are then linked by
 // several lanes at once instead of one long chain of finds and unions).  Up to kFewCells
-// cells, kFewCross of them with a neighbour in another stretch, which leave most of the chip
-// idle, every cell is a segment: FoF of a 24k Plummer sphere 397 -> 339 us (its first round 113 ->
-// 60), 98k clump stars 279 -> 255, 654k 430 -> 405, 240k bridged 427 -> 405, 800k (650k cells) 670
-// and 667; 2.4M 1325 -> 1339.  With more between stretches the lanes fill the chip as
-// segments of kSegCells: 200k uniform points 0.8-1.2 linking lengths apart 485 -> 427 and 434 -> 401 us
-// (100k, all of them between stretches: 360 and 323 either way).  Lane order:
+// cells, which leave most of the chip idle, every cell is a segment: FoF of a 24k Plummer
+// sphere 397 -> 339 us (its first round 113 -> 60), 98k clump stars 279 -> 255, 654k 430 -> 405, 240k
+// bridged 427 -> 405, 800k (650k cells) 670 and 667; 2.4M 1325 -> 1339.  Not so where that makes
+// more than kFewMore segments more, which fill the chip: 200k uniform points (columns of 5-25
+// cells, 1.2e5 more) 0.8 and 1.2 linking lengths apart take 480 and 433 us that way, 428 and 395 in
+// segments of kSegCells, 100k (7e4 more) 360 and 322 against 368 and 335.  Lane order:
 // segments grouped by the log2 of their particle count, largest first, so that the lanes
 // of a wavefront walk segments of similar length (a wavefront lasts as long as its
 // longest lane) and the longest start first.  A counting sort over kColClasses classes;
@@ -391,12 +391,16 @@ constexpr int kBigLists = 3;  // fillings of the list of large pairs: local, cro
 constexpr int kSegMin = 4;
 constexpr int kSegCells = 4;
 constexpr int64_t kFewCells = 1 << 19;
-constexpr int kFewCross = 1 << 17;
+constexpr int kFewMore = 3 << 15;
 static_assert(kSegCells < 1024 && kSegMin < 1024, "a segment's cell count has 10 bits");
 
-// whether every cell is a segment (counts: k_col_class_count's)
+// The segments per class as k_col_class_count has counted them: counts[0 .. 7] with every cell
+// a segment (up to kFewCells cells), counts[8 .. 15] in segments of kSegCells.
 __device__ __forceinline__ bool few_cells(int64_t ncell, const int* __restrict__ counts) {
-    return ncell <= kFewCells && counts[2 * kColClasses] <= kFewCross;
+    int more = 0;
+#pragma unroll
+    for (int k = 0; k < kColClasses; ++k) more += counts[k] - counts[kColClasses + k];
+    return ncell <= kFewCells && more <= kFewMore;
 }
 
 // cells per segment of a column of n cells
@@ -433,13 +437,9 @@ __global__ __launch_bounds__(256) void k_col_neigh(const int64_t* __restrict__ t
                                                    const int* __restrict__ col_cell,
                                                    const uint64_t* __restrict__ col_key, int by,
                                                    ColEntry* __restrict__ cols,
-                                                   ColNeigh* __restrict__ neigh,
-                                                   int* __restrict__ n_cross) {
+                                                   ColNeigh* __restrict__ neigh) {
     const int64_t ncol = totals[0] >> 32;
-    const int64_t ncell = totals[0] & 0xffffffff;
-    const int str = stretch_cells(ncell);
     const uint64_t ymask = (uint64_t{1} << by) - 1;
-    int cross = 0;  // cells with a neighbour in another stretch
     for (int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; q < ncol;
          q += static_cast<int64_t>(gridDim.x) * blockDim.x) {
         const uint64_t key = col_key[q];
@@ -477,38 +477,35 @@ __global__ __launch_bounds__(256) void k_col_neigh(const int64_t* __restrict__ t
         nb.mask = mask;
         nb.last = col_cell[last + 1] - 1;
         neigh[q] = nb;
-        cross += max(0, min(a1, nb.last / str * str) - a0);
     }
-    if (ncell > kFewCells) return;  // not asked for
-    for (int s = kWave / 2; s >= 1; s >>= 1) cross += __shfl_xor(cross, s, kWave);
-    if (__lane_id() == 0 && cross > 0) atomicAdd(n_cross, cross);
 }
 
-// counts[0..7]: segments per class; counts[8..15]: the class cursors (zero here);
-// counts[16]: k_col_neigh's count of cells with a neighbour in another stretch
+// counts: as few_cells has it, zero before; counts[16 .. 23] are the class cursors
 __global__ __launch_bounds__(256) void k_col_class_count(const int64_t* __restrict__ totals,
                                                          const int* __restrict__ col_cell,
                                                          const ColNeigh* __restrict__ neigh,
                                                          const int2* __restrict__ crec,
                                                          int* __restrict__ counts) {
-    __shared__ int h[kColClasses];
-    if (threadIdx.x < kColClasses) h[threadIdx.x] = 0;
+    __shared__ int h[2 * kColClasses];
+    if (threadIdx.x < 2 * kColClasses) h[threadIdx.x] = 0;
     __syncthreads();
     const int64_t ncol = totals[0] >> 32;
     const int64_t ncell = totals[0] & 0xffffffff;
     const int str = stretch_cells(ncell);
-    const bool few = few_cells(ncell, counts);
     const int64_t per = (ncol + gridDim.x - 1) / gridDim.x;
     const int64_t q0 = blockIdx.x * per, q1 = q0 + per < ncol ? q0 + per : ncol;
     for (int64_t q = q0 + threadIdx.x; q < q1; q += blockDim.x) {
         const int a0 = col_cell[q], a1 = col_cell[q + 1];
-        const int step = seg_step(a1 - a0, few);
         const int last = neigh[q].last / str;
+        const int step = seg_step(a1 - a0, false);
         for (int c = a0; c < a1; c += step)
-            if (c / str != last) atomicAdd(&h[seg_class(crec, c, min(c + step, a1))], 1);
+            if (c / str != last) atomicAdd(&h[kColClasses + seg_class(crec, c, min(c + step, a1))], 1);
+        if (ncell > kFewCells) continue;
+        for (int c = a0; c < a1 && c / str != last; ++c) atomicAdd(&h[seg_class(crec, c, c + 1)], 1);
     }
     __syncthreads();
-    if (threadIdx.x < kColClasses && h[threadIdx.x] > 0) atomicAdd(counts + threadIdx.x, h[threadIdx.x]);
+    if (threadIdx.x < 2 * kColClasses && h[threadIdx.x] > 0)
+        atomicAdd(counts + threadIdx.x, h[threadIdx.x]);
 }
 
 __global__ __launch_bounds__(256) void k_col_class_scatter(const int64_t* __restrict__ totals,
@@ -538,9 +535,10 @@ __global__ __launch_bounds__(256) void k_col_class_scatter(const int64_t* __rest
     __syncthreads();
     if (threadIdx.x < kColClasses) {
         int before = 0;  // segments of the higher classes: the longest come first
-        for (int k = threadIdx.x + 1; k < kColClasses; ++k) before += counts[k];
+        for (int k = threadIdx.x + 1; k < kColClasses; ++k)
+            before += counts[(few ? 0 : kColClasses) + k];
         base[threadIdx.x] =
-            h[threadIdx.x] > 0 ? before + atomicAdd(counts + kColClasses + threadIdx.x, h[threadIdx.x]) : 0;
+            h[threadIdx.x] > 0 ? before + atomicAdd(counts + 2 * kColClasses + threadIdx.x, h[threadIdx.x]) : 0;
         h[threadIdx.x] = 0;
     }
     __syncthreads();
@@ -826,11 +824,12 @@ __global__ __launch_bounds__(256) void k_fof_cross(
     double ll2, int* __restrict__ parent, int2* __restrict__ big, int64_t big_cap,
     unsigned long long* __restrict__ n_big, const int* __restrict__ seg_counts) {
     constexpr int K = DIST == 1 ? 5 : 13;  // own column + neighbour columns
+    const int str = stretch_cells(totals[0] & 0xffffffff);
+    const int form = few_cells(totals[0] & 0xffffffff, seg_counts) ? 0 : kColClasses;
     int64_t nseg = 0;
 #pragma unroll
-    for (int k = 0; k < kColClasses; ++k) nseg += seg_counts[k];
+    for (int k = 0; k < kColClasses; ++k) nseg += seg_counts[form + k];
     const int64_t total = nseg * K;
-    const int str = stretch_cells(totals[0] & 0xffffffff);
     for (int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
          idx < total; idx += static_cast<int64_t>(gridDim.x) * blockDim.x) {
         const ColRec col = lanes[idx / K];
@@ -1087,7 +1086,7 @@ FofWs carve_fof(void* base, int64_t n, size_t elt) {
     w.col_cell = c.take<int>(nn + 1);
     w.col_key = c.take<uint64_t>(nn);
     w.lanes = c.take<ColRec>(nn + nn / kSegCells + 1);  // segments <= columns + cells / 4
-    w.class_counts = c.take<int>(2 * kColClasses + 1);
+    w.class_counts = c.take<int>(3 * kColClasses);
     w.parent = c.take<int>(nn);
     w.root = c.take<int>(nn);
     w.comp_min = c.take<int>(nn);
@@ -1184,11 +1183,10 @@ int fof_run(const T* x, const T* y, const T* z, int64_t n, double ll, int* label
     HALMA_LAUNCH_CHECK();
     k_clear_words<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(w.n_big), 2 * kBigLists);
     HALMA_LAUNCH_CHECK();
-    k_clear_words<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(w.class_counts),
-                                     2 * kColClasses + 1);
+    k_clear_words<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(w.class_counts), 3 * kColClasses);
     HALMA_LAUNCH_CHECK();
     k_col_neigh<<<grid_cells, 256, 0, st>>>(w.totals, w.col_cell, w.col_key, g.by, w.cols,
-                                            w.neigh, w.class_counts + 2 * kColClasses);
+                                            w.neigh);
     HALMA_LAUNCH_CHECK();
     k_col_class_count<<<kClassBlocks, 256, 0, st>>>(w.totals, w.col_cell, w.neigh, w.crec,
                                                      w.class_counts);
