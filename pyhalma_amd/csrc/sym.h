@@ -59,6 +59,10 @@ struct SymPlan {
 int plan_sym(int64_t H, const int64_t* off, SymPlan& plan, bool with_items,
              int max_members = 0, int band = 0);
 
+// Workgroups of 256 threads for each of n merge segments {halo, first member, members, ...}: no
+// more than the largest needs, twice the mean at least, enough of them all for every CU.
+unsigned merge_width(const int4* segs, int64_t n);
+
 // Writes the items of plan.tiles (n_tiles, on the device) into items.
 int expand_sym_items(const int4* d_tiles, int64_t n_tiles, const SymDesc* d_halos, int4* items,
                      hipStream_t st);

@@ -269,8 +269,10 @@ __global__ __launch_bounds__(1024) void k_pot_sym_fine(const float4* __restrict_
 // before the first launch): segment s = {halo, first member, count, role << 24 | local
 // slots}; the member adds its local slots 0 .. nloc - 1 in order, then, on a diagonal
 // tile, the diagonal slot.  With one band a member's slots 0..nb are added in order.  Bound
-// by reading the slots: 128 workgroups to a segment, since a launch of few large haloes has
-// few segments (24 gas haloes of 1e3-2e5 cells: 62 -> 22.6 us a launch against 32).
+// by reading the slots: up to 128 workgroups to a segment (merge_width), since a launch of few
+// large haloes has few segments (24 gas haloes of 1e3-2e5 cells: 62 -> 22.6 us a launch against 32
+// for every segment); as many for each of 20000 haloes of 100 members, nearly all without a
+// member, took 555 us, 32 took 330, the one that they need 20.
 __global__ __launch_bounds__(256) void k_sym_merge_tile(const SymDesc* __restrict__ halos,
                                                         const int4* __restrict__ segs, int nseg,
                                                         const int64_t* __restrict__ member_base,
@@ -447,6 +449,18 @@ int plan_sym(int64_t H, const int64_t* off, SymPlan& plan, bool with_items, int 
     return 0;
 }
 
+unsigned merge_width(const int4* segs, int64_t n) {
+    int64_t most = 1, blocks = 0;
+    for (int64_t s = 0; s < n; ++s) {
+        const int64_t b = (segs[s].z + 255) / 256;
+        most = std::max(most, b);
+        blocks += b;
+    }
+    if (n <= 0) return 1;
+    const int64_t want = std::max((2 * blocks + n - 1) / n, (8192 + n - 1) / n);
+    return static_cast<unsigned>(std::min<int64_t>({want, most, 128}));
+}
+
 int expand_sym_items(const int4* d_tiles, int64_t n_tiles, const SymDesc* d_halos, int4* items,
                      hipStream_t st) {
     if (n_tiles <= 0) return 0;
@@ -561,7 +575,8 @@ int halma_pot_sum_self_batched(int64_t n_halo, const int64_t* offsets, const flo
             HALMA_LAUNCH_CHECK();
         }
         if (ns > 0) {
-            const dim3 mg(128, static_cast<unsigned>(std::min<int64_t>(ns, 4096)));
+            const dim3 mg(merge_width(plan.segs.data() + s0, ns),
+                          static_cast<unsigned>(std::min<int64_t>(ns, 65535)));
             k_sym_merge_tile<<<mg, 256, 0, st>>>(w.halos, w.segs + s0, static_cast<int>(ns),
                                                  w.base, w.part, o);
             HALMA_LAUNCH_CHECK();

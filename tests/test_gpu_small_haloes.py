@@ -1,0 +1,47 @@
+"""Many small haloes beside a few large ones in one call: the launches are shaped by all of them
+together, each halo's sums by itself alone."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _catalogue(sizes, seed):
+    rng = np.random.default_rng(seed)
+    h = np.repeat(np.arange(len(sizes)), sizes)
+    x = rng.uniform(-20, 20, (len(sizes), 3))[h] + 0.004 * rng.normal(size=(len(h), 3))
+    m = np.exp(rng.uniform(np.log(1e4), np.log(1e6), len(h)))
+    return x.astype(np.float32), m.astype(np.float32), np.concatenate([[0], np.cumsum(sizes)])
+
+
+SIZES = [[20] * 5000, [1, 0, 3, 257, 256, 255] * 700, [40] * 4200 + [9000, 1300],
+         [30000] + [0, 7] * 2000]
+
+
+@pytest.mark.parametrize("sizes", SIZES, ids=["equal", "edges", "last_large", "first_large"])
+def test_self_sums_of_many_small_haloes(gpu, sizes):
+    import torch
+
+    from pyhalma_amd import engine
+
+    x, m, off = _catalogue(np.array(sizes), len(sizes))
+    print(f"haloes={len(sizes)} members={len(m)}", flush=True)
+    S = engine.pot_sum_self(off, m, *x.T)
+    bound = engine.pot_sym_error_bound()
+    rng = np.random.default_rng(1)
+    for h in np.unique(np.concatenate([rng.integers(0, len(sizes), 40), np.argsort(sizes)[-3:],
+                                       [0, len(sizes) - 1]])):
+        a, b = off[h], off[h + 1]
+        if b == a:
+            continue
+        q = torch.from_numpy(x[a:b]).cuda().double()
+        want = torch.zeros(b - a, dtype=torch.float64, device=q.device)
+        mm = torch.from_numpy(m[a:b]).cuda().double()
+        for i in range(0, b - a, 1000):
+            d = q[i:i + 1000, None] - q[None]
+            w = d.pow(2).sum(2).rsqrt()
+            w[(d == 0).any(2)] = 0.0
+            want[i:i + 1000] = (w * mm).sum(1)
+        assert bool(((S[a:b] - want).abs() <= bound * want).all()), h
+        alone = engine.pot_sum_self(np.array([0, b - a]), m[a:b], *x[a:b].T)
+        assert torch.equal(alone, S[a:b]), h
