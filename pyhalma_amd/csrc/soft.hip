@@ -322,10 +322,13 @@ __global__ void k_soft_pack(const float* __restrict__ m, const float* __restrict
 struct SoftPlan {
     std::vector<SoftDesc> halos;
     std::vector<int4> tile_items, few_items;  // largest items first
+    int64_t n_tile = 0, n_few = 0;            // their counts
     int64_t n_src = 0, n_tst = 0, n_part = 0;
 };
 
-int plan_soft(int64_t H, const int64_t* src_off, const int64_t* tst_off, SoftPlan& plan) {
+// with_items false: the counts alone (a workspace query)
+int plan_soft(int64_t H, const int64_t* src_off, const int64_t* tst_off, SoftPlan& plan,
+              bool with_items = true) {
     plan = SoftPlan();
     plan.halos.resize(H);
     int64_t part = 0;
@@ -355,7 +358,17 @@ int plan_soft(int64_t H, const int64_t* src_off, const int64_t* tst_off, SoftPla
         const int64_t nch = ns > 0 ? (ns + d.chunk - 1) / d.chunk : 0;
         d.part_off = part;
         part += nch * nt;
+        if (d.few)
+            plan.n_few += nch * nt;
+        else
+            plan.n_tile += nch * ((nt + kWave - 1) / kWave);
     }
+    plan.n_src = src_off[H] - src_off[0];
+    plan.n_tst = tst_off[H] - tst_off[0];
+    plan.n_part = part;
+    if (plan.n_tile > INT32_MAX || plan.n_few > INT32_MAX)
+        return set_error(HALMA_E_LIMIT, "too many work items");
+    if (!with_items) return 0;
     // items, haloes by descending chunk (the cost of one item), ties by index
     std::vector<int32_t> order(H);
     for (int64_t h = 0; h < H; ++h) order[h] = static_cast<int32_t>(h);
@@ -377,12 +390,6 @@ int plan_soft(int64_t H, const int64_t* src_off, const int64_t* tst_off, SoftPla
                 for (int ti = 0; ti < tiles; ++ti) plan.tile_items.push_back(make_int4(h, ti, c, 0));
         }
     }
-    if (plan.tile_items.size() > static_cast<size_t>(INT32_MAX) ||
-        plan.few_items.size() > static_cast<size_t>(INT32_MAX))
-        return set_error(HALMA_E_LIMIT, "too many work items");
-    plan.n_src = src_off[H] - src_off[0];
-    plan.n_tst = tst_off[H] - tst_off[0];
-    plan.n_part = part;
     return 0;
 }
 
@@ -402,8 +409,8 @@ SoftWs carve_soft(void* base, const SoftPlan& p, bool pack) {
     SoftWs w;
     w.src4 = c.take<float4>(pack ? std::max<int64_t>(p.n_src, 1) : 1);
     w.halos = c.take<SoftDesc>(std::max<size_t>(p.halos.size(), 1));
-    w.tile_items = c.take<int4>(std::max<size_t>(p.tile_items.size(), 1));
-    w.few_items = c.take<int4>(std::max<size_t>(p.few_items.size(), 1));
+    w.tile_items = c.take<int4>(std::max<int64_t>(p.n_tile, 1));
+    w.few_items = c.take<int4>(std::max<int64_t>(p.n_few, 1));
     w.part = c.take<char>(8 * static_cast<size_t>(n_planes(kModeBoth)) *
                           static_cast<size_t>(std::max<int64_t>(p.n_part, 1)));
     w.tst_halo = c.take<int>(std::max<int64_t>(p.n_tst, 1));
@@ -545,7 +552,7 @@ size_t soft_ws_bytes(int64_t n_halo, const int64_t* src_off, const int64_t* tst_
     if (n_halo < 0 || !src_off || !tst_off) return 0;
     if (check_offsets(n_halo, src_off) || check_offsets(n_halo, tst_off)) return 0;
     SoftPlan plan;
-    if (plan_soft(n_halo, src_off, tst_off, plan)) return 0;
+    if (plan_soft(n_halo, src_off, tst_off, plan, false)) return 0;
     return carve_soft(nullptr, plan, pack).bytes;
 }
 

@@ -34,9 +34,11 @@
 #include <vector>
 
 #include "halma_common.h"
+#include "potential.h"
 #include "soft_pair.h"
 #include "soft_sym.h"
 #include "staging.h"
+#include "sym.h"
 #include "wave_reduce.h"
 
 namespace halma {
@@ -44,6 +46,8 @@ namespace halma {
 namespace {
 
 constexpr int kSsBand = 64;          // blocks per band
+constexpr int kSsQueues = 8;         // queues of a launch's items, heads in lines of their own
+constexpr int kSsHead = 16;
 constexpr int kSsBig = 16384;        // members from which a halo is cut into blocks of 512
 // Slot bytes of the haloes that share a launch, at 32 bytes a slot (room for S and a, whatever
 // the call asks for): the workspace grows by 2 kB a member up to here and no further, and a
@@ -154,13 +158,18 @@ __global__ __launch_bounds__(256, 2) void k_soft_sym(const float4* __restrict__ 
     constexpr int kBlock = T * kWave;
     const int lane = __lane_id();
     const int n_waves = static_cast<int>(gridDim.x * (blockDim.x / kWave));
+    // the items after the first ones from a queue, of blocks of 128 from kSsQueues of them in
+    // turn: one queue's additions follow one another by 7 ns (300 haloes of 5000 members have
+    // 246k: S 2.8 ms, 1.6 this way)
+    const int nq = T == 8 ? 1 : min(kSsQueues, static_cast<int>(gridDim.x));
+    const int queue = static_cast<int>(blockIdx.x) % nq;
     int k = __builtin_amdgcn_readfirstlane(
         static_cast<int>(blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave));
     for (bool first = true;; first = false) {
         if (!first) {
             int t = 0;
-            if (lane == 0) t = atomicAdd(head, 1);
-            k = n_waves + __builtin_amdgcn_readfirstlane(t);
+            if (lane == 0) t = atomicAdd(head + kSsHead * queue, 1);
+            k = n_waves + __builtin_amdgcn_readfirstlane(t) * nq + queue;
         }
         if (k >= n_items) break;
         SsDesc d;
@@ -255,8 +264,10 @@ __global__ __launch_bounds__(256) void k_soft_sym_merge(const SsDesc* __restrict
     }
 }
 
-__global__ void k_soft_sym_clear(int* __restrict__ p, int n) {
-    for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0;
+__global__ void k_soft_sym_clear(int* __restrict__ p, int64_t n) {
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
+         i += static_cast<int64_t>(gridDim.x) * blockDim.x)
+        p[i] = 0;
 }
 
 struct SsLaunch {
@@ -271,24 +282,32 @@ struct SsPlan {
     int64_t n_part = 0;  // slots of the largest group of haloes
 };
 
+// a halo of n members from row `off` on
+SsDesc ss_desc(int64_t n, int64_t off) {
+    SsDesc d;
+    d.off = off;
+    d.part_off = 0;
+    d.n = static_cast<int32_t>(std::min<int64_t>(n, INT32_MAX));  // larger: not taken
+    d.bs = n >= kSsBig ? 512 : 128;
+    d.nb = static_cast<int32_t>((n + d.bs - 1) / d.bs);
+    d.wb = std::max(1, std::min(d.nb, kSsBand));
+    return d;
+}
+
 int plan_ss(int64_t H, const int64_t* off, SsPlan& p) {
     p = SsPlan();
     p.halos.resize(static_cast<size_t>(H));
-    std::vector<int32_t> order;
+    std::vector<int64_t> key(static_cast<size_t>(H), 0);
+    size_t taken = 0;
     for (int64_t h = 0; h < H; ++h) {
-        SsDesc& d = p.halos[h];
         const int64_t n = off[h + 1] - off[h];
-        d.off = off[h] - off[0];
-        d.n = static_cast<int32_t>(std::min<int64_t>(n, INT32_MAX));  // larger: not taken
-        d.bs = n >= kSsBig ? 512 : 128;
-        d.nb = static_cast<int32_t>((n + d.bs - 1) / d.bs);
-        d.wb = std::max(1, std::min(d.nb, kSsBand));
-        d.part_off = 0;
+        p.halos[h] = ss_desc(n, off[h] - off[0]);
         if (n == 0 || !soft_sym_takes(n)) continue;
-        order.push_back(static_cast<int32_t>(h));
+        key[h] = n;
+        ++taken;
     }
-    std::stable_sort(order.begin(), order.end(),
-                     [&](int32_t a, int32_t b) { return p.halos[a].n > p.halos[b].n; });
+    std::vector<int32_t> order = order_desc(key);
+    order.resize(taken);
     size_t at = 0;
     while (at < order.size()) {
         // a group: haloes of one block size whose slots (at most four planes) fit together
@@ -359,14 +378,15 @@ struct SsWs {
     size_t bytes;
 };
 
-SsWs carve_ss(void* base, const SsPlan& p) {
+SsWs carve_ss(void* base, size_t halos, size_t tiles, size_t segs, size_t launches,
+              int64_t n_part) {
     Carver c(base);
     SsWs w;
-    w.halos = c.take<SsDesc>(std::max<size_t>(p.halos.size(), 1));
-    w.tiles = c.take<int4>(std::max<size_t>(p.tiles.size(), 1));
-    w.segs = c.take<int4>(std::max<size_t>(p.segs.size(), 1));
-    w.heads = c.take<int>(std::max<size_t>(p.launches.size(), 1));
-    w.part = c.take<double>(4 * static_cast<size_t>(std::max<int64_t>(p.n_part, 1)));
+    w.halos = c.take<SsDesc>(std::max<size_t>(halos, 1));
+    w.tiles = c.take<int4>(std::max<size_t>(tiles, 1));
+    w.segs = c.take<int4>(std::max<size_t>(segs, 1));
+    w.heads = c.take<int>(kSsQueues * kSsHead * std::max<size_t>(launches, 1));
+    w.part = c.take<double>(4 * static_cast<size_t>(std::max<int64_t>(n_part, 1)));
     w.bytes = c.used;
     return w;
 }
@@ -375,7 +395,8 @@ template <int MODE>
 int launch_ss(const SsPlan& p, const SsWs& w, const float4* rows, float e2, double* pot,
               double* acc, hipStream_t st) {
     const int cus = std::max(device_cu_count(), 1);
-    k_soft_sym_clear<<<1, 256, 0, st>>>(w.heads, static_cast<int>(p.launches.size()));
+    k_soft_sym_clear<<<16, 256, 0, st>>>(
+        w.heads, static_cast<int64_t>(kSsQueues * kSsHead) * static_cast<int64_t>(p.launches.size()));
     HALMA_LAUNCH_CHECK();
     for (size_t q = 0; q < p.launches.size(); ++q) {
         const SsLaunch& l = p.launches[q];
@@ -383,14 +404,14 @@ int launch_ss(const SsPlan& p, const SsWs& w, const float4* rows, float e2, doub
         if (l.big)
             k_soft_sym<MODE, 8><<<std::min(blocks, cus * 2), 256, 0, st>>>(
                 rows, w.halos, w.tiles + l.tile0, l.n_tiles, l.n_items, e2, w.part, p.n_part,
-                w.heads + q);
+                w.heads + kSsQueues * kSsHead * q);
         else
             k_soft_sym<MODE, 2><<<std::min(blocks, cus * 4), 256, 0, st>>>(
                 rows, w.halos, w.tiles + l.tile0, l.n_tiles, l.n_items, e2, w.part, p.n_part,
-                w.heads + q);
+                w.heads + kSsQueues * kSsHead * q);
         HALMA_LAUNCH_CHECK();
-        const dim3 grid(l.big ? 128 : 16, static_cast<unsigned>(std::min(l.n_segs, 4096)),
-                        ss_planes(MODE));
+        const dim3 grid(merge_width(p.segs.data() + l.seg0, l.n_segs),
+                        static_cast<unsigned>(std::min(l.n_segs, 65535)), ss_planes(MODE));
         k_soft_sym_merge<MODE><<<grid, 256, 0, st>>>(w.halos, w.segs + l.seg0, l.n_segs, w.part,
                                                      p.n_part, pot, acc);
         HALMA_LAUNCH_CHECK();
@@ -403,9 +424,26 @@ int launch_ss(const SsPlan& p, const SsWs& w, const float4* rows, float e2, doub
 bool soft_sym_takes(int64_t n) { return n <= kSsMax; }
 
 size_t soft_sym_bytes(int64_t H, const int64_t* off) {
-    SsPlan p;
-    if (plan_ss(H, off, p)) return 0;
-    return carve_ss(nullptr, p).bytes;
+    // at least what the plan needs, without its tables: a group of haloes fits kSsSlots, two
+    // after one another would not, and a group's largest halo has no more bands than any
+    size_t tiles = 0, segs = 0, bands[2] = {0, 0};
+    int64_t slots[2] = {0, 0};
+    for (int64_t h = 0; h < H; ++h) {
+        const SsDesc d = ss_desc(off[h + 1] - off[h], 0);
+        if (d.n == 0 || !soft_sym_takes(d.n)) continue;
+        const size_t K = static_cast<size_t>((d.nb + d.wb - 1) / d.wb);
+        tiles += K * (K + 1) / 2;
+        segs += K * K;
+        slots[d.bs == 512] += static_cast<int64_t>(d.wb) * d.n;
+        bands[d.bs == 512] = std::max(bands[d.bs == 512], K);
+    }
+    const int64_t room = static_cast<int64_t>(kSsSlots / kSsSlotBytes);
+    size_t launches = 0;
+    for (int c = 0; c < 2; ++c)
+        launches += (static_cast<size_t>(2 * slots[c] / room) + 1) * (bands[c] * (bands[c] + 1) / 2);
+    return carve_ss(nullptr, static_cast<size_t>(H), tiles, segs, std::min(launches, tiles),
+                    std::min(std::max(slots[0], slots[1]), room))
+        .bytes;
 }
 
 int soft_sym_run(int64_t H, const int64_t* off, const float4* rows, float e2, double* pot,
@@ -413,7 +451,7 @@ int soft_sym_run(int64_t H, const int64_t* off, const float4* rows, float e2, do
     SsPlan p;
     int rc = plan_ss(H, off, p);
     if (rc) return rc;
-    SsWs w = carve_ss(ws, p);
+    SsWs w = carve_ss(ws, p.halos.size(), p.tiles.size(), p.segs.size(), p.launches.size(), p.n_part);
     if (ws_bytes < w.bytes)
         return set_error(HALMA_E_WORKSPACE, "workspace %zu < required %zu", ws_bytes, w.bytes);
     rc = upload_async(w.halos, p.halos.data(), p.halos.size() * sizeof(SsDesc), st);

@@ -45,3 +45,27 @@ def test_self_sums_of_many_small_haloes(gpu, sizes):
         assert bool(((S[a:b] - want).abs() <= bound * want).all()), h
         alone = engine.pot_sum_self(np.array([0, b - a]), m[a:b], *x[a:b].T)
         assert torch.equal(alone, S[a:b]), h
+
+
+@pytest.mark.parametrize("sizes", SIZES, ids=["equal", "edges", "last_large", "first_large"])
+def test_softened_sums_of_many_small_haloes(gpu, sizes):
+    import torch
+
+    from pyhalma_amd import engine
+
+    eps = 5e-4
+    x, m, off = _catalogue(np.array(sizes), 7 + len(sizes))
+    print(f"haloes={len(sizes)} members={len(m)}", flush=True)
+    rows = torch.from_numpy(np.concatenate([x, m[:, None]], 1)).cuda()
+    r = engine.pot_soft_self(off, rows, eps, pot=True, acc=True)
+    one = engine.pot_soft_self(off, rows, eps, pot=True, acc=True, wsum=True)  # one-sided
+    # 13u and 15u of S; 26u and 28u of the sum of |terms| of a, no term beyond 0.1 Mpc
+    assert bool(((r["pot"] - one["pot"]).abs() <= 28 * 2.0 ** -24 * one["pot"]).all())
+    scale = one["wsum"][:, None] * 0.1
+    assert bool(((r["acc"] - one["acc"]).abs() <= 54 * 2.0 ** -24 * scale + 1e-30).all())
+    rng = np.random.default_rng(1)
+    for h in np.unique(np.concatenate([rng.integers(0, len(sizes), 30), np.argsort(sizes)[-3:]])):
+        a, b = off[h], off[h + 1]
+        alone = engine.pot_soft_self(np.array([0, b - a]), rows[a:b], eps, pot=True, acc=True)
+        assert torch.equal(alone["pot"], r["pot"][a:b])
+        assert torch.equal(alone["acc"], r["acc"][a:b])
