@@ -344,8 +344,11 @@ __global__ __launch_bounds__(W * kWave) void k_ball_count(int64_t H, Grid g, Que
                 dd_add_dd(th, tl, shm[2 * v], shm[2 * v + 1]);
             }
             count[h] = t;
-            atomicMax(reinterpret_cast<unsigned long long*>(most),
-                      static_cast<unsigned long long>(t));
+            // the largest count only grows: a count that is not above what is read of it needs no
+            // atomic, however old the read (100000 spheres with one each 1156 us, 335 this way)
+            if (t > __hip_atomic_load(most, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))
+                atomicMax(reinterpret_cast<unsigned long long*>(most),
+                          static_cast<unsigned long long>(t));
             if (mass) mass[h] = th + tl;
         }
         __syncthreads();

@@ -69,3 +69,24 @@ def test_softened_sums_of_many_small_haloes(gpu, sizes):
         alone = engine.pot_soft_self(np.array([0, b - a]), rows[a:b], eps, pot=True, acc=True)
         assert torch.equal(alone["pot"], r["pot"][a:b])
         assert torch.equal(alone["acc"], r["acc"][a:b])
+
+
+@pytest.mark.parametrize("large", [0, 1, 7])
+def test_many_tiny_spheres(gpu, large):
+    """Spheres of no or a few points, alone and with some of thousands among them (the largest
+    count decides how the hits are sorted)."""
+    from scipy.spatial import cKDTree
+
+    from pyhalma_amd import engine
+
+    rng = np.random.default_rng(large)
+    x = rng.uniform(0, 10, (60000, 3))
+    c = rng.uniform(0, 10, (20000, 3))
+    r = np.full(len(c), 0.08)
+    r[rng.integers(0, len(c), large)] = rng.uniform(1.0, 4.5, large)
+    print(f"spheres={len(c)} large={large}", flush=True)
+    off, idx, mass = engine.ball_query(*x.T, c, r, m=np.ones(len(x)))
+    want = [np.sort(k) for k in cKDTree(x).query_ball_point(c, r)]
+    assert np.array_equal(np.diff(off), [len(k) for k in want])
+    assert np.array_equal(idx.cpu().numpy(), np.concatenate(want))
+    assert np.array_equal(mass, np.diff(off))
