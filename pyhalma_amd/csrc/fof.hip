@@ -480,6 +480,38 @@ __global__ __launch_bounds__(256) void k_col_neigh(const int64_t* __restrict__ t
     }
 }
 
+// f(column, its cells [a0, a1), lim, first, stride) for the block's share of the columns: their
+// segments with a neighbour in another stretch begin before cell lim, and the caller takes
+// those numbered first, first + stride, ...  A column of more than kLongCol cells is spread
+// over its wavefront: a line of 2e5 cells along z takes one lane 20 ms in each of the two
+// kernels.
+constexpr int kLongCol = 256;
+
+template <typename F>
+__device__ __forceinline__ void for_columns(int64_t ncol, int64_t ncell,
+                                            const int* __restrict__ col_cell,
+                                            const ColNeigh* __restrict__ neigh, F&& f) {
+    const int lane = __lane_id();
+    const int str = stretch_cells(ncell);
+    const int64_t per = (ncol + gridDim.x - 1) / gridDim.x;
+    const int64_t q0 = blockIdx.x * per, q1 = q0 + per < ncol ? q0 + per : ncol;
+    for (int64_t b = q0 + (threadIdx.x & ~(kWave - 1)); b < q1; b += blockDim.x) {
+        const int64_t q = b + lane;
+        int a0 = 0, a1 = 0, lim = 0;
+        if (q < q1) {
+            a0 = col_cell[q];
+            a1 = col_cell[q + 1];
+            lim = min(a1, neigh[q].last / str * str);
+        }
+        const bool is_long = a1 - a0 > kLongCol;
+        if (!is_long) f(q, a0, a1, lim, 0, 1);
+        for (unsigned long long left = __ballot(is_long); left != 0; left &= left - 1) {
+            const int l = __ffsll(left) - 1;
+            f(b + l, __shfl(a0, l, kWave), __shfl(a1, l, kWave), __shfl(lim, l, kWave), lane, kWave);
+        }
+    }
+}
+
 // counts: as few_cells has it, zero before; counts[16 .. 23] are the class cursors
 __global__ __launch_bounds__(256) void k_col_class_count(const int64_t* __restrict__ totals,
                                                          const int* __restrict__ col_cell,
@@ -491,18 +523,14 @@ __global__ __launch_bounds__(256) void k_col_class_count(const int64_t* __restri
     __syncthreads();
     const int64_t ncol = totals[0] >> 32;
     const int64_t ncell = totals[0] & 0xffffffff;
-    const int str = stretch_cells(ncell);
-    const int64_t per = (ncol + gridDim.x - 1) / gridDim.x;
-    const int64_t q0 = blockIdx.x * per, q1 = q0 + per < ncol ? q0 + per : ncol;
-    for (int64_t q = q0 + threadIdx.x; q < q1; q += blockDim.x) {
-        const int a0 = col_cell[q], a1 = col_cell[q + 1];
-        const int last = neigh[q].last / str;
+    for_columns(ncol, ncell, col_cell, neigh, [&](int64_t, int a0, int a1, int lim,
+                                                int first, int stride) {
         const int step = seg_step(a1 - a0, false);
-        for (int c = a0; c < a1; c += step)
-            if (c / str != last) atomicAdd(&h[kColClasses + seg_class(crec, c, min(c + step, a1))], 1);
-        if (ncell > kFewCells) continue;
-        for (int c = a0; c < a1 && c / str != last; ++c) atomicAdd(&h[seg_class(crec, c, c + 1)], 1);
-    }
+        for (int c = a0 + first * step; c < lim; c += stride * step)
+            atomicAdd(&h[kColClasses + seg_class(crec, c, min(c + step, a1))], 1);
+        if (ncell > kFewCells) return;
+        for (int c = a0 + first; c < lim; c += stride) atomicAdd(&h[seg_class(crec, c, c + 1)], 1);
+    });
     __syncthreads();
     if (threadIdx.x < 2 * kColClasses && h[threadIdx.x] > 0)
         atomicAdd(counts + threadIdx.x, h[threadIdx.x]);
@@ -521,17 +549,13 @@ __global__ __launch_bounds__(256) void k_col_class_scatter(const int64_t* __rest
     __syncthreads();
     const int64_t ncol = totals[0] >> 32;
     const int64_t ncell = totals[0] & 0xffffffff;
-    const int str = stretch_cells(ncell);
     const bool few = few_cells(ncell, counts);
-    const int64_t per = (ncol + gridDim.x - 1) / gridDim.x;
-    const int64_t q0 = blockIdx.x * per, q1 = q0 + per < ncol ? q0 + per : ncol;
-    for (int64_t q = q0 + threadIdx.x; q < q1; q += blockDim.x) {
-        const int a0 = col_cell[q], a1 = col_cell[q + 1];
+    for_columns(ncol, ncell, col_cell, neigh, [&](int64_t, int a0, int a1, int lim,
+                                                int first, int stride) {
         const int step = seg_step(a1 - a0, few);
-        const int last = neigh[q].last / str;
-        for (int c = a0; c < a1; c += step)
-            if (c / str != last) atomicAdd(&h[seg_class(crec, c, min(c + step, a1))], 1);
-    }
+        for (int c = a0 + first * step; c < lim; c += stride * step)
+            atomicAdd(&h[seg_class(crec, c, min(c + step, a1))], 1);
+    });
     __syncthreads();
     if (threadIdx.x < kColClasses) {
         int before = 0;  // segments of the higher classes: the longest come first
@@ -542,12 +566,10 @@ __global__ __launch_bounds__(256) void k_col_class_scatter(const int64_t* __rest
         h[threadIdx.x] = 0;
     }
     __syncthreads();
-    for (int64_t q = q0 + threadIdx.x; q < q1; q += blockDim.x) {
-        const int a0 = col_cell[q], a1 = col_cell[q + 1];
+    for_columns(ncol, ncell, col_cell, neigh, [&](int64_t q, int a0, int a1, int lim,
+                                                int first, int stride) {
         const int step = seg_step(a1 - a0, few);
-        const int last = neigh[q].last / str;
-        for (int c = a0; c < a1; c += step) {
-            if (c / str == last) continue;
+        for (int c = a0 + first * step; c < lim; c += stride * step) {
             const int c1 = min(c + step, a1);
             const int k = seg_class(crec, c, c1);
             ColRec r;
@@ -557,7 +579,7 @@ __global__ __launch_bounds__(256) void k_col_class_scatter(const int64_t* __rest
             r.col = static_cast<int32_t>(q);
             lanes[base[k] + atomicAdd(&h[k], 1)] = r;
         }
-    }
+    });
 }
 
 // Between the rounds, after k_flatten (parent[c] is then c's root): the root shared by

@@ -58,3 +58,17 @@ def test_fof_slabs_about_a_stretch(gpu, side, spacing):
         parts.append(np.concatenate([np.full((len(yz), 1), k), yz], 1))
     x = np.concatenate(parts) * spacing
     _check(x[rng.permutation(len(x))], 1.0)
+
+
+@pytest.mark.parametrize("n", [255, 256, 257, 258, 5000, 70001])
+def test_fof_long_columns(gpu, n):
+    """Columns of about 256 cells and far beyond along z (spread over a wavefront when they are
+    listed), beside short ones, with gaps and side links."""
+    rng = np.random.default_rng(n)
+    z = np.arange(n) * 0.58 + rng.uniform(0, 1e-3, n)
+    z[n // 3:] += 2.0
+    a = np.stack([np.zeros(n), np.zeros(n), z], 1) + rng.uniform(0, 1e-3, (n, 3))
+    b = np.stack([np.full(n, 1.1), np.full(n, 0.7), z[::-1]], 1)[:: 7]
+    c = rng.uniform(0, 3, (500, 3)) + [0, 0, 0.58 * n / 2]
+    x = np.concatenate([a, b, c])
+    _check(x[rng.permutation(len(x))], 1.0)
