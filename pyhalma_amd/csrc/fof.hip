@@ -45,6 +45,8 @@ namespace {
 
 constexpr double kCellLimit = 2097152.0;  // 2^21 cells per axis
 constexpr int kBoxBlocks = 1024;
+constexpr int kColClasses = 8;  // classes of column segments
+constexpr int kBigLists = 3;    // fillings of the list of large pairs: local, cross 1, cross 2
 
 // A column's word: its key (x | y, at most 42 bits) in the low bits and its cell count
 // (at most 2^21) above them.
@@ -155,8 +157,19 @@ __global__ __launch_bounds__(256) void k_bbox_partial(const T* __restrict__ x,
     }
 }
 
+// ... also clears the call's error word and counters (a launch of their own each would be a
+// tenth of a call of a few points)
+struct Clear {
+    int* err;
+    int* class_counts;
+    unsigned long long* n_big;
+};
+
 __global__ __launch_bounds__(256) void k_bbox_final(const double* __restrict__ part, int nb,
-                                                    double* __restrict__ box) {
+                                                    double* __restrict__ box, Clear z) {
+    if (threadIdx.x == 0) *z.err = 0;
+    if (threadIdx.x < 3 * kColClasses) z.class_counts[threadIdx.x] = 0;
+    if (threadIdx.x < kBigLists) z.n_big[threadIdx.x] = 0;
     __shared__ double sh[4][6];
     double v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
     for (int b = threadIdx.x; b < nb; b += blockDim.x)
@@ -177,11 +190,6 @@ __global__ __launch_bounds__(256) void k_bbox_final(const double* __restrict__ p
             r = threadIdx.x < 3 ? fmin(r, sh[k][threadIdx.x]) : fmax(r, sh[k][threadIdx.x]);
         box[threadIdx.x] = r;
     }
-}
-
-__global__ void k_fill_i32n(int* p, int64_t n, int v) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
 }
 
 // (x, y, z, 0) in one vector: float4 for FP32 coordinates, double4 for FP64
@@ -385,9 +393,7 @@ __device__ __forceinline__ int stretch_cells(int64_t ncell) {
 // each block takes one contiguous stretch of columns, counts their segments, reserves
 // their places with one atomic per class, and writes them (the order within a class is
 // not fixed; the links do not depend on it).
-constexpr int kColClasses = 8;
 constexpr int kClassBlocks = 256;
-constexpr int kBigLists = 3;  // fillings of the list of large pairs: local, cross 1, cross 2
 constexpr int kSegMin = 4;
 constexpr int kSegCells = 4;
 constexpr int64_t kFewCells = 1 << 19;
@@ -1124,12 +1130,6 @@ FofWs carve_fof(void* base, int64_t n, size_t elt) {
     return w;
 }
 
-__global__ void k_clear_words(uint32_t* __restrict__ p, int64_t n) {
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-         i += static_cast<int64_t>(gridDim.x) * blockDim.x)
-        p[i] = 0u;
-}
-
 inline unsigned blocks_for(int64_t n, int t = 256) {
     return static_cast<unsigned>((n + t - 1) / t);
 }
@@ -1145,11 +1145,10 @@ int fof_run(const T* x, const T* y, const T* z, int64_t n, double ll, int* label
             const FofWs& w, hipStream_t st) {
     const int cus = std::max(1, device_cu_count());
     const int grid_cells = cus * 8;
-    k_fill_i32n<<<1, 64, 0, st>>>(w.err, 1, 0);
-    HALMA_LAUNCH_CHECK();
     k_bbox_partial<T><<<kBoxBlocks, 256, 0, st>>>(x, y, z, n, w.box_part);
     HALMA_LAUNCH_CHECK();
-    k_bbox_final<<<1, 256, 0, st>>>(w.box_part, kBoxBlocks, w.box);
+    k_bbox_final<<<1, 256, 0, st>>>(w.box_part, kBoxBlocks, w.box,
+                                    Clear{w.err, w.class_counts, w.n_big});
     HALMA_LAUNCH_CHECK();
     // the box fixes the grid (one small read-back)
     long long* hw = pinned_words(8);
@@ -1202,10 +1201,6 @@ int fof_run(const T* x, const T* y, const T* z, int64_t n, double ll, int* label
     k_fof_cells<<<blocks_for(n), 256, 0, st>>>(w.skey, perm, w.heads, w.before, n, g,
                                                w.crec, w.cell_min, w.cell_col, w.comp_min,
                                                w.col_cell, w.col_key);
-    HALMA_LAUNCH_CHECK();
-    k_clear_words<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(w.n_big), 2 * kBigLists);
-    HALMA_LAUNCH_CHECK();
-    k_clear_words<<<1, 64, 0, st>>>(reinterpret_cast<uint32_t*>(w.class_counts), 3 * kColClasses);
     HALMA_LAUNCH_CHECK();
     k_col_neigh<<<grid_cells, 256, 0, st>>>(w.totals, w.col_cell, w.col_key, g.by, w.cols,
                                             w.neigh);
