@@ -61,7 +61,12 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kIncChunk = 256;      // smallest source chunk of an incremental pass
-constexpr int kCounters = 16;       // words of the counters (EnergyArgs)
+// Words of the counters (EnergyArgs): sixteen, then the pairs of the workgroup passes in
+// kPairSlots words a cache line apart (an addition for each of 100000 haloes to one word takes
+// 0.7 ms).
+constexpr int kPairSlots = 16;
+constexpr int kPairStride = 8;
+constexpr int kCounters = 16 + kPairSlots * kPairStride;
 constexpr int kRetestBlock = 2048;  // live sets from this size are re-summed by a block
 
 // member states
@@ -154,8 +159,11 @@ __device__ __forceinline__ bool too_stale(int stale, int live) {
     return kStaleDiv * static_cast<int64_t>(stale) > live;
 }
 
-// k_halo_tail's workgroup, and the most it takes on (see there)
+// k_halo_tail's workgroups (for haloes of more than kTailSmall members and for the others),
+// and the most they take on (see there)
 constexpr int kTailThreads = 512;
+constexpr int kTailSmallThreads = 64;
+constexpr int kTailSmall = 256;
 constexpr int kTailLive = 4096;         // live members
 constexpr int64_t kTailPairs = 1 << 20;  // pairs of an incremental pass
 constexpr int64_t kTailFull = 1 << 19;   // pairs of a full pass
@@ -164,7 +172,7 @@ constexpr int64_t kTailFull = 1 << 19;   // pairs of a full pass
 constexpr uint32_t kStaleBit = 0x80000000u;
 
 __global__ void k_zero_counters(unsigned long long* __restrict__ c, int n) {
-    if (static_cast<int>(threadIdx.x) < n) c[threadIdx.x] = 0;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) c[i] = 0;
 }
 
 // block-wide exclusive scan of one int per thread; returns the block total
@@ -500,7 +508,7 @@ struct EnergyArgs {
                                    // [3] pairs, [4] symmetric-kernel pairs, [5] haloes
                                    // still active after the pass, [6] members re-summed
                                    // for their error bound alone, [8] the band
-                                   // count of large live sets, [9] haloes still active
+                                   // count of large live sets, [9] set while a halo is active
                                    // after k_halo_tail, [10] most passes of a halo, [11] active
                                    // haloes of more than kTailLive members
     double* s_out;     // optional: S per member position (FP64)
@@ -829,16 +837,21 @@ __global__ __launch_bounds__(kThreads) void k_finish(EnergyArgs a) {
 // members is active, launched passes go on anyway and the small haloes ride along: then
 // nothing is done here (the clump step, its largest haloes at 20000 members and 8 passes,
 // 4.55 ms; with this kernel after every launched pass 4.67).  512 threads: 1024 take
-// 5.8 ms on the pairs, 256 5.2.
+// 5.8 ms on the pairs, 256 5.2.  Haloes of at most kTailSmall members take a wavefront each,
+// eight times as many at once: 100000 of 20 members 9.0 -> 3.4 ms a call (8.4 with launched
+// passes alone), 10000 of 256 3.3 -> 1.55.
 constexpr int kTailRem = 736;            // removed members: at most half the live ones in an
                                          // incremental pass, so fewer than sqrt(kTailPairs / 2)
 static_assert(2 * int64_t(kTailRem) * kTailRem > kTailPairs, "removed members of a pass");
+constexpr int kTailSmallRem = kTailSmall / 2;
+static_assert(3 * kTailSmallRem >= kTailSmall, "a third of a set at most, as above");
 
+template <int T, int REM>
 struct TailShared {
-    float4 rem[kTailRem];
-    double dd[kTailThreads / kWave][8];
+    float4 rem[REM];
+    double dd[T / kWave][8];
     double vcm[3];
-    int scan[kTailThreads / kWave];
+    int scan[T / kWave];
     int n_gone, n_stale, n_list;
 };
 
@@ -862,14 +875,15 @@ __device__ __forceinline__ double tail_sum(const float4* src, int n, float4 t) {
     return S;
 }
 
-__global__ __launch_bounds__(kTailThreads, 4) void k_halo_tail(
+template <int T, int REM>
+__global__ __launch_bounds__(T, 4) void k_halo_tail(
     EnergyArgs a, const int32_t* __restrict__ order, const int64_t* __restrict__ off,
     const double* __restrict__ m64, float4* src4, int32_t* cidx) {
-    __shared__ TailShared sh;
+    __shared__ TailShared<T, REM> sh;
     const int h = order[blockIdx.x];
     if (!a.active[h]) return;
     if (a.counters[11] != 0) {  // launched passes go on anyway
-        if (threadIdx.x == 0) atomicAdd(a.counters + 9, 1ull);
+        if (threadIdx.x == 0) a.counters[9] = 1;
         return;
     }
     const int lane = __lane_id();
@@ -895,7 +909,7 @@ __global__ __launch_bounds__(kTailThreads, 4) void k_halo_tail(
         // at or before their own places), masses and momenta of the kept
         double acc[4][2] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
         int kept = 0, rem = 0;
-        for (int base = 0; base < n; base += kTailThreads) {
+        for (int base = 0; base < n; base += T) {
             const int i = base + tid;
             const bool in = i < n;
             const int k = in ? idx[i] : 0;
@@ -915,7 +929,7 @@ __global__ __launch_bounds__(kTailThreads, 4) void k_halo_tail(
             __syncthreads();
             int before = x - f, tot = 0;
 #pragma unroll
-            for (int q = 0; q < kTailThreads / kWave; ++q) {
+            for (int q = 0; q < T / kWave; ++q) {
                 if (q < wv) before += sh.scan[q];
                 tot += sh.scan[q];
             }
@@ -928,7 +942,7 @@ __global__ __launch_bounds__(kTailThreads, 4) void k_halo_tail(
                 for (int d = 0; d < 3; ++d) dd_add(acc[1 + d][0], acc[1 + d][1], m * v[d]);
             } else if (st == kJustGone) {
                 const int at = rem + (before >> 16);
-                if (at < kTailRem) sh.rem[at] = p;  // read in an incremental pass only
+                if (at < REM) sh.rem[at] = p;  // read in an incremental pass only
                 a.state[k] = kGone;
             }
             kept += tot & 0xffff;
@@ -951,7 +965,7 @@ __global__ __launch_bounds__(kTailThreads, 4) void k_halo_tail(
         __syncthreads();
         if (tid == 0) {
             double s[4][2] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
-            for (int w = 0; w < kTailThreads / kWave; ++w)
+            for (int w = 0; w < T / kWave; ++w)
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
                     dd_add_dd(s[q][0], s[q][1], sh.dd[w][2 * q], sh.dd[w][2 * q + 1]);
@@ -964,7 +978,7 @@ __global__ __launch_bounds__(kTailThreads, 4) void k_halo_tail(
         const double vc[3] = {sh.vcm[0], sh.vcm[1], sh.vcm[2]};
         // S and the decisions outside the band, a member per lane
         const int ns = full ? kept : rem;
-        for (int i0 = wv * kWave; i0 < kept; i0 += kTailThreads) {
+        for (int i0 = wv * kWave; i0 < kept; i0 += T) {
             const int i = min(i0 + lane, kept - 1);
             const int64_t k = idx[i];
             const double s_old = full ? 0.0 : a.sacc[k], e_old = full ? 0.0 : a.eacc[k];
@@ -1005,7 +1019,7 @@ __global__ __launch_bounds__(kTailThreads, 4) void k_halo_tail(
         // band members: the oracle's sum and decision; stale ones, when few, a fresh S
         const int n_list = sh.n_list, n_stale = sh.n_stale;
         const bool resum = !too_stale(n_stale, kept);
-        for (int e = wv; e < n_list; e += kTailThreads / kWave) {
+        for (int e = wv; e < n_list; e += T / kWave) {
             const uint32_t entry = static_cast<uint32_t>(list[e]);
             const int i = static_cast<int>(entry & ~kStaleBit);
             const bool stale = (entry & kStaleBit) != 0;
@@ -1051,9 +1065,13 @@ __global__ __launch_bounds__(kTailThreads, 4) void k_halo_tail(
         a.refresh[h] = refresh;
         a.hpass[h] = passes;
         a.iters[h] = iters;
-        if (pairs) atomicAdd(a.counters + 3, pairs);
-        if (on) atomicAdd(a.counters + 9, 1ull);
-        atomicMax(a.counters + 10, static_cast<unsigned long long>(passes));
+        if (pairs)
+            atomicAdd(a.counters + 16 + kPairStride * (blockIdx.x % kPairSlots), pairs);
+        if (on) a.counters[9] = 1;
+        // the most passes only grows: no atomic where it does not
+        if (static_cast<unsigned long long>(passes) >
+            __hip_atomic_load(a.counters + 10, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))
+            atomicMax(a.counters + 10, static_cast<unsigned long long>(passes));
     }
     if (n_retest) atomicAdd(a.counters + 2, n_retest);
     if (n_resum) atomicAdd(a.counters + 6, n_resum);
@@ -1257,6 +1275,7 @@ struct UnbWs {
     float2* part;
     // the symmetric kernel of the full passes
     SymDesc* sym;     // per halo (in the tables region)
+    int32_t* tail;    // haloes in k_halo_tail's order
     int4* sym_items;
     int64_t* sym_icnt;
     int64_t* sym_ioff;
@@ -1273,7 +1292,7 @@ struct UnbWs {
     int64_t n_chunks;
     // host tables (off, halos, order, chunks, cfirst) sit in one region, uploaded at once
     char* tables;
-    size_t t_off, t_halos, t_order, t_chunks, t_cfirst, t_sym, t_bytes;
+    size_t t_off, t_halos, t_order, t_chunks, t_cfirst, t_sym, t_tail, t_bytes;
     size_t bytes;
 };
 
@@ -1303,6 +1322,8 @@ UnbWs carve_unb(void* base, int64_t H, int64_t nm, const PotPlan& plan, const Sy
     t.take<int32_t>(h1 + 1);
     w.t_sym = t.used;
     t.take<SymDesc>(h1);
+    w.t_tail = t.used;
+    t.take<int32_t>(h1);
     w.t_bytes = t.used;
     w.tables = c.take<char>(w.t_bytes);
     w.off = reinterpret_cast<int64_t*>(w.tables + w.t_off);
@@ -1311,6 +1332,7 @@ UnbWs carve_unb(void* base, int64_t H, int64_t nm, const PotPlan& plan, const Sy
     w.chunks = reinterpret_cast<int2*>(w.tables + w.t_chunks);
     w.cfirst = reinterpret_cast<int32_t*>(w.tables + w.t_cfirst);
     w.sym = reinterpret_cast<SymDesc*>(w.tables + w.t_sym);
+    w.tail = reinterpret_cast<int32_t*>(w.tables + w.t_tail);
     w.n_chunks = n_chunks;
     w.ccnt = c.take<int32_t>(2 * c1);
     w.csum = c.take<double>(8 * c1);
@@ -1565,14 +1587,20 @@ int unbind_run(int64_t H, const int64_t* h_off, const int32_t* members, Inputs i
         }
         cfirst[H] = q;
     }
-    const UploadPiece pieces[6] = {
+    // the haloes as k_halo_tail takes them: the larger ones first, each part in the plan's order
+    std::vector<int32_t> tail(plan.order);
+    const auto small_from = std::stable_partition(
+        tail.begin(), tail.end(), [&](int32_t h) { return rel[h + 1] - rel[h] > kTailSmall; });
+    const int64_t n_tail_large = small_from - tail.begin();
+    const UploadPiece pieces[7] = {
         {w.t_off, rel.data(), (H + 1) * sizeof(int64_t)},
         {w.t_halos, plan.halos.data(), plan.halos.size() * sizeof(HaloDesc)},
         {w.t_order, plan.order.data(), plan.order.size() * sizeof(int32_t)},
         {w.t_chunks, chunks.data(), chunks.size() * sizeof(int2)},
         {w.t_cfirst, cfirst.data(), cfirst.size() * sizeof(int32_t)},
-        {w.t_sym, splan.halos.data(), splan.halos.size() * sizeof(SymDesc)}};
-    rc = upload_pieces(w.tables, w.t_bytes, pieces, 6, st);
+        {w.t_sym, splan.halos.data(), splan.halos.size() * sizeof(SymDesc)},
+        {w.t_tail, tail.data(), tail.size() * sizeof(int32_t)}};
+    rc = upload_pieces(w.tables, w.t_bytes, pieces, 7, st);
     if (rc) return rc;
     const int32_t* mem = members + h_off[0];
     if (nm > 0) {
@@ -1724,9 +1752,18 @@ int unbind_run(int64_t H, const int64_t* h_off, const int32_t* members, Inputs i
         if (!r) r = run_part(3);
         if (!r && timing) r = record(ev[q][3]);
         if (r) return r;
-        k_halo_tail<<<static_cast<unsigned>(H), kTailThreads, 0, st>>>(L.ea, w.order, w.off,
-                                                                       w.m64, w.src4, w.cidx);
-        HALMA_LAUNCH_CHECK();
+        if (n_tail_large > 0) {
+            k_halo_tail<kTailThreads, kTailRem>
+                <<<static_cast<unsigned>(n_tail_large), kTailThreads, 0, st>>>(
+                    L.ea, w.tail, w.off, w.m64, w.src4, w.cidx);
+            HALMA_LAUNCH_CHECK();
+        }
+        if (H > n_tail_large) {
+            k_halo_tail<kTailSmallThreads, kTailSmallRem>
+                <<<static_cast<unsigned>(H - n_tail_large), kTailSmallThreads, 0, st>>>(
+                    L.ea, w.tail + n_tail_large, w.off, w.m64, w.src4, w.cidx);
+            HALMA_LAUNCH_CHECK();
+        }
         if (timing) r = record(ev[q][4]);
         if (r) return r;
         const hipError_t e = hipMemcpyAsync(host + kCounters * q, w.counters,
@@ -1794,6 +1831,7 @@ int unbind_run(int64_t H, const int64_t* h_off, const int32_t* members, Inputs i
         stats[5] = static_cast<int64_t>(pot_ms * 1e6);  // ns
         stats[6] = pot_launches;
         stats[7] = last[3];
+        for (int q = 0; q < kPairSlots; ++q) stats[7] += last[16 + q * kPairStride];
         stats[8] = static_cast<int64_t>(sym_ms * 1e6);  // ns
         stats[9] = sym_launches;
         stats[10] = last[4];

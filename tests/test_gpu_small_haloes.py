@@ -90,3 +90,36 @@ def test_many_tiny_spheres(gpu, large):
     assert np.array_equal(np.diff(off), [len(k) for k in want])
     assert np.array_equal(idx.cpu().numpy(), np.concatenate(want))
     assert np.array_equal(mass, np.diff(off))
+
+
+@pytest.mark.parametrize("max_iter", [2, 5, 100])
+@pytest.mark.parametrize("sizes", [[20, 21] * 1500, [255, 256, 257, 63, 64, 65] * 15,
+                                   [10, 11] * 300 + [2001, 3000, 500, 501]],
+                         ids=["tiny", "edges", "mixed"])
+def test_unbinding_of_many_small_haloes(gpu, sizes, max_iter):
+    """Haloes of at most 256 members take a wavefront each for their further passes, larger ones
+    a workgroup: masks and pass counts of the plain FP64 comparator, v_cm of the bound ones."""
+    import torch
+    from test_gpu_unbind_tail import _groups, _haloes
+
+    from pyhalma_amd import engine
+
+    X, V, M = _haloes(sizes, 5)
+    print(f"haloes={len(sizes)} members={len(M)} max_iter={max_iter}", flush=True)
+    r = engine.unbind(_groups(sizes), *X.T, *V.T, M, max_iter=max_iter, with_pot=True)
+    bound, iters = engine.unbind_plain_f64(_groups(sizes), *X.T, *V.T, M, max_iter=max_iter)
+    assert torch.equal(r.bound, bound)
+    assert np.array_equal(r.iters.cpu().numpy(), iters)
+    assert r.stats["passes"] >= iters.max()
+    # the pairs of the reference's loop: every pass over the bound set it began with
+    n = np.array(sizes, float)
+    assert (n * n).sum() <= r.stats["pairs"] <= (n * n * iters).sum()
+    if max_iter < 100:
+        return
+    off = np.concatenate([[0], np.cumsum(sizes)])
+    b = r.bound.cpu().numpy().astype(bool)
+    m = M.astype(np.float64) * b
+    mass = np.add.reduceat(m, off[:-1])
+    want = np.add.reduceat(m[:, None] * V.astype(np.float64), off[:-1]) / np.maximum(mass, 1e-300)[:, None]
+    got = r.vcm.cpu().numpy()
+    assert np.abs(got - want)[mass > 0].max() <= 1e-12 * np.abs(V).max()
