@@ -237,15 +237,16 @@ int plan_pot(int64_t H, const int64_t* src_off, const int64_t* tst_off, PotPlan&
     const int64_t waves = static_cast<int64_t>(cus) * t.waves_per_cu;
     plan.grid = static_cast<int>(waves / 4);
     const int64_t target = waves * t.items_per_wave;
-    int64_t base_items = 0, min_items = 0;
+    int64_t base_items = 0, with_src = 0;  // test tiles, those that have sources
     double work = 0.0;
     for (int64_t h = 0; h < H; ++h) {
         const int64_t ns = src_off[h + 1] - src_off[h];
         const int64_t nt = tst_off[h + 1] - tst_off[h];
         if (ns < 0 || nt < 0 || ns > INT32_MAX || nt > INT32_MAX)
             return set_error(HALMA_E_ARG, "halo %lld: bad offsets", (long long)h);
-        base_items += (nt + tile - 1) / tile;
-        min_items += (nt + tile - 1) / tile * ((ns + t.min_chunk - 1) / t.min_chunk);
+        const int64_t tiles = (nt + tile - 1) / tile;
+        base_items += tiles;
+        with_src += ns > 0 ? tiles : 0;
         work += static_cast<double>(ns) * static_cast<double>(nt);
     }
     // A launch that leaves SIMDs without two wavefronts at the tuned smallest chunk is a
@@ -253,6 +254,13 @@ int plan_pot(int64_t H, const int64_t* src_off, const int64_t* tst_off, PotPlan&
     // smaller chunks until it has them, 64 sources at the least (329 items, 12 us).
     int64_t min_chunk = t.min_chunk;
     const int64_t two_waves = static_cast<int64_t>(cus) * 8;
+    int64_t min_items = with_src;  // an item each at the least
+    if (with_src < two_waves) {
+        min_items = 0;
+        for (int64_t h = 0; h < H; ++h)
+            min_items += (tst_off[h + 1] - tst_off[h] + tile - 1) / tile *
+                         ((src_off[h + 1] - src_off[h] + t.min_chunk - 1) / t.min_chunk);
+    }
     if (min_items < two_waves)
         min_chunk = std::min<int64_t>(
             min_chunk, std::max<int64_t>(64, min_chunk * min_items / two_waves / 8 * 8));
