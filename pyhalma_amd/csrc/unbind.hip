@@ -1752,13 +1752,14 @@ int unbind_run(int64_t H, const int64_t* h_off, const int32_t* members, Inputs i
         if (!r) r = run_part(3);
         if (!r && timing) r = record(ev[q][3]);
         if (r) return r;
-        if (n_tail_large > 0) {
+        const bool last_pass = p + 1 >= max_iter;  // of every halo: nothing follows
+        if (n_tail_large > 0 && !last_pass) {
             k_halo_tail<kTailThreads, kTailRem>
                 <<<static_cast<unsigned>(n_tail_large), kTailThreads, 0, st>>>(
                     L.ea, w.tail, w.off, w.m64, w.src4, w.cidx);
             HALMA_LAUNCH_CHECK();
         }
-        if (H > n_tail_large) {
+        if (H > n_tail_large && !last_pass) {
             k_halo_tail<kTailSmallThreads, kTailSmallRem>
                 <<<static_cast<unsigned>(H - n_tail_large), kTailSmallThreads, 0, st>>>(
                     L.ea, w.tail + n_tail_large, w.off, w.m64, w.src4, w.cidx);
