@@ -304,7 +304,7 @@ __device__ const double* block_group_reduce(double (&acc)[8][2], double (&mn)[8]
     return sh + nw * kGrpQ;
 }
 
-// One workgroup per group of first < members <= last: 1024 threads for the large groups,
+// One workgroup per group, in two launches: 1024 threads for the large groups,
 // 256 for those of at most kSmallGroup, of which a CU then holds several at once and whose
 // barriers, trees and folds span four wavefronts (2.1M members in 1000 groups of up to
 // 20000: 79 us with 1024 threads for every group, 68 us in the two launches; one group of 24k
@@ -314,14 +314,13 @@ constexpr int64_t kSmallGroup = 4096;
 template <int DT, int T>
 __global__ __launch_bounds__(T, 4) void k_group_reduce(Src s, const int64_t* __restrict__ off,
                                                     const int32_t* __restrict__ mem, int64_t G,
-                                                    int64_t first, int64_t last,
                                                     const double* __restrict__ centres,
                                                     double* __restrict__ out) {
     __shared__ double sh[kGrpQ * (T / kWave + 1)];
     __shared__ double cen[3];
     for (int64_t g = blockIdx.x; g < G; g += gridDim.x) {
         const int64_t b = off[g], e = off[g + 1];
-        if (e - b <= first || e - b > last) continue;  // block-uniform
+        if ((e - b > kSmallGroup) != (T == kBig)) continue;  // block-uniform
         double acc[8][2];  // M, Mx, My, Mz, Mvx, Mvy, Mvz, sum |m|
         for (int k = 0; k < 8; ++k) acc[k][0] = acc[k][1] = 0.0;
         double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
@@ -891,11 +890,9 @@ template <int DT>
 int run_group_reduce(const Src& s, const int64_t* off, const int32_t* mem, int64_t G,
                      const double* centres, double* out, hipStream_t st) {
     const unsigned grid = static_cast<unsigned>(G < 65536 ? G : 65536);
-    k_group_reduce<DT, kBig><<<grid, kBig, 0, st>>>(s, off, mem, G, kSmallGroup, INT64_MAX,
-                                                    centres, out);
+    k_group_reduce<DT, kBig><<<grid, kBig, 0, st>>>(s, off, mem, G, centres, out);
     HALMA_LAUNCH_CHECK();
-    k_group_reduce<DT, kThreads><<<grid, kThreads, 0, st>>>(s, off, mem, G, -1, kSmallGroup,
-                                                            centres, out);
+    k_group_reduce<DT, kThreads><<<grid, kThreads, 0, st>>>(s, off, mem, G, centres, out);
     HALMA_LAUNCH_CHECK();
     return 0;
 }
