@@ -1741,6 +1741,9 @@ int unbind_run(int64_t H, const int64_t* h_off, const int32_t* members, Inputs i
                    ? 0
                    : set_error(HALMA_E_STATE, "event record failed");
     };
+    std::fill(host, host + 2 * kCounters, 0ll);
+    const long long* last = host;  // the counters of the last round read back
+    bool with_tail[2] = {false, false};
     auto launch_round = [&](int p) -> int {
         const int q = p & 1;
         int r = run_part(0);
@@ -1752,14 +1755,17 @@ int unbind_run(int64_t H, const int64_t* h_off, const int32_t* members, Inputs i
         if (!r) r = run_part(3);
         if (!r && timing) r = record(ev[q][3]);
         if (r) return r;
-        const bool last_pass = p + 1 >= max_iter;  // of every halo: nothing follows
-        if (n_tail_large > 0 && !last_pass) {
+        // nothing for k_halo_tail after every halo's last pass, nor while a large halo is
+        // active: as the last round read back has it (a round or two late, which only leaves
+        // passes to the launched ones)
+        with_tail[q] = p + 1 < max_iter && last[11] == 0;
+        if (n_tail_large > 0 && with_tail[q]) {
             k_halo_tail<kTailThreads, kTailRem>
                 <<<static_cast<unsigned>(n_tail_large), kTailThreads, 0, st>>>(
                     L.ea, w.tail, w.off, w.m64, w.src4, w.cidx);
             HALMA_LAUNCH_CHECK();
         }
-        if (H > n_tail_large && !last_pass) {
+        if (H > n_tail_large && with_tail[q]) {
             k_halo_tail<kTailSmallThreads, kTailSmallRem>
                 <<<static_cast<unsigned>(H - n_tail_large), kTailSmallThreads, 0, st>>>(
                     L.ea, w.tail + n_tail_large, w.off, w.m64, w.src4, w.cidx);
@@ -1792,9 +1798,7 @@ int unbind_run(int64_t H, const int64_t* h_off, const int32_t* members, Inputs i
         }
         return 0;
     };
-    std::fill(host, host + 2 * kCounters, 0ll);
     // every launched pass takes each active halo a pass further, so max_iter rounds do
-    const long long* last = host;
     int rounds = 0, launched = 0;
     int status = max_iter > 0 ? launch_round(0) : 0;
     if (max_iter > 0) launched = 1;
@@ -1809,7 +1813,8 @@ int unbind_run(int64_t H, const int64_t* h_off, const int32_t* members, Inputs i
         if (status) break;
         last = host + kCounters * (p & 1);
         rounds = p + 1;
-        if (last[9] == 0) break;  // no halo left: a queued round, if any, does nothing
+        if (last[with_tail[p & 1] ? 9 : 5] == 0)
+            break;  // no halo left: a queued round, if any, does nothing
     }
     // the queued round after convergence: its (empty) kernels are counted like the others
     if (!status && launched > rounds) status = collect(rounds);
