@@ -37,8 +37,8 @@
 //                    reset to that value); stale members: a fresh FP32 S;
 //   5. k_finish      per-halo pass counts, convergence flags, the removed total (a thread
 //                    per halo);
-//   6. k_halo_tail   the passes that follow, a workgroup per halo, where none of the active
-//                    haloes is large and until a halo's next pass is too much for a
+//   6. k_halo_tail   the passes that follow, a workgroup per halo (a wavefront for a small
+//                    one), where none of the active haloes is large and until a halo's next pass is too much for a
 //                    workgroup.
 // The parts are plain launches (or, on request, hipGraphs captured once and replayed);
 // the host reads one counter per pass to stop.
