@@ -482,8 +482,9 @@ int halma_energy_test_self_batched(int64_t n_halo, const int64_t *tst_off, const
  * over the pairs computes them all.  FP32 terms in plain sub-tiles of eight, the sub-tiles
  * in Kahan pairs (self sums without wsum: in FP64), the chunks in FP64.  Against FP64: pot
  * within 2^-20 relative, acc and wsum within 2^-19 relative to sum_j |term_j|, whatever the
- * tuning (halma_pot_error_bound() is the plain sums').  A halo with at most 8 tests spreads each test's sources over the lanes
- * of a wavefront (chunks of 4096 sources); larger haloes hold 64 tests per wavefront.
+ * tuning (halma_pot_error_bound() is the plain sums').  A halo with at most 8 tests
+ * spreads each test's sources over the lanes of a wavefront (chunks of 4096 sources);
+ * larger haloes hold 64 tests per wavefront.
  * Chunk sizes follow from each halo's own source and test counts and the chunk
  * partials are added in chunk order, so a test's bits depend on its halo's inputs only
  * (not on the other haloes of the call).  The pair terms are recomputed, never stored.

@@ -382,11 +382,12 @@ __device__ __forceinline__ int stretch_cells(int64_t ncell) {
 // cells, and each segment takes its own lanes (a long column's cells are then linked by
 // several lanes at once instead of one long chain of finds and unions).  Up to kFewCells
 // cells, which leave most of the chip idle, every cell is a segment: FoF of a 24k Plummer
-// sphere 397 -> 339 us (its first round 113 -> 60), 98k clump stars 279 -> 255, 654k 430 -> 405, 240k
-// bridged 427 -> 405, 800k (650k cells) 670 and 667; 2.4M 1325 -> 1339.  Not so where that makes
-// more than kFewMore segments more, which fill the chip: 200k uniform points (columns of 5-25
-// cells, 1.2e5 more) 0.8 and 1.2 linking lengths apart take 480 and 433 us that way, 428 and 395 in
-// segments of kSegCells, 100k (7e4 more) 360 and 322 against 368 and 335.  Lane order:
+// sphere 397 -> 339 us (its first round 113 -> 60), 98k clump stars 279 -> 255, 654k 430 ->
+// 405, 240k bridged 427 -> 405, 800k (650k cells) 670 and 667; 2.4M 1325 -> 1339.  Not so where
+// that makes more than kFewMore segments more, which fill the chip: 200k uniform points
+// (columns of 5-25 cells, 1.2e5 more) 0.8 and 1.2 linking lengths apart take 480 and 433 us
+// that way, 428 and 395 in segments of kSegCells, 100k (7e4 more) 360 and 322 against 368 and
+// 335.  Lane order:
 // segments grouped by the log2 of their particle count, largest first, so that the lanes
 // of a wavefront walk segments of similar length (a wavefront lasts as long as its
 // longest lane) and the longest start first.  A counting sort over kColClasses classes;
@@ -568,7 +569,9 @@ __global__ __launch_bounds__(256) void k_col_class_scatter(const int64_t* __rest
         for (int k = threadIdx.x + 1; k < kColClasses; ++k)
             before += counts[(few ? 0 : kColClasses) + k];
         base[threadIdx.x] =
-            h[threadIdx.x] > 0 ? before + atomicAdd(counts + 2 * kColClasses + threadIdx.x, h[threadIdx.x]) : 0;
+            h[threadIdx.x] > 0
+                ? before + atomicAdd(counts + 2 * kColClasses + threadIdx.x, h[threadIdx.x])
+                : 0;
         h[threadIdx.x] = 0;
     }
     __syncthreads();

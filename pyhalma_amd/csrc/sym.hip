@@ -10,8 +10,8 @@
 //   - test side: per test an FP32 sum of the eight terms, added in FP64 over the segment,
 //     the segments' sums in FP64 in order;
 //   - source side: per source two FP32 chains over a lane's tests 0-3 and 4-7, their sum
-//     through a fixed tree over the lanes (reduce8, its last levels in FP64).  The lanes hold every test of the
-//     item, so the total goes straight to the member's slot.
+//     through a fixed tree over the lanes (reduce8, its last three levels in FP64).  The lanes
+//     hold every test of the item, so the total goes straight to the member's slot.
 // In a diagonal item (A == B) a source of strip s meets the strips t < s on both sides and
 // strip s on the test side alone (all its ordered pairs); the strips above it are another
 // source's.  Every member then has partial sums in nb + 1 slots (nb = blocks of its halo),

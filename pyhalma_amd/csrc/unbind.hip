@@ -38,8 +38,8 @@
 //   5. k_finish      per-halo pass counts, convergence flags, the removed total (a thread
 //                    per halo);
 //   6. k_halo_tail   the passes that follow, a workgroup per halo (a wavefront for a small
-//                    one), where none of the active haloes is large and until a halo's next pass is too much for a
-//                    workgroup.
+//                    one), where none of the active haloes is large and until a halo's next
+//                    pass is too much for a workgroup.
 // The parts are plain launches (or, on request, hipGraphs captured once and replayed);
 // the host reads one counter per pass to stop.
 #include <math.h>
@@ -143,8 +143,8 @@ __device__ __forceinline__ bool pass_is_full(int pass_no, int run, int rrun, int
 // is stale.  Its decision is exact (it lies outside the decision band), so it only needs
 // a fresh S: when its halo has few stale members (at most 1/kStaleDiv of the live set)
 // the re-test kernel re-sums them, FP32 terms added in FP64 (bound 6u = 3.6e-7);
-// otherwise the halo's next pass is a full one (the symmetric kernel recomputes every S), and a halo
-// that removed nobody takes that full pass only to refresh its S (not counted as an
+// otherwise the halo's next pass is a full one (the symmetric kernel recomputes every S), and
+// a halo that removed nobody takes that full pass only to refresh its S (not counted as an
 // iteration: its decisions are exact and do not change).  Both full-pass kernels stay
 // below the limit (halma_pot_error_bound at sub-tiles of 4 or 8, halma_pot_sym_error_bound).
 constexpr double kPotRelMax = 1e-6;
