@@ -39,26 +39,27 @@ def _cols(p):
 _src_cache = {}
 
 
+def _key(t):
+    t = t.detach()
+    return (t.device, t.data_ptr(), tuple(t.shape), t.stride(), t.dtype, t._version,
+            torch.cuda.current_stream().cuda_stream if t.is_cuda else 0)
+
+
 def _src_cols(src_pos):
     """FP32 columns of the source positions, kept for the next call on the same unchanged
-    tensor (an iteration over soft_potential passes one source array to every forward and
-    backward).
-    The key holds the storage address, shape, strides, dtype and the version counter
-    (bumped by every in-place change); the entry holds the tensor itself, so its storage
-    cannot be freed and reused under the same address while it is cached."""
+    tensor and stream (an iteration over soft_potential passes one source array to every
+    forward and backward).  The key holds the storage address, shape, strides, dtype, the
+    version counter (bumped by every in-place change) and the stream, whose work the columns
+    are ordered with; the entry holds the tensor itself, so its storage cannot be freed and
+    reused under the same address while it is cached."""
     p = src_pos.detach()
-    key = (p.device, p.data_ptr(), tuple(p.shape), p.stride(), p.dtype, p._version)
+    key = _key(p)
     hit = _src_cache.get("src")
     if hit is not None and hit[0] == key:
         return hit[2]
     cols = _cols(p.float())
     _src_cache["src"] = (key, p, cols)
     return cols
-
-
-def _key(t):
-    t = t.detach()
-    return (t.device, t.data_ptr(), tuple(t.shape), t.stride(), t.dtype, t._version)
 
 
 def _src_packed(src_pos, src_m):

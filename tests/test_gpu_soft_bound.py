@@ -35,3 +35,27 @@ def test_soft_sums_within_their_bounds(gpu, tests, n):
     assert bool(((r["pot"] - S).abs() <= 2.0 ** -20 * S).all())
     assert bool(((r["acc"] - a).abs() <= 2.0 ** -19 * mag).all())
     assert bool(((r["wsum"] - w3.sum(1)).abs() <= 2.0 ** -19 * w3.sum(1)).all())
+
+
+def test_kept_sources_stay_on_their_stream(gpu):
+    """The packed sources that soft_potential keeps are ordered with the stream that packed
+    them: another stream packs its own, the same one finds them."""
+    import torch
+
+    from pyhalma_amd import centring
+
+    centring.clear_cache()
+    pos, m = torch.rand(1000, 3, device="cuda"), torch.rand(1000, device="cuda")
+    print("streams", flush=True)
+    a = centring._src_packed(pos, m)
+    assert centring._src_packed(pos, m) is a
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        b = centring._src_packed(pos, m)
+        cols = centring._src_cols(pos)
+        assert b is not a and centring._src_packed(pos, m) is b
+    assert centring._src_cols(pos)[0] is not cols[0]
+    torch.cuda.synchronize()
+    assert torch.equal(a, b)
+    centring.clear_cache()
